@@ -147,6 +147,41 @@ def run(st):
     return w, ids, sorted_ids, expert_ids[: ids.numel() // st["block"]], npost
 
 
+def _quantised(x):
+    """Rows as e4m3 holds them (scale = largest magnitude / 448, in 32 bits), back in 64 bits."""
+    scale = x.abs().amax(dim=1, keepdim=True).float() / 448.0
+    scale = torch.where(scale > 0, scale, torch.ones_like(scale))
+    return (x.float() / scale).to(torch.float8_e4m3fn).double() * scale.double()
+
+
+def exact(case, seed):
+    """run()'s floating outputs in 64 bits with plain torch, from the same inputs."""
+    st, topk = prepare({**case, "prepared": False}, seed), SHAPES[case["shape"]]["topk"]
+    logits = (st["x"].double() @ st["gate"].double()) if case["kind"] == "gate" else st["logits"].double()
+    top, ids = torch.sort(logits, dim=1, descending=True, stable=True)
+    top, ids = top[:, :topk], ids[:, :topk]
+    if case["kind"] == "route":
+        return torch.softmax(top, dim=1), None, None, None, None
+    weights, fp8 = torch.softmax(top, dim=1), case["kind"] == "fp8"
+    x = _quantised(st["x"].double()) if fp8 else st["x"].double()
+    out = torch.zeros_like(x)
+    for e in range(st["E"]):
+        token, slot = (ids == e).nonzero(as_tuple=True)
+        if token.numel() == 0:
+            continue
+        if fp8:
+            w1 = st["w1q"][e].view(torch.float8_e4m3fn).double() * st["w1s"][e].double()[:, None]
+            w2 = st["w2q"][e].view(torch.float8_e4m3fn).double() * st["w2s"][e].double()[:, None]
+        else:
+            w1, w2 = st["w1"][e].double(), st["w2"][e].double()
+        gate, up = (x[token] @ w1.t()).chunk(2, dim=1)
+        act = torch.nn.functional.silu(gate) * up
+        if fp8:  # the path's own formats: activated rows in bf16, quantised per row
+            act = _quantised(act.bfloat16().double())
+        out.index_add_(0, token, (act @ w2.t()) * weights[token, slot][:, None])
+    return out
+
+
 def _active_experts(M, E, topk, zipf):
     """Experts that a batch of M tokens hits, from one sample of the case's logits."""
     gen = torch.Generator(device="cpu").manual_seed(1)
