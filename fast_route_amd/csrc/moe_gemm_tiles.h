@@ -14,8 +14,8 @@ namespace fr {
 //                   in the 256-row tile one wavefront per SIMD issues the loads of both;
 //   64 rows:        3-slot ring, 8 wavefronts (4 with 256-byte row segments for the gate/up GEMM, persistent);
 //                   (the register-staged double buffer of STAGES == 0 is no longer used by any tile);
-//   32 / 16 rows:   decode regime, 16x16 MFMA, 3-slot ring, two workgroups per CU:
-//                   weight streaming at HBM rate.  The gate/up GEMM (short weight rows
+//   32 / 16 rows:   decode regime, 16x16 MFMA, 3-slot ring, two workgroups per CU (the 16-row tile
+//                   persistent or plain, see dispatch_block): weight streaming at HBM rate.  The gate/up GEMM (short weight rows
 //                   of H elements, many of them) streams faster with 512-byte row
 //                   segments: T32L / T16L, used when H allows.
 template <typename T> struct Tiles {  // bf16 / fp16
@@ -131,11 +131,29 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       fill(32, TL::T32::BF, TL::T32::BKB);
       return launch_gemm<T, typename TL::T32, EPI>(a, splits, st);
     case 16:
-      if (EPI == EPI_SILU && a.K % (TL::T16L::BKB / static_cast<int>(sizeof(T))) == 0) {
-        fill(16, TL::T16L::BF, TL::T16L::BKB);
-        return launch_gemm<T, typename TL::T16L, EPI>(a, splits, st);
+      // Plain or persistent.  A plain launch has two workgroups per CU that come and go: every tile pays its start-up
+      // (block table -> sorted ids -> first K tiles) and its drain, and rounds of tiles do not overlap.  The persistent
+      // form refills the ring across tiles, which pays where a tile's K loop is short or there are several rounds.
+      if constexpr (EPI == EPI_SILU) {
+        // Rows of up to 4 KB (16 K tiles of 256 bytes): persistent.  Plain 512-byte / persistent 256-byte segments,
+        // layer: H = 2048, F = 1408, 64 experts, top-6, 32 / 48 / 128 tokens 93 / 131 / 191 against 88 / 126 / 177 us;
+        // H = 1024, F = 3584, 8 experts, 16 / 128 tokens 47.3 / 77 against 46.0 / 63; fp8, H = 4096, F = 14336, 24 tokens
+        // 239 against 233.  Longer rows stream faster in 512-byte pieces (bf16, H = 4096: 428 against 445 us).
+        if (a.K * static_cast<int>(sizeof(T)) <= 4096) {
+          fill(16, TL::T16::BF, TL::T16::BKB);
+          return launch_gemm_persistent<T, typename TL::T16, EPI>(a, splits, st);
+        }
+        if (a.K % (TL::T16L::BKB / static_cast<int>(sizeof(T))) == 0) {
+          fill(16, TL::T16L::BF, TL::T16L::BKB);
+          return launch_gemm<T, typename TL::T16L, EPI>(a, splits, st);
+        }
       }
       fill(16, TL::T16::BF, TL::T16::BKB);
+      // The layer's down projection from 8 KB of K per slice on (32 K tiles): persistent.  H = 4096, F = 8192, 16 experts,
+      // 24 / 64 tokens 498 / 554 us plain, 490 / 525 persistent (two rounds of tiles); one round (8 experts, F = 14336)
+      // 428 either way; 2.8 KB (F = 1408) loses 1 %.
+      if (EPI != EPI_SILU && a.long_k && a.k_per_split * static_cast<int>(sizeof(T)) >= 8192)
+        return launch_gemm_persistent<T, typename TL::T16, EPI>(a, splits, st);
       return launch_gemm<T, typename TL::T16, EPI>(a, splits, st);
     default: return fail(FR_E_SHAPE, "routing block %d not in {16, 32, 64, 128, 160, 256}", block);
   }
@@ -158,7 +176,7 @@ int prepare_tiles() {
   if (rc == FR_OK) rc = launch_gemm<T, typename TL::T128, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm<T, typename TL::T64, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32, EPI>(a, 1, nullptr);
-  if (rc == FR_OK) rc = launch_gemm<T, typename TL::T16, EPI>(a, 1, nullptr);
+  if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T16, EPI>(a, 1, nullptr);  // and its plain form
   if constexpr (EPI == EPI_SILU) {
     if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64U, EPI>(a, 1, nullptr);
     if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32L, EPI>(a, 1, nullptr);
