@@ -85,8 +85,23 @@ constexpr int kChunkBlocks = 8;    // token blocks per chunk, at most (measured 
 // off[e] = first token block of expert e among the nt real blocks, off[E] = nt; off[kMaxExperts + 1] = 1
 // if expert_ids does not ascend (routing arrays of another producer, legal for the op-level GEMM): then
 // every tile takes the plain row-major walk, since the table describes no partition of the blocks.
+// One pass up to kOnePassExperts experts: thread b compares blocks b - 1 and b and fills the entries that start at b, one
+// load latency where a binary search per expert is a chain of log2(nt) of them (and another pass for the order) in front
+// of the first tile of every launch.  With more experts one thread might have to fill a thousand entries: the search.
+constexpr int kOnePassExperts = 256;
 __device__ __forceinline__ void expert_block_offsets(const GemmArgs& a, int nt, int* off, int tid, int nthreads) {
   if (tid == 0) off[kMaxExperts + 1] = 0;
+  if (a.num_experts <= kOnePassExperts) {
+    __syncthreads();
+    for (int b = tid; b <= nt; b += nthreads) {
+      const int prev = b > 0 ? a.expert_ids[b - 1] : -1, cur = b < nt ? a.expert_ids[b] : a.num_experts;
+      if (b > 0 && b < nt && cur < prev) off[kMaxExperts + 1] = 1;
+      const int last = min(cur, a.num_experts);
+      for (int e = max(prev + 1, 0); e <= last; ++e) off[e] = b;
+    }
+    __syncthreads();
+    return;
+  }
   for (int e = tid; e <= a.num_experts; e += nthreads) {
     int lo = 0, hi = nt;
     while (lo < hi) {
