@@ -617,50 +617,74 @@ __global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int n
   const float* first = a.tail_ws + static_cast<int64_t>(xcd * nper + t) * (BT * BF);
   const int64_t slice_stride = static_cast<int64_t>(xs.rest) * (BT * BF);
   const int cg = threadIdx.x % CG;
+  // Memory bound (every slice read once): the rows of a thread are taken together, slice by slice, so that all their loads
+  // are in flight at once.  A padding row's address is that of the tile's first row (one line for all of them).
+  constexpr int P = kFixupRows / RPP;  // rows per thread
+  const int row0 = rb * kFixupRows + threadIdx.x / CG;
+  if constexpr (EPI != EPI_SILU) {
+    int sid[P];
+    const float* src[P];
+    f32x4 sum[P];
 #pragma unroll
-  for (int p = 0; p < kFixupRows / RPP; ++p) {
-    const int row = rb * kFixupRows + p * RPP + threadIdx.x / CG;
-    const int slot = pid_t * BT + row;
-    const float* src = first + row * BF + cg * 4;
-    if constexpr (EPI != EPI_SILU) {
-      const int sid = a.sorted[slot];
-      if (sid >= a.num_valid) continue;
-      f32x4 sum = *reinterpret_cast<const f32x4*>(src);
-      for (int s = 1; s < xs.slices; ++s) sum += *reinterpret_cast<const f32x4*>(src + s * slice_stride);
-      float rw = a.mul_weight ? a.topk_w[sid] : 1.f;
+    for (int p = 0; p < P; ++p) sid[p] = a.sorted[pid_t * BT + row0 + p * RPP];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      src[p] = first + (sid[p] < a.num_valid ? (row0 + p * RPP) * BF : 0) + cg * 4;
+      sum[p] = *reinterpret_cast<const f32x4*>(src[p]);
+    }
+    for (int s = 1; s < xs.slices; ++s)
+#pragma unroll
+      for (int p = 0; p < P; ++p) sum[p] += *reinterpret_cast<const f32x4*>(src[p] + s * slice_stride);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      if (sid[p] >= a.num_valid) continue;
+      float rw = a.mul_weight ? a.topk_w[sid[p]] : 1.f;
       if constexpr (E::SCALED) {  // per-row scales of both fp8 operands
-        rw *= a.top_k > 0 ? a.x_scale[sid / a.top_k] : a.x_scale[slot];
+        rw *= a.top_k > 0 ? a.x_scale[sid[p] / a.top_k] : a.x_scale[pid_t * BT + row0 + p * RPP];
         const f32x4 ws = *reinterpret_cast<const f32x4*>(wsc + pid_f * BF + cg * 4);
-        sum *= ws;
+        sum[p] *= ws;
       }
-      const int64_t at = static_cast<int64_t>(sid) * a.ldo + pid_f * BF + cg * 4;
+      const int64_t at = static_cast<int64_t>(sid[p]) * a.ldo + pid_f * BF + cg * 4;
       if constexpr (EPI == EPI_DOWN) {
-        const f32x4 o = {sum[0] * rw, sum[1] * rw, sum[2] * rw, sum[3] * rw};
+        const f32x4 o = {sum[p][0] * rw, sum[p][1] * rw, sum[p][2] * rw, sum[p][3] * rw};
         *reinterpret_cast<f32x4*>(static_cast<float*>(a.out) + at) = o;
       } else {
         out4 o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = static_cast<out_t>(sum[r] * rw);
-        if (a.add_div) atomic_add4(static_cast<out_t*>(a.out) + static_cast<int64_t>(sid / a.add_div) * a.ldo + pid_f * BF + cg * 4, o);
+        for (int r = 0; r < 4; ++r) o[r] = static_cast<out_t>(sum[p][r] * rw);
+        if (a.add_div) atomic_add4(static_cast<out_t*>(a.out) + static_cast<int64_t>(sid[p] / a.add_div) * a.ldo + pid_f * BF + cg * 4, o);
         else *reinterpret_cast<out4*>(static_cast<out_t*>(a.out) + at) = o;
       }
-    } else {
-      f32x4 g = *reinterpret_cast<const f32x4*>(src), u = *reinterpret_cast<const f32x4*>(src + BF / 2);
-      for (int s = 1; s < xs.slices; ++s) {
-        g += *reinterpret_cast<const f32x4*>(src + s * slice_stride);
-        u += *reinterpret_cast<const f32x4*>(src + s * slice_stride + BF / 2);
+    }
+  } else {
+    f32x4 g[P], u[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const float* src = first + (row0 + p * RPP) * BF + cg * 4;
+      g[p] = *reinterpret_cast<const f32x4*>(src);
+      u[p] = *reinterpret_cast<const f32x4*>(src + BF / 2);
+    }
+    for (int s = 1; s < xs.slices; ++s)
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const float* src = first + s * slice_stride + (row0 + p * RPP) * BF + cg * 4;
+        g[p] += *reinterpret_cast<const f32x4*>(src);
+        u[p] += *reinterpret_cast<const f32x4*>(src + BF / 2);
       }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int slot = pid_t * BT + row0 + p * RPP;
       if constexpr (E::SCALED) {
         const int sid = a.sorted[slot];
         const float xsc = a.top_k > 0 ? (sid < a.num_valid ? a.x_scale[sid / a.top_k] : 1.f) : a.x_scale[slot];
         const f32x4 gs = *reinterpret_cast<const f32x4*>(wsc + pid_f * (BF / 2) + cg * 4);
         const f32x4 us = *reinterpret_cast<const f32x4*>(wsc + a.N + pid_f * (BF / 2) + cg * 4);
-        g *= gs * xsc;
-        u *= us * xsc;
+        g[p] *= gs * xsc;
+        u[p] *= us * xsc;
       }
       out4 o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = static_cast<out_t>(silu(g[r]) * u[r]);
+      for (int r = 0; r < 4; ++r) o[r] = static_cast<out_t>(silu(g[p][r]) * u[p][r]);
       out_t* orow = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot) * a.ldo + pid_f * (BF / 2) + cg * 4;
       *reinterpret_cast<out4*>(orow) = o;
     }
