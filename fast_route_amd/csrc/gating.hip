@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kGateThreads) void gating_topk_blocked_kernel(
   for (int64_t it = 0; it < rounds; ++it, token += stride) {
     const bool live = token < M;
     const T* row = logits + (live ? token : 0) * ld;
-    gate_token_blocked<G, NV>([&](int e0) { return load4_as_float(row + e0); }, live, E, topk, renorm,
+    gate_token_blocked<G, NV>([&](int e0) { return load4_as_float(row + e0); }, [&](int e) { return to_float(row[e]); }, live, E, topk, renorm,
                               w_out + token * topk, ids_out + token * topk);
   }
 }

@@ -206,14 +206,26 @@ __device__ __forceinline__ void gate_token(Load load, bool live, int E, int topk
 // instruction per step per token) shrink to log2(G) steps shared by 64/G tokens.  Inside a
 // lane expert indices rise with the slot number, across lanes ties go to the lower index,
 // so the order is still (value descending, index ascending).  load4(e0) returns logits
-// e0..e0+3; E must be a multiple of 4.
+// e0..e0+3, load1(e) logit e; E must be a multiple of 4.
+//
+// Bound by vector instructions (a lane looks at 4*NV logits in every round), so the selection runs on packed keys:
+// the upper bits of a logit's order key over the complement of its expert index, which no two experts of a token
+// share.  The largest key below the previous winner is the largest key minus the winner modulo 2^32 (keys above or
+// equal wrap to small values, those below to large ones, nearest first): a subtraction and half a three-way maximum
+// per logit and round where comparing exact keys and remembering the slot took five instructions.
+// The packed order is the exact one unless two logits differ only in the bits the index displaced; that shows as two
+// successive winners (one more than asked for is drawn) with equal upper bits while some logit of the token has a bit
+// set down there, and the wavefront then selects again on exact keys.  Logits that came from 16-bit values have no such
+// bits.  65536 tokens, 64 experts, top-6, fp32: 11.6 -> 7.8 us.
 constexpr int kBlockedSlots = 4;  // result slots per lane: topk <= kBlockedSlots * G
 
-template <int G, int NV, typename Load4>
-__device__ __forceinline__ void gate_token_blocked(Load4 load4, bool live, int E, int topk, int renorm,
+template <int G, int NV, typename Load4, typename Load1>
+__device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, bool live, int E, int topk, int renorm,
                                                    float* __restrict__ w_row, int32_t* __restrict__ id_row) {
   constexpr int VPL = 4 * NV;
   static_assert(G <= 16, "the all-reduce uses the in-row DPP steps only");
+  constexpr unsigned kIndexMask = G * VPL - 1;
+  static_assert((G * VPL & (G * VPL - 1)) == 0, "expert indices fill whole bits");
   const int g = threadIdx.x % G;
   float v[VPL];
 #pragma unroll
@@ -224,72 +236,110 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, bool live, int E
 #pragma unroll
     for (int c = 0; c < 4; ++c) v[4 * j + c] = t[c];
   }
-  float m = v[0];
-  float s = (v[0] == -INFINITY) ? 0.f : 1.f;
-#pragma unroll
-  for (int i = 1; i < VPL; ++i) {
-    if (v[i] == -INFINITY) continue;
-    const float mn = fmaxf(m, v[i]);
-    s = (m == -INFINITY ? 0.f : s * __expf(m - mn)) + __expf(v[i] - mn);
-    m = mn;
-  }
-  group_online_softmax<G>(m, s);
 
-  // Order keys of this lane's logits (0 = not a candidate).  Inside the lane a strict
-  // "greater" scan keeps the lowest slot, i.e. the lowest expert index, among equal keys.
-  unsigned k[VPL];
+  // Packed keys of this lane's logits (0 = not a candidate); + 0.f: -0 and +0 are the same value.
+  unsigned pk[VPL], low = 0u;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int e = 4 * (G * (i / 4) + g) + (i % 4);
-    k[i] = (e < E) ? float_key(v[i] + 0.f) : 0u;  // + 0.f: -0 and +0 are the same value
+    const float x = v[i] + 0.f;
+    if (live) low |= __float_as_uint(x);
+    pk[i] = (e < E) ? (float_key(x) & ~kIndexMask) | (kIndexMask - static_cast<unsigned>(e)) : 0u;
   }
-  float sel_v[kBlockedSlots];
   int sel_i[kBlockedSlots];
 #pragma unroll
-  for (int i = 0; i < kBlockedSlots; ++i) {
-    sel_v[i] = -INFINITY;
-    sel_i[i] = 0;
+  for (int i = 0; i < kBlockedSlots; ++i) sel_i[i] = 0;
+  unsigned win = 0u;  // previous winner; with 0 the first round's difference is the key itself
+  bool equal_upper = false;
+  int top = 0;        // expert of the largest logit
+  for (int r = 0; r <= topk; ++r) {
+    unsigned best = 0u;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) best = max(best, pk[i] - win);
+    if constexpr (G > 1) best = max(best, static_cast<unsigned>(partner_i32<1>(static_cast<int>(best))));
+    if constexpr (G > 2) best = max(best, static_cast<unsigned>(partner_i32<2>(static_cast<int>(best))));
+    if constexpr (G > 4) best = max(best, static_cast<unsigned>(partner_i32<4>(static_cast<int>(best))));
+    if constexpr (G > 8) best = max(best, static_cast<unsigned>(partner_i32<8>(static_cast<int>(best))));
+    const unsigned next = best + win;
+    if (r > 0) equal_upper |= ((next ^ win) & ~kIndexMask) == 0u;
+    win = next;
+    const int be = static_cast<int>(kIndexMask - (win & kIndexMask));
+    if (r == 0) top = be;
+    if (r < topk) {
+#pragma unroll
+      for (int sl = 0; sl < kBlockedSlots; ++sl)
+        if (r == sl * G + g) sel_i[sl] = be;
+    }
   }
-  int last = -1;  // slot this lane gave away in the previous round
-  float sel_sum = 0.f;
-  for (int r = 0; r < topk; ++r) {
-    unsigned bk = 0u;
-    int bs = 0;
+  const bool has_low = (low & kIndexMask) != 0u;
+  if (__any(equal_upper) && __any(has_low)) {
+    // exact keys; inside the lane a strict "greater" scan keeps the lowest slot, i.e. the lowest expert index, among equal keys
+    unsigned k[VPL];
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      if (i == last) k[i] = 0u;
-      if (k[i] > bk) {
-        bk = k[i];
-        bs = i;
-      }
+      const int e = 4 * (G * (i / 4) + g) + (i % 4);
+      k[i] = (e < E) ? float_key(v[i] + 0.f) : 0u;
     }
-    int be = 4 * (G * (bs >> 2) + g) + (bs & 3);
-    // all-reduce over the group: larger key wins, equal keys go to the lower expert index
-    auto step = [&](auto tag) {
-      constexpr int S = decltype(tag)::value;
-      const unsigned ok = static_cast<unsigned>(partner_i32<S>(static_cast<int>(bk)));
-      const int oe = partner_i32<S>(be);
-      if (ok > bk || (ok == bk && oe < be)) {
-        bk = ok;
-        be = oe;
-      }
-    };
-    if constexpr (G > 1) step(std::integral_constant<int, 1>{});
-    if constexpr (G > 2) step(std::integral_constant<int, 2>{});
-    if constexpr (G > 4) step(std::integral_constant<int, 4>{});
-    if constexpr (G > 8) step(std::integral_constant<int, 8>{});
-    last = ((be >> 2) % G == g) ? (4 * (be / (4 * G)) + (be & 3)) : -1;
-    const float bv = key_float(bk);
-    sel_sum += __expf(bv - m);
+    int last = -1;  // slot this lane gave away in the previous round
+    for (int r = 0; r < topk; ++r) {
+      unsigned bk = 0u;
+      int bs = 0;
 #pragma unroll
-    for (int sl = 0; sl < kBlockedSlots; ++sl) {
-      if (r == sl * G + g) {
-        sel_v[sl] = bv;
-        sel_i[sl] = be;
+      for (int i = 0; i < VPL; ++i) {
+        if (i == last) k[i] = 0u;
+        if (k[i] > bk) {
+          bk = k[i];
+          bs = i;
+        }
       }
+      int be = 4 * (G * (bs >> 2) + g) + (bs & 3);
+      // all-reduce over the group: larger key wins, equal keys go to the lower expert index
+      auto step = [&](auto tag) {
+        constexpr int S = decltype(tag)::value;
+        const unsigned ok = static_cast<unsigned>(partner_i32<S>(static_cast<int>(bk)));
+        const int oe = partner_i32<S>(be);
+        if (ok > bk || (ok == bk && oe < be)) {
+          bk = ok;
+          be = oe;
+        }
+      };
+      if constexpr (G > 1) step(std::integral_constant<int, 1>{});
+      if constexpr (G > 2) step(std::integral_constant<int, 2>{});
+      if constexpr (G > 4) step(std::integral_constant<int, 4>{});
+      if constexpr (G > 8) step(std::integral_constant<int, 8>{});
+      last = ((be >> 2) % G == g) ? (4 * (be / (4 * G)) + (be & 3)) : -1;
+      if (r == 0) top = be;
+#pragma unroll
+      for (int sl = 0; sl < kBlockedSlots; ++sl)
+        if (r == sl * G + g) sel_i[sl] = be;
     }
   }
-  const float denom = renorm ? sel_sum : s;
+
+  // The winners' logits again from the cache the row was just read through: they are spread over the lanes' registers.
+  // top-1 first: with renormalised weights it is all the softmax statistics there are.
+  float sel_v[kBlockedSlots];
+#pragma unroll
+  for (int sl = 0; sl < kBlockedSlots; ++sl) sel_v[sl] = (live && sl * G + g < topk) ? load1(sel_i[sl]) + 0.f : -INFINITY;
+  float m = live ? load1(top) + 0.f : 0.f;
+  float denom;
+  if (renorm) {
+    denom = 0.f;
+#pragma unroll
+    for (int sl = 0; sl < kBlockedSlots; ++sl)
+      if (sl * G < topk) denom += group_sum<G>((live && sl * G + g < topk) ? __expf(sel_v[sl] - m) : 0.f);
+  } else {
+    m = v[0];
+    float s = (v[0] == -INFINITY) ? 0.f : 1.f;
+#pragma unroll
+    for (int i = 1; i < VPL; ++i) {
+      if (v[i] == -INFINITY) continue;
+      const float mn = fmaxf(m, v[i]);
+      s = (m == -INFINITY ? 0.f : s * __expf(m - mn)) + __expf(v[i] - mn);
+      m = mn;
+    }
+    group_online_softmax<G>(m, s);
+    denom = s;
+  }
   if (live) {
 #pragma unroll
     for (int sl = 0; sl < kBlockedSlots; ++sl) {

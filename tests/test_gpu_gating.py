@@ -84,6 +84,25 @@ def test_gating_ties_many_experts(native, E, topk):
     assert torch.equal(ids2, oracle.gating_topk(logits, topk, True)[1])
 
 
+@pytest.mark.parametrize("E,topk", [(20, 3), (32, 16), (64, 6), (64, 15), (128, 8), (256, 32)])
+def test_gating_near_ties_many_experts(native, E, topk):
+    """fp32 logits a few units in the last place apart: the few-lanes-per-token form packs the expert index into the low
+    bits of its keys and has to notice that such neighbours need the exact ones.  Rows of clear-cut logits share the
+    wavefronts; masked experts (-inf) tie among themselves."""
+    _say(f"gating near ties E={E} topk={topk}")
+    g = torch.Generator().manual_seed(E * 17 + topk)
+    for sign in (1.0, -1.0):
+        logits = sign * (1.0 + torch.randint(0, 70, (1300, E), generator=g).float() * 2.0 ** -23)
+        logits[::3] = torch.randn(logits[::3].shape, generator=g)
+        logits[1::7] = logits[1::7] * (1 + 2.0 ** -20 * torch.randn(logits[1::7].shape, generator=g))
+        logits[2::5, topk:] = float("-inf")
+        for renorm in (True, False):
+            w, ids = _run_gating(logits.cuda(), topk, renorm)
+            rw, rid = oracle.gating_topk(logits, topk, renorm)
+            assert torch.equal(ids, rid)
+            torch.testing.assert_close(w, rw, atol=W_ATOL, rtol=0)
+
+
 def test_gating_reference_route_test_recipe(native):
     """tests/test_route.py:12-77 of the reference: weights vs topk(softmax(h@gate)), atol 1e-2."""
     for seed in range(3):
