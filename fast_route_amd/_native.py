@@ -5,6 +5,8 @@ import ctypes
 import os
 from ctypes import c_char_p, c_int, c_int32, c_int64, c_void_p
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 # FR_NATIVE_LIB: another build of the library (a measurement build, see build.py); bench.py records which one ran
 LIB_PATH = os.environ.get("FR_NATIVE_LIB") or os.path.join(HERE, "libfast_route_hip.so")
@@ -90,18 +92,21 @@ def check(rc: int) -> None:
     raise RuntimeError("fast_route_amd native error %d: %s" % (rc, msg))
 
 
+_DTYPE_CODES = {torch.float16: FR_F16, torch.bfloat16: FR_BF16, torch.float32: FR_F32,
+                torch.int32: FR_I32, torch.int64: FR_I64}
+
+
 def dtype_code(dt) -> int:
-    import torch
-    table = {torch.float16: FR_F16, torch.bfloat16: FR_BF16, torch.float32: FR_F32,
-             torch.int32: FR_I32, torch.int64: FR_I64}
-    if dt not in table:
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
         raise AssertionError("unsupported dtype %s" % dt)
-    return table[dt]
+    return code
 
 
 def stream_ptr(device) -> int:
-    import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    """Handle of the current stream of a tensor's device, without the Stream object around it."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_cuda(*tensors) -> None:

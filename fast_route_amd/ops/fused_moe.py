@@ -28,10 +28,10 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     lib = N.lib()
     ws_bytes = lib.fr_moe_align_workspace_bytes(n, num_experts)
     assert ws_bytes >= 0, "num_experts=%d outside [1, 1024]" % num_experts
-    ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev) if ws_bytes else None  # small inputs sort in LDS
     N.check(lib.fr_moe_align(topk_ids.data_ptr(), N.dtype_code(topk_ids.dtype), n, num_experts, block_size,
                              sorted_ids.data_ptr(), expert_ids.data_ptr(), num_tokens_post_pad.data_ptr(),
-                             ws.data_ptr(), ws_bytes, N.stream_ptr(dev)))
+                             ws.data_ptr() if ws_bytes else 0, ws_bytes, N.stream_ptr(dev)))
     return sorted_ids, expert_ids, num_tokens_post_pad
 
 
