@@ -80,6 +80,16 @@ __device__ __forceinline__ void segment_ids(const IdT* __restrict__ ids, int64_t
     ev[r] = (p < hi) ? static_cast<int>(ids[p]) : -1;
   }
 }
+// Histogram of [lo, hi); `first` holds the ids of its first kScatterPF rounds (segment_ids), -1 behind hi: they are asked
+// for together instead of each round waiting for its own.
+template <typename IdT>
+__device__ __forceinline__ void segment_histogram(const IdT* __restrict__ ids, int64_t lo, int64_t hi,
+                                                  int E, int lane, int* hist, const int (&first)[kScatterPF]) {
+#pragma unroll
+  for (int r = 0; r < kScatterPF; ++r)
+    if (first[r] >= 0 && first[r] < E) atomicAdd(&hist[first[r]], 1);
+  segment_histogram(ids, lo + kScatterPF * kWave, hi, E, lane, hist);
+}
 // `first`: the ids of the first kScatterPF rounds, fetched by the caller ahead of time (segment_ids), or nullptr
 template <typename IdT>
 __device__ __forceinline__ void segment_scatter(const IdT* __restrict__ ids, int64_t lo, int64_t hi,
@@ -155,6 +165,23 @@ __device__ __forceinline__ void write_block_table(const int* total, const int* s
 }
 
 // ---------------------------------------------------------------- small path
+// table[w][e]: pairs of expert e in segment w -> in the segments before w; total[e]: in all.  The counts are read before
+// any of them is overwritten: the reads then do not wait for one another (16 LDS latencies, about a microsecond).
+__device__ __forceinline__ void scan_segments(int* table, int* total, int E, int tid) {
+  for (int e = tid; e < E; e += kSmallThreads) {
+    int c[kSmallWaves];
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) c[w] = table[w * E + e];
+    int running = 0;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) {
+      table[w * E + e] = running;
+      running += c[w];
+    }
+    total[e] = running;
+  }
+}
+
 template <typename IdT>
 __global__ __launch_bounds__(kSmallThreads) void align_small_kernel(
     const IdT* __restrict__ ids, int64_t n, int E, int B, int seg_len, int64_t sorted_len,
@@ -163,28 +190,22 @@ __global__ __launch_bounds__(kSmallThreads) void align_small_kernel(
   __shared__ int total[kSmallMaxE];
   __shared__ int start[kSmallMaxE + 1];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] = 0;
-  __syncthreads();
   const int64_t lo = min64(n, static_cast<int64_t>(wave) * seg_len);
   const int64_t hi = min64(n, lo + seg_len);
-  segment_histogram(ids, lo, hi, E, lane, &table[wave * E]);
+  int first[kScatterPF];  // read once for the histogram and the placement
+  segment_ids(ids, lo, hi, lane, first);
+  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] = 0;
   __syncthreads();
-  for (int e = tid; e < E; e += kSmallThreads) {
-    int running = 0;
-    for (int w = 0; w < kSmallWaves; ++w) {
-      const int c = table[w * E + e];
-      table[w * E + e] = running;
-      running += c;
-    }
-    total[e] = running;
-  }
+  segment_histogram(ids, lo, hi, E, lane, &table[wave * E], first);
+  __syncthreads();
+  scan_segments(table, total, E, tid);
   __syncthreads();
   if (wave == 0) scan_padded_totals(total, start, E, B, lane);
   __syncthreads();
   for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] += start[i % E];
   write_block_table(total, start, E, B, n, sorted_len, tid, kSmallThreads, sorted, expert_ids, npost_out);
   __syncthreads();
-  segment_scatter(ids, lo, hi, E, bits_for(E), lane, &table[wave * E], sorted);
+  segment_scatter(ids, lo, hi, E, bits_for(E), lane, &table[wave * E], sorted, first);
 }
 
 // bf16 token rows [M, K] to quantise to e4m3 alongside (x == nullptr: none)
@@ -206,6 +227,7 @@ __global__ __launch_bounds__(kSmallThreads) void route_align_small_kernel(
   __shared__ int table[kSmallWaves * kSmallMaxE];
   __shared__ int total[kSmallMaxE];
   __shared__ int start[kSmallMaxE + 1];
+  __shared__ int32_t pair_id[kRouteAlignMaxN];  // the ids stay here for the sort: no way out to memory and back
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   if (blockIdx.x > 0) {  // the fp8 layer's token rows are quantised by further workgroups of the same launch
     const int64_t row = static_cast<int64_t>(blockIdx.x - 1) * kSmallWaves + wave;
@@ -219,31 +241,25 @@ __global__ __launch_bounds__(kSmallThreads) void route_align_small_kernel(
     const bool live = token < M;
     const T* row = logits + (live ? token : 0) * E;
     gate_token<G, VPL>([&](int e) { return to_float(row[e]); }, live, E, topk, renorm, w_out + token * topk,
-                       ids_out + token * topk);
+                       pair_id + static_cast<int>(live ? token : 0) * topk);
   }
-  __threadfence_block();
-  __syncthreads();  // the ids written above are read back below by other lanes of this workgroup
+  __syncthreads();
   const int64_t n = M * topk;
   const int64_t lo = min64(n, static_cast<int64_t>(wave) * seg_len);
   const int64_t hi = min64(n, lo + seg_len);
-  segment_histogram(ids_out, lo, hi, E, lane, &table[wave * E]);
+  int first[kScatterPF];
+  segment_ids(pair_id, lo, hi, lane, first);
+  segment_histogram(pair_id, lo, hi, E, lane, &table[wave * E], first);
+  for (int i = tid; i < n; i += kSmallThreads) ids_out[i] = pair_id[i];
   __syncthreads();
-  for (int e = tid; e < E; e += kSmallThreads) {
-    int running = 0;
-    for (int w = 0; w < kSmallWaves; ++w) {
-      const int c = table[w * E + e];
-      table[w * E + e] = running;
-      running += c;
-    }
-    total[e] = running;
-  }
+  scan_segments(table, total, E, tid);
   __syncthreads();
   if (wave == 0) scan_padded_totals(total, start, E, B, lane);
   __syncthreads();
   for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] += start[i % E];
   write_block_table(total, start, E, B, n, sorted_len, tid, kSmallThreads, sorted, expert_ids, npost_out);
   __syncthreads();
-  segment_scatter(ids_out, lo, hi, E, bits_for(E), lane, &table[wave * E], sorted);
+  segment_scatter(pair_id, lo, hi, E, bits_for(E), lane, &table[wave * E], sorted, first);
 }
 
 // ---------------------------------------------------------------- large path
@@ -345,13 +361,13 @@ __global__ __launch_bounds__(kSeg2Threads) void align_count2_kernel(
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int seg0 = blockIdx.x * kSeg2Waves, seg = seg0 + wave;
   int* mine = hist + wave * E;
+  const int64_t lo = min64(n, static_cast<int64_t>(seg) * seg_len);
+  const int64_t hi = seg < S ? min64(n, lo + seg_len) : lo;
+  int first[kScatterPF];
+  segment_ids(ids, lo, hi, lane, first);
   for (int e = lane; e < E; e += kWave) mine[e] = 0;
   __builtin_amdgcn_wave_barrier();
-  if (seg < S) {
-    const int64_t lo = static_cast<int64_t>(seg) * seg_len;
-    const int64_t hi = min64(n, lo + seg_len);
-    segment_histogram(ids, lo, hi, E, lane, mine);
-  }
+  segment_histogram(ids, lo, hi, E, lane, mine, first);
   __syncthreads();
   for (int i = tid; i < E * kSeg2Waves; i += kSeg2Threads) {  // (expert, segment of this workgroup)
     const int e = i % E, w = i / E;
@@ -383,13 +399,25 @@ __global__ __launch_bounds__(kSeg2Threads) void align_scatter2_kernel(
   const int in_wg0 = (seg < S && lane < E) ? counts[static_cast<int64_t>(lane) * S + seg] : 0;
   for (int e = tid; e < E; e += kSeg2Threads) total[e] = before[e] = 0;
   __syncthreads();
-  for (int i = tid; i < E * NB; i += kSeg2Threads) {  // expert e: all pairs, and the pairs in the workgroups before this one
-    const int b = i / E, e = i % E;
-    const int c = wgcnt[i];
+  // expert e: all pairs, and the pairs in the workgroups before this one.  A thread keeps one expert and sums every
+  // (1024 / E)-th workgroup in registers: independent loads, two LDS atomics at the end.  E <= 512 (the launcher).
+  const int per_pass = kSeg2Threads / E, my_e = tid % E, b0 = tid / E;
+  if (E * NB <= kSeg2Threads) {
+    const int c = tid < E * NB ? wgcnt[tid] : 0;
     if (c != 0) {
-      atomicAdd(&total[e], c);
-      if (b < wg) atomicAdd(&before[e], c);
+      atomicAdd(&total[my_e], c);
+      if (b0 < wg) atomicAdd(&before[my_e], c);
     }
+  } else if (b0 < per_pass) {
+    int all = 0, below = 0;
+#pragma unroll 4
+    for (int b = b0; b < NB; b += per_pass) {
+      const int c = wgcnt[static_cast<int64_t>(b) * E + my_e];
+      all += c;
+      below += b < wg ? c : 0;
+    }
+    if (all != 0) atomicAdd(&total[my_e], all);
+    if (below != 0) atomicAdd(&before[my_e], below);
   }
   __syncthreads();
   if (wave == 0) scan_padded_totals(total, start, E, B, lane);
