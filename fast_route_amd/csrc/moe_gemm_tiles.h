@@ -135,11 +135,13 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       // (block table -> sorted ids -> first K tiles) and its drain, and rounds of tiles do not overlap.  The persistent
       // form refills the ring across tiles, which pays where a tile's K loop is short or there are several rounds.
       if constexpr (EPI == EPI_SILU) {
-        // Rows of up to 4 KB (16 K tiles of 256 bytes): persistent.  Plain 512-byte / persistent 256-byte segments,
-        // layer: H = 2048, F = 1408, 64 experts, top-6, 32 / 48 / 128 tokens 93 / 131 / 191 against 88 / 126 / 177 us;
-        // H = 1024, F = 3584, 8 experts, 16 / 128 tokens 47.3 / 77 against 46.0 / 63; fp8, H = 4096, F = 14336, 24 tokens
-        // 239 against 233.  Longer rows stream faster in 512-byte pieces (bf16, H = 4096: 428 against 445 us).
-        if (a.K * static_cast<int>(sizeof(T)) <= 4096) {
+        // Rows of up to 2 KB (8 K tiles of 256 bytes; fp8: up to 4 KB): persistent.  Plain 512-byte / persistent 256-byte
+        // segments, layer, on weights that no cache holds (several layers' in turn): H = 1024, F = 3584, 8 experts,
+        // 16 / 128 tokens 49.2 / 78.7 against 47.2 / 68.8 us; fp8, H = 4096, F = 14336, 16 tokens 245.9 against 243.1.
+        // H = 2048, F = 1408, 64 experts, top-6, 32 tokens: 108 / 111 against 116 / 113 (on the previous pass's weights it
+        // is the other way round, 102 against 98: part of them is still in the Infinity Cache).  Longer rows stream
+        // faster in 512-byte pieces (bf16, H = 4096: 428 against 445 us).
+        if (a.K * static_cast<int>(sizeof(T)) <= (sizeof(T) == 1 ? 4096 : 2048)) {
           fill(16, TL::T16::BF, TL::T16::BKB);
           return launch_gemm_persistent<T, typename TL::T16, EPI>(a, splits, st);
         }
