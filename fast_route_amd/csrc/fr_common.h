@@ -19,7 +19,19 @@ int check_launch(const char* what);
 // gateup: N counts the activated features (the weight has 2N rows).
 int64_t tail_scratch_bytes(int block, int dtype, int64_t K, int64_t N, bool gateup);
 
-int quant_rows(const void* x, int dtype, int64_t rows, const int32_t* rows_dev, int64_t K, int64_t ldx, void* q_out,
+// Rows a quantisation leaves out: those from *limit on and those whose slot of `sorted` holds a padding id (>= valid);
+// null pointers leave out none.  With 512 pairs per expert in 256-row blocks a fifth of the rows are padding: the activated
+// rows of 2048 tokens (H = 4096, F = 14336, 8 experts, top-2) 42.0 -> 33.9 us.
+struct RowFilter {
+  const int32_t* limit = nullptr;
+  const int32_t* sorted = nullptr;
+  int64_t valid = 0;
+  __device__ __forceinline__ bool skips(int64_t row) const {
+    const int32_t id = sorted ? sorted[row] : 0;
+    return (limit && row >= limit[0]) || (sorted && id >= valid);
+  }
+};
+int quant_rows(const void* x, int dtype, int64_t rows, RowFilter rf, int64_t K, int64_t ldx, void* q_out,
                float* scale_out, hipStream_t st);
 
 // the study knobs set through fr_moe_set_tunables (all zero: the library decides)

@@ -250,7 +250,7 @@ int route_and_align(const void* logits, int logits_dtype, int64_t M, int E, int 
   if (rc != FR_OK) return rc;
   rc = fr_moe_align(c.topk_ids, FR_I32, M * topk, E, block, c.sorted, c.expert_ids, c.npost, c.align_ws, c.align_ws_bytes, stream);
   if (rc != FR_OK || !qx) return rc;
-  return quant_rows(qx, FR_BF16, M, nullptr, H, H, c.xq, c.x_scale, st);
+  return quant_rows(qx, FR_BF16, M, RowFilter{}, H, H, c.xq, c.x_scale, st);
 }
 }  // namespace
 }  // namespace fr
@@ -322,7 +322,8 @@ extern "C" int fr_fused_moe_fp8(const void* x, int x_dtype, const void* w1q, con
   if (rc != FR_OK) return rc;
   rc = fr_moe_gateup_silu_fp8(c.xq, c.x_scale, w1q, w1_scale, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, c.act, stream);
   if (rc != FR_OK) return rc;
-  rc = quant_rows(c.act, FR_BF16, p.sorted_len, c.npost, F, F, c.actq, c.act_scale, st);
+  // only slots that hold a pair: nothing of a padding slot's row is used by the down projection
+  rc = quant_rows(c.act, FR_BF16, p.sorted_len, RowFilter{c.npost, c.sorted, M * topk}, F, F, c.actq, c.act_scale, st);
   if (rc != FR_OK) return rc;
   return fr_moe_down_combine_fp8(c.actq, c.act_scale, w2q, w2_scale, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E,
                                  topk, p.block, p.split_k, x_dtype | w2_flag, c.partial, out, c.tail, stream);
