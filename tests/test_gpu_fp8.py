@@ -69,6 +69,26 @@ def test_fp8_layer_vs_oracle(native, M):
     assert (o - full).norm() / full.norm() < 0.08
 
 
+@pytest.mark.parametrize("M", [1, 16, 200, 700, 2048])
+def test_fp8_layer_does_not_use_padding_rows(native, M):
+    """Padding slots' activated rows are not quantised: whatever the scratch held in their place (NaN codes and scales
+    here, zeros there), the output is the same bit for bit."""
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8
+    from fast_route_amd import _native as N
+    from fast_route_amd.layers.fused_moe import plan
+    _say(f"fp8 padding rows M={M}")
+    H, Fd, E, k = 512, 1024, 8, 2
+    x, logits, w1, w2 = oracle.make_inputs(M, H, Fd, E, seed=78)
+    w = prepare_weights_fp8(w1.bfloat16().cuda(), w2.bfloat16().cuda())
+    ws = torch.empty(plan(M, H, Fd, E, k, None, code=N.FR_FP8_E4M3).workspace_bytes, dtype=torch.uint8, device="cuda")
+    outs = []
+    for fill in (0xFF, 0):
+        out = fused_moe_fp8(x.bfloat16().cuda(), *w, logits.cuda(), k, True, workspace_buf=ws.fill_(fill))
+        torch.cuda.synchronize()
+        outs.append(out.clone())
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
 def test_fp8_layer_with_64_row_blocks(native):
     """H = 4096 with 40 pairs per expert: the plan takes 64-row routing blocks for fp8 too."""
     from fast_route_amd import fused_moe_fp8, prepare_weights_fp8

@@ -790,6 +790,52 @@ def test_out_of_range_expert_ids_are_dropped_pairs(native, M, E, k, H, Fd):
     assert torch.count_nonzero(out0) == 0, "all pairs masked: output must be zero"
 
 
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_combine_over_every_slot_count(native, k, split):
+    """The combine kernel takes the rows of two, three or four slots at a time: every remainder, over one and two K
+    slices, with dropped pairs whose rows are never written (the scratch is filled with NaN beforehand)."""
+    from fast_route_amd import _native as N
+    from fast_route_amd import fused_experts
+    from fast_route_amd.layers.fused_moe import workspace
+    M, E, H, Fd = 70, 12, 512, 1024
+    _say(f"combine k={k} split={split}")
+    x, logits, w1, w2 = _inputs(M, H, Fd, E, 53, torch.bfloat16)
+    tw, ti = oracle.gating_topk(logits, k, True)
+    ti = ti.clone()
+    ti[torch.rand(M, k, generator=torch.Generator().manual_seed(k)) < 0.25] = E
+    t = N.FrMoeTunables()
+    t.split_k = split
+    N.check(N.lib().fr_moe_set_tunables(t))
+    try:
+        ws = workspace(M, H, Fd, E, k, torch.bfloat16, "cuda").fill_(0xFF)
+        out = fused_experts(x.cuda(), w1.cuda(), w2.cuda(), tw.cuda(), ti.cuda(), workspace_buf=ws)
+        torch.cuda.synchronize()
+    finally:
+        N.check(N.lib().fr_moe_set_tunables(None))
+    _assert_close(out, oracle.moe_experts(x, w1, w2, tw, ti), torch.bfloat16, f"combine k={k} split={split}")
+
+
+@pytest.mark.parametrize("E", [3, 64, 256, 257, 300])
+def test_persistent_tiles_with_experts_missing(native, E):
+    """The walk table of the persistent tiles where most experts have no block (runs of equal entries at the front, in
+    between and at the end), below and above the expert count up to which it is built in one pass."""
+    from fast_route_amd.ops.fused_moe import invoke_fused_moe_kernel, moe_align_block_size
+    n, N_, K, block = 700, 256, 512, 128
+    _say(f"experts missing E={E}")
+    g = torch.Generator().manual_seed(E)
+    used = torch.tensor(sorted({1, E // 3, E // 2, E - 2}))
+    ids = used[torch.randint(0, len(used), (n, 1), generator=g)].int()
+    a = (torch.randn(n, K, generator=g) / 8).bfloat16()
+    b = (torch.randn(E, N_, K, generator=g) / 8).bfloat16()
+    s, e, npost = moe_align_block_size(ids.cuda(), block, E)
+    c = torch.zeros(n, 1, N_, dtype=torch.bfloat16, device="cuda")
+    invoke_fused_moe_kernel(a.cuda(), b.cuda(), c, None, ids.cuda(), s, e, npost, False, 1, {"BLOCK_SIZE_M": block})
+    torch.cuda.synchronize()
+    ref = torch.stack([b[int(ids[p])].float() @ a[p].float() for p in range(n)])
+    _assert_close(c.view(n, N_), ref, torch.bfloat16, f"experts missing E={E}")
+
+
 @pytest.mark.parametrize("E", [8, 100, 256])
 @pytest.mark.parametrize("M", [3, 40])
 def test_nan_logit_rows_do_not_reach_the_weights(native, E, M):
