@@ -215,8 +215,15 @@ __device__ __forceinline__ void gate_token(Load load, bool live, int E, int topk
 // per logit and round where comparing exact keys and remembering the slot took five instructions.
 // The packed order is the exact one unless two logits differ only in the bits the index displaced; that shows as two
 // successive winners (one more than asked for is drawn) with equal upper bits while some logit of the token has a bit
-// set down there, and the wavefront then selects again on exact keys.  Logits that came from 16-bit values have no such
-// bits.  65536 tokens, 64 experts, top-6, fp32: 11.6 -> 8.3 us.
+// set down there.  A wavefront that sees it in any of its tokens puts these right: where the class of equal upper bits
+// reaches beyond the last winner, the places it holds are filled again in the exact order of that class alone (its keys
+// are the displaced bits over the index), then the winners' own logits are sorted, which takes one pass over a list
+// that is all but sorted.  Logits that came from 16-bit values have no such bits.
+// Random fp32 logits, us: 65536 tokens, 64 experts, top-6 9.9 (13.0 with exact keys compared in every round), 16384 tokens,
+// 256 experts, top-8 / top-32 10.0 / 18.1 (14.6 / 37.8; 12.0 / 35.6 with every such wavefront selecting again on exact
+// keys).  Every wavefront with a collision, 65536 tokens, 64 experts: 16-bit logits scaled in fp32 10.8 (12.7; 12.6),
+// all but topk - 1 experts masked 9.8 (11.7; 12.2).  The worst case, all 64 logits within 70 units in the last place:
+// 14.9 (12.4; 12.2); 256 experts, top-8: 11.9 (14.4; 14.6).
 constexpr int kBlockedSlots = 4;  // result slots per lane: topk <= kBlockedSlots * G
 
 template <int G, int NV, typename Load4, typename Load1>
@@ -249,8 +256,8 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, boo
   int sel_i[kBlockedSlots];
 #pragma unroll
   for (int i = 0; i < kBlockedSlots; ++i) sel_i[i] = 0;
-  unsigned win = 0u;  // previous winner; with 0 the first round's difference is the key itself
-  bool equal_upper = false;
+  unsigned win = 0u, prev = 0u;  // this and the previous round's winner; with 0 the first round's difference is the key itself
+  unsigned equal = 0u;  // the first winner with the upper bits of the one before it
   int top = 0;        // expert of the largest logit
   for (int r = 0; r <= topk; ++r) {
     unsigned best = 0u;
@@ -261,7 +268,8 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, boo
     if constexpr (G > 4) best = max(best, static_cast<unsigned>(partner_i32<4>(static_cast<int>(best))));
     if constexpr (G > 8) best = max(best, static_cast<unsigned>(partner_i32<8>(static_cast<int>(best))));
     const unsigned next = best + win;
-    if (r > 0) equal_upper |= ((next ^ win) & ~kIndexMask) == 0u;
+    if (r > 0 && equal == 0u && ((next ^ win) & ~kIndexMask) == 0u) equal = next;
+    prev = win;
     win = next;
     const int be = static_cast<int>(kIndexMask - (win & kIndexMask));
     if (r == 0) top = be;
@@ -271,56 +279,109 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, boo
         if (r == sl * G + g) sel_i[sl] = be;
     }
   }
-  const bool has_low = (low & kIndexMask) != 0u;
-  if (__any(equal_upper) && __any(has_low)) {
-    // exact keys; inside the lane a strict "greater" scan keeps the lowest slot, i.e. the lowest expert index, among equal keys
-    unsigned k[VPL];
+  bool unsorted = false;  // winners whose order among themselves is in doubt
+  if (__any(equal != 0u) && __any((low & kIndexMask) != 0u)) {
+    // prev: the last winner, win: the one drawn beyond it
+    int above = 0;  // logits of the token in higher classes than the last winner's
+    unsigned ck[VPL];  // keys of that class, 0 for the rest
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
       const int e = 4 * (G * (i / 4) + g) + (i % 4);
-      k[i] = (e < E) ? float_key(v[i] + 0.f) : 0u;
+      above += pk[i] > (prev | kIndexMask) ? 1 : 0;
+      ck[i] = (e < E && ((pk[i] ^ prev) & ~kIndexMask) == 0u)
+                  ? (float_key(v[i] + 0.f) & kIndexMask) * (kIndexMask + 1) + (pk[i] & kIndexMask) + 1u : 0u;
     }
-    int last = -1;  // slot this lane gave away in the previous round
-    for (int r = 0; r < topk; ++r) {
-      unsigned bk = 0u;
-      int bs = 0;
+    if constexpr (G > 1) above += partner_i32<1>(above);
+    if constexpr (G > 2) above += partner_i32<2>(above);
+    if constexpr (G > 4) above += partner_i32<4>(above);
+    if constexpr (G > 8) above += partner_i32<8>(above);
+    const int places = (live && ((win ^ prev) & ~kIndexMask) == 0u) ? topk - above : 0;
+    // a refilled class comes out in order: left to sort are higher classes, or one that ends with the last winner
+    unsorted = live && equal != 0u && (places == 0 || equal > (prev | kIndexMask));
+    unsigned cw = 0u;
+    for (int q = 0; __any(q < places); ++q) {
+      unsigned best = 0u;
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) {
-        if (i == last) k[i] = 0u;
-        if (k[i] > bk) {
-          bk = k[i];
-          bs = i;
-        }
+      for (int i = 0; i < VPL; ++i) best = max(best, ck[i] - cw);
+      if constexpr (G > 1) best = max(best, static_cast<unsigned>(partner_i32<1>(static_cast<int>(best))));
+      if constexpr (G > 2) best = max(best, static_cast<unsigned>(partner_i32<2>(static_cast<int>(best))));
+      if constexpr (G > 4) best = max(best, static_cast<unsigned>(partner_i32<4>(static_cast<int>(best))));
+      if constexpr (G > 8) best = max(best, static_cast<unsigned>(partner_i32<8>(static_cast<int>(best))));
+      cw += best;
+      if (q < places) {
+#pragma unroll
+        for (int sl = 0; sl < kBlockedSlots; ++sl)
+          if (above + q == sl * G + g) sel_i[sl] = static_cast<int>(kIndexMask - ((cw - 1u) & kIndexMask));
       }
-      int be = 4 * (G * (bs >> 2) + g) + (bs & 3);
-      // all-reduce over the group: larger key wins, equal keys go to the lower expert index
-      auto step = [&](auto tag) {
-        constexpr int S = decltype(tag)::value;
-        const unsigned ok = static_cast<unsigned>(partner_i32<S>(static_cast<int>(bk)));
-        const int oe = partner_i32<S>(be);
-        if (ok > bk || (ok == bk && oe < be)) {
-          bk = ok;
-          be = oe;
-        }
-      };
-      if constexpr (G > 1) step(std::integral_constant<int, 1>{});
-      if constexpr (G > 2) step(std::integral_constant<int, 2>{});
-      if constexpr (G > 4) step(std::integral_constant<int, 4>{});
-      if constexpr (G > 8) step(std::integral_constant<int, 8>{});
-      last = ((be >> 2) % G == g) ? (4 * (be / (4 * G)) + (be & 3)) : -1;
-      if (r == 0) top = be;
-#pragma unroll
-      for (int sl = 0; sl < kBlockedSlots; ++sl)
-        if (r == sl * G + g) sel_i[sl] = be;
     }
   }
 
   // The winners' logits again from the cache the row was just read through: they are spread over the lanes' registers.
-  // top-1 first: with renormalised weights it is all the softmax statistics there are.
-  float sel_v[kBlockedSlots];
+  // Asked for together and unconditionally: slots that are not in use hold expert 0, groups without a token read token 0.
+  float sel_v[kBlockedSlots], top_v = load1(top);
 #pragma unroll
-  for (int sl = 0; sl < kBlockedSlots; ++sl) sel_v[sl] = (live && sl * G + g < topk) ? load1(sel_i[sl]) + 0.f : -INFINITY;
-  float m = live ? load1(top) + 0.f : 0.f;
+  for (int sl = 0; sl < kBlockedSlots; ++sl) sel_v[sl] = load1(sel_i[sl]);
+  top_v += 0.f;
+#pragma unroll
+  for (int sl = 0; sl < kBlockedSlots; ++sl) sel_v[sl] = sl * G + g < topk ? sel_v[sl] + 0.f : -INFINITY;
+
+  if (__any(unsorted)) {
+    // Odd-even transposition of the winners, place sl * G + g in slot sl of lane g, until nothing moves: every exchange
+    // takes away an inversion of a strict order.
+    const int lane = threadIdx.x & 63, base = lane & ~(G - 1);
+    bool moved = true;
+    while (__any(moved)) {
+      moved = false;
+#pragma unroll
+      for (int odd = 0; odd < 2; ++odd) {
+        const bool first = (g & 1) == odd;  // this lane's places are the earlier ones of their pairs
+        auto partner = [&](int x) -> int {  // lane g ^ 1; odd: g + 1 and g - 1 around the group
+          if (!odd) return partner_i32<1>(x);
+          if constexpr (G == 4) return partner_i32<1>(partner_i32<2>(x));
+          return __shfl(x, base | ((first ? g + 1 : g + G - 1) % G));
+        };
+        float ov[kBlockedSlots] = {};
+        int oe[kBlockedSlots] = {};
+#pragma unroll
+        for (int sl = 0; sl < kBlockedSlots; ++sl) {
+          if (sl * G >= topk) continue;
+          ov[sl] = __int_as_float(partner(__float_as_int(sel_v[sl])));
+          oe[sl] = partner(sel_i[sl]);
+        }
+        float nv[kBlockedSlots];
+        int ne[kBlockedSlots];
+#pragma unroll
+        for (int sl = 0; sl < kBlockedSlots; ++sl) {
+          nv[sl] = sel_v[sl];
+          ne[sl] = sel_i[sl];
+          if (sl * G >= topk) continue;
+          // across the end of the group: the next slot of its first lane, the previous slot of its last
+          const int down = sl > 0 ? sl - 1 : 0, up = sl + 1 < kBlockedSlots ? sl + 1 : sl;
+          const bool wraps = odd && (g == 0 || g == G - 1);
+          const float pv = wraps ? (g == 0 ? ov[down] : ov[up]) : ov[sl];
+          const int pe = wraps ? (g == 0 ? oe[down] : oe[up]) : oe[sl];
+          const int r = sl * G + g;
+          const unsigned mine = float_key(sel_v[sl]), other = float_key(pv);
+          const bool other_first = other > mine || (other == mine && pe < sel_i[sl]);
+          const bool pair = live && (first ? r + 1 < topk : (r > 0 && r < topk));
+          if (pair && first == other_first) {
+            nv[sl] = pv;
+            ne[sl] = pe;
+            moved = true;
+          }
+        }
+#pragma unroll
+        for (int sl = 0; sl < kBlockedSlots; ++sl) {
+          sel_v[sl] = nv[sl];
+          sel_i[sl] = ne[sl];
+        }
+      }
+    }
+    top_v = __shfl(sel_v[0], base);
+  }
+
+  // top-1 first: with renormalised weights it is all the softmax statistics there are
+  float m = top_v;
   float denom;
   if (renorm) {
     denom = 0.f;

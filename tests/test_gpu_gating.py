@@ -103,6 +103,48 @@ def test_gating_near_ties_many_experts(native, E, topk):
             torch.testing.assert_close(w, rw, atol=W_ATOL, rtol=0)
 
 
+@pytest.mark.parametrize("E,topk", [(20, 16), (32, 5), (64, 1), (64, 6), (64, 16), (128, 8), (128, 32), (252, 9), (256, 8), (256, 64)])
+@pytest.mark.parametrize("spread", [2, 40, 700, 20000])
+def test_gating_packed_key_classes(native, E, topk, spread):
+    """fp32 logits that share the upper bits of their packed keys in every way: classes that end with the last winner or
+    reach beyond it, several classes in one row, exact duplicates with low bits set (16-bit logits scaled in fp32), masked
+    experts.  `spread` is the width of a row's logits in units in the last place."""
+    _say(f"gating classes E={E} topk={topk} spread={spread}")
+    g = torch.Generator().manual_seed(E * 31 + topk * 7 + spread)
+    for sign in (1.0, -1.0):
+        logits = sign * (1.0 + torch.randint(0, spread, (1100, E), generator=g).float() * 2.0 ** -23)
+        logits[1::5] = torch.randn(logits[1::5].shape, generator=g).bfloat16().float() * 0.37
+        logits[2::5, max(topk - 1, 1):] = float("-inf")
+        logits[3::5, ::3] += torch.randint(0, 3, logits[3::5, ::3].shape, generator=g).float()
+        for renorm in (True, False):
+            w, ids = _run_gating(logits.cuda(), topk, renorm)
+            rw, rid = oracle.gating_topk(logits, topk, renorm)
+            assert torch.equal(ids, rid)
+            torch.testing.assert_close(w, rw, atol=W_ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("E,topk", [(32, 4), (64, 6), (128, 8), (256, 8)])
+def test_gating_nan_and_infinite_rows_many_experts(native, E, topk):
+    """Rows with NaN or +inf next to ordinary ones: NaN orders above +inf (the order of the keys), such a row's weights are
+    NaN, and the other rows of its wavefront are what they are without it."""
+    _say(f"gating nan / inf rows E={E} topk={topk}")
+    g = torch.Generator().manual_seed(E + topk)
+    logits = torch.randn(1200, E, generator=g)
+    logits[::7, E // 3] = float("nan")
+    logits[3::11, E - 1] = float("inf")
+    logits[::14, 1] = float("nan")
+    bad = (logits.isnan() | (logits == float("inf"))).any(dim=1)
+    masked = ~bad & (torch.arange(1200) % 5 == 0)
+    logits[masked, topk // 2:] = float("-inf")
+    lifted = torch.where(logits.isnan(), 9e30, torch.where(logits == float("inf"), 8e30, logits))
+    for renorm in (True, False):
+        w, ids = _run_gating(logits.cuda(), topk, renorm)
+        rw, rid = oracle.gating_topk(lifted, topk, renorm)
+        assert torch.equal(ids, rid)
+        assert w[bad].isnan().all()
+        torch.testing.assert_close(w[~bad], rw[~bad], atol=W_ATOL, rtol=0)
+
+
 def test_gating_reference_route_test_recipe(native):
     """tests/test_route.py:12-77 of the reference: weights vs topk(softmax(h@gate)), atol 1e-2."""
     for seed in range(3):
