@@ -8,10 +8,13 @@ namespace fr {
 // P = float (one fp32 slice per K split) or the operand type (single slice: each pair's row
 // rounded once before the sum over its token's slots, as the reference's second GEMM writes it,
 // fast_route/fast_route/ops/fused_moe.py:117-123, before torch.sum).
-// HBM bound: the rows of JB (slot, split) terms are asked for together - the check of a pair's expert id would otherwise
-// put every row's load behind the previous row's id - and added in the order of the terms.  JB is a divisor of the number
-// of terms where one of 2, 3, 4 is; a term beyond the last, or of a pair without a row, reads the token's first row (in
-// cache) and is not added.  8192 tokens, H = 2048, top-6: 45.2 -> 40.6 us (5.8 TB/s); 16384 tokens, H = 4096, top-2: 71.1 -> 65.5.
+// HBM bound: the rows of JB (slot, split) terms are asked for together, after their pairs' expert ids (also together; a row
+// behind each id in turn leaves one load in flight), and added in the order of the terms.  JB: 3 where it divides the
+// number of terms, 1 and 2 for so many, else 4.  A term beyond the last, or of a pair without a row, reads the first
+// row of `partial` (in cache, the same for all tokens) and is not added.
+// 8192 tokens, H = 2048, 64 experts, top-6, kernel in us, all pairs / half / an eighth of them on these experts: 34.5 / 20.8 /
+// 17.1 (one row at a time 39.5 / 22.4 / 15.0; rows asked for before the ids are known 36.3 / 35.7 / 37.6); 16384 tokens,
+// H = 4096, 8 experts, top-2: 74.1 / 53.0 / 31.1 (74.8 / 58.0 / 26.2; 73.4 / 71.4 / 66.0).
 template <typename T, typename P, int V, int JB>
 __global__ __launch_bounds__(256) void combine_kernel(const P* __restrict__ partial,
                                                       int64_t split_stride, int splits, int topk,
@@ -26,20 +29,28 @@ __global__ __launch_bounds__(256) void combine_kernel(const P* __restrict__ part
   float s[V];
 #pragma unroll
   for (int r = 0; r < V; ++r) s[r] = 0.f;
-  const P* first = partial + m * topk * H + h;
+  const P *first = partial + m * topk * H + h, *spare = partial + h;
   const int terms = topk * splits;
   for (int t0 = 0; t0 < terms; t0 += JB) {
+    int j[JB], e[JB];
     bool ok[JB];
+    const P* at[JB];
     pv v[JB];
 #pragma unroll
     for (int i = 0; i < JB; ++i) {
-      const int t = t0 + i < terms ? t0 + i : 0, j = splits == 1 ? t : t / splits, sp = t - j * splits;
-      ok[i] = t0 + i < terms;
-      v[i] = *reinterpret_cast<const pv*>(first + sp * split_stride + static_cast<int64_t>(j) * H);
-      if (pair_ids) {  // a pair whose expert id lies outside [0, E) got no slot in the routing arrays: no row was written for it
-        const int e = pair_ids[m * topk + j];
-        ok[i] = ok[i] && e >= 0 && e < E;
-      }
+      const int t = min(t0 + i, terms - 1);
+      j[i] = splits == 1 ? t : t / splits;
+      at[i] = first + (t - j[i] * splits) * split_stride + static_cast<int64_t>(j[i]) * H;
+      e[i] = 0;
+    }
+    if (pair_ids) {  // a pair whose expert id lies outside [0, E) got no slot in the routing arrays: no row was written for it
+#pragma unroll
+      for (int i = 0; i < JB; ++i) e[i] = pair_ids[m * topk + j[i]];
+    }
+#pragma unroll
+    for (int i = 0; i < JB; ++i) {
+      ok[i] = t0 + i < terms && e[i] >= 0 && e[i] < E;
+      v[i] = *reinterpret_cast<const pv*>(ok[i] ? at[i] : spare);
     }
 #pragma unroll
     for (int i = 0; i < JB; ++i)

@@ -798,7 +798,7 @@ def test_combine_over_every_slot_count(native, k, split):
     from fast_route_amd import _native as N
     from fast_route_amd import fused_experts
     from fast_route_amd.layers.fused_moe import workspace
-    M, E, H, Fd = 70, 12, 512, 1024
+    M, E, H, Fd = 70, 12, 512, 2048  # 8 K tiles of the 16-row block's 128 elements per slice: k = 1 is really cut in two
     _say(f"combine k={k} split={split}")
     x, logits, w1, w2 = _inputs(M, H, Fd, E, 53, torch.bfloat16)
     tw, ti = oracle.gating_topk(logits, k, True)
