@@ -11,10 +11,10 @@ namespace fr {
 // HBM bound: the rows of JB (slot, split) terms are asked for together, after their pairs' expert ids (also together; a row
 // behind each id in turn leaves one load in flight), and added in the order of the terms.  JB: 3 where it divides the
 // number of terms, 1 and 2 for so many, else 4.  A term beyond the last, or of a pair without a row, reads the first
-// row of `partial` (in cache, the same for all tokens) and is not added.
-// 8192 tokens, H = 2048, 64 experts, top-6, kernel in us, all pairs / half / an eighth of them on these experts: 34.5 / 20.8 /
-// 17.1 (one row at a time 39.5 / 22.4 / 15.0; rows asked for before the ids are known 36.3 / 35.7 / 37.6); 16384 tokens,
-// H = 4096, 8 experts, top-2: 74.1 / 53.0 / 31.1 (74.8 / 58.0 / 26.2; 73.4 / 71.4 / 66.0).
+// row of `partial` (in cache, the same for all tokens) and is not added; a wavefront without any row in the group goes on.
+// 8192 tokens, H = 2048, 64 experts, top-6, kernel in us, all pairs / half / an eighth of them on these experts: 34.7 / 20.8 /
+// 13.4 (one row at a time 39.0 / 22.4 / 15.1; rows asked for before the ids are known 35.9 / 35.7 / 37.6); 16384 tokens,
+// H = 4096, 8 experts, top-2: 73.4 / 51.0 / 27.1 (74.8 / 58.4 / 27.8; 74.2 / 71.6 / 65.9).
 template <typename T, typename P, int V, int JB>
 __global__ __launch_bounds__(256) void combine_kernel(const P* __restrict__ partial,
                                                       int64_t split_stride, int splits, int topk,
@@ -47,11 +47,15 @@ __global__ __launch_bounds__(256) void combine_kernel(const P* __restrict__ part
 #pragma unroll
       for (int i = 0; i < JB; ++i) e[i] = pair_ids[m * topk + j[i]];
     }
+    bool any = false;
 #pragma unroll
     for (int i = 0; i < JB; ++i) {
       ok[i] = t0 + i < terms && e[i] >= 0 && e[i] < E;
-      v[i] = *reinterpret_cast<const pv*>(ok[i] ? at[i] : spare);
+      any = any || ok[i];
     }
+    if (!__any(any)) continue;  // no row for this wavefront in the group
+#pragma unroll
+    for (int i = 0; i < JB; ++i) v[i] = *reinterpret_cast<const pv*>(ok[i] ? at[i] : spare);
 #pragma unroll
     for (int i = 0; i < JB; ++i)
 #pragma unroll
