@@ -58,7 +58,7 @@ struct GemmArgs {
   int group_t;
   int mul_weight;
   int num_experts;      // E (persistent form: walk order by expert)
-  int long_k;           // down projection (few feature tiles, long K): hint for the 128-row tile's form
+  int long_k;           // down projection (few feature tiles, long K): hint for the form of the 128- and 16-row tiles
   float* tail_ws;       // persistent form only: slice buffers for splitting the last round of tiles along K, or nullptr
   unsigned x_span;      // bytes of X the tile loads may address (from X in gather mode, from a block's first row otherwise), or 0:
                         // with it, the loads of padding slots fall outside the buffer resource and fetch nothing

@@ -3,9 +3,10 @@
 // one output tile are being multiplied, the ring is already refilled with the first K
 // tiles of the workgroup's next output tile (whose routing data was fetched a whole tile
 // earlier), so the start-up of a tile (dependent loads of block table, sorted ids, first
-// operand tiles) and the memory side of its epilogue hide behind MFMA work.  It pays for
-// tiles that leave room for one workgroup per CU only (256 x 256); smaller tiles already
-// overlap one workgroup's start-up with the other's MFMAs.
+// operand tiles) and the memory side of its epilogue hide behind MFMA work.  It pays most for
+// tiles that leave room for one workgroup per CU only (64 rows and up).  With two workgroups per
+// CU (16 rows) one's start-up already overlaps the other's work; there it pays where a tile's K
+// loop is short or a launch has several rounds of tiles (dispatch_block has the figures).
 //
 // Same tile shapes, LDS layout, swizzle, fragment double buffering, barrier placement and
 // epilogues as moe_gemm_kernel (STAGES >= 2, refill in one group); see there.

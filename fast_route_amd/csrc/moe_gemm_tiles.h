@@ -15,9 +15,8 @@ namespace fr {
 //   64 rows:        3-slot ring, 8 wavefronts (4 with 256-byte row segments for the gate/up GEMM, persistent);
 //                   (the register-staged double buffer of STAGES == 0 is no longer used by any tile);
 //   32 / 16 rows:   decode regime, 16x16 MFMA, 3-slot ring, two workgroups per CU (the 16-row tile
-//                   persistent or plain, see dispatch_block): weight streaming at HBM rate.  The gate/up GEMM (short weight rows
-//                   of H elements, many of them) streams faster with 512-byte row
-//                   segments: T32L / T16L, used when H allows.
+//                   persistent or plain, see dispatch_block): weight streaming at HBM rate.  The gate/up GEMM
+//                   streams long weight rows faster in 512-byte segments: T32L (when H allows), T16L (rows over 2 KB, fp8 4 KB).
 template <typename T> struct Tiles {  // bf16 / fp16
   typedef Cfg<256, 256, 128, 2, 4, 32, 1, 2, 0, 2> T256;
   // The same tile on v_mfma_f32_16x16x32: half the accumulator-register traffic per flop of the 32x32x16 shape.
@@ -135,12 +134,18 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       // (block table -> sorted ids -> first K tiles) and its drain, and rounds of tiles do not overlap.  The persistent
       // form refills the ring across tiles, which pays where a tile's K loop is short or there are several rounds.
       if constexpr (EPI == EPI_SILU) {
-        // Rows of up to 2 KB (8 K tiles of 256 bytes; fp8: up to 4 KB): persistent.  Plain 512-byte / persistent 256-byte
-        // segments, layer, on weights that no cache holds (several layers' in turn): H = 1024, F = 3584, 8 experts,
-        // 16 / 128 tokens 49.2 / 78.7 against 47.2 / 68.8 us; fp8, H = 4096, F = 14336, 16 tokens 245.9 against 243.1.
-        // H = 2048, F = 1408, 64 experts, top-6, 32 tokens: 108 / 111 against 116 / 113 (on the previous pass's weights it
-        // is the other way round, 102 against 98: part of them is still in the Infinity Cache).  Longer rows stream
-        // faster in 512-byte pieces (bf16, H = 4096: 428 against 445 us).
+        // Rows of up to 2 KB (8 K tiles of 256 bytes; fp8: up to 4 KB): 256-byte segments, persistent from 5 K tiles on and
+        // up to 1022 experts, else plain (up to 1 KB).  Kernel in us on weights that no cache holds (several layers' in
+        // turn), plain 512-byte segments / this form, 16 tokens, 8 experts unless said otherwise:
+        //   bf16  H = 512, F = 3584 (plain) 17.9 / 16.3; 64 experts, top-6, F = 1408 35.9 / 31.8, 64 tokens 45.2 / 40.0
+        //         H = 768 22.2 / 20.4, H = 1024 26.1 / 23.8, 64 experts, F = 1408, 32 tokens 65.4 / 59.6
+        //   fp8   H = 512 (plain) 14.7 / 13.2, H = 1024 (plain) 18.6 / 16.9, H = 2048, F = 7168 48.6 / 42.2
+        //         H = 3072, F = 8192 75.0 / 66.9, H = 3584 85.5 / 76.4
+        //         H = 4096, F = 14336, 5 / 16 / 28 tokens 116 / 150 / 151 against 111 / 145 / 145 (another card: 118 / 153 / 153
+        //         against 126 / 154 / 155); 64 experts, F = 1536, 32 tokens 124.7 / 125.0; 16 experts, F = 8192 169 / 167
+        // bf16, H = 2048, F = 1408, 64 experts, top-6, 32 tokens, layer: 108 / 111 against 116 / 113 (on the previous pass's
+        // weights it is the other way round, 102 against 98: part of them is still in the Infinity Cache).  Longer rows
+        // stream faster in 512-byte pieces (bf16, H = 4096, layer: 428 against 445 us).
         if (a.K * static_cast<int>(sizeof(T)) <= (sizeof(T) == 1 ? 4096 : 2048)) {
           fill(16, TL::T16::BF, TL::T16::BKB);
           return launch_gemm_persistent<T, typename TL::T16, EPI>(a, splits, st);
@@ -151,9 +156,10 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
         }
       }
       fill(16, TL::T16::BF, TL::T16::BKB);
-      // The layer's down projection from 8 KB of K per slice on (32 K tiles): persistent.  H = 4096, F = 8192, 16 experts,
-      // 24 / 64 tokens 498 / 554 us plain, 490 / 525 persistent (two rounds of tiles); one round (8 experts, F = 14336)
-      // 428 either way; 2.8 KB (F = 1408) loses 1 %.
+      // The layer's down projection from 8 KB of K per slice on (32 K tiles): persistent.  Kernel, plain / persistent: bf16,
+      // H = 4096, F = 8192, 16 experts, 24 / 64 tokens (two rounds of tiles) 208 / 178 us, H = 2048, F = 4096, 64 experts, top-6,
+      // 8 / 40 tokens 114 / 99 and 201 / 159; fp8, 16 experts 102 / 94; one round (8 experts, F = 14336) 151.5 either way,
+      // fp8 72 / 71; 2.8 KB (F = 1408) loses 1 %.
       if (EPI != EPI_SILU && a.long_k && a.k_per_split * static_cast<int>(sizeof(T)) >= 8192)
         return launch_gemm_persistent<T, typename TL::T16, EPI>(a, splits, st);
       return launch_gemm<T, typename TL::T16, EPI>(a, splits, st);

@@ -347,8 +347,8 @@ __global__ __launch_bounds__(kSegThreads) void align_scatter_kernel(
 // (a) each expert's total and (b) the pairs of each expert in the segments before its own.  Here a count
 // workgroup covers 16 segments, leaves each segment's offset INSIDE the workgroup in counts[e][seg] and the
 // workgroup's sums in wgcnt[b][e]; a scatter workgroup then gets (a) and (b) from one pass over the NB x E
-// workgroup sums (6144 values for 64 experts and 393 216 pairs: six loads per thread, summed with integer
-// LDS atomics, so the order does not matter).  Used while NB x E stays small.
+// workgroup sums (6144 values for 64 experts and 393 216 pairs: six loads per thread, all of one expert, summed in
+// registers before two integer LDS atomics, so the order does not matter).  Used while NB x E stays small.
 constexpr int kSeg2Threads = 1024;
 constexpr int kSeg2Waves = kSeg2Threads / kWave;
 constexpr int64_t kTwoLevelMaxEntries = 16384;

@@ -89,6 +89,50 @@ def test_fp8_layer_does_not_use_padding_rows(native, M):
     assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("split,Fd", [(1, 8192), (2, 16384)])
+def test_fp8_sixteen_row_down_projection_over_several_rounds(native, split, Fd):
+    """Persistent 16-row tiles in fp8 (8 KB of K per slice of the down projection) with more tiles than workgroups: the ring
+    is handed over between full blocks, blocks of one pair and the two blocks of an expert with 17 pairs.  Tolerance as for
+    the layer against the oracle: the reference quantises the same activations, in fp32 on dequantised operands."""
+    from fast_route_amd import _native as N
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8, quantize_rows_e4m3
+    E, H = 40, 1024
+    _say(f"fp8 16-row down rounds split={split}")
+    g = torch.Generator().manual_seed(93)
+    counts = [(16, 1, 9, 17)[e % 4] if e < 8 else 1 + (e * 7) % 16 for e in range(E)]
+    ti = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    M = ti.numel()
+    ti = ti[torch.randperm(M, generator=g)]
+    logits = torch.randn(M, E, generator=g)
+    logits[torch.arange(M), ti] += 20.0
+    gd = torch.Generator(device="cuda").manual_seed(94)
+    w = prepare_weights_fp8(torch.empty(E, 2 * Fd, H, dtype=torch.bfloat16, device="cuda").normal_(0, 0.02, generator=gd),
+                            torch.empty(E, H, Fd, dtype=torch.bfloat16, device="cuda").normal_(0, 0.02, generator=gd))
+    x = torch.randn(M, H, generator=g).bfloat16().cuda()
+    t = N.FrMoeTunables()
+    t.block, t.split_k = 16, split
+    N.check(N.lib().fr_moe_set_tunables(t))
+    try:
+        out = fused_moe_fp8(x, *w, logits.cuda(), 1, True)
+        torch.cuda.synchronize()
+    finally:
+        N.check(N.lib().fr_moe_set_tunables(None))
+
+    def wide(codes, scale):
+        return codes.view(torch.float8_e4m3fn).float() * scale[:, None]
+
+    ref = torch.empty(M, H)
+    xq = wide(*quantize_rows_e4m3(x))
+    for e in range(E):
+        rows = (ti == e).nonzero()[:, 0]
+        h = xq[rows.cuda()] @ wide(w[0][e], w[1][e]).t()
+        act = (torch.nn.functional.silu(h[:, :Fd]) * h[:, Fd:]).bfloat16()
+        ref[rows] = (wide(*quantize_rows_e4m3(act)) @ wide(w[2][e], w[3][e]).t()).cpu()
+    o = out.float().cpu()
+    assert torch.isfinite(o).all()
+    assert (o - ref).norm() <= 1e-2 * ref.norm() and (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
 def test_fp8_layer_with_64_row_blocks(native):
     """H = 4096 with 40 pairs per expert: the plan takes 64-row routing blocks for fp8 too."""
     from fast_route_amd import fused_moe_fp8, prepare_weights_fp8

@@ -816,12 +816,49 @@ def test_combine_over_every_slot_count(native, k, split):
     _assert_close(out, oracle.moe_experts(x, w1, w2, tw, ti), torch.bfloat16, f"combine k={k} split={split}")
 
 
+@pytest.mark.parametrize("split,Fd", [(1, 4096), (2, 8192)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_sixteen_row_down_projection_over_several_rounds(native, dtype, split, Fd):
+    """The 16-row down projection with 8 KB of K per slice is persistent: 42 blocks x 16 feature tiles are more than its
+    512 workgroups (two K slices: 256 each), so workgroups hand their ring over to a second and third tile - between full
+    blocks, blocks of one pair and the two blocks of an expert with 17 pairs."""
+    from fast_route_amd import _native as N
+    from fast_route_amd import fused_experts
+    E, H = 40, 1024
+    _say(f"16-row down rounds {dtype} split={split}")
+    g = torch.Generator().manual_seed(91)
+    counts = [(16, 1, 9, 17)[e % 4] if e < 8 else 1 + (e * 7) % 16 for e in range(E)]
+    ti = torch.repeat_interleave(torch.arange(E, dtype=torch.int32), torch.tensor(counts))
+    M = ti.numel()
+    ti = ti[torch.randperm(M, generator=g)].view(M, 1).contiguous()
+    gd = torch.Generator(device="cuda").manual_seed(92)
+    w1 = torch.empty(E, 2 * Fd, H, dtype=dtype, device="cuda").normal_(0, 0.02, generator=gd)
+    w2 = torch.empty(E, H, Fd, dtype=dtype, device="cuda").normal_(0, 0.02, generator=gd)
+    x = torch.randn(M, H, generator=g).to(dtype).cuda()
+    tw = torch.rand(M, 1, generator=g).cuda()
+    t = N.FrMoeTunables()
+    t.block, t.split_k = 16, split
+    N.check(N.lib().fr_moe_set_tunables(t))
+    try:
+        out = fused_experts(x, w1, w2, tw, ti.cuda())
+        torch.cuda.synchronize()
+    finally:
+        N.check(N.lib().fr_moe_set_tunables(None))
+    ref = torch.empty(M, H)
+    for e in range(E):
+        rows = (ti[:, 0] == e).nonzero()[:, 0]
+        h = x[rows.cuda()].float() @ w1[e].float().t()
+        act = (torch.nn.functional.silu(h[:, :Fd]) * h[:, Fd:]).to(dtype).float()
+        ref[rows] = ((act @ w2[e].float().t()) * tw[rows.cuda()]).cpu()
+    _assert_close(out, ref, dtype, f"16-row down rounds split={split}")
+
+
 @pytest.mark.parametrize("E", [3, 64, 256, 257, 300])
 def test_persistent_tiles_with_experts_missing(native, E):
     """The walk table of the persistent tiles where most experts have no block (runs of equal entries at the front, in
     between and at the end), below and above the expert count up to which it is built in one pass."""
     from fast_route_amd.ops.fused_moe import invoke_fused_moe_kernel, moe_align_block_size
-    n, N_, K, block = 700, 256, 512, 128
+    n, N_, K, block = 700, 256, 512, 160  # 160 rows: persistent at op level too, from 5 K tiles on
     _say(f"experts missing E={E}")
     g = torch.Generator().manual_seed(E)
     used = torch.tensor(sorted({1, E // 3, E // 2, E - 2}))
