@@ -217,13 +217,13 @@ __device__ __forceinline__ void gate_token(Load load, bool live, int E, int topk
 // successive winners (one more than asked for is drawn) with equal upper bits while some logit of the token has a bit
 // set down there.  A wavefront that sees it in any of its tokens puts these right: where the class of equal upper bits
 // reaches beyond the last winner, the places it holds are filled again in the exact order of that class alone (its keys
-// are the displaced bits over the index), then the winners' own logits are sorted, which takes one pass over a list
-// that is all but sorted.  Logits that came from 16-bit values have no such bits.
-// Random fp32 logits, us: 65536 tokens, 64 experts, top-6 9.9 (13.0 with exact keys compared in every round), 16384 tokens,
-// 256 experts, top-8 / top-32 10.0 / 18.1 (14.6 / 37.8; 12.0 / 35.6 with every such wavefront selecting again on exact
-// keys).  Every wavefront with a collision, 65536 tokens, 64 experts: 16-bit logits scaled in fp32 10.8 (12.7; 12.6),
-// all but topk - 1 experts masked 9.8 (11.7; 12.2).  The worst case, all 64 logits within 70 units in the last place:
-// 14.9 (12.4; 12.2); 256 experts, top-8: 11.9 (14.4; 14.6).
+// are the displaced bits over the index), then every winner's place is counted from the winners' own logits.  Logits that
+// came from 16-bit values have no such bits.  (Sorting the winners by exchanges of neighbours took 15.1 us where the count
+// takes 12.3, 64 experts, top-6, all in one class; 256 experts, top-32, it was 10 % faster.)
+// Random fp32 logits, us, exact keys compared in every round / a whole second selection on exact keys after a collision /
+// now: 65536 tokens, 64 experts, top-6 13.1 / 10.0 / 9.3; 16384 tokens, 256 experts, top-8 16.1 / 11.9 / 10.8, top-32 40.7 /
+// 36.5 / 21.2.  A collision in every wavefront, 65536 tokens, 64 experts: 16-bit logits scaled in fp32 12.3 / 12.6 / 10.5,
+// all but topk - 1 experts masked 11.5 / 12.7 / 9.9, all 64 logits within 70 units in the last place 12.5 / 12.5 / 12.3.
 constexpr int kBlockedSlots = 4;  // result slots per lane: topk <= kBlockedSlots * G
 
 template <int G, int NV, typename Load4, typename Load1>
@@ -325,59 +325,48 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, boo
 #pragma unroll
   for (int sl = 0; sl < kBlockedSlots; ++sl) sel_v[sl] = sl * G + g < topk ? sel_v[sl] + 0.f : -INFINITY;
 
+  int place[kBlockedSlots];
+#pragma unroll
+  for (int sl = 0; sl < kBlockedSlots; ++sl) place[sl] = sl * G + g;
   if (__any(unsorted)) {
-    // Odd-even transposition of the winners, place sl * G + g in slot sl of lane g, until nothing moves: every exchange
-    // takes away an inversion of a strict order.
-    const int lane = threadIdx.x & 63, base = lane & ~(G - 1);
-    bool moved = true;
-    while (__any(moved)) {
-      moved = false;
+    // Every winner's place is the number of winners before it: the lanes' winners go round the group (Gray code over the
+    // four exchanges), each compared with this lane's.  Slots that are not in use come after all others.
+    unsigned key[kBlockedSlots], ok[kBlockedSlots];
+    int oe[kBlockedSlots];
+    unsigned top_key = 0u;
 #pragma unroll
-      for (int odd = 0; odd < 2; ++odd) {
-        const bool first = (g & 1) == odd;  // this lane's places are the earlier ones of their pairs
-        auto partner = [&](int x) -> int {  // lane g ^ 1; odd: g + 1 and g - 1 around the group
-          if (!odd) return partner_i32<1>(x);
-          if constexpr (G == 4) return partner_i32<1>(partner_i32<2>(x));
-          return __shfl(x, base | ((first ? g + 1 : g + G - 1) % G));
+    for (int sl = 0; sl < kBlockedSlots; ++sl) {
+      key[sl] = ok[sl] = sl * G + g < topk ? float_key(sel_v[sl]) : 0u;
+      oe[sl] = sl * G + g < topk ? sel_i[sl] : INT_MAX;
+      place[sl] = 0;
+      top_key = max(top_key, key[sl]);
+    }
+#pragma unroll
+    for (int step = 0; step < G; ++step) {
+#pragma unroll
+      for (int o = 0; o < kBlockedSlots; ++o) {
+        if (o * G >= topk) continue;
+        auto exchange = [&](auto tag) {
+          constexpr int S = decltype(tag)::value;
+          ok[o] = static_cast<unsigned>(partner_i32<S>(static_cast<int>(ok[o])));
+          oe[o] = partner_i32<S>(oe[o]);
         };
-        float ov[kBlockedSlots] = {};
-        int oe[kBlockedSlots] = {};
+        if (step & 1) exchange(std::integral_constant<int, 1>{});
+        else if (step & 2) exchange(std::integral_constant<int, 2>{});
+        else if (step & 4) exchange(std::integral_constant<int, 4>{});
+        else if (step & 8) exchange(std::integral_constant<int, 8>{});
 #pragma unroll
         for (int sl = 0; sl < kBlockedSlots; ++sl) {
           if (sl * G >= topk) continue;
-          ov[sl] = __int_as_float(partner(__float_as_int(sel_v[sl])));
-          oe[sl] = partner(sel_i[sl]);
-        }
-        float nv[kBlockedSlots];
-        int ne[kBlockedSlots];
-#pragma unroll
-        for (int sl = 0; sl < kBlockedSlots; ++sl) {
-          nv[sl] = sel_v[sl];
-          ne[sl] = sel_i[sl];
-          if (sl * G >= topk) continue;
-          // across the end of the group: the next slot of its first lane, the previous slot of its last
-          const int down = sl > 0 ? sl - 1 : 0, up = sl + 1 < kBlockedSlots ? sl + 1 : sl;
-          const bool wraps = odd && (g == 0 || g == G - 1);
-          const float pv = wraps ? (g == 0 ? ov[down] : ov[up]) : ov[sl];
-          const int pe = wraps ? (g == 0 ? oe[down] : oe[up]) : oe[sl];
-          const int r = sl * G + g;
-          const unsigned mine = float_key(sel_v[sl]), other = float_key(pv);
-          const bool other_first = other > mine || (other == mine && pe < sel_i[sl]);
-          const bool pair = live && (first ? r + 1 < topk : (r > 0 && r < topk));
-          if (pair && first == other_first) {
-            nv[sl] = pv;
-            ne[sl] = pe;
-            moved = true;
-          }
-        }
-#pragma unroll
-        for (int sl = 0; sl < kBlockedSlots; ++sl) {
-          sel_v[sl] = nv[sl];
-          sel_i[sl] = ne[sl];
+          place[sl] += (ok[o] > key[sl] || (ok[o] == key[sl] && oe[o] < sel_i[sl])) ? 1 : 0;
         }
       }
     }
-    top_v = __shfl(sel_v[0], base);
+    if constexpr (G > 1) top_key = max(top_key, static_cast<unsigned>(partner_i32<1>(static_cast<int>(top_key))));
+    if constexpr (G > 2) top_key = max(top_key, static_cast<unsigned>(partner_i32<2>(static_cast<int>(top_key))));
+    if constexpr (G > 4) top_key = max(top_key, static_cast<unsigned>(partner_i32<4>(static_cast<int>(top_key))));
+    if constexpr (G > 8) top_key = max(top_key, static_cast<unsigned>(partner_i32<8>(static_cast<int>(top_key))));
+    top_v = key_float(top_key);
   }
 
   // top-1 first: with renormalised weights it is all the softmax statistics there are
@@ -406,8 +395,8 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, boo
     for (int sl = 0; sl < kBlockedSlots; ++sl) {
       const int r = sl * G + g;
       if (r < topk) {
-        w_row[r] = __expf(sel_v[sl] - m) / denom;
-        id_row[r] = sel_i[sl];
+        w_row[place[sl]] = __expf(sel_v[sl] - m) / denom;
+        id_row[place[sl]] = sel_i[sl];
       }
     }
   }
