@@ -53,13 +53,31 @@ int gateup_rows_routed(const void* x, const void* w1, const void* logits, int lo
 // Looks up (once per device) the device address of the static scratch behind fr_fused_moe_noalloc on the current device.
 int prepare_static_scratch();
 
+constexpr int kTailDescBytes = 8192;  // what TailScratch::cuts points to
+
+// Scratch of a grouped GEMM for cutting the tiles of its last round along K (plan.tail_bytes, or nullptr), a place for the
+// list of the tiles cut (kTailDescBytes, or nullptr: taken from the scratch's end), and whether the tiles' heights may
+// differ from the routing block's: the layers leave them to the kernel, the staged entry points' callers choose a tile by
+// the block they route with.
+struct TailScratch {
+  float* buffers = nullptr;
+  int* cuts = nullptr;
+  bool any_height = false;
+};
+
+// Gate/up projection + SiLU * up (what fr_moe_gateup_silu / fr_moe_gateup_silu_fp8 launch).
+int gateup_impl(const void* x, const float* x_scale, const void* w1, const float* w1_scale,
+                const int32_t* sorted, const int32_t* expert_ids, const int32_t* npost, int64_t M, int64_t H,
+                int64_t F, int E, int topk, int block, int dtype, void* act, TailScratch tail, hipStream_t st,
+                const char* who, int w_tiled);
+
 // Down projection + routed weight + top-k combine (what fr_moe_down_combine / fr_moe_down_combine_fp8 launch).  pair_ids:
 // the [M, topk] expert ids, or nullptr; with them a pair whose id lies outside [0, E) - it has no slot in the routing
 // arrays - contributes nothing to its token's sum (without them its never-written partial row would be added).
 int down_impl(const void* act, const float* act_scale, const void* w2, const float* w2_scale,
               const float* topk_weights, const int32_t* sorted, const int32_t* expert_ids, const int32_t* npost,
               int64_t M, int64_t H, int64_t F, int E, int topk, int block, int split_k, int dtype, int out_dtype,
-              float* partial, void* out, float* tail_ws, hipStream_t st, const char* who, int w_tiled,
+              float* partial, void* out, TailScratch tail, hipStream_t st, const char* who, int w_tiled,
               const int32_t* pair_ids);
 
 #define FR_REQUIRE(cond, code, ...) \

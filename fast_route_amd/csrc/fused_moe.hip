@@ -9,6 +9,32 @@ namespace {
 constexpr int64_t kAlign = 256;
 int64_t aligned(int64_t bytes) { return round_up(bytes, kAlign); }
 
+fr_moe_tunables g_tunables = {0, 0, 0, 0, 0};
+
+// expected multiples of `rows` that hold an expert's pairs: `avg` pairs per expert, spread as under uniform routing
+double expected_blocks(double avg, int E, int rows) {
+  const double sigma = sqrt(avg * (1.0 - 1.0 / E)) + 1e-9;
+  double sum = 1.0;
+  for (int k = 1; k * rows < avg + 8 * sigma; ++k) sum += 0.5 * erfc((static_cast<double>(k) * rows - avg) / (sigma * 1.4142135623730951));
+  return sum;
+}
+
+// A layer whose plan routes for 128 or 160 rows and runs the one-wavefront-per-SIMD kernel all the same, with tiles as tall as
+// the experts' runs (moe_gemm_quad.h): where the runs' own length in units of 32 rows is under 0.95 of the rows of whole
+// blocks.  Layer in us, 8 experts, H = 4096, F = 14336, top-2, blocks / runs: 1300 tokens 1056 / 967, 1400 1080 / 1000, 1500
+// 1180 / 1033, 2300 (0.92) 1525 / 1520; 1200 tokens (0.99) 870 / 932.  From 310 pairs per expert on: below, with one tile or
+// two per expert, the three-slot ring of the smaller tiles streams the weights faster (1031 tokens 860 / 853, 900 781 / 820,
+// 768 715 / 760, 512 585 / 690).  H = 2048, F = 1408, 64 experts, Zipf-skewed: 6000 tokens (562 pairs per expert) 753 / 730,
+// 5000 tokens (469) 666 / 672.
+bool any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block) {
+  const fr_moe_tunables& t = g_tunables;
+  if ((block != 128 && block != 160) || t.no_quad || t.block || t.split_k > 1 || E > 1022) return false;
+  const int es = dtype == FR_FP8_E4M3 ? 1 : 2;
+  if (H * es < 2048 || F * es < 2048 || H < 256) return false;  // 16 K tiles in both GEMMs, a feature tile in the narrower one
+  const double avg = static_cast<double>(M) * topk / E;
+  return avg >= (H >= 4096 ? 310.0 : 520.0) && expected_blocks(avg, E, 32) * 32 < 0.95 * expected_blocks(avg, E, block) * block;
+}
+
 struct Carve {
   float* topk_w;
   int32_t* topk_ids;
@@ -20,11 +46,15 @@ struct Carve {
   void* act;
   float* partial;
   float* tail;       // scratch for splitting the last round of 256-row tiles, or nullptr
+  int* tail_cuts;    // and the list of the tiles cut
+  bool any_height;   // the GEMMs' tiles need not be the plan's blocks
+  int splits;        // K slices of the down projection
   void* xq;          // fp8 layer only
   float* x_scale;
   void* actq;
   float* act_scale;
   int64_t total;
+  TailScratch tail_scratch() const { return TailScratch{tail, tail_cuts, any_height}; }
 };
 
 // the activated intermediate is stored in half precision also on the fp8 path
@@ -46,6 +76,9 @@ Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dt
   c.act = take(p.sorted_len * F * act_elem_size(dtype));
   c.partial = reinterpret_cast<float*>(take(static_cast<int64_t>(p.split_k) * n * H * 4));
   c.tail = p.tail_bytes > 0 ? reinterpret_cast<float*>(take(p.tail_bytes)) : nullptr;
+  c.any_height = any_height(M, H, F, E, topk, dtype, p.block);
+  c.splits = c.any_height ? 1 : p.split_k;
+  c.tail_cuts = p.tail_bytes > 0 ? reinterpret_cast<int*>(take(kTailDescBytes)) : nullptr;
   c.xq = nullptr; c.x_scale = nullptr; c.actq = nullptr; c.act_scale = nullptr;
   if (dtype == FR_FP8_E4M3) {
     c.xq = take(M * H);
@@ -56,8 +89,6 @@ Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dt
   c.total = off;
   return c;
 }
-
-fr_moe_tunables g_tunables = {0, 0, 0, 0, 0};
 
 int check_layer_shapes(const char* who, int64_t M, int64_t H, int64_t F, int E, int topk, int dtype) {
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16 || dtype == FR_FP8_E4M3, FR_E_DTYPE, "%s: dtype %d not in {f16, bf16, fp8_e4m3}", who, dtype);
@@ -141,13 +172,7 @@ extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk,
   // go - 128 / 160 / 256 rows: 512 tokens 435 / 392, 1024: 543 / 505, 2560: 1145 / 1006 / 1063 us, but 2048: 853 / 877
   // / 899 - and below 900 pairs per expert (4096 tokens: 1506 against 1495 us with 256 rows).
   const bool two_byte = dtype == FR_BF16 || dtype == FR_F16;
-  const double sigma = sqrt(avg * (1.0 - 1.0 / E)) + 1e-9;  // spread of an expert's pairs under uniform routing
-  auto tail = [&](double x) { return 0.5 * erfc((x - avg) / (sigma * 1.4142135623730951)); };  // P(pairs of an expert > x)
-  auto expected = [&](int rows) {  // expected multiples of `rows` that hold an expert's pairs
-    double sum = 1.0;
-    for (int k = 1; k * rows < avg + 8 * sigma; ++k) sum += tail(static_cast<double>(k) * rows);
-    return sum;
-  };
+  auto expected = [&](int rows) { return expected_blocks(avg, E, rows); };
   if ((block == 128 || block == 256) && H >= 2048 && F >= 1024 && E <= 1022 && avg >= 112 &&
       avg < (H >= 4096 ? (two_byte ? 1200.0 : 900.0) : t256)) {
     const double b128 = expected(128), b160 = expected(160);
@@ -268,10 +293,11 @@ extern "C" int fr_fused_experts(const void* x, const void* w1, const void* w2, c
   Carve c = carve(workspace, M, H, F, E, topk, dtype & ~FR_W_TILED, p);
   rc = fr_moe_align(topk_ids, FR_I32, M * topk, E, p.block, c.sorted, c.expert_ids, c.npost, c.align_ws, c.align_ws_bytes, stream);
   if (rc != FR_OK) return rc;
-  rc = fr_moe_gateup_silu(x, w1, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, dtype, c.act, c.tail, stream);
+  rc = gateup_impl(x, nullptr, w1, nullptr, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, dtype & ~FR_W_TILED, c.act, c.tail_scratch(),
+                   static_cast<hipStream_t>(stream), "fr_fused_experts", (dtype & FR_W1_TILED) ? 1 : 0);
   if (rc != FR_OK) return rc;
   return down_impl(c.act, nullptr, w2, nullptr, topk_weights, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
-                   p.split_k, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail, static_cast<hipStream_t>(stream),
+                   c.splits, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
                    "fr_fused_experts", (dtype & FR_W2_TILED) ? 1 : 0, topk_ids);
 }
 
@@ -294,11 +320,12 @@ extern "C" int fr_fused_moe(const void* x, const void* w1, const void* w2, const
   if (rc == 1) {
     rc = route_and_align(logits, logits_dtype, M, E, topk, renormalize, p.block, c, nullptr, H, stream);
     if (rc != FR_OK) return rc;
-    rc = fr_moe_gateup_silu(x, w1, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, dtype, c.act, c.tail, stream);
+    rc = gateup_impl(x, nullptr, w1, nullptr, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, dtype & ~FR_W_TILED, c.act, c.tail_scratch(),
+                   static_cast<hipStream_t>(stream), "fr_fused_moe", (dtype & FR_W1_TILED) ? 1 : 0);
     if (rc != FR_OK) return rc;
   }
   return down_impl(c.act, nullptr, w2, nullptr, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
-                   p.split_k, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail, static_cast<hipStream_t>(stream),
+                   c.splits, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
                    "fr_fused_moe", (dtype & FR_W2_TILED) ? 1 : 0, c.topk_ids);
 }
 
@@ -320,13 +347,15 @@ extern "C" int fr_fused_moe_fp8(const void* x, int x_dtype, const void* w1q, con
   Carve c = carve(workspace, M, H, F, E, topk, FR_FP8_E4M3, p);
   rc = route_and_align(logits, logits_dtype, M, E, topk, renormalize, p.block, c, x, H, stream);
   if (rc != FR_OK) return rc;
-  rc = fr_moe_gateup_silu_fp8(c.xq, c.x_scale, w1q, w1_scale, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, c.act, stream);
+  // the eight-wavefront kernels' gate/up GEMM does not cut its last round in fp8
+  rc = gateup_impl(c.xq, c.x_scale, w1q, w1_scale, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, FR_FP8_E4M3, c.act,
+                   p.block == 256 || c.any_height ? c.tail_scratch() : TailScratch{}, st, "fr_fused_moe_fp8", 0);
   if (rc != FR_OK) return rc;
   // only slots that hold a pair: nothing of a padding slot's row is used by the down projection
   rc = quant_rows(c.act, FR_BF16, p.sorted_len, RowFilter{c.npost, c.sorted, M * topk}, F, F, c.actq, c.act_scale, st);
   if (rc != FR_OK) return rc;
-  return fr_moe_down_combine_fp8(c.actq, c.act_scale, w2q, w2_scale, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E,
-                                 topk, p.block, p.split_k, x_dtype | w2_flag, c.partial, out, c.tail, stream);
+  return down_impl(c.actq, c.act_scale, w2q, w2_scale, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
+                   c.splits, FR_FP8_E4M3, x_dtype, c.partial, out, c.tail_scratch(), st, "fr_fused_moe_fp8", w2_flag ? 1 : 0, nullptr);
 }
 
 // ---- one entry point that allocates nothing ------------------------------------

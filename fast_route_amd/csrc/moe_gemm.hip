@@ -161,8 +161,8 @@ int64_t tail_scratch_bytes(int block, int dtype, int64_t K, int64_t N, bool gate
 
 int gateup_impl(const void* x, const float* x_scale, const void* w1, const float* w1_scale,
                 const int32_t* sorted, const int32_t* expert_ids, const int32_t* npost, int64_t M, int64_t H,
-                int64_t F, int E, int topk, int block, int dtype, void* act, float* tail_ws, hipStream_t st,
-                const char* who, int w_tiled = 0) {
+                int64_t F, int E, int topk, int block, int dtype, void* act, TailScratch tail, hipStream_t st,
+                const char* who, int w_tiled) {
   if (M == 0) return FR_OK;
   FR_REQUIRE(!w_tiled || (F % kTileRows == 0 && (H * elem_bytes(dtype)) % kTileBytes == 0), FR_E_SHAPE,
              "%s: prepared weights need F %% %d == 0 and whole %d-byte K tiles", who, kTileRows, kTileBytes);
@@ -171,7 +171,7 @@ int gateup_impl(const void* x, const float* x_scale, const void* w1, const float
   FR_REQUIRE(H > 0 && H % k_multiple(dtype, block) == 0, FR_E_SHAPE, "%s: H=%lld must be a multiple of %d for block %d", who, (long long)H, k_multiple(dtype, block), block);
   FR_REQUIRE(F > 0 && F % 8 == 0, FR_E_SHAPE, "%s: F=%lld must be a positive multiple of 8", who, (long long)F);
   FR_REQUIRE(topk >= 1 && E >= 1 && M * topk < (int64_t(1) << 30), FR_E_SHAPE, "%s: M*topk too large", who);
-  FR_REQUIRE(aligned16(x) && aligned16(w1) && aligned16(act) && aligned16(tail_ws), FR_E_ALIGN, "%s: operands must be 16-byte aligned", who);
+  FR_REQUIRE(aligned16(x) && aligned16(w1) && aligned16(act) && aligned16(tail.buffers), FR_E_ALIGN, "%s: operands must be 16-byte aligned", who);
   const int64_t n = M * topk, sorted_len = n + int64_t(E) * (block - 1);
   GemmArgs a = {};
   a.X = x; a.ldx = H; a.W = w1; a.w_expert_stride = 2 * F * H; a.ldw = H; a.out = act; a.ldo = F;
@@ -179,7 +179,9 @@ int gateup_impl(const void* x, const float* x_scale, const void* w1, const float
   a.x_scale = x_scale; a.w_scale = w1_scale; a.w_rows = static_cast<int>(2 * F);
   a.num_valid = (int)n; a.top_k = topk; a.N = (int)F; a.K = (int)H;
   a.num_experts = E;
-  a.tail_ws = tail_ws;
+  a.tail_ws = tail.buffers;
+  a.tail_desc = tail.cuts;
+  a.any_height = tail.any_height;
   a.w_tiled = w_tiled;
   // batches the routed form of the row kernel takes run the row kernel here too (same kernel, same sums, whoever
   // did the routing); the row kernels read whole weight rows and take the row-major layout only
@@ -216,7 +218,7 @@ int gateup_rows_routed(const void* x, const void* w1, const void* logits, int lo
 int down_impl(const void* act, const float* act_scale, const void* w2, const float* w2_scale,
               const float* topk_weights, const int32_t* sorted, const int32_t* expert_ids, const int32_t* npost,
               int64_t M, int64_t H, int64_t F, int E, int topk, int block, int split_k, int dtype, int out_dtype,
-              float* partial, void* out, float* tail_ws, hipStream_t st, const char* who, int w_tiled,
+              float* partial, void* out, TailScratch tail, hipStream_t st, const char* who, int w_tiled,
               const int32_t* pair_ids) {
   if (M == 0) return FR_OK;
   FR_REQUIRE(!w_tiled || (H % kTileRows == 0 && (F * elem_bytes(dtype)) % kTileBytes == 0), FR_E_SHAPE,
@@ -227,7 +229,7 @@ int down_impl(const void* act, const float* act_scale, const void* w2, const flo
   FR_REQUIRE(H > 0 && H % 4 == 0, FR_E_SHAPE, "%s: H=%lld must be a positive multiple of 4", who, (long long)H);
   FR_REQUIRE(split_k >= 1 && split_k <= 64, FR_E_SHAPE, "%s: split_k=%d outside [1, 64]", who, split_k);
   FR_REQUIRE(topk >= 1 && E >= 1 && M * topk < (int64_t(1) << 30), FR_E_SHAPE, "%s: M*topk too large", who);
-  FR_REQUIRE(aligned16(act) && aligned16(w2) && aligned16(partial) && aligned16(out) && aligned16(tail_ws), FR_E_ALIGN, "%s: operands must be 16-byte aligned", who);
+  FR_REQUIRE(aligned16(act) && aligned16(w2) && aligned16(partial) && aligned16(out) && aligned16(tail.buffers), FR_E_ALIGN, "%s: operands must be 16-byte aligned", who);
   const int64_t n = M * topk, sorted_len = n + int64_t(E) * (block - 1);
   const int splits = usable_splits(split_k, F, k_multiple(dtype, block));
   GemmArgs a = {};
@@ -238,7 +240,9 @@ int down_impl(const void* act, const float* act_scale, const void* w2, const flo
   a.topk_w = topk_weights; a.num_valid = (int)n; a.top_k = 0; a.N = (int)H; a.K = (int)F;
   a.mul_weight = 1;
   a.num_experts = E;
-  a.tail_ws = tail_ws;
+  a.tail_ws = tail.buffers;
+  a.tail_desc = tail.cuts;
+  a.any_height = tail.any_height;
   a.long_k = 1;
   a.w_tiled = w_tiled;
   if (!w_tiled && down_rows_fits(n, F, H, sorted_len, elem_bytes(dtype)) && out_dtype == dtype) {
@@ -347,7 +351,7 @@ extern "C" int fr_moe_gateup_silu(const void* x, const void* w1, const int32_t* 
   dtype &= ~FR_W_TILED;
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_gateup_silu: dtype %d not in {f16, bf16}", dtype);
   return gateup_impl(x, nullptr, w1, nullptr, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F, E, topk,
-                     block, dtype, act, static_cast<float*>(tail_ws), static_cast<hipStream_t>(stream), "fr_moe_gateup_silu", w_tiled);
+                     block, dtype, act, TailScratch{static_cast<float*>(tail_ws)}, static_cast<hipStream_t>(stream), "fr_moe_gateup_silu", w_tiled);
 }
 
 extern "C" int fr_moe_gateup_silu_fp8(const void* xq, const float* x_scale, const void* w1q, const float* w1_scale,
@@ -356,7 +360,7 @@ extern "C" int fr_moe_gateup_silu_fp8(const void* xq, const float* x_scale, cons
                                       int topk, int block, void* act_bf16, void* stream) {
   FR_REQUIRE(x_scale && w1_scale, FR_E_NULL, "fr_moe_gateup_silu_fp8: null scale pointer");
   return gateup_impl(xq, x_scale, w1q, w1_scale, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F, E, topk,
-                     block, FR_FP8_E4M3, act_bf16, nullptr, static_cast<hipStream_t>(stream), "fr_moe_gateup_silu_fp8");
+                     block, FR_FP8_E4M3, act_bf16, TailScratch{}, static_cast<hipStream_t>(stream), "fr_moe_gateup_silu_fp8", 0);
 }
 
 extern "C" int fr_moe_down_combine(const void* act, const void* w2, const float* topk_weights,
@@ -368,7 +372,7 @@ extern "C" int fr_moe_down_combine(const void* act, const void* w2, const float*
   dtype &= ~FR_W_TILED;
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_down_combine: dtype %d not in {f16, bf16}", dtype);
   return down_impl(act, nullptr, w2, nullptr, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F,
-                   E, topk, block, split_k, dtype, dtype, partial, out, static_cast<float*>(tail_ws),
+                   E, topk, block, split_k, dtype, dtype, partial, out, TailScratch{static_cast<float*>(tail_ws)},
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine", w_tiled, nullptr);
 }
 
@@ -381,7 +385,7 @@ extern "C" int fr_moe_down_combine_fp8(const void* actq, const float* act_scale,
   out_dtype &= ~FR_W_TILED;
   FR_REQUIRE(act_scale && w2_scale, FR_E_NULL, "fr_moe_down_combine_fp8: null scale pointer");
   return down_impl(actq, act_scale, w2q, w2_scale, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M,
-                   H, F, E, topk, block, split_k, FR_FP8_E4M3, out_dtype, partial, out, static_cast<float*>(tail_ws),
+                   H, F, E, topk, block, split_k, FR_FP8_E4M3, out_dtype, partial, out, TailScratch{static_cast<float*>(tail_ws)},
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine_fp8", w_tiled, nullptr);
 }
 

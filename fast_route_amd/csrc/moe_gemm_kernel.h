@@ -60,9 +60,14 @@ struct GemmArgs {
   int num_experts;      // E (persistent form: walk order by expert)
   int long_k;           // down projection (few feature tiles, long K): hint for the form of the 128- and 16-row tiles
   float* tail_ws;       // persistent form only: slice buffers for splitting the last round of tiles along K, or nullptr
+  int* tail_desc;       // one-wavefront-per-SIMD form only: kTailDescBytes next to tail_ws, or nullptr (they are taken from its end)
+  int tail_buffers;     // slice buffers of 256 x 256 fp32 per XCD
   unsigned x_span;      // bytes of X the tile loads may address (from X in gather mode, from a block's first row otherwise), or 0:
                         // with it, the loads of padding slots fall outside the buffer resource and fetch nothing
   int add_div;          // EPI_PLAIN: 0 = store row `sorted id` of out; k > 0 = add into row (sorted id / k) of a zero-filled out (packed atomics)
+  unsigned div_mul;     // division by top_k of the one-wavefront-per-SIMD form (quad_divisor)
+  int div_shift;
+  int any_height;       // the tiles' heights need not be the routing block's (routing arrays of this library's own layers)
   int w_tiled;          // W is in the prepared layout (see w_byte_offset), not [E, w_rows, K] row-major
   int setup_only;       // do the per-device set-up of the kernel a launch would take (LDS limit, occupancy) and launch nothing
 };
@@ -244,10 +249,12 @@ __device__ __forceinline__ f32x16 acc_fetch(const f32x16& v) {
   return o;
 }
 
-// AG: the accumulators live in the accumulation registers (one wavefront per SIMD) and are fetched tile by tile.
-template <typename T, typename C, int EPI, bool HOIST = true, bool AG = false, typename AccT>
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::JF][C::IT], int pid_t, int pid_f,
-                                              int expert, int split, int wt, int wf, int frow, int kgrp) {
+// slot0, f0: the tile's first sorted slot and output column.  AG: the accumulators of the first AG token tiles live in the accumulation registers (one
+// wavefront per SIMD) and are fetched tile by tile; slots from row_end on then belong to another tile, their rows of the
+// accumulators are nobody's.
+template <typename T, typename C, int EPI, bool HOIST = true, int AG = 0, typename AccT>
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::JF][C::IT], int slot0, int f0,
+                                              int expert, int split, int wt, int wf, int frow, int kgrp, int row_end = 0) {
   typedef Elem<T> E;
   typedef typename E::out_t out_t;
   typedef typename E::out4 out4;
@@ -259,7 +266,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
   // starting at g*8 + kgrp*4 (TILE==32) or kgrp*4 (TILE==16) inside the MFMA tile.
   constexpr int GROUPS = ACC_N / 4;
   // accumulators in the accumulation registers: results are fetched, computed and stored group by group
-  constexpr bool kFence = AG;
+  constexpr bool kFence = AG > 0;
   // fp8: with HOIST the scales of the lane's weight rows (the same for every token tile) and of its token rows
   // are fetched up front, all loads in flight together, instead of one by one between the stores (which the
   // compiler may not move them across).  That takes JF * ACC_N registers: the persistent kernel, which keeps
@@ -275,7 +282,15 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
   }
   if constexpr (EPI != EPI_SILU || E::SCALED) {
 #pragma unroll
-    for (int i = 0; i < C::IT; ++i) sids[i] = a.sorted[pid_t * BT + wt * C::TT + i * C::TILE + frow];
+    for (int i = 0; i < C::IT; ++i) {
+      const int slot = slot0 + wt * C::TT + i * C::TILE + frow;
+      if constexpr (kFence) {
+        sids[i] = a.sorted[min(slot, row_end - 1)];
+        if (slot >= row_end) sids[i] = a.num_valid;
+      } else {
+        sids[i] = a.sorted[slot];
+      }
+    }
   }
   float routed[C::IT];  // routed weight of the lane's pair in each token tile (all fetched before the first store)
 #pragma unroll
@@ -291,10 +306,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
     int f;
     if constexpr (EPI == EPI_SILU) {
       constexpr int HJ = C::JF / 2;
-      const int fl = pid_f * (BF / 2) + wf * (C::TF / 2) + (j % HJ) * C::TILE + g * 8 + kgrp * 4 + r;
+      const int fl = f0 + wf * (C::TF / 2) + (j % HJ) * C::TILE + g * 8 + kgrp * 4 + r;
       f = (j / HJ) * a.N + (fl < a.N ? fl : a.N - 1);
     } else {
-      const int fl = pid_f * BF + wf * C::TF + j * C::TILE + g * 8 + kgrp * 4 + r;
+      const int fl = f0 + wf * C::TF + j * C::TILE + g * 8 + kgrp * 4 + r;
       f = fl < a.N ? fl : a.N - 1;
     }
     return wsc[f];
@@ -315,12 +330,12 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
 #pragma unroll
     for (int i = 0; i < C::IT; ++i) {
       if (a.top_k > 0) xscale[i] = sids[i] < a.num_valid ? a.x_scale[sids[i] / a.top_k] : 1.f;
-      else xscale[i] = a.x_scale[pid_t * BT + wt * C::TT + i * C::TILE + frow];
+      else xscale[i] = a.x_scale[kFence ? min(slot0 + wt * C::TT + i * C::TILE + frow, row_end - 1) : slot0 + wt * C::TT + i * C::TILE + frow];
     }
   }
 #pragma unroll
   for (int i = 0; i < C::IT; ++i) {
-    const int slot = pid_t * BT + wt * C::TT + i * C::TILE + frow;
+    const int slot = slot0 + wt * C::TT + i * C::TILE + frow;
     const int sid = sids[i];
     const float xs = xscale[i];
     if constexpr (EPI == EPI_SILU) {
@@ -328,10 +343,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
       out_t* orow = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot) * a.ldo;
 #pragma unroll
       for (int j = 0; j < HJ; ++j) {
-        const AccT ga = AG ? acc_fetch(acc[j][i]) : acc[j][i], ua = AG ? acc_fetch(acc[j + HJ][i]) : acc[j + HJ][i];
+        const AccT ga = i < AG ? acc_fetch(acc[j][i]) : acc[j][i], ua = i < AG ? acc_fetch(acc[j + HJ][i]) : acc[j + HJ][i];
 #pragma unroll
         for (int g = 0; g < GROUPS; ++g) {
-          const int f = pid_f * (BF / 2) + wf * (C::TF / 2) + j * C::TILE + g * 8 + kgrp * 4;
+          const int f = f0 + wf * (C::TF / 2) + j * C::TILE + g * 8 + kgrp * 4;
           out4 o;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -342,6 +357,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
             }
             o[r] = static_cast<out_t>(silu(gv) * uv);
           }
+          if (kFence && slot >= row_end) continue;
           if (f + 3 < a.N) *reinterpret_cast<out4*>(orow + f) = o;
           else
             for (int r = 0; r < 4; ++r)
@@ -354,10 +370,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
         const float rw = routed[i] * xs;
 #pragma unroll
         for (int j = 0; j < C::JF; ++j) {
-          const AccT ca = AG ? acc_fetch(acc[j][i]) : acc[j][i];
+          const AccT ca = i < AG ? acc_fetch(acc[j][i]) : acc[j][i];
 #pragma unroll
           for (int g = 0; g < GROUPS; ++g) {
-            const int f = pid_f * BF + wf * C::TF + j * C::TILE + g * 8 + kgrp * 4;
+            const int f = f0 + wf * C::TF + j * C::TILE + g * 8 + kgrp * 4;
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -753,7 +769,7 @@ _Pragma("unroll") \
 #undef FR_XD
 #undef FR_WD
 
-  gemm_epilogue<T, C, EPI>(a, acc, pid_t, pid_f, expert, split, wt, wf, frow, kgrp);
+  gemm_epilogue<T, C, EPI>(a, acc, pid_t * BT, pid_f * (EPI == EPI_SILU ? BF / 2 : BF), expert, split, wt, wf, frow, kgrp);
 }
 
 template <typename T, typename C, int EPI>

@@ -41,7 +41,8 @@ struct XcdSchedule {
 // kernel streams every weight tile once from HBM, and there an XCD that stays inside one expert's weights is
 // faster (256 tokens: 357 against 412 us for the gate/up GEMM), so the rule follows the blocks per expert.
 __device__ __forceinline__ bool schedule_by_rounds(int token_blocks, int num_experts) { return 2 * token_blocks >= 5 * num_experts; }
-__device__ __forceinline__ XcdSchedule xcd_schedule(int total, int nper, int xcd, int k_tiles, bool split_tail, bool by_rounds) {
+// tail_units: slice buffers per XCD.
+__device__ __forceinline__ XcdSchedule xcd_schedule(int total, int nper, int xcd, int k_tiles, bool split_tail, bool by_rounds, int tail_units) {
   XcdSchedule s;
   if (by_rounds) {
     const int grid = nper * 8;
@@ -63,7 +64,7 @@ __device__ __forceinline__ XcdSchedule xcd_schedule(int total, int nper, int xcd
     // fix-up's: one fp32 tile written and read back per slice plus a launch, in units of
     // about a twelfth of a K tile's time (measured: 10 tiles in 3 slices of 21 K tiles each
     // break even or gain, 6 tiles in 5 slices of 45 gain a fifth of the kernel's time).
-    const int sl = min(min(nper / s.rest, k_tiles / kTailMinSlice), kTailMaxSplit);
+    const int sl = min(min(min(nper, tail_units) / s.rest, k_tiles / kTailMinSlice), kTailMaxSplit);
     if (sl >= 2 && k_tiles * (7 * sl - 10) >= 3 * sl * (s.rest * sl + 10)) s.slices = sl;
   }
   return s;
@@ -117,19 +118,13 @@ __device__ __forceinline__ void expert_block_offsets(const GemmArgs& a, int nt, 
     if (a.expert_ids[b] < a.expert_ids[b - 1]) off[kMaxExperts + 1] = 1;
   __syncthreads();
 }
-// A tile's place among the tiles that share its weight tile: the `count` token blocks of its chunk, of which it
-// is number `index` (1 and 0 without a walk table).
-struct TileShare {
-  int count, index;
-};
 __device__ __forceinline__ void tile_coords(const GemmArgs& a, const int* off, int lin, int& pid_t, int& pid_f,
-                                            int& expert, TileShare* share = nullptr) {
+                                            int& expert) {
   const int F = a.num_f_tiles;
   if (off[kMaxExperts + 1]) {
     pid_t = lin / F;
     pid_f = lin % F;
     expert = a.expert_ids[pid_t];
-    if (share) *share = TileShare{1, 0};
     return;
   }
   expert = a.expert_ids[lin / F];  // lin / F is one of the expert's blocks: its tiles are [off[e] * F, off[e + 1] * F)
@@ -152,7 +147,6 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& a, const int* off, i
   }
   pid_t = start + q % gsz;
   pid_f = q / gsz;
-  if (share) *share = TileShare{gsz, q % gsz};
 }
 // Tile column of accumulator tile j of feature wavefront wf (= row of the weight tile in LDS).
 template <typename C, int EPI>
@@ -165,7 +159,7 @@ __device__ __forceinline__ int acc_tile_col(int wf, int j) {
   }
 }
 // fp32 accumulators of one K slice, as they are, to the slice's [BT][BF] buffer
-template <typename C, int EPI, bool AG = false, typename AccT>
+template <typename C, int EPI, int AG = 0, typename AccT>
 __device__ __forceinline__ void tail_store(float* tile, AccT (&acc)[C::JF][C::IT], int wt, int wf, int frow, int kgrp) {
   constexpr int GROUPS = ((C::TILE == 32) ? 16 : 4) / 4;
 #pragma unroll
@@ -173,12 +167,12 @@ __device__ __forceinline__ void tail_store(float* tile, AccT (&acc)[C::JF][C::IT
     float* row = tile + (wt * C::TT + i * C::TILE + frow) * C::BF;
 #pragma unroll
     for (int j = 0; j < C::JF; ++j) {
-      const AccT ca = AG ? acc_fetch(acc[j][i]) : acc[j][i];
+      const AccT ca = i < AG ? acc_fetch(acc[j][i]) : acc[j][i];
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g) {
         const f32x4 o = {ca[g * 4 + 0], ca[g * 4 + 1], ca[g * 4 + 2], ca[g * 4 + 3]};
         *reinterpret_cast<f32x4*>(row + acc_tile_col<C, EPI>(wf, j) + g * 8 + kgrp * 4) = o;
-        if constexpr (AG) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (AG > 0) __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
@@ -237,7 +231,7 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   const int split = blockIdx.y;
   const int k0 = split * a.k_per_split;
   const int k_all = min(a.k_per_split, a.K - k0) / BK;  // K tiles of a whole unit, >= S + 2 (checked by the launcher)
-  const XcdSchedule xs = xcd_schedule(total, nper, xcd, k_all, a.tail_ws != nullptr, schedule_by_rounds(nt, a.num_experts));
+  const XcdSchedule xs = xcd_schedule(total, nper, xcd, k_all, a.tail_ws != nullptr, schedule_by_rounds(nt, a.num_experts), nper);
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
   if (n_units == 0) return;
   __shared__ int expert_off[kWalkTable];
@@ -516,7 +510,7 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
       FR_KTILE(ISS_, false, A, 0, true, 0)                                                                 \
     }                                                                                                      \
     FR_STAMP(1)                                                                                            \
-    if (tu < 0) gemm_epilogue<T, C, EPI, HOIST>(a, acc, pid_t, pid_f, expert, split, wt, wf, frow, kgrp);         \
+    if (tu < 0) gemm_epilogue<T, C, EPI, HOIST>(a, acc, pid_t * BT, pid_f * (EPI == EPI_SILU ? BF / 2 : BF), expert, split, wt, wf, frow, kgrp);         \
     else tail_store<C, EPI>(a.tail_ws + static_cast<int64_t>(xcd * nper + tu) * (BT * BF), acc, wt, wf, frow, kgrp); \
   }
   // Fill of the ring with the first S K tiles of set A and the first fragments.
@@ -594,46 +588,35 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
 // Grid: 8 XCDs x nper/2 tiles (a split tail has at most that many) x BT/32 row groups; blocks
 // without a split tile leave at once.  nper = workgroups per XCD of the GEMM launch.
 constexpr int kFixupRows = 32;
-template <typename T, typename C, int EPI>
-__global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int nper) {
+// kFixupRows rows [r0, + kFixupRows) of a tile whose `slices` slice buffers ([rows][BF] fp32) lie `slice_stride` floats apart
+// from `first` on; slot0, f0: the tile's first sorted slot and output column.
+template <typename T, int BF, int EPI>
+__device__ __forceinline__ void fixup_rows(const GemmArgs& a, const float* first, int64_t slice_stride, int slices, int slot0, int r0, int f0, int expert) {
   typedef Elem<T> E;
   typedef typename E::out_t out_t;
   typedef typename E::out4 out4;
-  constexpr int BT = C::BT, BF = C::BF, BK = C::BKB / static_cast<int>(sizeof(T));
   constexpr int COLS = (EPI == EPI_SILU) ? BF / 2 : BF;  // output columns of a tile
   constexpr int CG = COLS / 4, RPP = 256 / CG;           // 4-column groups per row, rows per pass
-  static_assert(256 % CG == 0 && kFixupRows % RPP == 0 && BT % kFixupRows == 0, "fix-up thread map");
-  constexpr int BPT = BT / kFixupRows;
-  const int half = nper / 2;
-  const int xcd = blockIdx.x / (half * BPT), t = (blockIdx.x / BPT) % half, rb = blockIdx.x % BPT;
-  const int nt = min(a.npost[0] / BT, a.num_t_blocks);
-  const XcdSchedule xs = xcd_schedule(nt * a.num_f_tiles, nper, xcd, a.K / BK, true, schedule_by_rounds(nt, a.num_experts));
-  if (xs.slices < 2 || t >= xs.rest) return;
-  __shared__ int expert_off[kWalkTable];
-  expert_block_offsets(a, nt, expert_off, threadIdx.x, 256);
-  int pid_t, pid_f, expert;
-  tile_coords(a, expert_off, xs.tail_base + t, pid_t, pid_f, expert);
+  static_assert(256 % CG == 0 && kFixupRows % RPP == 0, "fix-up thread map");
   const float* wsc = nullptr;
   if constexpr (E::SCALED) wsc = a.w_scale + static_cast<int64_t>(expert) * a.w_rows;
-  const float* first = a.tail_ws + static_cast<int64_t>(xcd * nper + t) * (BT * BF);
-  const int64_t slice_stride = static_cast<int64_t>(xs.rest) * (BT * BF);
   const int cg = threadIdx.x % CG;
   // Memory bound (every slice read once): the rows of a thread are taken together, slice by slice, so that all their loads
   // are in flight at once.  A padding row's address is that of the tile's first row (one line for all of them).
   constexpr int P = kFixupRows / RPP;  // rows per thread
-  const int row0 = rb * kFixupRows + threadIdx.x / CG;
+  const int row0 = r0 + threadIdx.x / CG;
   if constexpr (EPI != EPI_SILU) {
     int sid[P];
     const float* src[P];
     f32x4 sum[P];
 #pragma unroll
-    for (int p = 0; p < P; ++p) sid[p] = a.sorted[pid_t * BT + row0 + p * RPP];
+    for (int p = 0; p < P; ++p) sid[p] = a.sorted[slot0 + row0 + p * RPP];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       src[p] = first + (sid[p] < a.num_valid ? (row0 + p * RPP) * BF : 0) + cg * 4;
       sum[p] = *reinterpret_cast<const f32x4*>(src[p]);
     }
-    for (int s = 1; s < xs.slices; ++s)
+    for (int s = 1; s < slices; ++s)
 #pragma unroll
       for (int p = 0; p < P; ++p) sum[p] += *reinterpret_cast<const f32x4*>(src[p] + s * slice_stride);
 #pragma unroll
@@ -641,11 +624,11 @@ __global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int n
       if (sid[p] >= a.num_valid) continue;
       float rw = a.mul_weight ? a.topk_w[sid[p]] : 1.f;
       if constexpr (E::SCALED) {  // per-row scales of both fp8 operands
-        rw *= a.top_k > 0 ? a.x_scale[sid[p] / a.top_k] : a.x_scale[pid_t * BT + row0 + p * RPP];
-        const f32x4 ws = *reinterpret_cast<const f32x4*>(wsc + pid_f * BF + cg * 4);
+        rw *= a.top_k > 0 ? a.x_scale[sid[p] / a.top_k] : a.x_scale[slot0 + row0 + p * RPP];
+        const f32x4 ws = *reinterpret_cast<const f32x4*>(wsc + f0 + cg * 4);
         sum[p] *= ws;
       }
-      const int64_t at = static_cast<int64_t>(sid[p]) * a.ldo + pid_f * BF + cg * 4;
+      const int64_t at = static_cast<int64_t>(sid[p]) * a.ldo + f0 + cg * 4;
       if constexpr (EPI == EPI_DOWN) {
         const f32x4 o = {sum[p][0] * rw, sum[p][1] * rw, sum[p][2] * rw, sum[p][3] * rw};
         *reinterpret_cast<f32x4*>(static_cast<float*>(a.out) + at) = o;
@@ -653,7 +636,7 @@ __global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int n
         out4 o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = static_cast<out_t>(sum[p][r] * rw);
-        if (a.add_div) atomic_add4(static_cast<out_t*>(a.out) + static_cast<int64_t>(sid[p] / a.add_div) * a.ldo + pid_f * BF + cg * 4, o);
+        if (a.add_div) atomic_add4(static_cast<out_t*>(a.out) + static_cast<int64_t>(sid[p] / a.add_div) * a.ldo + f0 + cg * 4, o);
         else *reinterpret_cast<out4*>(static_cast<out_t*>(a.out) + at) = o;
       }
     }
@@ -665,7 +648,7 @@ __global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int n
       g[p] = *reinterpret_cast<const f32x4*>(src);
       u[p] = *reinterpret_cast<const f32x4*>(src + BF / 2);
     }
-    for (int s = 1; s < xs.slices; ++s)
+    for (int s = 1; s < slices; ++s)
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         const float* src = first + s * slice_stride + (row0 + p * RPP) * BF + cg * 4;
@@ -674,22 +657,40 @@ __global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int n
       }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      const int slot = pid_t * BT + row0 + p * RPP;
+      const int slot = slot0 + row0 + p * RPP;
       if constexpr (E::SCALED) {
         const int sid = a.sorted[slot];
         const float xsc = a.top_k > 0 ? (sid < a.num_valid ? a.x_scale[sid / a.top_k] : 1.f) : a.x_scale[slot];
-        const f32x4 gs = *reinterpret_cast<const f32x4*>(wsc + pid_f * (BF / 2) + cg * 4);
-        const f32x4 us = *reinterpret_cast<const f32x4*>(wsc + a.N + pid_f * (BF / 2) + cg * 4);
+        const f32x4 gs = *reinterpret_cast<const f32x4*>(wsc + f0 + cg * 4);
+        const f32x4 us = *reinterpret_cast<const f32x4*>(wsc + a.N + f0 + cg * 4);
         g[p] *= gs * xsc;
         u[p] *= us * xsc;
       }
       out4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = static_cast<out_t>(silu(g[p][r]) * u[p][r]);
-      out_t* orow = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot) * a.ldo + pid_f * (BF / 2) + cg * 4;
+      out_t* orow = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot) * a.ldo + f0 + cg * 4;
       *reinterpret_cast<out4*>(orow) = o;
     }
   }
+}
+
+template <typename T, typename C, int EPI>
+__global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int nper) {
+  constexpr int BT = C::BT, BF = C::BF, BK = C::BKB / static_cast<int>(sizeof(T));
+  constexpr int BPT = BT / kFixupRows;
+  static_assert(BT % kFixupRows == 0, "whole groups of rows");
+  const int half = nper / 2;
+  const int xcd = blockIdx.x / (half * BPT), t = (blockIdx.x / BPT) % half, rb = blockIdx.x % BPT;
+  const int nt = min(a.npost[0] / BT, a.num_t_blocks);
+  const XcdSchedule xs = xcd_schedule(nt * a.num_f_tiles, nper, xcd, a.K / BK, true, schedule_by_rounds(nt, a.num_experts), nper);
+  if (xs.slices < 2 || t >= xs.rest) return;
+  __shared__ int expert_off[kWalkTable];
+  expert_block_offsets(a, nt, expert_off, threadIdx.x, 256);
+  int pid_t, pid_f, expert;
+  tile_coords(a, expert_off, xs.tail_base + t, pid_t, pid_f, expert);
+  fixup_rows<T, BF, EPI>(a, a.tail_ws + static_cast<int64_t>(xcd * nper + t) * (BT * BF), static_cast<int64_t>(xs.rest) * (BT * BF), xs.slices,
+                         pid_t * BT, rb * kFixupRows, pid_f * (EPI == EPI_SILU ? BF / 2 : BF), expert);
 }
 
 // Workgroups resident at once on the current device (a multiple of 8, one share per XCD).

@@ -1,151 +1,380 @@
-// Persistent grouped GEMM with ONE wavefront per SIMD: 256 sorted slots x 256 features per workgroup, four
-// wavefronts of 128 x 128 each, 16x16x32 MFMAs (2-byte operands) or 32x32x64 MFMAs (fp8).
+// Persistent grouped GEMM with ONE wavefront per SIMD: up to 288 sorted slots x 256 features per workgroup, 16x16x32
+// MFMAs (2-byte operands) or 32x32x64 MFMAs (fp8).
 //
 // Why.  In the eight-wavefront tiles a wavefront owns 128 x 64 outputs and reads twelve operand fragments from
 // LDS for thirty-two MFMAs; with 128 x 128 per wavefront it reads sixteen for sixty-four, a third less LDS traffic
 // for the same arithmetic and half as many wavefronts issuing instructions, and the part's clock under MFMA load
-// follows the energy a flop costs.  The 256 accumulator registers of a lane live in the accumulation half of the
-// register file (one wavefront per SIMD has 512 registers per lane); the ordinary half holds two fragment buffers
-// of one K-step each (128 registers) and the two address sets of the persistent hand-off.
+// follows the energy a flop costs.  The accumulators live in the accumulation half of the register file (one
+// wavefront per SIMD has 512 registers per lane), those of a 288-row tile's last token tiles in the ordinary half.
+//
+// Tile heights.  A tile is 1 to 9 units of 32 token rows: an expert's run of slots is cut into as few tiles as 288 rows
+// allow (quad_tiles, quad_walk, quad_tile_at), whatever the routing block.  No tile crosses into the padding behind a
+// run: an expert with 1030 pairs is multiplied as 1056 rows in four tiles where 256-row blocks made it 1280 rows in
+// five.  Layer in us, 8 experts, H = 4096, F = 14336, top-2, whole and half blocks of 256 / runs: 2048 tokens 1374 / 1200,
+// 3000 1814 / 1713, 4096 2325 / 2174, 5800 3154 / 3107, 16384 8528 / 8356; fp8 2048 769 / 680, 3100 1077 / 1007, 2500
+// 900 / 904; H = 2048, F = 1408, 64 experts, top-6, Zipf-skewed 7000 816 / 799, 8192 930 / 937.  Where the blocks had no
+// padding to lose (every expert a multiple of 256) gate/up is even and the down projection 1.5 % slower.  A K loop exists per height (kernel code per height, chosen per work unit); the height of the next
+// unit is known a tile ahead, and the hand-over always loads 288 rows' worth of addresses (rows beyond the tile are
+// outside the buffer resource and fetch nothing), so any height may follow any other.
 //
 // Stream.  With a single wavefront per SIMD nobody fills the issue slots a burst of loads or a wait leaves, so the
-// wavefront's own instruction stream is even: a K tile of 64 elements is two K-steps of 64 MFMAs; during a K-step
-// the sixteen fragments of the following K-step are read, one after every third or fourth MFMA, into the other
-// fragment buffer; the one barrier per K tile sits between its two K-steps, where every fragment of the tile has
-// been read: the tile's ring slot is free from there on and takes the sixteen loads per wavefront of the K tile
-// after next, one after every fourth MFMA of the second K-step, which leaves them the first K-step of the next
-// K tile to land.
+// wavefront's own instruction stream is even: a K tile of 128 bytes per row is two K-steps; the one barrier per K tile
+// sits between them, where every fragment of the tile has been read: the tile's ring slot is free from there on and takes
+// the loads of the K tile after next, spread over the second K-step, which leaves them the first K-step of the next K tile
+// to land.  The operand the MFMAs walk slowest (2-byte: the eight weight fragments; fp8: the token fragments) has one
+// register set, each fragment read again behind its last MFMA of the K-step, except the last ones, whose reads would end
+// up right before the barrier; the other operand and those last ones have two sets.
 //
 // What such a stream cannot hide is a load that misses L2: the ring has two slots, so at most one K tile per
 // workgroup is in flight, and a wavefront that finds the memory pipeline backed up stalls at the issue of its
 // next load with its MFMAs behind it.  Hence the L2 touch: the workgroups an XCD runs at one time share their
-// operand tiles (the token blocks of one chunk share a weight tile, the feature tiles of one token block its
+// operand tiles (the token tiles of one chunk share a weight tile, the feature tiles of one token tile its
 // rows), and each of them asks for its share of the rows of a K tile several K tiles ahead - one dword per
 // 128-byte row piece, into a sink in LDS - so that the tile loads proper find their lines in L2.
 //
-// Half tiles.  A block whose upper 128 slots are all padding (the last block of every other expert) is multiplied
-// as 128 rows x 256 features with the FEATURES split four ways over the wavefronts (128 x 64 each): half the MFMAs
-// per K-step, 12 loads per K tile.  Both forms of the K loop exist for every place in the persistent walk; the kind
-// of the next unit is known a tile ahead, and the hand-over always loads a whole tile's first two K tiles, so any
-// kind may follow any other.
-//
-// Same tile walk, tail split, LDS swizzle, epilogues and fix-up kernel as moe_gemm_persistent_kernel; the result
-// is bit-identical to the eight-wavefront kernels on the same MFMA shape (same K order per accumulator).
-//
-// Measurement switches (compile time, -D): FQ_TOUCH=0 no L2 touch, FQ_HALF=0 no half tiles, FQ_AHEAD=n touch
-// distance in K tiles, FQ_XSHARE=n ways the token rows' touch is shared; results stay correct with all of them.
+// Same tail split, LDS swizzle and epilogues as moe_gemm_persistent_kernel; the result is bit-identical to the
+// eight-wavefront kernels on the same MFMA shape (same K order per accumulator).
 #pragma once
 #include "moe_gemm_persistent.h"
 
 namespace fr {
 
-// 2-byte operands: 16x16x32 MFMAs (8 x 8 accumulator tiles of 4 registers per wavefront); fp8: 32x32x64 (4 x 4 tiles of
-// 16 registers).  Either way a K tile of 128 bytes per row is two K-steps, a K-step's fragments are 16 reads of 16
-// bytes per lane and 64 registers, and a wavefront issues 16 tile loads per K tile.
-template <typename T> struct QuadTile { static constexpr int kTile = sizeof(T) == 1 ? 32 : 16; };
-template <typename T> using QuadCfg = Cfg<256, 256, 128, 2, 2, QuadTile<T>::kTile, 1, 2, 0, 1>;
-// output geometry of a half tile: 128 rows, a quarter of the features per wavefront
-template <typename T> using QuadHalfCfg = Cfg<128, 256, 128, 1, 4, QuadTile<T>::kTile, 1, 2, 0, 1>;
-constexpr int kQuadMinTiles = 8;    // K tiles per work unit, at least (two peeled at each end, the touch distance)
-#ifndef FQ_AHEAD
-#define FQ_AHEAD 3
-#endif
-constexpr int kQuadTouchAhead = FQ_AHEAD;  // K tiles between a touch and the tile loads of the same rows
-constexpr int kQuadSink = 1024;     // bytes of LDS the touches land in (256 per wavefront)
+constexpr int kUnitRows = 32;   // a tile's height in units of
+constexpr int kMaxUnits = 9;
+// 2 x 2 wavefronts of (half the rows) x 128 features; 16x16x32 MFMAs, fp8 32x32x64.  fp8 tiles of an odd number of units: 1 x 4
+// wavefronts of (all rows) x 64 features, a fifth more LDS reads per MFMA (6000 tokens with 1 x 4 throughout: down
+// projection 567 against 548 us) but no unit of padding.
+template <typename T, int UN>
+using QuadCfg = typename std::conditional<sizeof(T) == 2, Cfg<kUnitRows * UN, 256, 128, 2, 2, 16, 1, 2, 0, 1>,
+                                          typename std::conditional<UN % 2 == 0, Cfg<kUnitRows * UN, 256, 128, 2, 2, UN % 2 == 0 ? 32 : 16, 1, 2, 0, 1>,
+                                                                    Cfg<kUnitRows * UN, 256, 128, 1, 4, 32, 1, 2, 0, 1>>::type>::type;
+constexpr int kQuadMinTiles = 8;       // K tiles per work unit, at least (one peeled at its start, five at its end)
+constexpr int kQuadXShare = 4;         // ways the touch of a tile's token rows is shared, at most
+constexpr int kQuadSink = 1024;        // bytes of LDS the touches land in (256 per wavefront)
+constexpr int kTileCost = 26;          // what a tile costs besides its height, in tenths of a unit (weight rows, barriers, epilogue)
+constexpr int kQuadRing = 2 * (kUnitRows * kMaxUnits + 256) * 128;
+// Slice buffers of the cut last round, per XCD of 32 workgroups: 32 of 256 x 256 fp32 or, with 288-row tiles, 28 of 288 x 256.
+// What the fix-up launch needs to know about a cut tile is left next to them (QuadCut), in the scratch itself where the
+// caller has no other place for it: then there are 31 buffers of 256 rows.
+constexpr int kQuadTallBuffers = 28;
+__device__ __forceinline__ int quad_buffer_rows(int tallest) { return tallest > 8 ? kUnitRows * kMaxUnits : 256; }
+__device__ __forceinline__ int quad_buffers(const GemmArgs& a, int tallest) { return tallest > 8 ? kQuadTallBuffers : a.tail_buffers; }
+struct QuadCut {
+  int row0, units, f, expert, slices, rest, buffers, buffer_rows;  // slices 0: tile is not cut
+};
+static_assert(sizeof(QuadCut) * kTailUnits <= kTailDescBytes, "a tile per workgroup");
+static_assert(8 * kQuadTallBuffers * kUnitRows * kMaxUnits * 256 * 4 + kTailDescBytes <= kTailUnits * 256 * 256 * 4 &&
+                  8 * 31 * 256 * 256 * 4 + kTailDescBytes <= kTailUnits * 256 * 256 * 4, "fits the scratch");
 
-#ifndef FQ_TAIL_LONG_K  // measurement switches of the host side: K tiles from which a K loop counts as long, and
-#define FQ_TAIL_LONG_K 112
-#endif
-#ifndef FQ_TAIL_ROUNDS_SHORT  // whole rounds after which a shorter one stops splitting its last round
-#define FQ_TAIL_ROUNDS_SHORT 8
-#endif
-#ifndef FQ_XSHARE
-#define FQ_XSHARE 4
-#endif
-#ifndef FQ_HALF
-#define FQ_HALF 1
-#endif
-#ifndef FQ_TOUCH
-#define FQ_TOUCH 1
+// Tiles an expert's run of `units` units is cut into when a tile may have `limit` of them: as few as fit, of heights as equal
+// as units allow.  With the largest limit a multiple of 256 rows keeps 256-row tiles.
+__device__ __forceinline__ int quad_tiles(int units, int limit) {
+  return limit == kMaxUnits && units % 8 == 0 ? units / 8 : (units + limit - 1) / limit;
+}
+
+// Walk table: off[e] = first routing block of expert e, units[e] = units of its run up to the last one that holds a
+// pair, tiles[e] = tiles of the experts before e.  off[kMaxExperts + 1]: the blocks are in no order (legal for the op-level
+// GEMM): every block is a tile of its own, tiles and units are not written.
+struct QuadWalk {
+  int off[kWalkTable], units[kWalkTable], tiles[kWalkTable];
+  int tallest;  // units of the tallest tile
+};
+// all 256 threads; `block` rows per routing block (a multiple of 32, at most 256), nt > 0 blocks
+__device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int block, int nt, int tid, int workgroups) {
+  expert_block_offsets(a, nt, w.off, tid, 256);
+  if (w.off[kMaxExperts + 1]) {
+    if (tid == 0) w.tallest = block / kUnitRows;
+    __syncthreads();
+    return;
+  }
+  const int E = a.num_experts, lane = tid & 63, wave = tid >> 6;
+  // the last block of every run: its last 32-slot group with a pair (sixteen experts' ids in flight per wavefront)
+  constexpr int XE = 16;
+  for (int e0 = wave; e0 < E; e0 += 4 * XE) {
+    int id[XE][4];
+#pragma unroll
+    for (int x = 0; x < XE; ++x) {
+      if (e0 + 4 * x >= E) break;
+      const int last = max(w.off[e0 + 4 * x + 1] - 1, 0);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) id[x][p] = a.sorted[last * block + min(p * kWave + lane, block - 1)];
+    }
+#pragma unroll
+    for (int x = 0; x < XE; ++x) {
+      const int e = e0 + 4 * x;
+      if (e >= E) break;
+      int groups = 0;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const unsigned long long b = __ballot(p * kWave + lane < block && id[x][p] < a.num_valid);
+        if (b) groups = 2 * p + (b >> 32 ? 2 : 1);
+      }
+      if (lane == 0) {
+        const int len = w.off[e + 1] - w.off[e];
+        w.units[e] = len > 0 ? (len - 1) * (block / kUnitRows) + groups : 0;
+      }
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // The limit of a tile's height.  Tall tiles cost least per row, but a launch of few rounds is over when its busiest
+    // workgroup is: a round takes as long as kTileCost + height, and the tiles behind the whole rounds as long as a round
+    // unless they can be cut along K.  (Down projection, 8 experts x 16 feature tiles: with 8 or 9 units each, tiles of 8 or 9
+    // leave half the chip idle and 4 and 5 fill it; 33 units are best in four tiles, not five.)
+    constexpr int NL = 6;  // limits 9 to 4
+    int count[NL] = {}, high[NL] = {};
+    for (int e0 = 0; e0 < E; e0 += kWave) {
+      const int u = e0 + lane < E ? w.units[e0 + lane] : 0;
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {
+        const int c = quad_tiles(u, kMaxUnits - l);
+        count[l] += c;
+        high[l] = max(high[l], c ? (u + c - 1) / c : 0);
+      }
+    }
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1)
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {  // the limits' chains of exchanges overlap
+        count[l] += __shfl_xor(count[l], d);
+        high[l] = max(high[l], __shfl_xor(high[l], d));
+      }
+    unsigned cost = ~0u;  // lane l: of limit 9 - l
+    {
+      int n = 0, tall = 0;
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {
+        n = lane == l ? count[l] : n;
+        tall = lane == l ? high[l] : tall;
+      }
+      const unsigned total = n * a.num_f_tiles, whole = total / static_cast<unsigned>(workgroups), rest = total - whole * workgroups;
+      const unsigned tile = kTileCost + 10 * tall, cuts = 8 * quad_buffers(a, tall) / max(rest, 1u);
+      const unsigned slices = a.tail_ws ? min(cuts, static_cast<unsigned>(kTailMaxSplit)) : 1u;
+      if (lane < NL) cost = 32 * whole * tile + (rest == 0 ? 0 : slices < 2 ? 32 * tile : 32 * tile / slices + 3 * tile);
+    }
+    int best = kMaxUnits;
+    unsigned least = __builtin_amdgcn_readlane(cost, 0);
+#pragma unroll
+    for (int l = 1; l < NL; ++l) {  // a lower limit has to be 3 % cheaper
+      const unsigned c = __builtin_amdgcn_readlane(cost, l);
+      if (c < least - least / 32) {
+        least = c;
+        best = kMaxUnits - l;
+      }
+    }
+    int base = 0, tall = 0;
+    for (int e0 = 0; e0 <= E; e0 += kWave) {
+      const int e = e0 + lane, u = e < E ? w.units[e] : 0, c = e < E ? quad_tiles(u, best) : 0;
+      int s = c;
+#pragma unroll
+      for (int d = 1; d < kWave; d <<= 1) {
+        const int up = __shfl_up(s, d);
+        if (lane >= d) s += up;
+      }
+      if (e <= E) w.tiles[e] = base + s - c;
+      base += __shfl(s, kWave - 1);
+      for (int h = tall + 1; h <= kMaxUnits; ++h)
+        if (__any(c && (u + c - 1) / c >= h)) tall = h;
+    }
+    if (lane == 0) w.tallest = tall;
+  }
+  __syncthreads();
+}
+
+// A work unit: an output tile, or a K slice of one.
+struct QuadUnit {
+  int row0, units;    // first slot, height
+  int f, expert;      // feature tile, expert
+  int kb, kn, tu;     // first K tile, K tiles, slice buffer (-1: a whole tile)
+  int share;          // tiles of its chunk (which share its weight tile) and its index among them: count << 16 | index
+};
+constexpr int kUnitTable = 64;  // units a wavefront works out at a time, one per lane
+
+// Tile number lin of the walk: experts in order, an expert's run in chunks of at most group_t tiles, a chunk tile-fastest
+// over all feature tiles (see tile_coords).  even_heights: all tiles
+// of an expert but the last have the mean height rounded up to even, the last what is left.
+__device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& w, int block, bool even_heights, int lin, QuadUnit& u) {
+  const int F = a.num_f_tiles, t = lin / F;
+  if (w.off[kMaxExperts + 1]) {
+    u.row0 = t * block;
+    u.units = block / kUnitRows;
+    u.f = lin - t * F;
+    u.expert = a.expert_ids[t];
+    u.share = 1 << 16;
+    return;
+  }
+  int lo = 0, hi = a.num_experts - 1;  // the last expert whose tiles start at or before t: it has some
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (w.tiles[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  const int first = w.tiles[lo], len = w.tiles[lo + 1] - first, un = w.units[lo];
+  const int chunks = (len + a.group_t - 1) / a.group_t, base = len / chunks, rem = len - base * chunks;
+  int q = lin - first * F, gsz = base + 1, start = 0;
+  const int big = rem * gsz * F;  // the first rem chunks hold one tile more
+  if (q >= big) {
+    q -= big;
+    start = rem * gsz;
+    gsz = base;
+  }
+  const int c = q / (gsz * F);
+  q -= c * gsz * F;
+  start += c * gsz;
+  u.f = q / gsz;
+  const int index = q - u.f * gsz, b = start + index;
+  const int even = (un + 2 * len - 1) / (2 * len) * 2;  // the mean height, rounded up to even
+  if (even_heights && un <= 8 * len + 1 && min(even, 8) * (len - 1) < un) {
+    const int h = min(even, 8);
+    u.row0 = w.off[lo] * block + b * h * kUnitRows;
+    u.units = b < len - 1 ? h : un - h * (len - 1);
+  } else {
+    const int ub = un / len, ur = un - ub * len;  // the first ur tiles are one unit taller
+    u.row0 = w.off[lo] * block + (b * ub + min(b, ur)) * kUnitRows;
+    u.units = ub + (b < ur ? 1 : 0);
+  }
+  u.expert = lo;
+  u.share = gsz << 16 | index;
+}
+
+// One MFMA, written out so that an accumulator stays in the registers it has: those of the first kQuadAgpr token tiles in
+// the accumulation half of the register file (all 256 of them in a tile of 256 rows or more), the rest in the ordinary
+// half.  Left to the compiler's three-operand form, with no register of that half to spare, accumulators wandered through
+// ordinary registers around the K loop and address registers were spilled inside it (288 rows, 4096 tokens: down projection
+// 906 against 740 us).  What the compiler does not know about these instructions: an accumulator may be read by another
+// instruction 19 wait states after its last MFMA (run_unit's s_nop); MFMAs on one accumulator are as many MFMAs apart as
+// a K-step has.
+constexpr int kQuadAgpr = 8;
+#if defined(__HIP_DEVICE_COMPILE__)
+#define FQ_MFMA(name_, reg_)                                                                                     \
+  if constexpr (FIRST) asm volatile(name_ " %0, %1, %2, 0" : "=&" reg_(acc) : "v"(wf), "v"(xf));                 \
+  else asm volatile(name_ " %0, %1, %2, %0" : "+" reg_(acc) : "v"(wf), "v"(xf));
+template <typename T, bool AGPR, bool FIRST, typename AccT>
+__device__ __forceinline__ void quad_mfma(AccT& acc, const u32x4* w, const u32x4* x) {
+  if constexpr (sizeof(T) == 1) {
+    const i32x8 wf = Elem<T>::join(w), xf = Elem<T>::join(x);
+    if constexpr (AGPR) { FQ_MFMA("v_mfma_f32_32x32x64_f8f6f4", "a") } else { FQ_MFMA("v_mfma_f32_32x32x64_f8f6f4", "v") }
+  } else {
+    const u32x4 wf = w[0], xf = x[0];
+    if constexpr (std::is_same<T, bf16_t>::value) {
+      if constexpr (AGPR) { FQ_MFMA("v_mfma_f32_16x16x32_bf16", "a") } else { FQ_MFMA("v_mfma_f32_16x16x32_bf16", "v") }
+    } else {
+      if constexpr (AGPR) { FQ_MFMA("v_mfma_f32_16x16x32_f16", "a") } else { FQ_MFMA("v_mfma_f32_16x16x32_f16", "v") }
+    }
+  }
+}
+#undef FQ_MFMA
 #endif
 
 template <typename T, int EPI>
-__global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a FR_PROF_PARAM) {
+__global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  typedef QuadCfg<T> C;
-  typedef QuadHalfCfg<T> CH;
+  typedef QuadCfg<T, kMaxUnits> CM;
   typedef Elem<T> E;
   typedef __attribute__((address_space(3))) void* lptr_t;
-  typedef typename std::conditional<C::TILE == 32, f32x16, f32x4>::type acc_t;
+  typedef typename std::conditional<CM::TILE == 32, f32x16, f32x4>::type acc_t;
   constexpr int ES = static_cast<int>(sizeof(T));
-  constexpr int BT = C::BT, BF = C::BF, CPR = C::CPR, BK = C::BKB / ES, EPC = 16 / ES, FC = E::FC;
-  constexpr int TILE = C::TILE, KG = C::KGROUPS;
-  constexpr int NF = 128 / TILE;              // fragments per operand and K-step (8, fp8: 4)
-  constexpr int NM = NF * NF;                 // MFMAs per K-step (64 of 16 cycles, fp8: 16 of 64 cycles)
-  constexpr int NW = 4, XI = 8, WI = 8, NL = XI + WI;  // tile loads per wavefront and K tile
-  constexpr int XBYTES = C::XCH * 16, WBYTES = C::WCH * 16, SLOT = XBYTES + WBYTES;  // a ring slot: X rows, then W rows
-  // Whole tile, 2-byte operands: one fragment read after every 3rd / 4th MFMA of the first / second K-step, tile
-  // load q after MFMA 2 + 4 q of the second.  fp8 has a quarter of the MFMAs, four times as long: two fragment reads
-  // after each of the first eight, one tile load after every one of the second K-step.
-  constexpr int RD0 = FC == 1 ? 3 : 1, RD1 = FC == 1 ? 4 : 1, RPS = FC;
-  constexpr int LD_POS = FC == 1 ? 2 : 0, LD_EVERY = FC == 1 ? 4 : 1;
-  static_assert(C::IT == NF && C::JF == NF && C::XIW == XI && C::WIW == WI && CPR == 8 && CPR / (KG * FC) == 2, "128 x 128 per wavefront, two K-steps per K tile");
+  constexpr int BF = CM::BF, CPR = CM::CPR, BKB = CM::BKB, BK = BKB / ES, FC = E::FC;
+  constexpr int TILE = CM::TILE, KG = CM::KGROUPS;
+  constexpr int COLS = EPI == EPI_SILU ? BF / 2 : BF;
+  constexpr int NW = 4, XI = kMaxUnits, WI = 8;        // tile loads per wavefront and K tile, at most: a load per unit of rows
+  constexpr int XBYTES = kUnitRows * kMaxUnits * BKB, SLOT = XBYTES + BF * BKB;  // a ring slot: X rows, then W rows
+  static_assert(2 * SLOT == kQuadRing && CM::WIW == WI && CM::XIW == XI && CPR == 8 && CPR / (KG * FC) == 2, "two K-steps per K tile");
 
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  __shared__ QuadWalk walk;
+  __shared__ QuadUnit unit_table[2][kUnitTable];
 
-  // ---- schedule (as in moe_gemm_persistent_kernel) -----------------------------------------
-  const int npost = a.npost[0];
-  const int nt = min(npost / BT, a.num_t_blocks);
-  const int total = nt * a.num_f_tiles;
+  // ---- schedule (as in moe_gemm_persistent_kernel, over the tiles of quad_walk) -----------------
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int nt = min(a.npost[0] / block, a.num_t_blocks);
   const int xcd = blockIdx.x & 7, nper = gridDim.x >> 3, loc = blockIdx.x >> 3;
   const int k_all = a.K / BK;
-  const XcdSchedule xs = xcd_schedule(total, nper, xcd, k_all, a.tail_ws != nullptr, schedule_by_rounds(nt, a.num_experts));
+  // fp8's even heights have the geometry with fewer LDS reads, and short K loops are better off with whole tiles and one
+  // short one than with equal ones: layer in us, equal / even, fp8 2500 tokens 926 / 894, 4878 1570 / 1515; H = 2048, F = 1408
+  // (32 and 22 K tiles), 64 experts, 8192 tokens 952 / 940, 7000 806 / 800; H = 4096, F = 14336 (64 and 224) 2300 1460 / 1495,
+  // 3000 1713 / 1733, 5800 3116 / 3142.
+  const bool even_heights = sizeof(T) == 1 || k_all <= 32;
+  int tiles = 0, tallest = 0;
+  if (nt > 0) {
+    quad_walk(a, walk, block, nt, tid, 8 * nper);
+    tiles = __builtin_amdgcn_readfirstlane(walk.off[kMaxExperts + 1] ? nt : walk.tiles[a.num_experts]);
+    tallest = __builtin_amdgcn_readfirstlane(walk.tallest);
+  }
+  const XcdSchedule xs = xcd_schedule(tiles * a.num_f_tiles, nper, xcd, k_all, a.tail_ws != nullptr,
+                                      schedule_by_rounds(tiles, a.num_experts), quad_buffers(a, tallest));
+  if (a.tail_ws != nullptr && tid == 0) {
+    QuadCut c = {};
+    if (xs.slices > 1 && loc < xs.rest) {
+      QuadUnit u;
+      quad_tile_at(a, walk, block, even_heights, xs.tail_base + loc, u);
+      c = QuadCut{u.row0, u.units, u.f, u.expert, xs.slices, xs.rest, quad_buffers(a, tallest), quad_buffer_rows(tallest)};
+    }
+    reinterpret_cast<QuadCut*>(a.tail_desc)[xcd * nper + loc] = c;
+  }
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
   if (n_units == 0) return;
-  __shared__ int expert_off[kWalkTable];
-  expert_block_offsets(a, nt, expert_off, threadIdx.x, C::NT);
 
-  const int tid = threadIdx.x, lane = tid & 63;
   const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wt = wave_u >> 1, wf = wave_u & 1;
-  const int wstep = a.w_tiled ? (C::BKB / kTileBytes) * kTilePiece : C::BKB;  // bytes from one K tile of W to the next
+  const int wstep = a.w_tiled ? (BKB / kTileBytes) * kTilePiece : BKB;  // bytes from one K tile of W to the next
   const T* X = static_cast<const T*>(a.X);
 
-#define FQ_UNIT(j_, pt_, pf_, ex_, kb_, kn_, tu_, sh_)                                         \
-  {                                                                                            \
-    int lin_;                                                                                  \
-    if ((j_) < xs.rounds) {                                                                    \
-      lin_ = xcd_round_tile(xs, nper, xcd, loc, (j_));                                         \
-      kb_ = 0; kn_ = k_all; tu_ = -1;                                                          \
-    } else {                                                                                   \
-      const int t_ = loc % xs.rest, s_ = loc / xs.rest;                                        \
-      lin_ = xs.tail_base + t_;                                                                \
-      kb_ = s_ * k_all / xs.slices;                                                            \
-      kn_ = (s_ + 1) * k_all / xs.slices - kb_;                                                \
-      tu_ = xs.slices > 1 ? s_ * xs.rest + t_ : -1;                                            \
-    }                                                                                          \
-    tile_coords(a, expert_off, lin_, pt_, pf_, ex_, &sh_);                                     \
-  }
-  // load q of this wavefront fills LDS rows [8 * (q * NW + wave), + 8) of the X or W tile: lane -> (row, chunk)
-#define FQ_SLOT_ROW(q_, rr_, c_)                                   \
-  const int slot_ = ((q_) * NW + wave_u) * kWave + lane;           \
-  const int rr_ = slot_ / CPR, c_ = swizzle<CPR>(rr_, slot_ % CPR);
-  auto w_src_row = [&](int pf, int rr) -> int {
-    if constexpr (EPI == EPI_SILU) {
-      const int half = rr / (BF / 2), f = pf * (BF / 2) + rr % (BF / 2);
-      return half * a.N + (f < a.N ? f : a.N - 1);
+  // Units j0 .. j0 + 63, one per lane, into the table's half (j0 / 64) & 1.  Every wavefront writes the same values and
+  // reads what it wrote itself; no wavefront is a whole unit ahead of another, so the other half is never in use.
+  // With equal heights the workgroups of an XCD move on by one tile per round: tiles of a chunk differ by a unit, and with a
+  // power of two of them a workgroup would meet the same one in every round (5800 tokens 3133 -> 3107 us).
+  auto fill_units = [&](int j0) {
+    const int j = min(j0 + lane, n_units - 1);
+    QuadUnit u = {};
+    int lin;
+    if (j < xs.rounds) {
+      int l = even_heights ? loc : loc + j;
+      l -= l / nper * nper;
+      lin = xcd_round_tile(xs, nper, xcd, l, j);
+      u.kb = 0;
+      u.kn = k_all;
+      u.tu = -1;
     } else {
-      const int f = pf * BF + rr;
-      return f < a.N ? f : a.N - 1;
+      const int s = loc / xs.rest, t = loc - s * xs.rest;
+      lin = xs.tail_base + t;
+      u.kb = s * k_all / xs.slices;
+      u.kn = (s + 1) * k_all / xs.slices - u.kb;
+      u.tu = xs.slices > 1 ? s * xs.rest + t : -1;
     }
+    quad_tile_at(a, walk, block, even_heights, lin, u);
+    unit_table[(j0 / kUnitTable) & 1][lane] = u;
   };
+  auto unit_at = [&](int j) {
+    const QuadUnit& s = unit_table[(j / kUnitTable) & 1][j % kUnitTable];
+    QuadUnit u;
+    u.row0 = __builtin_amdgcn_readfirstlane(s.row0);
+    u.units = __builtin_amdgcn_readfirstlane(s.units);
+    u.f = __builtin_amdgcn_readfirstlane(s.f);
+    u.expert = __builtin_amdgcn_readfirstlane(s.expert);
+    u.kb = __builtin_amdgcn_readfirstlane(s.kb);
+    u.kn = __builtin_amdgcn_readfirstlane(s.kn);
+    u.tu = __builtin_amdgcn_readfirstlane(s.tu);
+    u.share = __builtin_amdgcn_readfirstlane(s.share);
+    return u;
+  };
+  // Features of a tile: the last tile of a width that is no multiple of the tile's starts early instead of ending short
+  // (its first columns are the previous tile's last ones, same operands, same sums).
+  auto first_col = [&](int f) { return min(f * COLS, a.N - COLS); };
+  // row of W behind row r of a weight tile whose first column is f0
+  auto w_row = [&](int f0, int r) { return EPI == EPI_SILU ? (r / COLS) * a.N + f0 + r % COLS : f0 + r; };
 
-  // ---- fragment addresses: one per operand and K-step, the fragments at immediate offsets ------
-  // Whole tile: wavefront (wt, wf) owns token rows [wt * 128, + 128) x the weight rows acc_tile_col<C>(wf, .).
-  // Half tile (the block's upper 128 slots are all padding): wavefront w owns token rows [0, 128) x the weight
-  // rows acc_tile_col<CH>(w, .) - a quarter of the features each, so that the four MFMA pipes share what is left.
-  // All of a lane's fragment rows lie multiples of 16 apart (one swizzle key), and the two forms differ by
-  // wavefront-uniform distances.
+  // sorted id -> token row, by multiplication (ids below 2^31; a.div_mul and a.div_shift from quad_divisor)
+  auto div_top_k = [&](int sid) { return a.top_k == 1 ? static_cast<unsigned>(sid) : __umulhi(static_cast<unsigned>(sid), a.div_mul) >> a.div_shift; };
+  const unsigned xpitch = static_cast<unsigned>(a.ldx * ES);
+
+  // ---- per-lane addresses ------------------------------------------------------------------
+  // Tile load q of wavefront w fills LDS rows [32 q + 8 w, + 8) of the X or W tile, lane -> (row, 16-byte chunk); rows 32
+  // apart share their swizzle key, so the weight rows of the eight loads differ by wavefront-uniform distances only.
+  const int lrow = wave_u * 8 + lane / CPR, lchunk = swizzle<CPR>(lrow, lane % CPR);
+  const unsigned wlane = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, lrow, lchunk * 16, ES));
+  const unsigned wgap1 = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, 32, 0, ES));
+  const unsigned wgap2 = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, 64, 0, ES));
+  // fragments: one address per operand and K-step, the fragments at immediate offsets
   const int frow = lane % TILE, kgrp = lane / TILE;
   const int key0 = swizzle<CPR>(frow, 0);
   int xadr[2][FC];  // byte addresses in slot 0 of the chunks of row frow of the X tile (the W tile: XBYTES further)
@@ -153,73 +382,80 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a 
   for (int s = 0; s < 2; ++s)
 #pragma unroll
     for (int c = 0; c < FC; ++c) xadr[s][c] = (frow * CPR + (((s * KG + kgrp) * FC + c) ^ key0)) * 16;
-  const int xbaseF = wt * C::TT * CPR * 16, wbaseF = acc_tile_col<C, EPI>(wf, 0) * CPR * 16;
-  const int wbaseH = acc_tile_col<CH, EPI>(wave_u, 0) * CPR * 16;
 #define FQ_XD(i_) ((i_) * TILE * CPR * 16)
-#define FQ_WD(HALF, j_) ((HALF) ? (acc_tile_col<CH, EPI>(0, (j_)) - acc_tile_col<CH, EPI>(0, 0)) * CPR * 16 \
-                               : (acc_tile_col<C, EPI>(0, (j_)) - acc_tile_col<C, EPI>(0, 0)) * CPR * 16)
-
-  acc_t acc[NF][NF];
-  u32x4 fw[2][NF][FC], fx[2][NF][FC];
+#define FQ_WD(j_) ((acc_tile_col<C, EPI>(0, (j_)) - acc_tile_col<C, EPI>(0, 0)) * CPR * 16)
 
   // ---- address sets: A = unit being multiplied, B = the workgroup's next unit ---------------------
-  int pid_t, pid_f, expert, kb, kn, tu;
-  int n_pid_t = 0, n_pid_f = 0, n_expert = 0, n_kb = 0, n_kn = 0, n_tu = -1;
-  bool half = false, n_half = false;  // the unit is a half tile
-  TileShare shA, shB;
-  int n_sid[XI], n_tsid = 0, n_up0 = 0, n_up1 = 0;
-  unsigned xsrcA[XI], wsrcA[WI], xsrcB[XI], wsrcB[WI];
-  unsigned twA = 0, txA = 0, twB = 0, txB = 0;  // touch offsets (weight rows, token rows) of this lane
+  QuadUnit uA, uB;
+  int n_sid[XI], n_tsid = 0;
+  unsigned xsrcA[XI], xsrcB[XI];
+  unsigned wlA = 0, whA = 0, wlB = 0, whB = 0;          // W: byte offset of loads 0..3 and 4..7 of the tile
+  unsigned twA = 0, txA = 0, twB = 0, txB = 0;          // touch offsets (weight rows, token rows) of this lane
   __amdgpu_buffer_rsrc_t xrsA, wrsA, xrsB, wrsB;
-  // Touch shares.  Weight K tile (256 rows): shared by the sh.count token blocks of the tile's chunk, block
-  // sh.index asks for rows [index * per, + per), per = ceil(256 / count), a quarter of them per wavefront.
-  // Token K tile (256 gathered rows): shared by the feature tiles of the block an XCD holds at one time, about
-  // 32 / count of them, at most FQ_XSHARE: feature tile f asks for share f % that many.
-#define FQ_TOUCH_ROWS(sh_, pf_, wrow_, xrow_, xon_)                                            \
+  // Touch shares.  Weight K tile (256 rows): shared by the share >> 16 token tiles of the chunk, tile `index` asks for
+  // rows [index * per, + per), per = ceil(256 / count), a quarter of them per wavefront.  Token K tile: shared by
+  // the feature tiles of the token tile an XCD holds at one time, about 32 / count of them, at most kQuadXShare.
+#define FQ_TOUCH_ROWS(u_, wrow_, xrow_, xon_)                                                  \
   {                                                                                            \
-    const int cnt_ = max(1, min((sh_).count, 32));                                             \
+    const int cnt_ = max(1, min((u_).share >> 16, 32));                                        \
     const int per_ = (BF + cnt_ - 1) / cnt_, pw_ = (per_ + NW - 1) / NW;                       \
-    wrow_ = min((sh_).index * per_ + wave_u * pw_ + (lane < pw_ ? lane : 0), BF - 1);          \
-    const int xs_ = max(1, min(FQ_XSHARE, 32 / cnt_)), xper_ = BT / xs_, xw_ = xper_ / NW;     \
-    xrow_ = ((pf_) % xs_) * xper_ + wave_u * xw_ + (lane < xw_ ? lane : 0);                    \
-    xon_ = lane < xw_;                                                                         \
+    wrow_ = min(((u_).share & 0xFFFF) * per_ + wave_u * pw_ + (lane < pw_ ? lane : 0), BF - 1); \
+    const int xs_ = max(1, min(kQuadXShare, 32 / cnt_)), rows_ = (u_).units * kUnitRows;       \
+    const int xper_ = (rows_ + xs_ - 1) / xs_, xw_ = (xper_ + NW - 1) / NW;                    \
+    xrow_ = ((u_).f % xs_) * xper_ + wave_u * xw_ + (lane < xw_ ? lane : 0);                   \
+    xon_ = lane < xw_ && xrow_ < rows_;                                                        \
+    xrow_ = min(xrow_, rows_ - 1);                                                             \
   }
-  // the sorted ids of the upper 128 slots of block pt_, two per lane: a block is a half tile when none holds a pair
-#define FQ_UPPER_IDS(pt_, u0_, u1_)                                \
-  {                                                                \
-    u0_ = a.sorted[(pt_) * BT + BT / 2 + lane];                    \
-    u1_ = a.sorted[(pt_) * BT + BT / 2 + kWave + lane];            \
+  // A lane constant as if it came to be here: the compiler works what depends on it out in place, instead of ahead of all
+  // units and keeping it in registers through the K loops (which cost 40 to 140 spilled registers, some of them reloaded
+  // in a K loop).
+#define FQ_HERE(v_) asm volatile("" : "+v"(v_));
+  // sorted ids of the unit's load rows; a row beyond the tile counts as padding
+#define FQ_IDS(u_, sid_, tsid_)                                                                \
+  {                                                                                            \
+    const int rows_i = (u_).units * kUnitRows;                                                 \
+    int lrow_ = lrow;                                                                          \
+    FQ_HERE(lrow_)                                                                             \
+    _Pragma("unroll") for (int q = 0; q < XI; ++q) {                                           \
+      const int rr = q * kUnitRows + lrow_;                                                    \
+      sid_[q] = a.sorted[(u_).row0 + min(rr, rows_i - 1)];                                     \
+    }                                                                                          \
+    int wr_, xr_; bool xo_;                                                                    \
+    FQ_TOUCH_ROWS(u_, wr_, xr_, xo_)                                                           \
+    (void)wr_; (void)xo_;                                                                      \
+    tsid_ = a.sorted[(u_).row0 + xr_];                                                         \
   }
-#define FQ_IS_HALF(u0_, u1_) (FQ_HALF && __ballot((u0_) < a.num_valid || (u1_) < a.num_valid) == 0)
-#define FQ_MAKE_SET(pt_, pf_, ex_, kb_, sh_, SIDOF, TSIDOF, xsrc_, wsrc_, xrs_, wrs_, tw_, tx_)                 \
+  // The set of unit u_ in parts, so that the parts can stand between MFMAs.  Offsets are bytes within 4 GiB (checked by the
+  // launcher).  live_: 1, or 0 for the set behind a workgroup's last unit, whose loads all fall outside empty resources.
+#define FQ_SET_RSRC(u_, live_, wl_, wh_, xrs_, wrs_)                                                         \
   {                                                                                                          \
-    const int64_t xrow0_ = a.top_k > 0 ? 0 : static_cast<int64_t>(pt_) * BT;                                 \
-    const int64_t kfirst_ = static_cast<int64_t>(kb_) * BK;                                                  \
-    xrs_ = uniform_rsrc(X + xrow0_ * a.ldx, a.x_span ? a.x_span : 0xFFFFFFFFu);                              \
-    wrs_ = uniform_rsrc(static_cast<const T*>(a.W) + static_cast<int64_t>(ex_) * a.w_expert_stride);         \
-    _Pragma("unroll") for (int q = 0; q < XI; ++q) {                                                         \
-      FQ_SLOT_ROW(q, rr, c)                                                                                  \
-      int64_t row_ = rr;                                                                                     \
-      const int sid_ = SIDOF;                                                                                \
-      if (a.top_k > 0) row_ = sid_ < a.num_valid ? sid_ / a.top_k : 0;                                       \
-      xsrc_[q] = static_cast<unsigned>((row_ * a.ldx + kfirst_ + c * EPC) * ES);                              \
-      if (a.x_span && sid_ >= a.num_valid) xsrc_[q] = kSkipOffset;                                           \
-    }                                                                                                        \
-    _Pragma("unroll") for (int q = 0; q < WI; ++q) {                                                         \
-      FQ_SLOT_ROW(q, rr, c)                                                                                  \
-      wsrc_[q] = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_src_row(pf_, rr), (kfirst_ + c * EPC) * ES, ES)); \
-    }                                                                                                        \
-    if (FQ_TOUCH) {                                                                                          \
-      int wrow_, xrow_; bool xon_;                                                                           \
-      FQ_TOUCH_ROWS(sh_, pf_, wrow_, xrow_, xon_)                                                            \
-      (void)xrow_;                                                                                           \
-      tw_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_src_row(pf_, wrow_), kfirst_ * ES, ES)); \
-      int64_t trow_ = xrow_;                                                                                 \
-      const int tsid_ = TSIDOF;                                                                              \
-      if (a.top_k > 0) trow_ = tsid_ < a.num_valid ? tsid_ / a.top_k : 0;                                    \
-      tx_ = static_cast<unsigned>((trow_ * a.ldx + kfirst_) * ES);                                            \
-      if (a.x_span && (tsid_ >= a.num_valid || !xon_)) tx_ = kSkipOffset;                                    \
-    }                                                                                                        \
+    const int64_t xrow0_ = a.top_k > 0 ? 0 : static_cast<int64_t>((u_).row0);                                \
+    xrs_ = uniform_rsrc(X + xrow0_ * a.ldx, (a.x_span ? a.x_span : 0xFFFFFFFFu) * static_cast<unsigned>(live_)); \
+    wrs_ = uniform_rsrc(static_cast<const T*>(a.W) + static_cast<int64_t>((u_).expert) * a.w_expert_stride, 0xFFFFFFFFu * static_cast<unsigned>(live_)); \
+    const int f0_ = first_col((u_).f);                                                                       \
+    const unsigned kbytes_ = static_cast<unsigned>((u_).kb) * wstep;                                         \
+    wl_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, f0_, 0, ES)) + kbytes_;                 \
+    wh_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_row(f0_, BF / 2), 0, ES)) + kbytes_;  \
+  }
+#define FQ_SET_ROW(u_, sid_, q_, xsrc_)                                                                      \
+  {                                                                                                          \
+    int lrow_ = lrow;                                                                                        \
+    FQ_HERE(lrow_)                                                                                           \
+    const bool pad_ = (q_) >= (u_).units || (sid_) >= a.num_valid;                                           \
+    unsigned row_ = a.top_k > 0 ? div_top_k(sid_) : (q_) * kUnitRows + lrow_;                                \
+    row_ = pad_ ? 0u : row_;                                                                                 \
+    const unsigned off_ = row_ * xpitch + static_cast<unsigned>((u_).kb) * BKB + lchunk * 16;                \
+    xsrc_ = a.x_span && pad_ ? kSkipOffset : off_;                                                           \
+  }
+#define FQ_SET_TOUCH(u_, tsid_, tw_, tx_)                                                                    \
+  {                                                                                                          \
+    int wrow_, xrow_; bool xon_;                                                                             \
+    FQ_TOUCH_ROWS(u_, wrow_, xrow_, xon_)                                                                    \
+    tw_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_row(first_col((u_).f), wrow_), 0, ES)) + static_cast<unsigned>((u_).kb) * wstep; \
+    const bool tpad_ = !xon_ || (tsid_) >= a.num_valid;                                                      \
+    unsigned trow_ = a.top_k > 0 ? div_top_k(tsid_) : static_cast<unsigned>(xrow_);                          \
+    trow_ = tpad_ ? 0u : trow_;                                                                              \
+    tx_ = a.x_span && tpad_ ? kSkipOffset : trow_ * xpitch + static_cast<unsigned>((u_).kb) * BKB;           \
   }
   // tile load q (weight rows first) of K tile tile_ of set SET into ring slot slot_
 #define FQ_ISSUE(SET, tile_, slot_, q_)                                                                     \
@@ -227,252 +463,241 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a 
     if ((q_) < WI) {                                                                                        \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                             \
           wrs##SET, (lptr_t)(lds_raw + (slot_) * SLOT + XBYTES + ((q_) * NW + wave_u) * (kWave * 16)),      \
-          16, wsrc##SET[(q_) < WI ? (q_) : 0], (tile_) * wstep, 0, 0);                                      \
+          16, wlane, (((q_) & 4) ? wh##SET : wl##SET) + (((q_) & 2) ? wgap2 : 0) + (((q_) & 1) ? wgap1 : 0) + (tile_) * wstep, 0, 0); \
     } else {                                                                                                \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                             \
           xrs##SET, (lptr_t)(lds_raw + (slot_) * SLOT + (((q_) - WI) * NW + wave_u) * (kWave * 16)),        \
-          16, xsrc##SET[(q_) < WI ? 0 : (q_) - WI], (tile_) * C::BKB, 0, 0);                                \
+          16, xsrc##SET[(q_) < WI ? 0 : (q_) - WI], (tile_) * BKB, 0, 0);                                   \
     }                                                                                                       \
   }
-  // touch of K tile tile_ of the unit whose set is (tw_, tx_, wrs_, xrs_)
-#define FQ_TOUCH_ISSUE(wrs_, xrs_, tw_, tx_, tile_)                                                         \
+  // touch of K tile tile_ of set SET
+#define FQ_TOUCH_ISSUE(SET, tile_)                                                                          \
   {                                                                                                         \
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs_, (lptr_t)(lds_raw + 2 * SLOT + wave_u * 256), 4, tw_, (tile_) * wstep, 0, 0);  \
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs_, (lptr_t)(lds_raw + 2 * SLOT + wave_u * 256), 4, tx_, (tile_) * C::BKB, 0, 0); \
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs##SET, (lptr_t)(lds_raw + 2 * SLOT + wave_u * 256), 4, tw##SET, (tile_) * wstep, 0, 0);  \
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs##SET, (lptr_t)(lds_raw + 2 * SLOT + wave_u * 256), 4, tx##SET, (tile_) * BKB, 0, 0); \
   }
-#define FQ_READ_W(HALF, buf_, j_, c_, s_, sl_)                                                             \
-  fw[buf_][j_][c_] = *reinterpret_cast<const u32x4*>(lds_raw + XBYTES + xadr[s_][c_] + ((HALF) ? wbaseH : wbaseF) + \
-                                                     (sl_) * SLOT + FQ_WD(HALF, j_));
-#define FQ_READ_X(HALF, buf_, i_, c_, s_, sl_) \
-  fx[buf_][i_][c_] = *reinterpret_cast<const u32x4*>(lds_raw + xadr[s_][c_] + ((HALF) ? 0 : xbaseF) + (sl_) * SLOT + FQ_XD(i_));
-  // read r of a K-step's fragment reads (FC chunks per fragment): whole tile X0 W0 X1 W1 ..., half tile X0 X1 W0
-  // X2 X3 W1 ... (twice as many token as weight fragments)
-#define FQ_READ_NTH(HALF, r_, buf_, s_, sl_)                                                               \
+#define FQ_FENCE __builtin_amdgcn_sched_barrier(0);
+  // One K-step: the MFMAs of fragment set S.  FIRST: the accumulators start from zero.  RD: the fragments of K-step
+  // S ^ 1 are read from ring slot rsl_.  NLD_ (0: none): the first NLD_ loads of K tile ltile_ of set LSET go into slot
+  // lsl_, and behind the last MFMA the touch of K tile ttile_ of set TSET goes out.
+  // Read r goes behind MFMA r * span / N2, load q behind MFMA (q + 1/2) * (NM - 1) / NLD_, out of the reads' way.
+#define FQ_KSTEP(S, FIRST, RD, rsl_, NLD_, LSET, ltile_, lsl_, TSET, ttile_, HOOK)                         \
   {                                                                                                        \
-    const int f_ = (r_) / FC, c_ = (r_) % FC;                                                          \
-    if (HALF) {                                                                                            \
-      if (f_ % 3 == 2) { FQ_READ_W(true, buf_, f_ / 3, c_, s_, sl_) }                                      \
-      else { FQ_READ_X(true, buf_, (f_ / 3) * 2 + f_ % 3, c_, s_, sl_) }                                   \
-    } else {                                                                                               \
-      if (f_ & 1) { FQ_READ_W(false, buf_, f_ >> 1, c_, s_, sl_) } else { FQ_READ_X(false, buf_, f_ >> 1, c_, s_, sl_) } \
+    _Pragma("unroll") for (int m = 0; m < NM; ++m) {                                                       \
+      const int j = WOUT ? m / IN : m % IN, i = WOUT ? m % IN : m / IN;                                    \
+      if (i < kQuadAgpr) quad_mfma<T, true, FIRST>(acc[j][i], fw[WOUT && j < OUT - KEEP2 ? 0 : (S)][j], fx[!WOUT && i < OUT - KEEP2 ? 0 : (S)][i]); \
+      else quad_mfma<T, false, FIRST>(acc[j][i], fw[WOUT && j < OUT - KEEP2 ? 0 : (S)][j], fx[!WOUT && i < OUT - KEEP2 ? 0 : (S)][i]); \
+      FQ_FENCE                                                                                             \
+      HOOK(m)                                                                                              \
+      if (RD) {                                                                                            \
+        if (m % IN == IN - 1 && m / IN < OUT - KEEP2) {                                                    \
+          if (WOUT) { FQ_READ_W(0, m / IN, (S) ^ 1, rsl_) } else { FQ_READ_X(0, m / IN, (S) ^ 1, rsl_) }   \
+        }                                                                                                  \
+        const int span_ = (S) == 0 ? RSPAN0 : RSPAN1, r = (m * N2 + span_ - 1) / span_;                    \
+        if (r < N2 && r * span_ < (m + 1) * N2) {                                                          \
+          if (r < IN) {                                                                                    \
+            if (WOUT) { FQ_READ_X((S) ^ 1, r, (S) ^ 1, rsl_) } else { FQ_READ_W((S) ^ 1, r, (S) ^ 1, rsl_) } \
+          } else {                                                                                         \
+            if (WOUT) { FQ_READ_W((S) ^ 1, OUT - KEEP2 + r - IN, (S) ^ 1, rsl_) }                          \
+            else { FQ_READ_X((S) ^ 1, OUT - KEEP2 + r - IN, (S) ^ 1, rsl_) }                               \
+          }                                                                                                \
+        }                                                                                                  \
+      }                                                                                                    \
+      if ((NLD_) > 0) {                                                                                    \
+        _Pragma("unroll") for (int x = 0; x < ((NLD_) + NM - 2) / (NM - 1) + 1; ++x) {                         \
+          const int q = (2 * m * (NLD_) + NM - 1) / (2 * (NM - 1)) + x;                                    \
+          if (q < (NLD_) && (2 * q + 1) * (NM - 1) < 2 * (m + 1) * (NLD_)) {                               \
+            FQ_ISSUE(LSET, ltile_, lsl_, q)                                                                \
+            FQ_FENCE                                                                                       \
+          }                                                                                                \
+        }                                                                                                  \
+        if (m == NM - 1) {                                                                                 \
+          FQ_TOUCH_ISSUE(TSET, ttile_)                                                                     \
+          FQ_FENCE                                                                                         \
+        }                                                                                                  \
+      }                                                                                                    \
     }                                                                                                      \
   }
-  // One K-step: the MFMAs of fragment buffer S (a half tile: half as many, its weight fragments are half).
-  // FIRST: the accumulators start from zero.  RD: the fragments of K-step S ^ 1 of ring slot rsl_ are read into
-  // the other buffer.  NLD_ (0: none): the first NLD_ loads of K tile ltile_ of set LSET go into slot lsl_.
-  // TCH: the touch (resources and offsets given) of K tile ttile_, behind the last load.
-#define FQ_KSTEP(HALF, S, FIRST, RD, rsl_, NLD_, LSET, ltile_, lsl_, TCH, twrs_, txrs_, tw_, tx_, ttile_)   \
+#define FQ_READ_W(set_, j_, s_, sl_)                                                                       \
   {                                                                                                        \
-    constexpr int NMk = (HALF) ? NM / 2 : NM, NR = ((HALF) ? NF + NF / 2 : 2 * NF) * FC;                   \
-    constexpr int RE = (HALF) ? (FC == 1 ? 2 : 1) : ((S) == 0 ? RD0 : RD1);                                \
-    constexpr int LP = (HALF) ? (FC == 1 ? 1 : 0) : LD_POS, LE = (HALF) ? (FC == 1 ? 2 : 1) : LD_EVERY;    \
-    constexpr int LPS = ((HALF) && FC == 2) ? 2 : 1;  /* loads per MFMA slot */                            \
-    static_assert(LP + ((NL + LPS - 1) / LPS - 1) * LE < NMk && ((NR + RPS - 1) / RPS - 1) * RE < NMk,     \
-                  "loads and reads fit the K-step");                                                       \
-    _Pragma("unroll") for (int m = 0; m < NMk; ++m) {                                                      \
-      const int j = m / NF, i = m % NF;                                                                    \
-      if (FIRST) {                                                                                         \
-        const acc_t z_ = {};                                                                               \
-        if constexpr (TILE == 32) acc[j][i] = E::m32(fw[S][j], fx[S][i], z_);                              \
-        else acc[j][i] = E::m16(fw[S][j], fx[S][i], z_);                                                   \
-      } else {                                                                                             \
-        if constexpr (TILE == 32) acc[j][i] = E::m32(fw[S][j], fx[S][i], acc[j][i]);                       \
-        else acc[j][i] = E::m16(fw[S][j], fx[S][i], acc[j][i]);                                            \
-      }                                                                                                    \
-      __builtin_amdgcn_sched_barrier(0);                                                                   \
-      if ((RD) && m % RE == 0) {                                                                           \
-        _Pragma("unroll") for (int rr = 0; rr < RPS; ++rr)                                                 \
-          if ((m / RE) * RPS + rr < NR) {                                                                  \
-            FQ_READ_NTH(HALF, (m / RE) * RPS + rr, (S) ^ 1, (S) ^ 1, rsl_)                                 \
-            __builtin_amdgcn_sched_barrier(0);                                                             \
-          }                                                                                                \
-      }                                                                                                    \
-      if ((NLD_) > 0 && m >= LP && (m - LP) % LE == 0) {                                                   \
-        _Pragma("unroll") for (int ll = 0; ll < LPS; ++ll)                                                 \
-          if (((m - LP) / LE) * LPS + ll < (NLD_)) {                                                       \
-            FQ_ISSUE(LSET, ltile_, lsl_, ((m - LP) / LE) * LPS + ll)                                       \
-            __builtin_amdgcn_sched_barrier(0);                                                             \
-          }                                                                                                \
-      }                                                                                                    \
-      if ((TCH) && FQ_TOUCH && m == NMk - 1) {                                                             \
-        FQ_TOUCH_ISSUE(twrs_, txrs_, tw_, tx_, ttile_)                                                     \
-        __builtin_amdgcn_sched_barrier(0);                                                                 \
-      }                                                                                                    \
+    _Pragma("unroll") for (int c = 0; c < FC; ++c) {                                                       \
+      fw[set_][j_][c] = *reinterpret_cast<const u32x4*>(lds_raw + xadr[s_][c] + wbase + (sl_) * SLOT + FQ_WD(j_)); \
+      FQ_FENCE                                                                                             \
+    }                                                                                                      \
+  }
+#define FQ_READ_X(set_, i_, s_, sl_)                                                                       \
+  {                                                                                                        \
+    _Pragma("unroll") for (int c = 0; c < FC; ++c) {                                                       \
+      fx[set_][i_][c] = *reinterpret_cast<const u32x4*>(lds_raw + xadr[s_][c] + xbase + (sl_) * SLOT + FQ_XD(i_)); \
+      FQ_FENCE                                                                                             \
     }                                                                                                      \
   }
   // the two newest memory operations of a wavefront at the barrier are the touches of the K tile before:
   // everything older - the tile loads the barrier publishes - has landed
-#define FQ_SYNC                                                                          \
+#define FQ_SYNC(newest_)                                                                 \
   {                                                                                      \
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(FQ_TOUCH ? 2 : 0) : "memory");   \
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(newest_) : "memory");            \
     __builtin_amdgcn_s_barrier();                                                        \
-    __builtin_amdgcn_sched_barrier(0);                                                   \
+    FQ_FENCE                                                                             \
   }
-#define FQ_SYNC0                                                                         \
+  // K tile t of the unit from ring slot par; its slot takes K tile ltile_ of set LSET
+#define FQ_PERIOD(FIRST, RDLAST, NLD_, LSET, ltile_, TSET, ttile_, HOOK)                 \
   {                                                                                      \
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");                          \
-    __builtin_amdgcn_s_barrier();                                                        \
-    __builtin_amdgcn_sched_barrier(0);                                                   \
+    FQ_KSTEP(0, FIRST, true, par, 0, LSET, 0, 0, TSET, 0, HOOK)                          \
+    FQ_SYNC((FIRST) ? 0 : 2)                                                             \
+    FQ_KSTEP(1, false, RDLAST, par ^ 1, NLD_, LSET, ltile_, par, TSET, ttile_, FQ_NO_HOOK) \
+    par ^= 1;                                                                            \
   }
-  // A period: K tile t of the unit from ring slot par; its slot takes K tile ltile_ of the unit (a half tile loads
-  // the weight rows and the lower 128 token rows: 12 loads).  Touch of K tile ttile_ of the unit.
-#define FQ_PERIOD_A(HALF, FIRST, ltile_, ttile_)                                                                   \
-  {                                                                                                                \
-    FQ_KSTEP(HALF, 0, FIRST, true, par, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                                \
-    if (FIRST) FQ_SYNC0 else FQ_SYNC                                                                               \
-    FQ_KSTEP(HALF, 1, false, true, par ^ 1, ((HALF) ? WI + XI / 2 : NL), A, ltile_, par, true, wrsA, xrsA, twA, txA, ttile_) \
-    par ^= 1;                                                                                                      \
+#define FQ_NO_HOOK(m_)
+  // The next unit's coordinates and the loads of its sorted ids, behind the second MFMA of a K tile; its address set between
+  // the MFMAs of the next K tile, a row in each gap.
+#define FQ_HOOK_IDS(m_)                                                                  \
+  if ((m_) == 1) {                                                                       \
+    uB = unit_at(unit + live);                                                           \
+    FQ_IDS(uB, n_sid, n_tsid)                                                            \
+    FQ_FENCE                                                                             \
   }
-  // One work unit (an output tile, or a K slice of one): kn >= kQuadMinTiles K tiles.  The ring holds the unit's
-  // first two K tiles when it starts.  NEXT: the workgroup has another unit after this one, whose routing data is
-  // asked for at the start, turned into the address set B after two K tiles, and whose first two K tiles (all 16
-  // loads: its kind need not be this unit's) refill the ring during the last two K tiles of this one.
-#define FQ_TILE(NEXT, HALF)                                                                                        \
-  {                                                                                                                \
-    FQ_STAMP(0)                                                                                                    \
-    _Pragma("unroll") for (int r = 0; r < ((HALF) ? NF + NF / 2 : 2 * NF) * FC; ++r) FQ_READ_NTH(HALF, r, 0, 0, par) \
-    if (NEXT) {                                                                                                    \
-      FQ_UNIT(unit + 1, n_pid_t, n_pid_f, n_expert, n_kb, n_kn, n_tu, shB)                                         \
-      _Pragma("unroll") for (int q = 0; q < XI; ++q) {                                                             \
-        FQ_SLOT_ROW(q, rr, c)                                                                                      \
-        (void)c;                                                                                                   \
-        n_sid[q] = a.sorted[n_pid_t * BT + rr];                                                                    \
-      }                                                                                                            \
-      FQ_UPPER_IDS(n_pid_t, n_up0, n_up1)                                                                          \
-      if (FQ_TOUCH) {                                                                                              \
-        int wrow_, xrow_; bool xon_;                                                                               \
-        FQ_TOUCH_ROWS(shB, n_pid_f, wrow_, xrow_, xon_)                                                            \
-        (void)wrow_; (void)xon_;                                                                                   \
-        n_tsid = a.sorted[n_pid_t * BT + xrow_];                                                                   \
-      }                                                                                                            \
-    }                                                                                                              \
-    FQ_PERIOD_A(HALF, true, 2, kQuadTouchAhead)                                                                    \
-    FQ_PERIOD_A(HALF, false, 3, 1 + kQuadTouchAhead)                                                               \
-    if (NEXT) {                                                                                                    \
-      FQ_MAKE_SET(n_pid_t, n_pid_f, n_expert, n_kb, shB, n_sid[q], n_tsid, xsrcB, wsrcB, xrsB, wrsB, twB, txB)     \
-      n_half = FQ_IS_HALF(n_up0, n_up1);                                                                           \
-    }                                                                                                              \
-    __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0): no scalar load pending inside the loop */                   \
-    for (int t = 2; t < kn - kQuadTouchAhead; ++t) FQ_PERIOD_A(HALF, false, t + 2, t + kQuadTouchAhead)            \
-    if (NEXT) {                                                                                                    \
-      /* the unit's last kQuadTouchAhead K tiles: touches go to the next unit's first K tiles */                   \
-      int tb_ = 0;                                                                                                 \
-      for (int t = kn - kQuadTouchAhead; t < kn - 2; ++t, ++tb_) {                                                 \
-        FQ_KSTEP(HALF, 0, false, true, par, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                            \
-        FQ_SYNC                                                                                                    \
-        FQ_KSTEP(HALF, 1, false, true, par ^ 1, ((HALF) ? WI + XI / 2 : NL), A, t + 2, par, true, wrsB, xrsB, twB, txB, tb_) \
-        par ^= 1;                                                                                                  \
-      }                                                                                                            \
-      FQ_KSTEP(HALF, 0, false, true, par, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                              \
-      FQ_SYNC                                                                                                      \
-      FQ_KSTEP(HALF, 1, false, true, par ^ 1, NL, B, 0, par, true, wrsB, xrsB, twB, txB, tb_)                      \
-      par ^= 1;                                                                                                    \
-      FQ_KSTEP(HALF, 0, false, true, par, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                              \
-      FQ_SYNC                                                                                                      \
-      FQ_KSTEP(HALF, 1, false, false, 0, NL, B, 1, par, true, wrsB, xrsB, twB, txB, tb_ + 1)                       \
-      par ^= 1;                                                                                                    \
-    } else {                                                                                                       \
-      for (int t = kn - kQuadTouchAhead; t < kn - 2; ++t) FQ_PERIOD_A(HALF, false, t + 2, kn - 1)                  \
-      FQ_KSTEP(HALF, 0, false, true, par, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                              \
-      FQ_SYNC                                                                                                      \
-      FQ_KSTEP(HALF, 1, false, true, par ^ 1, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                          \
-      par ^= 1;                                                                                                    \
-      FQ_KSTEP(HALF, 0, false, true, par, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                              \
-      FQ_SYNC0                                                                                                     \
-      FQ_KSTEP(HALF, 1, false, false, 0, 0, A, 0, 0, false, wrsA, xrsA, twA, txA, 0)                               \
-    }                                                                                                              \
-    FQ_STAMP(1)                                                                                                    \
-    /* the last MFMA's result is 16 cycles away: the fetches below are beyond the compiler's hazard checks */      \
-    asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");                                                               \
-    float* tws_ = a.tail_ws + static_cast<int64_t>(xcd * nper + (tu < 0 ? 0 : tu)) * (BT * BF);                    \
-    if (HALF) {                                                                                                    \
-      acc_t(&acch_)[NF / 2][NF] = reinterpret_cast<acc_t(&)[NF / 2][NF]>(acc);                                     \
-      if (tu < 0) gemm_epilogue<T, CH, EPI, true, true>(a, acch_, 2 * pid_t, pid_f, expert, 0, 0, wave_u, frow, kgrp); \
-      else tail_store<CH, EPI, true>(tws_, acch_, 0, wave_u, frow, kgrp);                                          \
-    } else {                                                                                                       \
-      if (tu < 0) gemm_epilogue<T, C, EPI, true, true>(a, acc, pid_t, pid_f, expert, 0, wt, wf, frow, kgrp);       \
-      else tail_store<C, EPI, true>(tws_, acc, wt, wf, frow, kgrp);                                                \
-    }                                                                                                              \
+#define FQ_HOOK_SET(m_)                                                                  \
+  if ((m_) == 0) {                                                                       \
+    FQ_SET_RSRC(uB, live, wlB, whB, xrsB, wrsB)                                          \
+    FQ_FENCE                                                                             \
+  }                                                                                      \
+  _Pragma("unroll") for (int x = 0; x < HPER; ++x)                                       \
+    if ((m_) >= 1 && ((m_) - 1) * HPER + x < XI) {                                       \
+      FQ_SET_ROW(uB, n_sid[((m_) - 1) * HPER + x < XI && (m_) >= 1 ? ((m_) - 1) * HPER + x : 0], ((m_) - 1) * HPER + x, \
+                 xsrcB[((m_) - 1) * HPER + x < XI && (m_) >= 1 ? ((m_) - 1) * HPER + x : 0]) \
+      FQ_FENCE                                                                           \
+    }                                                                                    \
+  if ((m_) == NM - 1) {                                                                  \
+    FQ_SET_TOUCH(uB, n_tsid, twB, txB)                                                   \
+    FQ_FENCE                                                                             \
   }
 
-  FQ_UNIT(0, pid_t, pid_f, expert, kb, kn, tu, shA)
+  fill_units(0);
+  uA = unit_at(0);
   {
-    int tsid0 = 0, up0, up1;
-    FQ_UPPER_IDS(pid_t, up0, up1)
-    half = FQ_IS_HALF(up0, up1);
-    if (FQ_TOUCH) {
-      int wrow_, xrow_; bool xon_;
-      FQ_TOUCH_ROWS(shA, pid_f, wrow_, xrow_, xon_)
-      (void)wrow_; (void)xon_;
-      tsid0 = a.sorted[pid_t * BT + xrow_];
-    }
-    FQ_MAKE_SET(pid_t, pid_f, expert, kb, shA, a.sorted[pid_t * BT + rr], tsid0, xsrcA, wsrcA, xrsA, wrsA, twA, txA)
+    int sid0[XI], tsid0;
+    FQ_IDS(uA, sid0, tsid0)
+    FQ_SET_RSRC(uA, 1, wlA, whA, xrsA, wrsA)
+#pragma unroll
+    for (int q = 0; q < XI; ++q) FQ_SET_ROW(uA, sid0[q], q, xsrcA[q])
+    FQ_SET_TOUCH(uA, tsid0, twA, txA)
   }
   // fill: K tiles 0 and 1 into slots 0 and 1
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int q = 0; q < NL; ++q) FQ_ISSUE(A, t, t, q)
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+    for (int q = 0; q < WI + XI; ++q) FQ_ISSUE(A, t, t, q)
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WI + XI) : "memory");
   __builtin_amdgcn_s_barrier();
-  int par = 0;
-  int unit = 0;
-#ifdef FR_PROF  // cycle counts of wavefront 0 of every workgroup: K loops / epilogues and hand-over / total / K tiles
-  long long pf_t[2] = {0, 0}, pf_last = __builtin_readcyclecounter(), pf_periods = 0;
-  const long long pf_begin = pf_last;
-#define FQ_STAMP(k_)                                                                   \
-  {                                                                                    \
-    const long long n_ = __builtin_readcyclecounter();                                 \
-    pf_t[(k_) == 1 ? 0 : 1] += n_ - pf_last;                                           \
-    pf_last = n_;                                                                      \
-    if ((k_) == 1) pf_periods += kn;                                                   \
-    if ((k_) == 2 && threadIdx.x == 0 && fr_prof_buf) {                                \
-      long long* o_ = fr_prof_buf + blockIdx.x * 4;                                    \
-      o_[0] = pf_t[0]; o_[1] = pf_t[1]; o_[2] = n_ - pf_begin; o_[3] = pf_periods;     \
-    }                                                                                  \
-  }
-#else
-#define FQ_STAMP(k_)
-#endif
-  for (; unit + 1 < n_units; ++unit) {
-    if (half) FQ_TILE(true, true) else FQ_TILE(true, false)
-    pid_t = n_pid_t; pid_f = n_pid_f; expert = n_expert; xrsA = xrsB; wrsA = wrsB;
-    kb = n_kb; kn = n_kn; tu = n_tu; twA = twB; txA = txB; half = n_half;
+  int par = 0, unit = 0;
+
+  // One work unit of UN units of rows (or fewer: rows beyond the tile are padding): kn >= kQuadMinTiles K tiles.  The ring
+  // holds the unit's first two K tiles when it starts.  The next unit's routing data is asked for five K tiles before the end
+  // and turned into the address set B in the next one (the K loop proper keeps one set in registers); the last three K tiles
+  // touch its first three, and its first two refill the ring during the last two.
+  auto run_unit = [&](auto height) __attribute__((always_inline)) {
+    constexpr int UN = decltype(height)::value;
+    typedef QuadCfg<T, UN> C;
+    // the operand walked slowest: the weights, or the token rows where a wavefront has all of them
+    constexpr bool WOUT = C::WT == 2;
+    constexpr int KEEP2 = FC == 1 ? 2 : 1;              // its last fragments, which have two register sets like the other operand
+    constexpr int IT = C::IT, JF = C::JF, OUT = WOUT ? JF : IT, IN = WOUT ? IT : JF, NM = OUT * IN;
+    const int wt = wave_u / C::WF, wf = wave_u % C::WF;
+    const int wbase = XBYTES + acc_tile_col<C, EPI>(wf, 0) * CPR * 16;
+    constexpr int N2 = IN + KEEP2;                      // fragments with two register sets
+    constexpr int HPER = (XI + NM - 3) / (NM - 2);      // rows of the next unit's address set per MFMA
+    // MFMAs their reads are spread over: in the first K-step they end well before the barrier that waits for them
+    constexpr int RSPAN0 = NM * 5 / 8 < N2 ? N2 : NM * 5 / 8, RSPAN1 = NM * 7 / 8 < N2 ? N2 : NM * 7 / 8;
+    const int xbase = wt * C::TT * CPR * 16;
+    acc_t acc[JF][IT];
+    u32x4 fw[2][JF][FC], fx[2][IT][FC];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) FQ_READ_X(0, i, 0, par)
+#pragma unroll
+    for (int j = 0; j < JF; ++j) FQ_READ_W(0, j, 0, par)
+    const int live = min(n_units - 1 - unit, 1);  // 0: this is the workgroup's last unit
+    if (live && (unit + 1) % kUnitTable == 0) fill_units(unit + 1);
+    const int kn = uA.kn;
+    FQ_PERIOD(true, true, WI + UN, A, 2, A, 3, FQ_NO_HOOK)
+    __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0): no scalar load pending inside the loop */
+    for (int t = 1; t < kn - 5; ++t) FQ_PERIOD(false, true, WI + UN, A, t + 2, A, t + 3, FQ_NO_HOOK)
+    FQ_PERIOD(false, true, WI + UN, A, kn - 3, A, kn - 2, FQ_HOOK_IDS)
+    FQ_PERIOD(false, true, WI + UN, A, kn - 2, A, kn - 1, FQ_HOOK_SET)
+    FQ_PERIOD(false, true, WI + UN, A, kn - 1, B, 0, FQ_NO_HOOK)
+    FQ_PERIOD(false, true, WI + XI, B, 0, B, 1, FQ_NO_HOOK)
+    FQ_PERIOD(false, false, WI + XI, B, 1, B, 2, FQ_NO_HOOK)
+    // the last MFMA's result is up to 19 wait states away, which the compiler does not know
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");
+    FQ_FENCE
+    int frow_e = frow, kgrp_e = kgrp;
+    FQ_HERE(frow_e)
+    FQ_HERE(kgrp_e)
+    if (uA.tu < 0)
+      gemm_epilogue<T, C, EPI, true, kQuadAgpr>(a, acc, uA.row0, first_col(uA.f), uA.expert, 0, wt, wf, frow_e, kgrp_e, uA.row0 + uA.units * kUnitRows);
+    else
+      tail_store<C, EPI, kQuadAgpr>(a.tail_ws + static_cast<int64_t>(xcd * quad_buffers(a, tallest) + uA.tu) * (quad_buffer_rows(tallest) * BF), acc, wt, wf, frow_e, kgrp_e);
+  };
+  for (;; ++unit) {
+    switch (sizeof(T) == 1 && uA.units < 8 ? (uA.units + 1) & ~1 : uA.units) {
+      case 9: run_unit(std::integral_constant<int, 9>()); break;
+      case 8: run_unit(std::integral_constant<int, 8>()); break;
+      case 7: run_unit(std::integral_constant<int, sizeof(T) == 1 ? 8 : 7>()); break;
+      case 6: run_unit(std::integral_constant<int, 6>()); break;
+      case 5: run_unit(std::integral_constant<int, sizeof(T) == 1 ? 6 : 5>()); break;
+      case 4:
+      case 3: run_unit(std::integral_constant<int, 4>()); break;
+      default: run_unit(std::integral_constant<int, 2>()); break;
+    }
+    if (unit + 1 >= n_units) break;
+    uA = uB; xrsA = xrsB; wrsA = wrsB; wlA = wlB; whA = whB; twA = twB; txA = txB;
 #pragma unroll
     for (int q = 0; q < XI; ++q) xsrcA[q] = xsrcB[q];
-#pragma unroll
-    for (int q = 0; q < WI; ++q) wsrcA[q] = wsrcB[q];
   }
-  if (half) FQ_TILE(false, true) else FQ_TILE(false, false)
-  FQ_STAMP(2)
-#undef FQ_STAMP
-#undef FQ_TILE
-#undef FQ_PERIOD_A
-#undef FQ_SYNC0
+  // the loads behind the last unit fetched nothing, but none may be pending when the workgroup gives its LDS back
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#undef FQ_HOOK_SET
+#undef FQ_HOOK_IDS
+#undef FQ_NO_HOOK
+#undef FQ_PERIOD
 #undef FQ_SYNC
 #undef FQ_KSTEP
-#undef FQ_READ_NTH
+#undef FQ_FENCE
 #undef FQ_READ_X
 #undef FQ_READ_W
 #undef FQ_TOUCH_ISSUE
 #undef FQ_ISSUE
-#undef FQ_MAKE_SET
-#undef FQ_IS_HALF
-#undef FQ_UPPER_IDS
+#undef FQ_SET_TOUCH
+#undef FQ_SET_ROW
+#undef FQ_SET_RSRC
+#undef FQ_HERE
+#undef FQ_IDS
 #undef FQ_TOUCH_ROWS
 #undef FQ_XD
 #undef FQ_WD
-#undef FQ_SLOT_ROW
-#undef FQ_UNIT
 #endif
+}
+
+// Sums the K slices of the last round's tiles and applies the epilogue: one workgroup per 32 rows of a tile.  What a tile is
+// the GEMM launch has written down; a launch without a cut tile costs 5 us (11 with the walk worked out again here).
+template <typename T, int EPI>
+__global__ __launch_bounds__(256) void quad_fixup_kernel(const GemmArgs a, int nper) {
+  constexpr int BF = QuadCfg<T, kMaxUnits>::BF;
+  const int half = nper / 2;
+  const int xcd = blockIdx.x / (half * kMaxUnits), t = (blockIdx.x / kMaxUnits) % half, rb = blockIdx.x % kMaxUnits;
+  const QuadCut c = reinterpret_cast<const QuadCut*>(a.tail_desc)[xcd * nper + t];
+  if (rb >= c.units || c.slices < 2) return;
+  const int64_t buffer = static_cast<int64_t>(c.buffer_rows) * BF;
+  const float* first = a.tail_ws + (xcd * c.buffers + t) * buffer;
+  // widths that are no multiple of a tile's are not cut: no tile starts early here
+  fixup_rows<T, BF, EPI>(a, first, c.rest * buffer, c.slices, c.row0, rb * kUnitRows, c.f * (EPI == EPI_SILU ? BF / 2 : BF), c.expert);
 }
 
 // Workgroups resident at once on the current device: one per CU (a multiple of 8, one share per XCD).
 template <typename T, int EPI>
 int quad_grid(int* grid_out) {
-  typedef QuadCfg<T> C;
   constexpr int kMaxDevices = 64;
-  constexpr int kLds = C::LDS_BYTES + kQuadSink;
+  constexpr int kLds = kQuadRing + kQuadSink;
   static int cached[kMaxDevices] = {};  // per device; a race between threads writes the same value twice
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -482,7 +707,7 @@ int quad_grid(int* grid_out) {
                             hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     int cus = 0, per_cu = 0;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_gemm_quad_kernel<T, EPI>, C::NT, kLds);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_gemm_quad_kernel<T, EPI>, 256, kLds);
     if (e != hipSuccess) {
       (void)hipGetLastError();  // reported here: not to be found again by the next launch check
       return fail(FR_E_LAUNCH, "quad GEMM set-up (%d B LDS): %s", kLds, hipGetErrorString(e));
@@ -494,20 +719,32 @@ int quad_grid(int* grid_out) {
   return FR_OK;
 }
 
-// Launches the one-wavefront-per-SIMD form of the 256-row tile for a single K split with at least kQuadMinTiles
-// K tiles per work unit.  Returns 1 when the shape is not one it takes (nothing launched: the caller takes
-// launch_gemm_persistent).
+// n / d as umulhi(n, mul) >> shift for n < 2^31 and 2 <= d < 2^31 (round-up reciprocal of 31 + ceil(log2 d) bits: its error
+// times n stays below one unit in the last place of the quotient).
+inline void quad_divisor(int d, unsigned* mul, int* shift) {
+  int l = 0;
+  while (l < 31 && (int64_t(1) << l) < d) ++l;
+  *mul = d >= 2 ? static_cast<unsigned>((uint64_t(1) << (31 + l)) / d + 1) : 0u;
+  *shift = l > 0 ? l - 1 : 0;
+}
+
+// Launches the one-wavefront-per-SIMD kernel on routing arrays of `block` rows (a multiple of 32, at most 256; num_t_blocks
+// and num_f_tiles filled for `block` rows and 256 features) for a single K split with at least kQuadMinTiles K tiles per work
+// unit.  Returns 1 when the shape is not one it takes (nothing launched: the caller takes another kernel).
 template <typename T, int EPI>
-int launch_gemm_quad(const GemmArgs& a_in, int splits, hipStream_t st) {
-  typedef QuadCfg<T> C;
+int launch_gemm_quad(const GemmArgs& a_in, int block, int splits, hipStream_t st) {
+  typedef QuadCfg<T, kMaxUnits> C;
   GemmArgs a = a_in;
   constexpr int ES = static_cast<int>(sizeof(T)), BK = C::BKB / ES;
+  constexpr int COLS = (EPI == EPI_SILU) ? C::BF / 2 : C::BF;
   if (a.setup_only) {
     int resident = 0;
     return quad_grid<T, EPI>(&resident);
   }
   // a K slice of the split tail has at least k tiles / kTailMaxSplit K tiles (and never under kTailMinSlice)
   if (splits != 1 || a.K % BK != 0 || a.K / BK < 2 * kQuadMinTiles || a.num_experts < 1 || a.num_experts > kMaxExperts) return 1;
+  // a width below a tile's has no last tile to start early; one that is no multiple adds columns twice in the atomic epilogue
+  if (a.N < COLS || (a.add_div && a.N % COLS != 0)) return 1;
   const int64_t x_rows = a.top_k > 0 ? a.num_valid / a.top_k : C::BT;
   const int64_t w_rows = EPI == EPI_SILU ? 2 * static_cast<int64_t>(a.N) : a.N;
   const int64_t lim = int64_t(1) << 32;
@@ -516,34 +753,35 @@ int launch_gemm_quad(const GemmArgs& a_in, int splits, hipStream_t st) {
                 (long long)x_rows, (long long)a.ldx, (long long)w_rows, (long long)a.ldw);
   a.group_t = tunables().group_m ? tunables().group_m : kChunkBlocks;
   if (tunables().no_tail_split) a.tail_ws = nullptr;
+  quad_divisor(a.top_k, &a.div_mul, &a.div_shift);
   a.x_span = x_rows * a.ldx * ES < (int64_t(1) << 31) ? static_cast<unsigned>(x_rows * a.ldx * ES) : 0u;
   int resident = 0;
   const int rc = quad_grid<T, EPI>(&resident);
   if (rc != FR_OK) return rc;
-  constexpr int COLS = (EPI == EPI_SILU) ? C::BF / 2 : C::BF;
   const int64_t worst = static_cast<int64_t>(a.num_t_blocks) * a.num_f_tiles;
-  // After many whole rounds the workgroups are no longer in step (half tiles, hand-overs), and cutting the last
+  // After many whole rounds the workgroups are no longer in step (tiles of several heights, hand-overs), and cutting the last
   // round buys less than its slices' fp32 round trip costs - the sooner the shorter a tile's K loop is: gate/up
   // (64 K tiles) with / without the split 681 / 684 us at 8.8 rounds (1536 tokens), 832 / 816 at 10.5, 1030 / 988
   // at 12.5, 1521 / 1505 at 17.5, 5743 / 5723 at 70; the down projection (224 K tiles) 785 / 915 at 2.7 rounds,
   // 2803 / 2979 at 11; fp8 down projection (112 K tiles) 1743 / 1794 at 8.5 rounds; 96 K tiles (H = 6144) 1138 / 1135
   // at 10 rounds, 1442 / 1437 at 12.
-  const int64_t max_rounds = a.K / BK >= FQ_TAIL_LONG_K ? 16 : FQ_TAIL_ROUNDS_SHORT;
-  const bool tail = a.tail_ws && a.K / BK >= kTailMinTiles && a.N % COLS == 0 && worst < max_rounds * static_cast<int64_t>(resident);
+  const int64_t max_rounds = a.K / BK >= 112 ? 16 : 8;
+  const bool tail = a.tail_ws && a.K / BK >= kTailMinTiles && a.N % COLS == 0 && worst * block < max_rounds * resident * 256;
   if (!tail) a.tail_ws = nullptr;
-  int64_t grid = resident;
-  if (tail) {
-    if (grid > kTailUnits) grid = kTailUnits;
-  } else if (grid > (worst + 7) / 8 * 8) {
-    grid = (worst + 7) / 8 * 8;
+  a.tail_buffers = 32;
+  if (tail && !a.tail_desc) {
+    a.tail_desc = reinterpret_cast<int*>(a.tail_ws + kTailUnits * 256 * 256) - kTailDescBytes / 4;
+    a.tail_buffers = 31;
   }
-  hipLaunchKernelGGL((moe_gemm_quad_kernel<T, EPI>), dim3(static_cast<unsigned>(grid)), dim3(C::NT), C::LDS_BYTES + kQuadSink, st, a FR_PROF_ARG);
+  int64_t grid = resident;
+  if (grid > kTailUnits && tail) grid = kTailUnits;
+  hipLaunchKernelGGL((moe_gemm_quad_kernel<T, EPI>), dim3(static_cast<unsigned>(grid)), dim3(256), kQuadRing + kQuadSink, st, a, block);
   int lrc = check_launch("moe_gemm_quad_kernel");
   if (lrc != FR_OK || !tail) return lrc;
   const int nper = static_cast<int>(grid / 8);
   if (nper >= 2) {
-    hipLaunchKernelGGL((tail_fixup_kernel<T, C, EPI>), dim3(8 * (nper / 2) * (C::BT / kFixupRows)), dim3(256), 0, st, a, nper);
-    lrc = check_launch("tail_fixup_kernel");
+    hipLaunchKernelGGL((quad_fixup_kernel<T, EPI>), dim3(8 * (nper / 2) * kMaxUnits), dim3(256), 0, st, a, nper);
+    lrc = check_launch("quad_fixup_kernel");
   }
   return lrc;
 }

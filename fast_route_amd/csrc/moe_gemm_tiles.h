@@ -85,10 +85,12 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       // faster for the down projection, but 6 % slower for the gate/up GEMM (short K, register-starved
       // epilogue: the hand-off K tiles spill; without the hand-off it is within 1 % of the plain kernel),
       // which keeps the plain kernel.
-      // one wavefront per SIMD, 128 x 128 outputs each (see moe_gemm_quad.h), where its K loop is long enough
-      if (!tunables().no_quad) {
-        const int rc = launch_gemm_quad<T, EPI>(a, splits, st);
-        if (rc != 1) return rc;
+      // one wavefront per SIMD, tiles as tall as the experts' runs (see moe_gemm_quad.h), where its K loop is long enough
+      if constexpr (EPI != EPI_DOWN) {
+        if (!tunables().no_quad) {
+          const int rc = launch_gemm_quad<T, EPI>(a, 256, splits, st);
+          if (rc != 1) return rc;
+        }
       }
       if constexpr (sizeof(T) == 1 && EPI == EPI_SILU) return launch_gemm<T, typename TL::T256G, EPI>(a, splits, st);
       else {
@@ -99,6 +101,13 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
         return launch_gemm_persistent<T, typename TL::T256, EPI>(a, splits, st);
       }
     case 128:
+      if constexpr (EPI != EPI_DOWN) {
+        if (a.any_height) {  // a layer that leaves the tiles' heights to the kernel
+          fill(128, TL::T256::BF, TL::T256::BKB);
+          const int rc = launch_gemm_quad<T, EPI>(a, 128, splits, st);
+          if (rc != 1) return rc;
+        }
+      }
       fill(128, TL::T128::BF, TL::T128::BKB);
       // The gate/up GEMM always takes the persistent form (its walk by expert fetches each expert's
       // weights once per chunk of token blocks); the down projection of the layer (few feature tiles,
@@ -110,6 +119,13 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       }
       return launch_gemm<T, typename TL::T128, EPI>(a, splits, st);
     case 160:
+      if constexpr (EPI != EPI_DOWN) {
+        if (a.any_height) {  // a layer that leaves the tiles' heights to the kernel
+          fill(160, TL::T256::BF, TL::T256::BKB);
+          const int rc = launch_gemm_quad<T, EPI>(a, 160, splits, st);
+          if (rc != 1) return rc;
+        }
+      }
       fill(160, TL::T160P::BF, TL::T160P::BKB);
       return launch_gemm_persistent<T, typename TL::T160P, EPI>(a, splits, st);
     case 64:
@@ -178,7 +194,9 @@ int prepare_tiles() {
   if constexpr (sizeof(T) == 2) {
     if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T256S, EPI>(a, 1, nullptr);
   }
-  if (rc == FR_OK) rc = launch_gemm_quad<T, EPI>(a, 1, nullptr);
+  if constexpr (EPI != EPI_DOWN) {
+    if (rc == FR_OK) rc = launch_gemm_quad<T, EPI>(a, 256, 1, nullptr);
+  }
   if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T128P, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T160P, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm<T, typename TL::T128, EPI>(a, 1, nullptr);

@@ -210,6 +210,33 @@ def test_fp8_down_projection_tail_split(native, rows256):
     assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
 
 
+def test_fp8_tiles_as_tall_as_the_experts_runs(native):
+    """Runs that end one slot before, at and behind every unit of 32 rows, up to several tiles, and experts without a pair:
+    the one-wavefront-per-SIMD kernel against the eight-wavefront kernels, bit for bit (same MFMAs, same order)."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8
+    _say("fp8 tile heights")
+    counts = [32 * u + d for u in range(1, 10) for d in (-1, 0, 1)] + [0, 320, 289, 575, 1060]
+    H, Fd, E, M = 2048, 2048, len(counts), sum(counts)
+    g = torch.Generator().manual_seed(95)
+    x = torch.randn(M, H, generator=g).bfloat16()
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g) * 0.02).bfloat16()
+    w2 = (torch.randn(E, H, Fd, generator=g) * 0.02).bfloat16()
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(M, generator=g)]
+    logits = torch.nn.functional.one_hot(ids, E).float() * 20.0
+    w1q, w1s, w2q, w2s = prepare_weights_fp8(w1.cuda(), w2.cuda())
+    res = []
+    try:
+        for no_quad in (False, True):
+            with fr.tunables(block=256, no_quad=no_quad):
+                res.append(fused_moe_fp8(x.cuda(), w1q, w1s, w2q, w2s, logits.cuda(), 1, True))
+        torch.cuda.synchronize()
+    finally:
+        fr.reset_tunables()
+    assert torch.isfinite(res[0].float()).all() and res[0].float().abs().max() > 0
+    assert torch.equal(res[0], res[1]), "the two 256-row fp8 kernels differ"
+
+
 def test_fp8_one_wavefront_per_simd_tile_equals_the_eight_wavefront_tile(native):
     """fp8 on 256-row blocks with 16 K tiles (2048 elements) or more runs on four wavefronts of 128 x 128 outputs
     (moe_gemm_quad_kernel, 32x32x64 MFMAs); the no_quad knob sends the call to the eight-wavefront kernels.  Same

@@ -710,6 +710,70 @@ def test_one_wavefront_per_simd_tile_equals_the_eight_wavefront_tile(native, dty
         fr.reset_tunables()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", ["heights", "many_experts", "odd_width", "plan_of_128", "plan_of_160"])
+def test_tiles_as_tall_as_the_experts_runs(native, dtype, case):
+    """The one-wavefront-per-SIMD kernel cuts an expert's run into tiles of 1 to 9 units of 32 rows, whatever the routing
+    block.  heights: runs that end one slot before, at and behind every unit, of one to five tiles, and an expert without a
+    pair; many_experts: 130 experts (more than a wavefront's lanes) with a
+    few pairs each and two long runs; odd_width: the staged entry points at widths whose last feature tile starts early
+    (F = 1088, H = 1152); plan_of_128 / plan_of_160: layers whose plan routes for smaller blocks and leaves the heights to the
+    kernel."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_experts, fused_moe
+    from fast_route_amd.layers.fused_moe import plan
+    _say(f"tile heights {case} {dtype}")
+    if case.startswith("plan_of"):
+        M, H, Fd, E, k = (1400, 4096, 1024, 8, 2) if case == "plan_of_128" else (2300, 4096, 1152, 8, 2)
+        assert plan(M, H, Fd, E, k, dtype).block == int(case[-3:])
+        x, logits, w1, w2 = _inputs(M, H, Fd, E, 83, dtype)
+        out = fused_moe(x.cuda(), w1.cuda(), w2.cuda(), logits.cuda(), k, True)
+        torch.cuda.synchronize()
+        _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, case)
+        return
+    H, Fd = (1152, 1088) if case == "odd_width" else (1024, 1024)
+    if case == "many_experts":
+        counts = [1 + (e * 7) % 5 for e in range(130)]
+        counts[3], counts[64], counts[129] = 700, 0, 290
+    else:
+        counts = [32 * u + d for u in range(1, 10) for d in (-1, 0, 1)] + [0, 320, 289, 575, 800, 1060, 1]
+    ids = torch.from_numpy(np.repeat(np.arange(len(counts)), counts)).int()
+    ids = ids[torch.from_numpy(np.random.default_rng(6).permutation(ids.numel()))].view(-1, 1)
+    M, E = ids.shape[0], len(counts)
+    x, _, w1, w2 = _inputs(M, H, Fd, E, 82, dtype)
+    wts = torch.rand(M, 1) + 0.5
+    args = [t.cuda() for t in (x, w1, w2, wts, ids)]
+
+    def staged(x, w1, w2, wts, ids):
+        from fast_route_amd import _native as N
+        from fast_route_amd.ops.fused_moe import moe_align_block_size
+        s, e, npost = moe_align_block_size(ids, 256, E)
+        act = torch.zeros(s.numel(), Fd, dtype=dtype, device="cuda")
+        partial = torch.empty(M * H, dtype=torch.float32, device="cuda")
+        out = torch.empty(M, H, dtype=dtype, device="cuda")
+        lib, st, code = N.lib(), torch.cuda.current_stream().cuda_stream, N.dtype_code(dtype)
+        N.check(lib.fr_moe_gateup_silu(x.data_ptr(), w1.data_ptr(), s.data_ptr(), e.data_ptr(), npost.data_ptr(), M, H, Fd, E, 1, 256, code,
+                                       act.data_ptr(), None, st))
+        N.check(lib.fr_moe_down_combine(act.data_ptr(), w2.data_ptr(), wts.data_ptr(), s.data_ptr(), e.data_ptr(), npost.data_ptr(), M, H,
+                                        Fd, E, 1, 256, 1, code, partial.data_ptr(), out.data_ptr(), None, st))
+        return out
+
+    experts = staged if case == "odd_width" else fused_experts
+    try:
+        with fr.tunables(block=256):
+            out = experts(*args)
+        with fr.tunables(block=256, no_quad=True):
+            eight = experts(*args)
+        torch.cuda.synchronize()
+    finally:
+        fr.reset_tunables()
+    _assert_close(out, oracle.moe_experts(x, w1, w2, wts, ids), dtype, case)
+    # K below 4096 puts the eight-wavefront kernel on 32x32 MFMAs: the same products, another order of the sums inside one
+    # MFMA, so up to an ulp of the operand type after the two roundings on the way
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    assert ((out.float() - eight.float()).abs() <= 2 * ulp * eight.float().abs().max()).all()
+
+
 @pytest.mark.parametrize("E,k,H", [(8, 2, 4096), (64, 6, 4096), (100, 3, 4096), (256, 8, 4096), (4, 4, 4096), (16, 1, 4096),
                                    (64, 6, 2048), (8, 2, 3072), (16, 4, 2560)])
 @pytest.mark.parametrize("ldtype", [torch.float32, torch.bfloat16])
