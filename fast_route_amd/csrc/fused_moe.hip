@@ -26,9 +26,12 @@ double expected_blocks(double avg, int E, int rows) {
 // two per expert, the three-slot ring of the smaller tiles streams the weights faster (1031 tokens 860 / 853, 900 781 / 820,
 // 768 715 / 760, 512 585 / 690).  H = 2048, F = 1408, 64 experts, Zipf-skewed: 6000 tokens (562 pairs per expert) 753 / 730,
 // 5000 tokens (469) 666 / 672.
-bool any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block) {
+// Only where the plan has a single K slice: that kernel writes a pair's row once, in the operands' 2-byte type, where several
+// slices are summed from fp32 rows.
+bool any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
   const fr_moe_tunables& t = g_tunables;
-  if ((block != 128 && block != 160) || t.no_quad || t.block || t.split_k > 1 || E > 1022) return false;
+  const int block = p.block;
+  if ((block != 128 && block != 160) || p.split_k > 1 || t.no_quad || t.block || E > 1022) return false;
   const int es = dtype == FR_FP8_E4M3 ? 1 : 2;
   if (H * es < 2048 || F * es < 2048 || H < 256) return false;  // 16 K tiles in both GEMMs, a feature tile in the narrower one
   const double avg = static_cast<double>(M) * topk / E;
@@ -48,7 +51,6 @@ struct Carve {
   float* tail;       // scratch for splitting the last round of 256-row tiles, or nullptr
   int* tail_cuts;    // and the list of the tiles cut
   bool any_height;   // the GEMMs' tiles need not be the plan's blocks
-  int splits;        // K slices of the down projection
   void* xq;          // fp8 layer only
   float* x_scale;
   void* actq;
@@ -76,8 +78,7 @@ Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dt
   c.act = take(p.sorted_len * F * act_elem_size(dtype));
   c.partial = reinterpret_cast<float*>(take(static_cast<int64_t>(p.split_k) * n * H * 4));
   c.tail = p.tail_bytes > 0 ? reinterpret_cast<float*>(take(p.tail_bytes)) : nullptr;
-  c.any_height = any_height(M, H, F, E, topk, dtype, p.block);
-  c.splits = c.any_height ? 1 : p.split_k;
+  c.any_height = any_height(M, H, F, E, topk, dtype, p);
   c.tail_cuts = p.tail_bytes > 0 ? reinterpret_cast<int*>(take(kTailDescBytes)) : nullptr;
   c.xq = nullptr; c.x_scale = nullptr; c.actq = nullptr; c.act_scale = nullptr;
   if (dtype == FR_FP8_E4M3) {
@@ -297,7 +298,7 @@ extern "C" int fr_fused_experts(const void* x, const void* w1, const void* w2, c
                    static_cast<hipStream_t>(stream), "fr_fused_experts", (dtype & FR_W1_TILED) ? 1 : 0);
   if (rc != FR_OK) return rc;
   return down_impl(c.act, nullptr, w2, nullptr, topk_weights, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
-                   c.splits, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
+                   p.split_k, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
                    "fr_fused_experts", (dtype & FR_W2_TILED) ? 1 : 0, topk_ids);
 }
 
@@ -325,7 +326,7 @@ extern "C" int fr_fused_moe(const void* x, const void* w1, const void* w2, const
     if (rc != FR_OK) return rc;
   }
   return down_impl(c.act, nullptr, w2, nullptr, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
-                   c.splits, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
+                   p.split_k, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
                    "fr_fused_moe", (dtype & FR_W2_TILED) ? 1 : 0, c.topk_ids);
 }
 
@@ -355,7 +356,7 @@ extern "C" int fr_fused_moe_fp8(const void* x, int x_dtype, const void* w1q, con
   rc = quant_rows(c.act, FR_BF16, p.sorted_len, RowFilter{c.npost, c.sorted, M * topk}, F, F, c.actq, c.act_scale, st);
   if (rc != FR_OK) return rc;
   return down_impl(c.actq, c.act_scale, w2q, w2_scale, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
-                   c.splits, FR_FP8_E4M3, x_dtype, c.partial, out, c.tail_scratch(), st, "fr_fused_moe_fp8", w2_flag ? 1 : 0, nullptr);
+                   p.split_k, FR_FP8_E4M3, x_dtype, c.partial, out, c.tail_scratch(), st, "fr_fused_moe_fp8", w2_flag ? 1 : 0, nullptr);
 }
 
 // ---- one entry point that allocates nothing ------------------------------------

@@ -774,6 +774,28 @@ def test_tiles_as_tall_as_the_experts_runs(native, dtype, case):
     assert ((out.float() - eight.float()).abs() <= 2 * ulp * eight.float().abs().max()).all()
 
 
+@pytest.mark.parametrize("M,H,Fd,E,k", [(1055, 2048, 5632, 4, 2), (2150, 1024, 3584, 8, 2), (328, 4096, 4096, 2, 2)])
+def test_a_plan_of_several_k_slices_keeps_their_fp32_rows(native, M, H, Fd, E, k):
+    """Runs that would suit the one-wavefront-per-SIMD kernel (it writes a pair's row once, in the operands' type) under a
+    plan of several K slices: the slices are summed from fp32 rows, as without that kernel, bit for bit."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_moe
+    from fast_route_amd.layers.fused_moe import plan
+    _say(f"K slices in fp32 M={M} H={H} F={Fd} E={E}")
+    p = plan(M, H, Fd, E, k, torch.bfloat16)
+    assert p.split_k > 1 and p.block in (128, 160)
+    g = torch.Generator(device="cuda").manual_seed(90)
+    x = torch.randn(M, H, generator=g, device="cuda").bfloat16()
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g, device="cuda") * 0.02).bfloat16()
+    w2 = (torch.randn(E, H, Fd, generator=g, device="cuda") * 0.02).bfloat16()
+    logits = torch.randn(M, E, generator=g, device="cuda")
+    out = fused_moe(x, w1, w2, logits, k, True)
+    with fr.tunables(no_quad=True):
+        q = plan(M, H, Fd, E, k, torch.bfloat16)
+        assert (q.block, q.split_k) == (p.block, p.split_k)
+        assert torch.equal(out, fused_moe(x, w1, w2, logits, k, True))
+
+
 @pytest.mark.parametrize("E,k,H", [(8, 2, 4096), (64, 6, 4096), (100, 3, 4096), (256, 8, 4096), (4, 4, 4096), (16, 1, 4096),
                                    (64, 6, 2048), (8, 2, 3072), (16, 4, 2560)])
 @pytest.mark.parametrize("ldtype", [torch.float32, torch.bfloat16])
