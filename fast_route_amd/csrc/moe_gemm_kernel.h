@@ -249,12 +249,10 @@ __device__ __forceinline__ f32x16 acc_fetch(const f32x16& v) {
   return o;
 }
 
-// slot0, f0: the tile's first sorted slot and output column.  AG: the accumulators of the first AG token tiles live in the accumulation registers (one
-// wavefront per SIMD) and are fetched tile by tile; slots from row_end on then belong to another tile, their rows of the
-// accumulators are nobody's.
-template <typename T, typename C, int EPI, bool HOIST = true, int AG = 0, typename AccT>
+// slot0, f0: the tile's first sorted slot and output column.
+template <typename T, typename C, int EPI, bool HOIST = true, typename AccT>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::JF][C::IT], int slot0, int f0,
-                                              int expert, int split, int wt, int wf, int frow, int kgrp, int row_end = 0) {
+                                              int expert, int split, int wt, int wf, int frow, int kgrp) {
   typedef Elem<T> E;
   typedef typename E::out_t out_t;
   typedef typename E::out4 out4;
@@ -265,8 +263,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
   // group g (TILE==32: 4 groups of 4 regs; TILE==16: one), 4 consecutive features
   // starting at g*8 + kgrp*4 (TILE==32) or kgrp*4 (TILE==16) inside the MFMA tile.
   constexpr int GROUPS = ACC_N / 4;
-  // accumulators in the accumulation registers: results are fetched, computed and stored group by group
-  constexpr bool kFence = AG > 0;
   // fp8: with HOIST the scales of the lane's weight rows (the same for every token tile) and of its token rows
   // are fetched up front, all loads in flight together, instead of one by one between the stores (which the
   // compiler may not move them across).  That takes JF * ACC_N registers: the persistent kernel, which keeps
@@ -282,15 +278,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
   }
   if constexpr (EPI != EPI_SILU || E::SCALED) {
 #pragma unroll
-    for (int i = 0; i < C::IT; ++i) {
-      const int slot = slot0 + wt * C::TT + i * C::TILE + frow;
-      if constexpr (kFence) {
-        sids[i] = a.sorted[min(slot, row_end - 1)];
-        if (slot >= row_end) sids[i] = a.num_valid;
-      } else {
-        sids[i] = a.sorted[slot];
-      }
-    }
+    for (int i = 0; i < C::IT; ++i) sids[i] = a.sorted[slot0 + wt * C::TT + i * C::TILE + frow];
   }
   float routed[C::IT];  // routed weight of the lane's pair in each token tile (all fetched before the first store)
 #pragma unroll
@@ -330,7 +318,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
 #pragma unroll
     for (int i = 0; i < C::IT; ++i) {
       if (a.top_k > 0) xscale[i] = sids[i] < a.num_valid ? a.x_scale[sids[i] / a.top_k] : 1.f;
-      else xscale[i] = a.x_scale[kFence ? min(slot0 + wt * C::TT + i * C::TILE + frow, row_end - 1) : slot0 + wt * C::TT + i * C::TILE + frow];
+      else xscale[i] = a.x_scale[slot0 + wt * C::TT + i * C::TILE + frow];
     }
   }
 #pragma unroll
@@ -343,7 +331,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
       out_t* orow = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot) * a.ldo;
 #pragma unroll
       for (int j = 0; j < HJ; ++j) {
-        const AccT ga = i < AG ? acc_fetch(acc[j][i]) : acc[j][i], ua = i < AG ? acc_fetch(acc[j + HJ][i]) : acc[j + HJ][i];
+        const AccT &ga = acc[j][i], &ua = acc[j + HJ][i];
 #pragma unroll
         for (int g = 0; g < GROUPS; ++g) {
           const int f = f0 + wf * (C::TF / 2) + j * C::TILE + g * 8 + kgrp * 4;
@@ -357,12 +345,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
             }
             o[r] = static_cast<out_t>(silu(gv) * uv);
           }
-          if (kFence && slot >= row_end) continue;
           if (f + 3 < a.N) *reinterpret_cast<out4*>(orow + f) = o;
           else
             for (int r = 0; r < 4; ++r)
               if (f + r < a.N) orow[f + r] = o[r];
-          if constexpr (kFence) __builtin_amdgcn_sched_barrier(0);
         }
       }
     } else {
@@ -370,7 +356,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
         const float rw = routed[i] * xs;
 #pragma unroll
         for (int j = 0; j < C::JF; ++j) {
-          const AccT ca = i < AG ? acc_fetch(acc[j][i]) : acc[j][i];
+          const AccT& ca = acc[j][i];
 #pragma unroll
           for (int g = 0; g < GROUPS; ++g) {
             const int f = f0 + wf * C::TF + j * C::TILE + g * 8 + kgrp * 4;
@@ -402,7 +388,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, AccT (&acc)[C::
                     if (f + r < a.N) orow[f + r] = o[r];
               }
             }
-            if constexpr (kFence) __builtin_amdgcn_sched_barrier(0);
           }
         }
       }

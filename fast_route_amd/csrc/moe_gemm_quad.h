@@ -266,6 +266,157 @@ __device__ __forceinline__ void quad_mfma(AccT& acc, const u32x4* w, const u32x4
 #undef FQ_MFMA
 #endif
 
+// Epilogue of a tile [row0, row_end) x columns from f0 on.  Every column exists (a width below a tile's is not taken, the last
+// tile starts early), rows from row_end on belong to another tile, in whole token tiles: one scalar test each.  With one
+// wavefront per SIMD nothing runs beside it, so a token tile has one row address and its columns are immediate offsets of
+// the stores, and fp8's weight scales come in 16-byte loads.  A token tile is fetched, computed and stored before the next
+// is looked at: what the compiler may not do across a fence is hold all accumulators in ordinary registers.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // a caller's scale array is aligned to its elements
+// fp16: a product and its conversion, rounded once (one instruction, which the compiler gives up for a packed conversion where
+// it sees two side by side) or twice, through fp32.  The other tile kernels do the first for the activated rows and for two
+// of every four values of a pair's row, and so does the epilogue here.
+#if defined(__HIP_DEVICE_COMPILE__)
+template <typename O>
+__device__ __forceinline__ O round_once(float product) {
+  O o = static_cast<O>(product);
+  if constexpr (std::is_same<O, f16_t>::value) asm("" : "+v"(o));
+  return o;
+}
+template <typename O>
+__device__ __forceinline__ O round_twice(float product) {
+  if constexpr (std::is_same<O, f16_t>::value) asm("" : "+v"(product));
+  return static_cast<O>(product);
+}
+// a loaded value is waited for here and not where it is used
+template <typename V>
+__device__ __forceinline__ void arrived(V& v) {
+  asm volatile("" : "+v"(v));
+}
+#else
+template <typename O>
+__device__ __forceinline__ O round_once(float product) { return static_cast<O>(product); }
+template <typename O>
+__device__ __forceinline__ O round_twice(float product) { return static_cast<O>(product); }
+template <typename V>
+__device__ __forceinline__ void arrived(V&) {}
+#endif
+template <typename T, typename C, int EPI, typename AccT>
+__device__ __forceinline__ void quad_epilogue(const GemmArgs& a, AccT (&acc)[C::JF][C::IT], int row0, int row_end, int f0, int expert,
+                                              int wt, int wf, int frow, int kgrp) {
+  typedef Elem<T> E;
+  typedef typename E::out_t out_t;
+  typedef typename E::out4 out4;
+  constexpr int GROUPS = (C::TILE == 32) ? 4 : 1;  // groups of 4 consecutive features of a lane and accumulator tile
+  constexpr int HJ = C::JF / 2;                    // EPI_SILU: gate tiles, then as many up tiles
+  constexpr int TF = (EPI == EPI_SILU) ? C::TF / 2 : C::TF;
+  const int slot0 = row0 + wt * C::TT, col0 = f0 + wf * TF + kgrp * 4;
+  // What the rows need from memory, in two rounds: all loads of a round go out before the first is waited for, and the last
+  // wait is behind them, not between the stores (a wait there is one for the stores before it, too).
+  int sids[C::IT];
+  float scale[C::IT];  // routed weight of the lane's pair in each token tile, times the token row's scale (fp8)
+  f32x4 wscale[E::SCALED ? C::JF * GROUPS : 1];
+  if constexpr (E::SCALED) {
+    const float* wsc = a.w_scale + static_cast<int64_t>(expert) * a.w_rows + col0;
+#pragma unroll
+    for (int j = 0; j < C::JF; ++j)
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g)
+        wscale[j * GROUPS + g] = *reinterpret_cast<const f32x4_a4*>(
+            EPI == EPI_SILU ? wsc + (j / HJ) * static_cast<int64_t>(a.N) + (j % HJ) * C::TILE + g * 8 : wsc + j * C::TILE + g * 8);
+  }
+  if constexpr (EPI != EPI_SILU || E::SCALED) {
+#pragma unroll
+    for (int i = 0; i < C::IT; ++i) sids[i] = a.sorted[min(slot0 + i * C::TILE + frow, row_end - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < C::IT; ++i) {
+      arrived(sids[i]);
+      if (slot0 + i * C::TILE + frow >= row_end) sids[i] = a.num_valid;
+      scale[i] = 1.f;
+    }
+    float xs[C::IT];
+    if constexpr (EPI != EPI_SILU) {
+      if (a.mul_weight) {
+#pragma unroll
+        for (int i = 0; i < C::IT; ++i) scale[i] = a.topk_w[min(sids[i], a.num_valid - 1)];
+      }
+    }
+    if constexpr (E::SCALED) {  // a padding row's scale is not used
+#pragma unroll
+      for (int i = 0; i < C::IT; ++i)
+        xs[i] = a.x_scale[a.top_k > 0 ? min(sids[i], a.num_valid - 1) / a.top_k : min(slot0 + i * C::TILE + frow, row_end - 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < C::IT; ++i) {
+      arrived(scale[i]);
+      if constexpr (E::SCALED) {
+        arrived(xs[i]);
+        scale[i] *= xs[i];
+      }
+    }
+    if constexpr (E::SCALED) {
+#pragma unroll
+      for (int x = 0; x < C::JF * GROUPS; ++x) arrived(wscale[x]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < C::IT; ++i) {
+    if (slot0 + i * C::TILE >= row_end) break;
+    if constexpr (EPI == EPI_SILU) {
+      out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot0 + i * C::TILE + frow) * a.ldo + col0;
+#pragma unroll
+      for (int j = 0; j < HJ; ++j) {
+        const AccT ga = i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i], ua = i < kQuadAgpr ? acc_fetch(acc[j + HJ][i]) : acc[j + HJ][i];
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) {
+          out4 o;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float gv = ga[g * 4 + r], uv = ua[g * 4 + r];
+            if constexpr (E::SCALED) {
+              gv *= scale[i] * wscale[j * GROUPS + g][r];
+              uv *= scale[i] * wscale[(j + HJ) * GROUPS + g][r];
+            }
+            o[r] = round_once<out_t>(silu(gv) * uv);
+          }
+          *reinterpret_cast<out4*>(row + j * C::TILE + g * 8) = o;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else if (sids[i] < a.num_valid) {
+      auto value = [&](const AccT& c, int j, int g) {
+        out4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float v = c[g * 4 + r] * scale[i];
+          if constexpr (E::SCALED) v *= wscale[j * GROUPS + g][r];
+          o[r] = r < 2 ? round_twice<out_t>(v) : round_once<out_t>(v);
+        }
+        return o;
+      };
+      if (a.add_div) {  // top-k combine in the epilogue
+        out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(sids[i] / a.add_div) * a.ldo + col0;
+#pragma unroll
+        for (int j = 0; j < C::JF; ++j) {
+          const AccT c = i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i];
+#pragma unroll
+          for (int g = 0; g < GROUPS; ++g) atomic_add4(row + j * C::TILE + g * 8, value(c, j, g));
+        }
+      } else {
+        out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(sids[i]) * a.ldo + col0;
+#pragma unroll
+        for (int j = 0; j < C::JF; ++j) {
+          const AccT c = i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i];
+#pragma unroll
+          for (int g = 0; g < GROUPS; ++g) *reinterpret_cast<out4*>(row + j * C::TILE + g * 8) = value(c, j, g);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 template <typename T, int EPI>
 __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -634,21 +785,22 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     FQ_HERE(frow_e)
     FQ_HERE(kgrp_e)
     if (uA.tu < 0)
-      gemm_epilogue<T, C, EPI, true, kQuadAgpr>(a, acc, uA.row0, first_col(uA.f), uA.expert, 0, wt, wf, frow_e, kgrp_e, uA.row0 + uA.units * kUnitRows);
+      quad_epilogue<T, C, EPI>(a, acc, uA.row0, uA.row0 + uA.units * kUnitRows, first_col(uA.f), uA.expert, wt, wf, frow_e, kgrp_e);
     else
       tail_store<C, EPI, kQuadAgpr>(a.tail_ws + static_cast<int64_t>(xcd * quad_buffers(a, tallest) + uA.tu) * (quad_buffer_rows(tallest) * BF), acc, wt, wf, frow_e, kgrp_e);
   };
   for (;; ++unit) {
-    switch (sizeof(T) == 1 && uA.units < 8 ? (uA.units + 1) & ~1 : uA.units) {
-      case 9: run_unit(std::integral_constant<int, 9>()); break;
-      case 8: run_unit(std::integral_constant<int, 8>()); break;
-      case 7: run_unit(std::integral_constant<int, sizeof(T) == 1 ? 8 : 7>()); break;
-      case 6: run_unit(std::integral_constant<int, 6>()); break;
-      case 5: run_unit(std::integral_constant<int, sizeof(T) == 1 ? 6 : 5>()); break;
-      case 4:
-      case 3: run_unit(std::integral_constant<int, 4>()); break;
-      default: run_unit(std::integral_constant<int, 2>()); break;
-    }
+    // a loop of its own for every height from 4 on (fp8: 9 and the even ones), 2 and 4 for those below
+    const int height = uA.units;
+    if (height == 9) run_unit(std::integral_constant<int, 9>());
+    else if (height == 8 || (sizeof(T) == 1 && height == 7)) run_unit(std::integral_constant<int, 8>());
+    else if (sizeof(T) != 1 && height == 7) {
+      if constexpr (sizeof(T) != 1) run_unit(std::integral_constant<int, 7>());
+    } else if (height == 6 || (sizeof(T) == 1 && height == 5)) run_unit(std::integral_constant<int, 6>());
+    else if (sizeof(T) != 1 && height == 5) {
+      if constexpr (sizeof(T) != 1) run_unit(std::integral_constant<int, 5>());
+    } else if (height >= 3) run_unit(std::integral_constant<int, 4>());
+    else run_unit(std::integral_constant<int, 2>());
     if (unit + 1 >= n_units) break;
     uA = uB; xrsA = xrsB; wrsA = wrsB; wlA = wlB; whA = whB; twA = twB; txA = txB;
 #pragma unroll
