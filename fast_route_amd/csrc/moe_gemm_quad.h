@@ -51,11 +51,21 @@ using QuadCfg = typename std::conditional<sizeof(T) == 2, Cfg<kUnitRows * UN, 25
 constexpr int kQuadMinTiles = 8;       // K tiles per work unit, at least (one peeled at its start, five at its end)
 constexpr int kQuadXShare = 4;         // ways the touch of a tile's token rows is shared, at most
 constexpr int kQuadSink = 1024;        // bytes of LDS the touches land in (256 per wavefront)
-constexpr int kTileCost = 26;          // what a tile costs besides its height, in tenths of a unit (weight rows, barriers, epilogue)
+// What a tile costs besides its height, in tenths of a unit (weight rows, barriers, epilogue): 64 experts x 8 feature tiles of the
+// 22-K-tile down projection, two tiles each (4 rounds), 10 / 12 / 16 / 18 units per expert 183 / 201 / 240 / 259 us with the
+// combine: 19.3 us per unit and about 47 + the combine's 40 at none.
+constexpr int kTileCost = 26;
+// What cutting the last round along K costs besides its slices, in 32nds of a tile, and how much longer than alone, in fifths,
+// the slices take behind whole rounds, whose workgroups are no longer in step.  Down projection, 8 experts x 16 feature tiles,
+// one round of whole tiles and 128 tiles in two slices / two whole rounds of lower tiles: 20 units per expert 574 / 498 us, 22
+// 608 / 547, 24 622 / 562; a round and 32 tiles in eight slices / two rounds, 2048 tokens 445 / 472; nothing but a cut round / a
+// whole one: 8 units 264 / 283, 4 experts, 16 units 203 / 231.
+constexpr int kCutCost = 4, kCutStretch = 8;
 constexpr int kQuadRing = 2 * (kUnitRows * kMaxUnits + 256) * 128;
 // Slice buffers of the cut last round, per XCD of 32 workgroups: 32 of 256 x 256 fp32 or, with 288-row tiles, 28 of 288 x 256.
 // What the fix-up launch needs to know about a cut tile is left next to them (QuadCut), in the scratch itself where the
-// caller has no other place for it: then there are 31 buffers of 256 rows.
+// caller has no other place for it: then there are 31 buffers of 256 rows.  (Working it out again in the fix-up launch instead
+// costs staged calls 8 to 12 us: down projection, 8 experts, 1300 tokens 302 / 314, 2048 381 / 393.)
 constexpr int kQuadTallBuffers = 28;
 __device__ __forceinline__ int quad_buffer_rows(int tallest) { return tallest > 8 ? kUnitRows * kMaxUnits : 256; }
 __device__ __forceinline__ int quad_buffers(const GemmArgs& a, int tallest) { return tallest > 8 ? kQuadTallBuffers : a.tail_buffers; }
@@ -79,8 +89,8 @@ struct QuadWalk {
   int off[kWalkTable], units[kWalkTable], tiles[kWalkTable];
   int tallest;  // units of the tallest tile
 };
-// all 256 threads; `block` rows per routing block (a multiple of 32, at most 256), nt > 0 blocks
-__device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int block, int nt, int tid, int workgroups) {
+// all 256 threads; `block` rows per routing block (a multiple of 32, at most 256), nt > 0 blocks, nper workgroups per XCD
+__device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int block, int nt, int tid, int nper, int k_tiles) {
   expert_block_offsets(a, nt, w.off, tid, 256);
   if (w.off[kMaxExperts + 1]) {
     if (tid == 0) w.tallest = block / kUnitRows;
@@ -119,8 +129,10 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
   if (wave == 0) {
     // The limit of a tile's height.  Tall tiles cost least per row, but a launch of few rounds is over when its busiest
     // workgroup is: a round takes as long as kTileCost + height, and the tiles behind the whole rounds as long as a round
-    // unless they can be cut along K.  (Down projection, 8 experts x 16 feature tiles: with 8 or 9 units each, tiles of 8 or 9
-    // leave half the chip idle and 4 and 5 fill it; 33 units are best in four tiles, not five.)
+    // unless the schedule cuts them along K.  (Down projection, 8 experts x 16 feature tiles, limit 9 / 8 / 7 / 6 / 5 / 4 in us:
+    // 20 units each 574 / 574 / 576 / 498 / 483 / 693 (6 taken), 26 units 715 / 622 / 622 / 790 / 767 / 923 (8 taken), 33 units
+    // 752 / 907 / 910 / 867 / 1002 / 1068 (9 taken).  Over 186 launches, 8 to 50 units on 1 to 16 experts, the limit taken costs
+    // 1.0 % more than the best on average.)
     constexpr int NL = 6;  // limits 9 to 4
     int count[NL] = {}, high[NL] = {};
     for (int e0 = 0; e0 < E; e0 += kWave) {
@@ -147,10 +159,10 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
         n = lane == l ? count[l] : n;
         tall = lane == l ? high[l] : tall;
       }
-      const unsigned total = n * a.num_f_tiles, whole = total / static_cast<unsigned>(workgroups), rest = total - whole * workgroups;
-      const unsigned tile = kTileCost + 10 * tall, cuts = 8 * quad_buffers(a, tall) / max(rest, 1u);
-      const unsigned slices = a.tail_ws ? min(cuts, static_cast<unsigned>(kTailMaxSplit)) : 1u;
-      if (lane < NL) cost = 32 * whole * tile + (rest == 0 ? 0 : slices < 2 ? 32 * tile : 32 * tile / slices + 3 * tile);
+      // XCD 0 has the largest share
+      const XcdSchedule xs = xcd_schedule(n * a.num_f_tiles, nper, 0, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(n, E), quad_buffers(a, tall));
+      const unsigned tile = kTileCost + 10 * tall, rounds = xs.rounds, slices = xs.slices;
+      if (lane < NL) cost = 32 * rounds * tile + (xs.rest == 0 ? 0 : slices < 2 ? 32 * tile : 32 * tile * (rounds ? kCutStretch : 5) / (5 * slices) + kCutCost * tile);
     }
     int best = kMaxUnits;
     unsigned least = __builtin_amdgcn_readlane(cost, 0);
@@ -417,6 +429,42 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& a, AccT (&acc)[C::
   }
 }
 
+// What the workgroups of an XCD have to do: all 256 threads, the walk table behind it.
+struct QuadPlan {
+  XcdSchedule xs;
+  int tallest;
+  bool even_heights;
+};
+template <typename T>
+__device__ __forceinline__ QuadPlan quad_plan(const GemmArgs& a, QuadWalk& walk, int block, int xcd, int nper, int tid) {
+  const int nt = min(a.npost[0] / block, a.num_t_blocks), k_tiles = a.K / (QuadCfg<T, kMaxUnits>::BKB / static_cast<int>(sizeof(T)));
+  QuadPlan p;
+  // fp8's even heights have the geometry with fewer LDS reads, and short K loops are better off with whole tiles and one
+  // short one than with equal ones: layer in us, equal / even, fp8 2500 tokens 926 / 894, 4878 1570 / 1515; H = 2048, F = 1408
+  // (32 and 22 K tiles), 64 experts, 8192 tokens 952 / 940, 7000 806 / 800; H = 4096, F = 14336 (64 and 224) 2300 1460 / 1495,
+  // 3000 1713 / 1733, 5800 3116 / 3142.
+  p.even_heights = sizeof(T) == 1 || k_tiles <= 32;
+  int tiles = 0;
+  p.tallest = 0;
+  if (nt > 0) {
+    quad_walk(a, walk, block, nt, tid, nper, k_tiles);
+    tiles = __builtin_amdgcn_readfirstlane(walk.off[kMaxExperts + 1] ? nt : walk.tiles[a.num_experts]);
+    p.tallest = __builtin_amdgcn_readfirstlane(walk.tallest);
+  }
+  p.xs = xcd_schedule(tiles * a.num_f_tiles, nper, xcd, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(tiles, a.num_experts), quad_buffers(a, p.tallest));
+  return p;
+}
+// tile t of the XCD's last round
+__device__ __forceinline__ QuadCut quad_cut(const GemmArgs& a, const QuadWalk& walk, int block, const QuadPlan& p, int t) {
+  QuadCut c = {};
+  if (p.xs.slices > 1 && t < p.xs.rest) {
+    QuadUnit u;
+    quad_tile_at(a, walk, block, p.even_heights, p.xs.tail_base + t, u);
+    c = QuadCut{u.row0, u.units, u.f, u.expert, p.xs.slices, p.xs.rest, quad_buffers(a, p.tallest), quad_buffer_rows(p.tallest)};
+  }
+  return c;
+}
+
 template <typename T, int EPI>
 __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -438,31 +486,11 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
 
   // ---- schedule (as in moe_gemm_persistent_kernel, over the tiles of quad_walk) -----------------
   const int tid = threadIdx.x, lane = tid & 63;
-  const int nt = min(a.npost[0] / block, a.num_t_blocks);
   const int xcd = blockIdx.x & 7, nper = gridDim.x >> 3, loc = blockIdx.x >> 3;
   const int k_all = a.K / BK;
-  // fp8's even heights have the geometry with fewer LDS reads, and short K loops are better off with whole tiles and one
-  // short one than with equal ones: layer in us, equal / even, fp8 2500 tokens 926 / 894, 4878 1570 / 1515; H = 2048, F = 1408
-  // (32 and 22 K tiles), 64 experts, 8192 tokens 952 / 940, 7000 806 / 800; H = 4096, F = 14336 (64 and 224) 2300 1460 / 1495,
-  // 3000 1713 / 1733, 5800 3116 / 3142.
-  const bool even_heights = sizeof(T) == 1 || k_all <= 32;
-  int tiles = 0, tallest = 0;
-  if (nt > 0) {
-    quad_walk(a, walk, block, nt, tid, 8 * nper);
-    tiles = __builtin_amdgcn_readfirstlane(walk.off[kMaxExperts + 1] ? nt : walk.tiles[a.num_experts]);
-    tallest = __builtin_amdgcn_readfirstlane(walk.tallest);
-  }
-  const XcdSchedule xs = xcd_schedule(tiles * a.num_f_tiles, nper, xcd, k_all, a.tail_ws != nullptr,
-                                      schedule_by_rounds(tiles, a.num_experts), quad_buffers(a, tallest));
-  if (a.tail_ws != nullptr && tid == 0) {
-    QuadCut c = {};
-    if (xs.slices > 1 && loc < xs.rest) {
-      QuadUnit u;
-      quad_tile_at(a, walk, block, even_heights, xs.tail_base + loc, u);
-      c = QuadCut{u.row0, u.units, u.f, u.expert, xs.slices, xs.rest, quad_buffers(a, tallest), quad_buffer_rows(tallest)};
-    }
-    reinterpret_cast<QuadCut*>(a.tail_desc)[xcd * nper + loc] = c;
-  }
+  const QuadPlan plan = quad_plan<T>(a, walk, block, xcd, nper, tid);
+  const XcdSchedule& xs = plan.xs;
+  if (a.tail_ws != nullptr && tid == 0) reinterpret_cast<QuadCut*>(a.tail_desc)[xcd * nper + loc] = quad_cut(a, walk, block, plan, loc);
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
   if (n_units == 0) return;
 
@@ -479,7 +507,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     QuadUnit u = {};
     int lin;
     if (j < xs.rounds) {
-      int l = even_heights ? loc : loc + j;
+      int l = plan.even_heights ? loc : loc + j;
       l -= l / nper * nper;
       lin = xcd_round_tile(xs, nper, xcd, l, j);
       u.kb = 0;
@@ -492,7 +520,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
       u.kn = (s + 1) * k_all / xs.slices - u.kb;
       u.tu = xs.slices > 1 ? s * xs.rest + t : -1;
     }
-    quad_tile_at(a, walk, block, even_heights, lin, u);
+    quad_tile_at(a, walk, block, plan.even_heights, lin, u);
     unit_table[(j0 / kUnitTable) & 1][lane] = u;
   };
   auto unit_at = [&](int j) {
@@ -787,7 +815,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     if (uA.tu < 0)
       quad_epilogue<T, C, EPI>(a, acc, uA.row0, uA.row0 + uA.units * kUnitRows, first_col(uA.f), uA.expert, wt, wf, frow_e, kgrp_e);
     else
-      tail_store<C, EPI, kQuadAgpr>(a.tail_ws + static_cast<int64_t>(xcd * quad_buffers(a, tallest) + uA.tu) * (quad_buffer_rows(tallest) * BF), acc, wt, wf, frow_e, kgrp_e);
+      tail_store<C, EPI, kQuadAgpr>(a.tail_ws + static_cast<int64_t>(xcd * quad_buffers(a, plan.tallest) + uA.tu) * (quad_buffer_rows(plan.tallest) * BF), acc, wt, wf, frow_e, kgrp_e);
   };
   for (;; ++unit) {
     // a loop of its own for every height from 4 on (fp8: 9 and the even ones), 2 and 4 for those below

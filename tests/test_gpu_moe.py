@@ -774,6 +774,67 @@ def test_tiles_as_tall_as_the_experts_runs(native, dtype, case):
     assert ((out.float() - eight.float()).abs() <= 2 * ulp * eight.float().abs().max()).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,E,Fd,cut", [(256, 8, 4096, ""), (256, 7, 4096, "down"), (288, 17, 2048, "gate/up, down"),
+                                           (257, 17, 2048, "gate/up, down"), (545, 9, 2048, "gate/up, down")])
+def test_cut_tiles_equal_whole_ones(native, rows, E, Fd, cut, dtype):
+    """The last round's tiles cut along K by the one-wavefront-per-SIMD kernel: tiles of 256 rows, in the down projection of 8
+    experts with every slice buffer of the layer's scratch in use (16 tiles per XCD in 2 slices; the staged entry points keep
+    their list of cut tiles in the scratch and have one buffer less: not cut there), and tiles of 9 units (buffers of 288
+    rows).  Operands are small integers times powers of two, whose sums are exact in any order: a cut tile equals the whole
+    one bit for bit (fp16: up to the one rounding more of the fix-up launch)."""
+    import fast_route_amd as fr
+    from fast_route_amd import _native as N, fused_experts
+    from fast_route_amd.ops.fused_moe import moe_align_block_size
+    H, M = 4096, rows * E
+    _say(f"cut tiles rows={rows} E={E} {dtype}")
+    g = torch.Generator(device="cuda").manual_seed(94)
+    ints = lambda hi, *shape: torch.randint(-hi, hi + 1, shape, generator=g, device="cuda").to(dtype)
+    x, act_in, w1, w2 = ints(1, M, H), ints(2, M + E * 255, Fd), ints(1, E, 2 * Fd, H) / 64, ints(1, E, H, Fd) / 64
+    x[:, 0] = 1
+    w1[:, :Fd] = 0
+    w1[:, :Fd, 0] = 64  # silu(64) is 64: the activated rows are sums times a power of two
+    ids = (torch.randperm(M, generator=g, device="cuda") % E).int().view(M, 1)
+    wts = torch.rand(M, 1, generator=g, device="cuda") + 0.5
+    lib, st, code = N.lib(), torch.cuda.current_stream().cuda_stream, N.dtype_code(dtype)
+    s, e, npost = moe_align_block_size(ids, 256, E)
+    tail = torch.full((256 * 256 * 256,), float("nan"), dtype=torch.float32, device="cuda")
+    pairs = (s < M).nonzero().view(-1)
+
+    def gate_up(scratch):
+        act = torch.zeros(s.numel(), Fd, dtype=dtype, device="cuda")
+        N.check(lib.fr_moe_gateup_silu(x.data_ptr(), w1.data_ptr(), s.data_ptr(), e.data_ptr(), npost.data_ptr(), M, H, Fd, E, 1,
+                                       256, code, act.data_ptr(), scratch, st))
+        return act
+
+    def down(act, scratch):
+        partial = torch.empty(M * H, dtype=torch.float32, device="cuda")
+        out = torch.empty(M, H, dtype=dtype, device="cuda")
+        N.check(lib.fr_moe_down_combine(act.data_ptr(), w2.data_ptr(), wts.data_ptr(), s.data_ptr(), e.data_ptr(), npost.data_ptr(),
+                                        M, H, Fd, E, 1, 256, 1, code, partial.data_ptr(), out.data_ptr(), scratch, st))
+        return out
+
+    def equal(a, b, what):
+        if dtype == torch.bfloat16:
+            assert torch.equal(a, b), what
+        else:  # an ulp: 2^-10 of the value
+            assert ((a.float() - b.float()).abs() <= 2.0 ** -10 * b.float().abs()).all(), what
+
+    for name, run in (("gate/up", lambda t: gate_up(t)[pairs]), ("down", lambda t: down(act_in, t))):
+        tail.fill_(float("nan"))
+        out = run(tail.data_ptr())
+        torch.cuda.synchronize()
+        buffers = tail[: 8 * 28 * 288 * 256]  # without the list of cut tiles
+        assert bool((~torch.isnan(buffers)).any()) == (name in cut), name
+        assert torch.isfinite(out.float()).all()
+        equal(out, run(None), name)
+    with fr.tunables(block=256, split_k=1):
+        layer = fused_experts(x, w1, w2, wts, ids)
+    with fr.tunables(block=256, split_k=1, no_tail_split=True):
+        equal(layer, fused_experts(x, w1, w2, wts, ids), "layer")
+    equal(layer, down(gate_up(tail.data_ptr()), tail.data_ptr()), "layer and staged entry points")
+
+
 @pytest.mark.parametrize("M,H,Fd,E,k", [(1055, 2048, 5632, 4, 2), (2150, 1024, 3584, 8, 2), (328, 4096, 4096, 2, 2)])
 def test_a_plan_of_several_k_slices_keeps_their_fp32_rows(native, M, H, Fd, E, k):
     """Runs that would suit the one-wavefront-per-SIMD kernel (it writes a pair's row once, in the operands' type) under a
