@@ -20,22 +20,27 @@ double expected_blocks(double avg, int E, int rows) {
 }
 
 // A layer whose plan routes for 128 or 160 rows and runs the one-wavefront-per-SIMD kernel all the same, with tiles as tall as
-// the experts' runs (moe_gemm_quad.h): where the runs' own length in units of 32 rows is under 0.95 of the rows of whole
-// blocks.  Layer in us, 8 experts, H = 4096, F = 14336, top-2, blocks / runs: 1300 tokens 1056 / 967, 1400 1080 / 1000, 1500
-// 1180 / 1033, 2300 (0.92) 1525 / 1520; 1200 tokens (0.99) 870 / 932.  From 310 pairs per expert on: below, with one tile or
-// two per expert, the three-slot ring of the smaller tiles streams the weights faster (1031 tokens 860 / 853, 900 781 / 820,
-// 768 715 / 760, 512 585 / 690).  H = 2048, F = 1408, 64 experts, Zipf-skewed: 6000 tokens (562 pairs per expert) 753 / 730,
-// 5000 tokens (469) 666 / 672.
+// the experts' runs (moe_gemm_quad.h).  Layer in us, the plan's own tiles / that kernel:
+//   H = 4096, F = 14336, 8 experts   bf16 1031 tokens (258 pairs per expert) 800 / 797, 1100 815 / 819, 1180 864 / 865,
+//                                    1240 (310) 973 / 893, 1280 995 / 908, 1430 1078 / 945, 1500 1133 / 969, 2300 1480 / 1406,
+//                                    2420 1520 / 1478; fp8 1100 511 / 524, 1180 542 / 564, 1250 614 / 556
+//   16 experts, F = 8192, fp16       2300 (288) 1022 / 1046, 2490 (311) 1108 / 1065, 4400 1727 / 1581
+//   H = 3072, F = 4096, 16 experts   4500 (562) 0.96, 5000 0.92 of the plan's tiles
+//   H = 2048, F = 1408, 64 experts, top-6, Zipf-skewed: 5600 (525) 1.04 to 1.06, 5900 (553) 0.96, 6200 0.96 to 0.99, 7100 0.97
+//   H = 2048, F = 8192, 8 experts    2200 (550) 0.98, 2500 0.92; fp8 0.92, 0.85
+//   H = 1024, F = 3584, 8 experts    2200 to 4096 0.93 to 1.03, 4142 (1036) 0.87
+// A few tiles leave the chip idle whatever their height, and the smaller ones less of it: one expert, F = 4096 (64 gate/up
+// tiles) 350 tokens 1.20, 570 1.11, F = 2048 1.21, 1.13; 8 experts, F = 1024 (128 and 192 tiles) 1400 1.02, 2300 1.07; but one
+// expert, F = 14336 (224) 0.97, 8 experts, F = 2048 (256) 1400 0.87.
 // Only where the plan has a single K slice: that kernel writes a pair's row once, in the operands' 2-byte type, where several
 // slices are summed from fp32 rows.
 bool any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
   const fr_moe_tunables& t = g_tunables;
-  const int block = p.block;
-  if ((block != 128 && block != 160) || p.split_k > 1 || t.no_quad || t.block || E > 1022) return false;
+  if ((p.block != 128 && p.block != 160) || p.split_k > 1 || t.no_quad || t.block || E > 1022) return false;
   const int es = dtype == FR_FP8_E4M3 ? 1 : 2;
-  if (H * es < 2048 || F * es < 2048 || H < 256) return false;  // 16 K tiles in both GEMMs, a feature tile in the narrower one
+  if (H * es < 2048 || F * es < 2048) return false;  // 16 K tiles in both GEMMs
   const double avg = static_cast<double>(M) * topk / E;
-  return avg >= (H >= 4096 ? 310.0 : 520.0) && expected_blocks(avg, E, 32) * 32 < 0.95 * expected_blocks(avg, E, block) * block;
+  return avg >= (H >= 4096 ? 310.0 : H >= 2048 ? 550.0 : 1030.0) && E * expected_blocks(avg, E, 288) * (F / 128) >= 200.0;
 }
 
 struct Carve {
@@ -181,24 +186,17 @@ extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk,
     const bool take160 = two_byte ? (b160 * 1.15 < b128 || c160 <= 0.98 * c128) : b160 * 1.2 < b128;
     if (take160) block = 160;
   }
-  // 256 rows on the one-wavefront-per-SIMD kernel (2-byte operands, 16 K tiles or more in both GEMMs): a row of its
-  // tiles costs about 8 % less than one of the 128- or 160-row tiles (4096 tokens 2365 against 2510 us with 160 rows,
-  // 16384: 8494 / 9349), which pays wherever its coarser blocks do not add more rows than that.  Its rows: the mean
-  // of whole blocks (the time of a tile) and whole half blocks (the wavefronts of an all-padding half idle: energy,
-  // and the clock follows the energy).  Measured 160 / 256 rows on 8 experts, H = 4096: 1280 tokens 982 / 1040 us
-  // (160 stays), 1536: 1148 / 1081, 1792: 1216 / 1102, 2048: 1395 / 1373, 2304: 1490 / 1626 (160 stays), 2560:
-  // 1664 / 1647, 3072: 1973 / 1815, 5120: 3059 / 2911, 8192: 4804 / 4339.  Below 350 pairs per expert the smaller
-  // tiles stream the weights faster (1024 tokens: 811 / 977 us).
-  // With a short K (H = 2048, F = 1408, 64 experts: 32 and 22 K tiles per output tile) a tile's epilogue and hand-over
-  // weigh more and the gain is smaller and later: 160 / 256 rows 4096 tokens (384 pairs per expert) 568 / 587 us,
-  // 8192: 941 / 918, 16384: 1698 / 1637; taken from 700 pairs per expert on.
-  // fp8 (32x32x64 MFMAs in that kernel; 16 K tiles are 2048 elements): 128 / 160 / 256 rows 2048 tokens 870 / - / 797 us,
-  // 2560: - / 1040 / 941, 4096: - / 1554 / 1383 (1511 on the eight-wavefront kernel), 16384: 5386 -> 4882.
+  // 256 rows, where both GEMMs run the one-wavefront-per-SIMD kernel (16 K tiles or more in both).  Its tiles follow the experts'
+  // runs in units of 32 rows (moe_gemm_quad.h), so the block decides the padding of the routing arrays only; what is priced
+  // here, the mean of whole and half blocks of 256 rows, bounds that padding.  Layer in us, 128 or 160 rows without that kernel
+  // / 256: H = 4096, F = 14336, 8 experts 1536 tokens 1117 / 983, 1792 1222 / 1077, 2048 1422 / 1184, 2560 1657 / 1547, 3000
+  // 1878 / 1694; fp8 1280 596 / 558, 1600 707 / 607, 2048 848 / 694, 2400 916 / 902; H = 2048, F = 1408, 64 experts, top-6,
+  // Zipf-skewed 7468 0.96, 8192 0.99, 10000 0.94.  Layers that keep smaller blocks by this rule may run that kernel, too
+  // (any_height); what it costs with one or two experts and F up to 4096 is that of few tiles (400 tokens, one expert 1.19).
   if (!g_tunables.no_quad && (block == 128 || block == 160) && H >= 2048 && F >= 2048 / (two_byte ? 2 : 1) && E <= 1022 &&
       avg >= (H >= 4096 ? (two_byte ? 350.0 : 300.0) : 700.0)) {
     const double other = expected(block) * block;
     const double quad = 0.5 * (expected(256) * 256 + expected(128) * 128);
-    // fp8 gains more per row (1280 tokens: 605 / 612 / 583 us with 128 / 160 / 256 rows, 2304: - / 882 / 870)
     if (quad <= (two_byte ? 1.08 : 1.18) * other) block = 256;
   }
   if (g_tunables.block) block = g_tunables.block;

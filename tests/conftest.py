@@ -26,3 +26,16 @@ def rows256():
     import fast_route_amd as fr
     with fr.tunables(block=256):
         yield
+
+
+@pytest.fixture(scope="session")
+def kernels_of():
+    """What a call returns and the names of the kernels it launched."""
+    import torch
+
+    def run(call):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            out = call()
+            torch.cuda.synchronize()
+        return out, [e.name for e in prof.events()]
+    return run

@@ -237,6 +237,50 @@ def test_fp8_tiles_as_tall_as_the_experts_runs(native):
     assert torch.equal(res[0], res[1]), "the two 256-row fp8 kernels differ"
 
 
+def test_fp8_layer_leaves_the_heights_to_the_kernel(native, kernels_of):
+    """A layer whose plan routes for 160 rows and whose runs suit the one-wavefront-per-SIMD kernel: both GEMMs take it."""
+    from fast_route_amd import _native as N, fused_moe_fp8, prepare_weights_fp8
+    from fast_route_amd.layers.fused_moe import plan
+    _say("fp8 plan of 160 rows, tiles as tall as the runs")
+    M, H, Fd, E, k = 1250, 4096, 2048, 8, 2
+    assert plan(M, H, Fd, E, k, None, code=N.FR_FP8_E4M3).block == 160
+    x, logits, w1, w2 = oracle.make_inputs(M, H, Fd, E, seed=97)
+    x, w1, w2 = x.bfloat16(), w1.bfloat16(), w2.bfloat16()
+    weights = prepare_weights_fp8(w1.cuda(), w2.cuda())
+    args = [x.cuda(), *weights, logits.cuda()]
+    out, names = kernels_of(lambda: fused_moe_fp8(*args, k, True))
+    assert sum("moe_gemm_quad_kernel" in n for n in names) == 2, names
+    ref, _ = oracle.fused_moe_fp8(x, w1, w2, logits, k, True)
+    o = out.float().cpu()
+    assert torch.isfinite(o).all()
+    assert (o - ref).norm() / ref.norm() <= 1e-2
+    assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
+def test_fp8_cut_tiles_of_nine_units(native):
+    """Both GEMMs' last round cut along K with tiles of 9 units (9 experts of two tiles each, 32 and 16 feature tiles, 32 K
+    tiles): the result differs from that of whole tiles by the order of fp32 sums (and the codes of activated rows that
+    round the other way)."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8
+    _say("fp8 cut tiles of nine units")
+    H, Fd, E, M = 4096, 4096, 9, 9 * 545
+    g = torch.Generator(device="cuda").manual_seed(98)
+    x = torch.randn(M, H, generator=g, device="cuda").bfloat16()
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g, device="cuda") * 0.02).bfloat16()
+    w2 = (torch.randn(E, H, Fd, generator=g, device="cuda") * 0.02).bfloat16()
+    ids = torch.randperm(M, generator=g, device="cuda") % E
+    logits = torch.nn.functional.one_hot(ids, E).float() * 20.0
+    weights = prepare_weights_fp8(w1, w2)
+    with fr.tunables(block=256, split_k=1):
+        cut = fused_moe_fp8(x, *weights, logits, 1, True).float()
+    with fr.tunables(block=256, split_k=1, no_tail_split=True):
+        whole = fused_moe_fp8(x, *weights, logits, 1, True).float()
+    assert torch.isfinite(cut).all() and not torch.equal(cut, whole), "nothing was cut"
+    assert (cut - whole).norm() / whole.norm() <= 1e-2
+    assert (cut - whole).abs().max() <= 2.0 ** -5 * whole.abs().max()
+
+
 def test_fp8_one_wavefront_per_simd_tile_equals_the_eight_wavefront_tile(native):
     """fp8 on 256-row blocks with 16 K tiles (2048 elements) or more runs on four wavefronts of 128 x 128 outputs
     (moe_gemm_quad_kernel, 32x32x64 MFMAs); the no_quad knob sends the call to the eight-wavefront kernels.  Same

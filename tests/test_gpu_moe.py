@@ -712,7 +712,7 @@ def test_one_wavefront_per_simd_tile_equals_the_eight_wavefront_tile(native, dty
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("case", ["heights", "many_experts", "odd_width", "plan_of_128", "plan_of_160"])
-def test_tiles_as_tall_as_the_experts_runs(native, dtype, case):
+def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
     """The one-wavefront-per-SIMD kernel cuts an expert's run into tiles of 1 to 9 units of 32 rows, whatever the routing
     block.  heights: runs that end one slot before, at and behind every unit, of one to five tiles, and an expert without a
     pair; many_experts: 130 experts (more than a wavefront's lanes) with a
@@ -724,11 +724,12 @@ def test_tiles_as_tall_as_the_experts_runs(native, dtype, case):
     from fast_route_amd.layers.fused_moe import plan
     _say(f"tile heights {case} {dtype}")
     if case.startswith("plan_of"):
-        M, H, Fd, E, k = (1400, 4096, 1024, 8, 2) if case == "plan_of_128" else (2300, 4096, 1152, 8, 2)
+        M, H, Fd, E, k = (1350, 4096, 2048, 8, 2) if case == "plan_of_128" else (2250, 4096, 2048, 8, 2)
         assert plan(M, H, Fd, E, k, dtype).block == int(case[-3:])
         x, logits, w1, w2 = _inputs(M, H, Fd, E, 83, dtype)
-        out = fused_moe(x.cuda(), w1.cuda(), w2.cuda(), logits.cuda(), k, True)
-        torch.cuda.synchronize()
+        args = [t.cuda() for t in (x, w1, w2, logits)]
+        out, names = kernels_of(lambda: fused_moe(*args, k, True))
+        assert sum("moe_gemm_quad_kernel" in n for n in names) == 2, names
         _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, case)
         return
     H, Fd = (1152, 1088) if case == "odd_width" else (1024, 1024)
@@ -772,6 +773,32 @@ def test_tiles_as_tall_as_the_experts_runs(native, dtype, case):
     # MFMA, so up to an ulp of the operand type after the two roundings on the way
     ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
     assert ((out.float() - eight.float()).abs() <= 2 * ulp * eight.float().abs().max()).all()
+
+
+@pytest.mark.parametrize("M,H,Fd,E,k,quad", [(1350, 4096, 2048, 8, 2, 2), (1430, 4096, 2048, 8, 2, 2), (2300, 2048, 2048, 8, 2, 2),
+                                              (1200, 4096, 2048, 8, 2, 0), (2100, 2048, 2048, 8, 2, 0), (2850, 1024, 3584, 8, 2, 0),
+                                              (350, 4096, 2048, 1, 1, 0), (1055, 2048, 5632, 4, 2, 0)])
+def test_plans_of_128_and_160_rows_that_leave_the_heights_to_the_kernel(native, kernels_of, M, H, Fd, E, k, quad):
+    """Layers whose plan routes for 128 or 160 rows: the one-wavefront-per-SIMD kernel for both GEMMs where the rule says so -
+    enough pairs per expert (at the first and behind the last count of every hidden size), enough tiles, one K slice -, the
+    plan's tiles elsewhere and under no_quad."""
+    import fast_route_amd as fr
+    from fast_route_amd.layers import stable_route
+    from fast_route_amd.layers.fused_moe import plan
+    _say(f"route of plans of 128 / 160 rows M={M} H={H} F={Fd} E={E}")
+    assert plan(M, H, Fd, E, k, torch.bfloat16).block in (128, 160)
+    g = torch.Generator(device="cuda").manual_seed(96)
+    x = torch.randn(M, H, generator=g, device="cuda").bfloat16()
+    gate = (torch.randn(H, E, generator=g, device="cuda") / 64).bfloat16()
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g, device="cuda") * 0.02).bfloat16()
+    w2 = (torch.randn(E, H, Fd, generator=g, device="cuda") * 0.02).bfloat16()
+    count = lambda names: sum("moe_gemm_quad_kernel" in n for n in names)
+    out, names = kernels_of(lambda: stable_route.fused_moe(x, gate, w1, w2, k, True))
+    assert count(names) == quad, names
+    with fr.tunables(no_quad=True):
+        tiles, names = kernels_of(lambda: stable_route.fused_moe(x, gate, w1, w2, k, True))
+    assert count(names) == 0, names
+    _assert_close(out, tiles.cpu(), torch.bfloat16, "one-wavefront-per-SIMD kernel against the plan's tiles")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
