@@ -57,13 +57,15 @@ constexpr int kTailDescBytes = 8192;  // what TailScratch::cuts points to
 
 // Scratch of a grouped GEMM for cutting the tiles of its last round along K (plan.tail_bytes, or nullptr), a place for the
 // list of the tiles cut (kTailDescBytes, or nullptr: taken from the scratch's end), and whether the tiles' heights may
-// differ from the routing block's: the layers leave them to the kernel, the staged entry points' callers choose a tile by
-// the block they route with.
+// differ from the routing block's: by the plan's rule, in the layers and for callers of the staged entry points who route
+// with the plan's block (plan_leaves_heights); another block chooses a tile.
 struct TailScratch {
   float* buffers = nullptr;
   int* cuts = nullptr;
   bool any_height = false;
 };
+
+bool plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block);
 
 // Gate/up projection + SiLU * up (what fr_moe_gateup_silu / fr_moe_gateup_silu_fp8 launch).
 int gateup_impl(const void* x, const float* x_scale, const void* w1, const float* w1_scale,

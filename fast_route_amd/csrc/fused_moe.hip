@@ -108,6 +108,13 @@ int check_layer_shapes(const char* who, int64_t M, int64_t H, int64_t F, int E, 
 
 }  // namespace
 const fr_moe_tunables& tunables() { return g_tunables; }
+
+bool plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block) {
+  const int mult = dtype == FR_FP8_E4M3 ? 256 : 128;
+  if ((block != 128 && block != 160) || H % mult || F % mult || E > 1022 || topk > E) return false;  // shapes without a plan among them
+  fr_moe_plan p;
+  return fr_moe_get_plan(M, H, F, E, topk, dtype, &p) == FR_OK && p.block == block && any_height(M, H, F, E, topk, dtype, p);
+}
 }  // namespace fr
 
 using namespace fr;

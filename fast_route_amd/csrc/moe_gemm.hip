@@ -351,7 +351,8 @@ extern "C" int fr_moe_gateup_silu(const void* x, const void* w1, const int32_t* 
   dtype &= ~FR_W_TILED;
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_gateup_silu: dtype %d not in {f16, bf16}", dtype);
   return gateup_impl(x, nullptr, w1, nullptr, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F, E, topk,
-                     block, dtype, act, TailScratch{static_cast<float*>(tail_ws)}, static_cast<hipStream_t>(stream), "fr_moe_gateup_silu", w_tiled);
+                     block, dtype, act, TailScratch{static_cast<float*>(tail_ws), nullptr, plan_leaves_heights(M, H, F, E, topk, dtype, block)},
+                     static_cast<hipStream_t>(stream), "fr_moe_gateup_silu", w_tiled);
 }
 
 extern "C" int fr_moe_gateup_silu_fp8(const void* xq, const float* x_scale, const void* w1q, const float* w1_scale,
@@ -360,7 +361,8 @@ extern "C" int fr_moe_gateup_silu_fp8(const void* xq, const float* x_scale, cons
                                       int topk, int block, void* act_bf16, void* stream) {
   FR_REQUIRE(x_scale && w1_scale, FR_E_NULL, "fr_moe_gateup_silu_fp8: null scale pointer");
   return gateup_impl(xq, x_scale, w1q, w1_scale, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F, E, topk,
-                     block, FR_FP8_E4M3, act_bf16, TailScratch{}, static_cast<hipStream_t>(stream), "fr_moe_gateup_silu_fp8", 0);
+                     block, FR_FP8_E4M3, act_bf16, TailScratch{nullptr, nullptr, plan_leaves_heights(M, H, F, E, topk, FR_FP8_E4M3, block)},
+                     static_cast<hipStream_t>(stream), "fr_moe_gateup_silu_fp8", 0);
 }
 
 extern "C" int fr_moe_down_combine(const void* act, const void* w2, const float* topk_weights,
@@ -372,7 +374,8 @@ extern "C" int fr_moe_down_combine(const void* act, const void* w2, const float*
   dtype &= ~FR_W_TILED;
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_down_combine: dtype %d not in {f16, bf16}", dtype);
   return down_impl(act, nullptr, w2, nullptr, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F,
-                   E, topk, block, split_k, dtype, dtype, partial, out, TailScratch{static_cast<float*>(tail_ws)},
+                   E, topk, block, split_k, dtype, dtype, partial, out,
+                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 && plan_leaves_heights(M, H, F, E, topk, dtype, block)},
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine", w_tiled, nullptr);
 }
 
@@ -385,7 +388,8 @@ extern "C" int fr_moe_down_combine_fp8(const void* actq, const float* act_scale,
   out_dtype &= ~FR_W_TILED;
   FR_REQUIRE(act_scale && w2_scale, FR_E_NULL, "fr_moe_down_combine_fp8: null scale pointer");
   return down_impl(actq, act_scale, w2q, w2_scale, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M,
-                   H, F, E, topk, block, split_k, FR_FP8_E4M3, out_dtype, partial, out, TailScratch{static_cast<float*>(tail_ws)},
+                   H, F, E, topk, block, split_k, FR_FP8_E4M3, out_dtype, partial, out,
+                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 && plan_leaves_heights(M, H, F, E, topk, FR_FP8_E4M3, block)},
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine_fp8", w_tiled, nullptr);
 }
 

@@ -67,7 +67,7 @@ struct GemmArgs {
   int add_div;          // EPI_PLAIN: 0 = store row `sorted id` of out; k > 0 = add into row (sorted id / k) of a zero-filled out (packed atomics)
   unsigned div_mul;     // division by top_k of the one-wavefront-per-SIMD form (quad_divisor)
   int div_shift;
-  int any_height;       // the tiles' heights need not be the routing block's (routing arrays of this library's own layers)
+  int any_height;       // the tiles' heights need not be the routing block's (TailScratch::any_height)
   int w_tiled;          // W is in the prepared layout (see w_byte_offset), not [E, w_rows, K] row-major
   int setup_only;       // do the per-device set-up of the kernel a launch would take (LDS limit, occupancy) and launch nothing
 };

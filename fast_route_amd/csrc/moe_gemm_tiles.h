@@ -85,7 +85,8 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       // faster for the down projection, but 6 % slower for the gate/up GEMM (short K, register-starved
       // epilogue: the hand-off K tiles spill; without the hand-off it is within 1 % of the plain kernel),
       // which keeps the plain kernel.
-      // one wavefront per SIMD, tiles as tall as the experts' runs (see moe_gemm_quad.h), where its K loop is long enough
+      // Before either: one wavefront per SIMD, tiles as tall as the experts' runs (see moe_gemm_quad.h), where its K loop is
+      // long enough.
       if constexpr (EPI != EPI_DOWN) {
         if (!tunables().no_quad) {
           const int rc = launch_gemm_quad<T, EPI>(a, 256, splits, st);
@@ -102,7 +103,7 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       }
     case 128:
       if constexpr (EPI != EPI_DOWN) {
-        if (a.any_height) {  // a layer that leaves the tiles' heights to the kernel
+        if (a.any_height) {  // tiles as tall as the experts' runs
           fill(128, TL::T256::BF, TL::T256::BKB);
           const int rc = launch_gemm_quad<T, EPI>(a, 128, splits, st);
           if (rc != 1) return rc;
@@ -120,7 +121,7 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       return launch_gemm<T, typename TL::T128, EPI>(a, splits, st);
     case 160:
       if constexpr (EPI != EPI_DOWN) {
-        if (a.any_height) {  // a layer that leaves the tiles' heights to the kernel
+        if (a.any_height) {  // tiles as tall as the experts' runs
           fill(160, TL::T256::BF, TL::T256::BKB);
           const int rc = launch_gemm_quad<T, EPI>(a, 160, splits, st);
           if (rc != 1) return rc;

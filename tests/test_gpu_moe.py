@@ -8,6 +8,7 @@ evaluated on the same rounded operands we require
     ||out - ref||_F <= 6e-3 * ||ref||_F     (bf16; 1.5e-3 for fp16)
 """
 import sys
+import tempfile
 
 import numpy as np
 import pytest
@@ -778,12 +779,13 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
 @pytest.mark.parametrize("M,H,Fd,E,k,quad", [(1350, 4096, 2048, 8, 2, 2), (1430, 4096, 2048, 8, 2, 2), (2300, 2048, 2048, 8, 2, 2),
                                               (1200, 4096, 2048, 8, 2, 0), (2100, 2048, 2048, 8, 2, 0), (2850, 1024, 3584, 8, 2, 0),
                                               (350, 4096, 2048, 1, 1, 0), (1055, 2048, 5632, 4, 2, 0)])
-def test_plans_of_128_and_160_rows_that_leave_the_heights_to_the_kernel(native, kernels_of, M, H, Fd, E, k, quad):
+def test_layers_and_staged_entry_points_take_the_same_kernels(native, kernels_of, M, H, Fd, E, k, quad):
     """Layers whose plan routes for 128 or 160 rows: the one-wavefront-per-SIMD kernel for both GEMMs where the rule says so -
     enough pairs per expert (at the first and behind the last count of every hidden size), enough tiles, one K slice -, the
-    plan's tiles elsewhere and under no_quad."""
+    plan's tiles elsewhere and under no_quad; the stage-by-stage twin, on the staged entry points with the plan's block,
+    takes the layer's kernels and has its result."""
     import fast_route_amd as fr
-    from fast_route_amd.layers import stable_route
+    from fast_route_amd.layers import profile_fused_route, stable_route
     from fast_route_amd.layers.fused_moe import plan
     _say(f"route of plans of 128 / 160 rows M={M} H={H} F={Fd} E={E}")
     assert plan(M, H, Fd, E, k, torch.bfloat16).block in (128, 160)
@@ -795,6 +797,10 @@ def test_plans_of_128_and_160_rows_that_leave_the_heights_to_the_kernel(native, 
     count = lambda names: sum("moe_gemm_quad_kernel" in n for n in names)
     out, names = kernels_of(lambda: stable_route.fused_moe(x, gate, w1, w2, k, True))
     assert count(names) == quad, names
+    with tempfile.TemporaryDirectory() as d:
+        twin, names = kernels_of(lambda: profile_fused_route.fused_moe(x, gate, w1, w2, k, True, save_dir=d))
+    assert count(names) == quad, names
+    assert torch.equal(out, twin)
     with fr.tunables(no_quad=True):
         tiles, names = kernels_of(lambda: stable_route.fused_moe(x, gate, w1, w2, k, True))
     assert count(names) == 0, names
