@@ -718,7 +718,7 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
     block.  heights: runs that end one slot before, at and behind every unit, of one to five tiles, and an expert without a
     pair; many_experts: 130 experts (more than a wavefront's lanes) with a
     few pairs each and two long runs; odd_width: the staged entry points at widths whose last feature tile starts early
-    (F = 1088, H = 1152); plan_of_128 / plan_of_160: layers whose plan routes for smaller blocks and leaves the heights to the
+    (F = 1088, H = 1152), with prepared weights, too; plan_of_128 / plan_of_160: layers whose plan routes for smaller blocks and leaves the heights to the
     kernel."""
     import fast_route_amd as fr
     from fast_route_amd import fused_experts, fused_moe
@@ -746,14 +746,14 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
     wts = torch.rand(M, 1) + 0.5
     args = [t.cuda() for t in (x, w1, w2, wts, ids)]
 
-    def staged(x, w1, w2, wts, ids):
+    def staged(x, w1, w2, wts, ids, flags=0):
         from fast_route_amd import _native as N
         from fast_route_amd.ops.fused_moe import moe_align_block_size
         s, e, npost = moe_align_block_size(ids, 256, E)
         act = torch.zeros(s.numel(), Fd, dtype=dtype, device="cuda")
         partial = torch.empty(M * H, dtype=torch.float32, device="cuda")
         out = torch.empty(M, H, dtype=dtype, device="cuda")
-        lib, st, code = N.lib(), torch.cuda.current_stream().cuda_stream, N.dtype_code(dtype)
+        lib, st, code = N.lib(), torch.cuda.current_stream().cuda_stream, N.dtype_code(dtype) | flags
         N.check(lib.fr_moe_gateup_silu(x.data_ptr(), w1.data_ptr(), s.data_ptr(), e.data_ptr(), npost.data_ptr(), M, H, Fd, E, 1, 256, code,
                                        act.data_ptr(), None, st))
         N.check(lib.fr_moe_down_combine(act.data_ptr(), w2.data_ptr(), wts.data_ptr(), s.data_ptr(), e.data_ptr(), npost.data_ptr(), M, H,
@@ -766,6 +766,10 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
             out = experts(*args)
         with fr.tunables(block=256, no_quad=True):
             eight = experts(*args)
+        if case == "odd_width":
+            from fast_route_amd.layers.fused_moe import prepare_weights
+            p1, p2, flags = prepare_weights(args[1], args[2], "both")
+            assert torch.equal(staged(args[0], p1, p2, *args[3:], flags), out), "prepared weights"
         torch.cuda.synchronize()
     finally:
         fr.reset_tunables()
@@ -805,6 +809,31 @@ def test_layers_and_staged_entry_points_take_the_same_kernels(native, kernels_of
         tiles, names = kernels_of(lambda: stable_route.fused_moe(x, gate, w1, w2, k, True))
     assert count(names) == 0, names
     _assert_close(out, tiles.cpu(), torch.bfloat16, "one-wavefront-per-SIMD kernel against the plan's tiles")
+
+
+def test_more_than_64_tiles_per_workgroup(native, kernels_of):
+    """The one-wavefront-per-SIMD kernel works a workgroup's tiles out 64 at a time: 131 tiles of up to 288 rows x 128 feature
+    tiles on 256 workgroups are 65 or 66 each.  Operands are small integers, whose sums are exact in any order: equal to the
+    eight-wavefront kernel bit for bit."""
+    import fast_route_amd as fr
+    from fast_route_amd.ops.fused_moe import invoke_fused_moe_kernel, moe_align_block_size
+    _say("more than 64 tiles per workgroup")
+    M, N_, K = 37500, 32768, 1024
+    g = torch.Generator(device="cuda").manual_seed(99)
+    a = torch.randint(-1, 2, (M, K), generator=g, device="cuda").bfloat16()
+    b = torch.randint(-1, 2, (1, N_, K), generator=g, device="cuda").bfloat16()
+    ids = torch.zeros(M, 1, dtype=torch.int32, device="cuda")
+    s, e, npost = moe_align_block_size(ids, 256, 1)
+    res = []
+    for no_quad in (False, True):
+        c = torch.zeros(M, 1, N_, dtype=torch.bfloat16, device="cuda")
+        with fr.tunables(no_quad=no_quad):
+            _, names = kernels_of(lambda: invoke_fused_moe_kernel(a, b, c, None, ids, s, e, npost, False, 1, {"BLOCK_SIZE_M": 256}))
+        assert any("moe_gemm_quad_kernel" in n for n in names) != no_quad, names
+        res.append(c)
+    assert torch.equal(res[0], res[1])
+    rows = torch.tensor([0, 287, 288, 20000, M - 1], device="cuda")
+    assert torch.equal(res[0][rows, 0], (a[rows].float() @ b[0].float().t()).bfloat16())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
