@@ -10,12 +10,14 @@
 // Tile heights.  A tile is 1 to 9 units of 32 token rows: an expert's run of slots is cut into as few tiles as 288 rows
 // allow (quad_tiles, quad_walk, quad_tile_at), whatever the routing block.  No tile crosses into the padding behind a
 // run: an expert with 1030 pairs is multiplied as 1056 rows in four tiles where 256-row blocks made it 1280 rows in
-// five.  Layer in us, 8 experts, H = 4096, F = 14336, top-2, whole and half blocks of 256 / runs: 2048 tokens 1374 / 1200,
-// 3000 1814 / 1713, 4096 2325 / 2174, 5800 3154 / 3107, 16384 8528 / 8356; fp8 2048 769 / 680, 3100 1077 / 1007, 2500
-// 900 / 904; H = 2048, F = 1408, 64 experts, top-6, Zipf-skewed 7000 816 / 799, 8192 930 / 937.  Where the blocks had no
-// padding to lose (every expert a multiple of 256) gate/up is even and the down projection 1.5 % slower.  A K loop exists per height (kernel code per height, chosen per work unit); the height of the next
-// unit is known a tile ahead, and the hand-over always loads 288 rows' worth of addresses (rows beyond the tile are
-// outside the buffer resource and fetch nothing), so any height may follow any other.
+// five.  Layer in us, 8 experts, H = 4096, F = 14336, top-2, whole and half blocks of 256 / runs: 2048 tokens 1374 / 1190,
+// 3000 1814 / 1694, 4096 2325 / 2155, 5800 3154 / 3107, 16384 8567 / 8440; fp8 2048 769 / 680, 3100 1077 / 1007; H = 2048,
+// F = 1408, 64 experts, top-6, Zipf-skewed 7000 816 / 790, 8192 922 / 900.  Where the blocks had no padding to lose (every
+// expert a multiple of 256) gate/up is even, the down projection 1 % slower with long K loops (8 experts, 256 / 512 / 1024 /
+// 2048 rows each 262 / 264, 369 / 374, 689 / 698, 1336 / 1348 us; staged calls, a slice buffer short, 262 / 286 on the first) and
+// 2 to 5 % faster with short ones (64 experts, 256 / 512 / 1024 rows 160 / 153, 234 / 222, 424 / 416).  A K loop exists per height (kernel code per height,
+// chosen per work unit); the height of the next unit is known a tile ahead, and the hand-over always loads 288 rows' worth of
+// addresses (rows beyond the tile are outside the buffer resource and fetch nothing), so any height may follow any other.
 //
 // Stream.  With a single wavefront per SIMD nobody fills the issue slots a burst of loads or a wait leaves, so the
 // wavefront's own instruction stream is even: a K tile of 128 bytes per row is two K-steps; the one barrier per K tile
@@ -32,8 +34,8 @@
 // rows), and each of them asks for its share of the rows of a K tile several K tiles ahead - one dword per
 // 128-byte row piece, into a sink in LDS - so that the tile loads proper find their lines in L2.
 //
-// Same tail split, LDS swizzle and epilogues as moe_gemm_persistent_kernel; the result is bit-identical to the
-// eight-wavefront kernels on the same MFMA shape (same K order per accumulator).
+// Same tail split and LDS swizzle as moe_gemm_persistent_kernel; the result is bit-identical to the eight-wavefront kernels on
+// the same MFMA shape (same K order per accumulator, same roundings in the epilogue).
 #pragma once
 #include "moe_gemm_persistent.h"
 
@@ -160,9 +162,11 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
         tall = lane == l ? high[l] : tall;
       }
       // XCD 0 has the largest share
-      const XcdSchedule xs = xcd_schedule(n * a.num_f_tiles, nper, 0, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(n, E), quad_buffers(a, tall));
+      const XcdSchedule xs = xcd_schedule(n * a.num_f_tiles, nper, 0, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(n, E),
+                                          quad_buffers(a, tall));
       const unsigned tile = kTileCost + 10 * tall, rounds = xs.rounds, slices = xs.slices;
-      if (lane < NL) cost = 32 * rounds * tile + (xs.rest == 0 ? 0 : slices < 2 ? 32 * tile : 32 * tile * (rounds ? kCutStretch : 5) / (5 * slices) + kCutCost * tile);
+      const unsigned cut = 32 * tile * (rounds ? kCutStretch : 5) / (5 * slices) + kCutCost * tile;
+      if (lane < NL) cost = 32 * rounds * tile + (xs.rest == 0 ? 0 : slices < 2 ? 32 * tile : cut);
     }
     int best = kMaxUnits;
     unsigned least = __builtin_amdgcn_readlane(cost, 0);
@@ -253,9 +257,12 @@ __device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& 
 // the accumulation half of the register file (all 256 of them in a tile of 256 rows or more), the rest in the ordinary
 // half.  Left to the compiler's three-operand form, with no register of that half to spare, accumulators wandered through
 // ordinary registers around the K loop and address registers were spilled inside it (288 rows, 4096 tokens: down projection
-// 906 against 740 us).  What the compiler does not know about these instructions: an accumulator may be read by another
-// instruction 19 wait states after its last MFMA (run_unit's s_nop); MFMAs on one accumulator are as many MFMAs apart as
-// a K-step has.
+// 906 against 740 us).  What the compiler sees to for MFMAs of its own, and not for these: a result may be read by another
+// instruction 18 wait states after the last MFMA on it at the earliest (run_unit's s_nops wait 20; MFMAs on one accumulator are
+// as many MFMAs apart as a K-step has), and no vector instruction may write an operand right before the MFMA (two wait states).
+// Operands are LDS reads, which are waited for, and accumulators start from zero in an MFMA, so there is nothing to write one;
+// a change here is checked in the assembly: the 4592 MFMAs of a 2-byte kernel and the 812 of an fp8 one have no vector write
+// of an operand among the four instructions before.
 constexpr int kQuadAgpr = 8;
 #if defined(__HIP_DEVICE_COMPILE__)
 #define FQ_MFMA(name_, reg_)                                                                                     \
@@ -282,7 +289,10 @@ __device__ __forceinline__ void quad_mfma(AccT& acc, const u32x4* w, const u32x4
 // tile starts early), rows from row_end on belong to another tile, in whole token tiles: one scalar test each.  With one
 // wavefront per SIMD nothing runs beside it, so a token tile has one row address and its columns are immediate offsets of
 // the stores, and fp8's weight scales come in 16-byte loads.  A token tile is fetched, computed and stored before the next
-// is looked at: what the compiler may not do across a fence is hold all accumulators in ordinary registers.
+// is looked at: what the compiler may not do across a fence is hold all accumulators in ordinary registers.  Against the
+// epilogue that the other kernels share (column tests and an address per group, ids loaded one by one): down projection,
+// H = 2048, F = 1408, 64 experts, 8192 tokens 332 -> 309 us, 256 rows each 170 -> 153; H = 4096, F = 14336, 8 experts, 4096 tokens
+// 727 -> 720; gate/up in fp8, 2048 tokens 478 -> 456.
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // a caller's scale array is aligned to its elements
 // fp16: a product and its conversion, rounded once (one instruction, which the compiler gives up for a packed conversion where
 // it sees two side by side) or twice, through fp32.  The other tile kernels do the first for the activated rows and for two
@@ -451,7 +461,8 @@ __device__ __forceinline__ QuadPlan quad_plan(const GemmArgs& a, QuadWalk& walk,
     tiles = __builtin_amdgcn_readfirstlane(walk.off[kMaxExperts + 1] ? nt : walk.tiles[a.num_experts]);
     p.tallest = __builtin_amdgcn_readfirstlane(walk.tallest);
   }
-  p.xs = xcd_schedule(tiles * a.num_f_tiles, nper, xcd, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(tiles, a.num_experts), quad_buffers(a, p.tallest));
+  p.xs = xcd_schedule(tiles * a.num_f_tiles, nper, xcd, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(tiles, a.num_experts),
+                      quad_buffers(a, p.tallest));
   return p;
 }
 // tile t of the XCD's last round
@@ -815,7 +826,9 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     if (uA.tu < 0)
       quad_epilogue<T, C, EPI>(a, acc, uA.row0, uA.row0 + uA.units * kUnitRows, first_col(uA.f), uA.expert, wt, wf, frow_e, kgrp_e);
     else
-      tail_store<C, EPI, kQuadAgpr>(a.tail_ws + static_cast<int64_t>(xcd * quad_buffers(a, plan.tallest) + uA.tu) * (quad_buffer_rows(plan.tallest) * BF), acc, wt, wf, frow_e, kgrp_e);
+      tail_store<C, EPI, kQuadAgpr>(
+          a.tail_ws + static_cast<int64_t>(xcd * quad_buffers(a, plan.tallest) + uA.tu) * (quad_buffer_rows(plan.tallest) * BF),
+          acc, wt, wf, frow_e, kgrp_e);
   };
   for (;; ++unit) {
     // a loop of its own for every height from 4 on (fp8: 9 and the even ones), 2 and 4 for those below

@@ -132,9 +132,13 @@ int fr_moe_prepare_weights(const void* w, int dtype, int64_t E, int64_t rows, in
 
 /* ---- fused expert MLPs ---------------------------------------------------
  * Tile plan chosen from the problem size: the routing block the fused kernels
- * want (pass it to fr_moe_align) and the split-K factor of the down GEMM. */
+ * want (pass it to fr_moe_align) and the split-K factor of the down GEMM.
+ * The block is the token rows per GEMM tile up to 64.  From 128 on the GEMMs
+ * may cut an expert's run of slots into tiles of 32 to 288 rows instead,
+ * whatever the block: always where the block is 256 and K is 16 tiles of 128
+ * bytes or more, under some plans of 128 and 160 with one K slice.           */
 typedef struct fr_moe_plan {
-  int32_t block;      /* routing block = token rows per GEMM tile            */
+  int32_t block;      /* routing block                                       */
   int32_t split_k;    /* K splits of the down projection                     */
   int64_t sorted_len; /* n + E*(block-1): length of sorted_token_ids         */
   int64_t workspace_bytes; /* bytes fr_fused_moe / fr_fused_experts need     */
@@ -167,9 +171,10 @@ int fr_moe_prepare(int dtype);
  *              combine kernel.  Off by default: measured slower - 16.7 M four-byte atomics at Mixtral
  *              shape and 4096 tokens cost the down stage 1015 us against 900 us (3650 against 3200 us at
  *              16384 tokens, 149 against 146 us at 16 tokens)
- *   no_quad    1: 256-row tiles of 2-byte operands never take the one-wavefront-per-SIMD kernel
- *              (four wavefronts of 128 x 128 outputs, the default where K has 16 K tiles or more) but the
- *              eight-wavefront one; same results bit for bit, for comparisons and tests
+ *   no_quad    1: no GEMM takes the one-wavefront-per-SIMD kernel (four wavefronts, tiles as tall as the experts' runs;
+ *              the default with 256-row blocks where K has 16 K tiles or more and the width is at least a
+ *              feature tile, and under some plans of 128 and 160 rows) but the eight-wavefront ones; same
+ *              results bit for bit on the same MFMA shape, for comparisons and tests
  * fr_moe_get_plan, fr_fused_moe, fr_fused_experts, fr_fused_moe_fp8 and the staged GEMM entry
  * points all see them.  fr_moe_set_tunables(NULL) restores the defaults.
  * The staged entry points read the knobs when they are called, not when the plan was made: a
@@ -195,8 +200,8 @@ int fr_moe_get_tunables(fr_moe_tunables* t);
 /* act[s, :] = silu(x[t] @ W1[e, :F]^T) * (x[t] @ W1[e, F:]^T) for every sorted
  * slot s < num_tokens_post_pad that holds a pair (t = sorted_token_ids[s] / topk),
  * written at row s of act[sorted_len, F].  Rows of padding slots are unspecified
- * (the tile kernels fill them from token 0, the decode form for up to 4 tokens
- * leaves them untouched); nothing downstream reads them.
+ * (some kernels fill them, some leave all or part of them untouched); nothing
+ * downstream uses them.
  * Replaces: grouped GEMM 1 + silu_and_mul,
  * fast_route/fast_route/layers/stable_route.py:85-90.
  * `tail_ws`: NULL, or 256-byte aligned device scratch of plan.tail_bytes.  With
