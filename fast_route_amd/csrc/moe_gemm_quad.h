@@ -288,40 +288,19 @@ __device__ __forceinline__ void quad_mfma(AccT& acc, const u32x4* w, const u32x4
 // Epilogue of a tile [row0, row_end) x columns from f0 on.  Every column exists (a width below a tile's is not taken, the last
 // tile starts early), rows from row_end on belong to another tile, in whole token tiles: one scalar test each.  With one
 // wavefront per SIMD nothing runs beside it, so a token tile has one row address and its columns are immediate offsets of
-// the stores, and fp8's weight scales come in 16-byte loads.  A token tile is fetched, computed and stored before the next
+// the stores, which are 16 bytes wide (join_features), and fp8's weight scales come in 16-byte loads.  A token tile is fetched, computed and stored before the next
 // is looked at: what the compiler may not do across a fence is hold all accumulators in ordinary registers.  Against the
 // epilogue that the other kernels share (column tests and an address per group, ids loaded one by one): down projection,
 // H = 2048, F = 1408, 64 experts, 8192 tokens 332 -> 309 us, 256 rows each 170 -> 153; H = 4096, F = 14336, 8 experts, 4096 tokens
 // 727 -> 720; gate/up in fp8, 2048 tokens 478 -> 456.
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // a caller's scale array is aligned to its elements
-// fp16: a product and its conversion, rounded once (one instruction, which the compiler gives up for a packed conversion where
-// it sees two side by side) or twice, through fp32.  The other tile kernels do the first for the activated rows and for two
-// of every four values of a pair's row, and so does the epilogue here.
-#if defined(__HIP_DEVICE_COMPILE__)
-template <typename O>
-__device__ __forceinline__ O round_once(float product) {
-  O o = static_cast<O>(product);
-  if constexpr (std::is_same<O, f16_t>::value) asm("" : "+v"(o));
-  return o;
-}
-template <typename O>
-__device__ __forceinline__ O round_twice(float product) {
-  if constexpr (std::is_same<O, f16_t>::value) asm("" : "+v"(product));
-  return static_cast<O>(product);
-}
 // a loaded value is waited for here and not where it is used
 template <typename V>
 __device__ __forceinline__ void arrived(V& v) {
+#if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("" : "+v"(v));
-}
-#else
-template <typename O>
-__device__ __forceinline__ O round_once(float product) { return static_cast<O>(product); }
-template <typename O>
-__device__ __forceinline__ O round_twice(float product) { return static_cast<O>(product); }
-template <typename V>
-__device__ __forceinline__ void arrived(V&) {}
 #endif
+}
 template <typename T, typename C, int EPI, typename AccT>
 __device__ __forceinline__ void quad_epilogue(const GemmArgs& a, AccT (&acc)[C::JF][C::IT], int row0, int row_end, int f0, int expert,
                                               int wt, int wf, int frow, int kgrp) {
@@ -382,31 +361,44 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& a, AccT (&acc)[C::
       for (int x = 0; x < C::JF * GROUPS; ++x) arrived(wscale[x]);
     }
   }
+  // pairs of accumulator groups, joined into 16-byte stores: (MFMA tile j, j + 1) or, with 32 x 32 tiles, groups (g, g + 1)
+  constexpr int JS = GROUPS == 1 ? 2 : 1, PAIRS = GROUPS == 1 ? 1 : GROUPS / 2;
+  typedef out_t out8 __attribute__((ext_vector_type(8), aligned(8)));  // rows of a width that is a multiple of 4
+  const int colw = f0 + wf * TF + kgrp * 8;
 #pragma unroll
   for (int i = 0; i < C::IT; ++i) {
     if (slot0 + i * C::TILE >= row_end) break;
+    auto fetch = [&](int j) { return i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i]; };
     if constexpr (EPI == EPI_SILU) {
-      out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot0 + i * C::TILE + frow) * a.ldo + col0;
+      out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(slot0 + i * C::TILE + frow) * a.ldo + colw;
+      auto value = [&](const AccT& ga, const AccT& ua, int j, int g) {
+        out4 o;
 #pragma unroll
-      for (int j = 0; j < HJ; ++j) {
-        const AccT ga = i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i], ua = i < kQuadAgpr ? acc_fetch(acc[j + HJ][i]) : acc[j + HJ][i];
-#pragma unroll
-        for (int g = 0; g < GROUPS; ++g) {
-          out4 o;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float gv = ga[g * 4 + r], uv = ua[g * 4 + r];
-            if constexpr (E::SCALED) {
-              gv *= scale[i] * wscale[j * GROUPS + g][r];
-              uv *= scale[i] * wscale[(j + HJ) * GROUPS + g][r];
-            }
-            o[r] = round_once<out_t>(silu(gv) * uv);
+        for (int r = 0; r < 4; ++r) {
+          float gv = ga[g * 4 + r], uv = ua[g * 4 + r];
+          if constexpr (E::SCALED) {
+            gv *= scale[i] * wscale[j * GROUPS + g][r];
+            uv *= scale[i] * wscale[(j + HJ) * GROUPS + g][r];
           }
-          *reinterpret_cast<out4*>(row + j * C::TILE + g * 8) = o;
+          o[r] = round_once<out_t>(silu(gv) * uv);
+        }
+        return o;
+      };
+#pragma unroll
+      for (int j = 0; j < HJ; j += JS) {
+        const AccT ga = fetch(j), ua = fetch(j + HJ);
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) {
+          out4 lo = value(ga, ua, j, GROUPS == 1 ? 0 : 2 * p), hi;
+          if constexpr (GROUPS == 1) hi = value(fetch(j + 1), fetch(j + 1 + HJ), j + 1, 0);
+          else hi = value(ga, ua, j, 2 * p + 1);
+          join_features<C::TILE>(lo, hi);
+          *reinterpret_cast<out8*>(row + j * C::TILE + p * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-    } else if (sids[i] < a.num_valid) {
+    } else {
+      const bool valid = sids[i] < a.num_valid;
       auto value = [&](const AccT& c, int j, int g) {
         out4 o;
 #pragma unroll
@@ -421,17 +413,24 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& a, AccT (&acc)[C::
         out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(sids[i] / a.add_div) * a.ldo + col0;
 #pragma unroll
         for (int j = 0; j < C::JF; ++j) {
-          const AccT c = i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i];
+          const AccT c = fetch(j);
 #pragma unroll
-          for (int g = 0; g < GROUPS; ++g) atomic_add4(row + j * C::TILE + g * 8, value(c, j, g));
+          for (int g = 0; g < GROUPS; ++g)
+            if (valid) atomic_add4(row + j * C::TILE + g * 8, value(c, j, g));
         }
       } else {
-        out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(sids[i]) * a.ldo + col0;
+        out_t* row = static_cast<out_t*>(a.out) + static_cast<int64_t>(sids[i]) * a.ldo + colw;
 #pragma unroll
-        for (int j = 0; j < C::JF; ++j) {
-          const AccT c = i < kQuadAgpr ? acc_fetch(acc[j][i]) : acc[j][i];
+        for (int j = 0; j < C::JF; j += JS) {
+          const AccT c = fetch(j);
 #pragma unroll
-          for (int g = 0; g < GROUPS; ++g) *reinterpret_cast<out4*>(row + j * C::TILE + g * 8) = value(c, j, g);
+          for (int p = 0; p < PAIRS; ++p) {
+            out4 lo = value(c, j, GROUPS == 1 ? 0 : 2 * p), hi;
+            if constexpr (GROUPS == 1) hi = value(fetch(j + 1), j + 1, 0);
+            else hi = value(c, j, 2 * p + 1);
+            join_features<C::TILE>(lo, hi);
+            if (valid) *reinterpret_cast<out8*>(row + j * C::TILE + p * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          }
         }
       }
     }

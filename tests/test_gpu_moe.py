@@ -413,6 +413,29 @@ def test_grouped_gemm_with_blocks_in_any_order(native, block):
     _assert_close(c1.view(M * k, -1), oracle.grouped_gemm(x, w1, w, ids, False, k), dtype, "reversed blocks")
 
 
+@pytest.mark.parametrize("N", [256, 260, 388, 516])
+@pytest.mark.parametrize("block", [16, 32, 64, 128, 160, 256])
+def test_rows_of_whole_and_partial_tiles(native, block, N):
+    """16-byte stores of whole tiles: output rows that start at multiples of 8 bytes only (N = 4 mod 8), with a last tile that is
+    narrower than the others; K long enough for the 256-row tile with one wavefront per SIMD.  What lies around C stays as it is."""
+    from fast_route_amd.ops.fused_moe import invoke_fused_moe_kernel, moe_align_block_size
+    _say(f"grouped GEMM, N={N}, block={block}")
+    M, K, E, k = 300, 1024, 5, 2
+    for dtype in (torch.bfloat16, torch.float16):
+        x, logits, _, w = _inputs(M, N, K, E, 43 + N, dtype)  # w: [E, N, K]
+        x = torch.randn(M, K, generator=torch.Generator().manual_seed(N)).to(dtype)
+        wt, ids = oracle.gating_topk(logits, k)
+        s, e, npost = moe_align_block_size(ids.cuda(), block, E)
+        cfg = {"BLOCK_SIZE_M": block, "BLOCK_SIZE_N": 64, "BLOCK_SIZE_K": 32, "GROUP_SIZE_M": 8}
+        guard = 8 * N
+        buf = torch.full((2 * guard + M * k * N,), 7.0, dtype=dtype, device="cuda")
+        c = buf[guard:-guard].view(M, k, N)
+        invoke_fused_moe_kernel(x.cuda(), w.cuda(), c, wt.cuda(), ids.cuda(), s, e, npost, True, k, cfg)
+        torch.cuda.synchronize()
+        assert (buf[:guard] == 7).all() and (buf[-guard:] == 7).all()
+        _assert_close(c.view(M * k, N), oracle.grouped_gemm(x, w, wt, ids, True, k), dtype, f"{dtype}")
+
+
 def test_stable_and_vllm_route_layers(native):
     """Gate-matrix entry points of both reference layers."""
     from fast_route_amd.layers import stable_route, vllm_route
