@@ -301,10 +301,11 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   // non-temporal the stream does not displace the token rows and its own neighbours in L2
   bool ntA = false, ntB = false;
   constexpr bool NTW = BT < 256;  // the 256-row tiles have no register to spare for the second form of the loads
-#define FR_MAKE_SET(pt_, pf_, ex_, kb_, SIDOF, xsrc_, wsrc_, xrs_, wrs_, nt_)                                   \
+#define FR_MAKE_SET(pt_, pf_, ex_, SIDOF, xsrc_, wsrc_, xrs_, wrs_, nt_)                                        \
   {                                                                                                          \
     const int64_t xrow0_ = a.top_k > 0 ? 0 : static_cast<int64_t>(pt_) * BT;                                 \
-    const int64_t kfirst_ = k0 + static_cast<int64_t>(kb_) * BK;                                             \
+    int64_t kfirst_ = k0;                                                                                    \
+    asm volatile("" : "+s"(kfirst_)); /* or the lanes' parts of the offsets stay in registers between units */ \
     xrs_ = uniform_rsrc(X + xrow0_ * a.ldx, a.x_span ? a.x_span : 0xFFFFFFFFu);                              \
     wrs_ = uniform_rsrc(static_cast<const T*>(a.W) + static_cast<int64_t>(ex_) * a.w_expert_stride);         \
     nt_ = NTW && !expert_off[kMaxExperts + 1] && expert_off[(ex_) + 1] - expert_off[ex_] == 1;               \
@@ -322,8 +323,26 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
                                                       (kfirst_ + c * EPC) * static_cast<int64_t>(sizeof(T)), sizeof(T))); \
     }                                                                                                        \
   }
+  // K tile a unit starts at: it walks its K tiles from there on, round the end.  The rows of a weight matrix are a power of two
+  // (or a multiple of 4 KB) long in most models, and workgroups that stream different rows of it at the same pace ask for the same
+  // columns, i.e. for a few of the memory channels, all at once: pure streaming with these loads and 128 token rows
+  // next to them reaches 5.4 TB/s (8 KB rows; 4 KB 5.6) and 6.5 (6.4) with the starts spread.  A tile that is alone on its
+  // weight tile starts at a place of its own (multiples of the golden ratio: any run of consecutive tiles is spread evenly); tiles
+  // that share theirs go on in step.  Layer in us, from column 0 / spread: H = 2048, F = 1408, 64 experts, top-6, 509 tokens
+  // 252 / 239, 1000 291 / 277, 2000 384 / 375; H = 4096, F = 14336, 8 experts 256 tokens 526 / 508, 400 547 / 520, 600 623 / 599; H = 6144,
+  // F = 16384 400 tokens 884 / 814; fp8 150 tokens 274 / 268, 300 330 / 307.  Two blocks per expert spread as well (1031 tokens
+  // 818 / 833, H = 6144 900 tokens 1297 / 1317): one of them finds its rows gone from L2.  Not for 2-byte tiles of 256-byte row pieces
+  // (64 rows, 150 tokens 452 / 461), which touch two channels' worth of every row at a time.
+  constexpr bool SPREAD_K = NTW && BT >= 64 && (C::BKB == 128 || sizeof(T) == 1);
+  auto first_k_tile = [&](bool alone, int ex, int pf, int kb_) -> int {
+    const int kb_u = __builtin_amdgcn_readfirstlane(kb_);
+    if (!SPREAD_K || !__builtin_amdgcn_readfirstlane(alone)) return kb_u;
+    const unsigned tile = __builtin_amdgcn_readfirstlane(ex * a.num_f_tiles + pf);
+    const int k = kb_u + static_cast<int>(__umulhi(tile * 2654435769u, static_cast<unsigned>(k_all)));
+    return k >= k_all ? k - k_all : k;
+  };
   FR_UNIT(0, pid_t, pid_f, expert, kb, kn, tu)
-  FR_MAKE_SET(pid_t, pid_f, expert, kb, a.sorted[pid_t * BT + rr], xsrcA, wsrcA, xrsA, wrsA, ntA)
+  FR_MAKE_SET(pid_t, pid_f, expert, a.sorted[pid_t * BT + rr], xsrcA, wsrcA, xrsA, wrsA, ntA)
 
   // Measurement switches (compile time; results are WRONG with any of them, only timings mean something):
   //   FR_ABL_NOLOAD  the ring is filled once and never refilled: MFMAs + fragment reads + barriers on real data
@@ -449,9 +468,9 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   }
   // One K tile of the current output tile.  REFILL: 0 none (the data is the last this
   // workgroup loads), else the slot of this K tile is refilled from set SET with K tile
-  // rtile_ after the barrier that publishes the next K tile; LAST: nothing follows this K
+  // kw after the barrier that publishes the next K tile; LAST: nothing follows this K
   // tile at all (no barrier, no fragment read-ahead).
-#define FR_KTILE(ISS_, REFILL, SET, rtile_, LAST, VMC)                                         \
+#define FR_KTILE(ISS_, REFILL, SET, LAST, VMC)                                                 \
   {                                                                                            \
     const int sn = (sl + 1 == S) ? 0 : sl + 1;                                                 \
     _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) {                                        \
@@ -462,10 +481,11 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
       } else {                                                                                 \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VMC) : "memory");                  \
         FR_KT_BARRIER                                                                          \
-        FR_KSTEP(ks & 1, true, sn, 0, (ISS_) && (REFILL), SET, rtile_, sl);                    \
+        FR_KSTEP(ks & 1, true, sn, 0, (ISS_) && (REFILL), SET, kw, sl);                        \
       }                                                                                        \
     }                                                                                          \
     sl = sn;                                                                                   \
+    if (REFILL) kw = kw + 1 == k_all ? 0 : kw + 1;                                             \
   }
   // One output tile.  NEXT (compile time): the workgroup has another tile after this one, whose
   // routing data is asked for at the start, turned into the address set B after two K tiles
@@ -498,16 +518,17 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
       _Pragma("unroll") for (int i = 0; i < C::IT; ++i)                                                    \
         _Pragma("unroll") for (int r = 0; r < ACC_N; ++r) acc[j][i][r] = 0.f;                              \
     /* vmcnt(0) once per tile: the previous tile's epilogue stores share the counter with the loads */     \
-    FR_KTILE(ISS_, true, A, S, false, 0)                                                                   \
-    FR_KTILE(ISS_, true, A, S + 1, false, (S - 2) * NLI)                                                   \
-    if (NEXT) FR_MAKE_SET(n_pid_t, n_pid_f, n_expert, n_kb, n_sid[ih], xsrcB, wsrcB, xrsB, wrsB, ntB)      \
+    FR_KTILE(ISS_, true, A, false, 0)                                                                      \
+    FR_KTILE(ISS_, true, A, false, (S - 2) * NLI)                                                          \
+    if (NEXT) FR_MAKE_SET(n_pid_t, n_pid_f, n_expert, n_sid[ih], xsrcB, wsrcB, xrsB, wrsB, ntB)            \
     __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0): no scalar load pending inside the loops */          \
-    for (int kt = 2; kt < kn - S; ++kt) FR_KTILE(ISS_, true, A, kt + S, false, (S - 2) * NLI)              \
+    for (int kt = 2; kt < kn - S; ++kt) FR_KTILE(ISS_, true, A, false, (S - 2) * NLI)                      \
     if (NEXT) {                                                                                            \
-      for (int kt = 0; kt < S; ++kt) FR_KTILE(ISS_, true, B, kt, false, (S - 2) * NLI)                     \
+      kw = first_k_tile(ntB, n_expert, n_pid_f, n_kb);                                                     \
+      for (int kt = 0; kt < S; ++kt) FR_KTILE(ISS_, true, B, false, (S - 2) * NLI)                         \
     } else {                                                                                               \
-      for (int kt = 0; kt < S - 1; ++kt) FR_KTILE(ISS_, false, A, 0, false, 0)                             \
-      FR_KTILE(ISS_, false, A, 0, true, 0)                                                                 \
+      for (int kt = 0; kt < S - 1; ++kt) FR_KTILE(ISS_, false, A, false, 0)                                \
+      FR_KTILE(ISS_, false, A, true, 0)                                                                    \
     }                                                                                                      \
     FR_STAMP(1)                                                                                            \
     if (tu < 0) gemm_epilogue<T, C, EPI, HOIST>(a, acc, pid_t * BT, pid_f * (EPI == EPI_SILU ? BF / 2 : BF), expert, split, wt, wf, frow, kgrp);         \
@@ -516,8 +537,10 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   // Fill of the ring with the first S K tiles of set A and the first fragments.
 #define FR_FILL(ISS_)                                                                                      \
   {                                                                                                        \
-    _Pragma("unroll") for (int t = 0; t < S; ++t)                                                          \
-      if (ISS_) { _Pragma("unroll") for (int q = 0; q < NLI; ++q) FR_ISSUE_REAL(A, t, t, q); }              \
+    _Pragma("unroll") for (int t = 0; t < S; ++t) {                                                        \
+      if (ISS_) { _Pragma("unroll") for (int q = 0; q < NLI; ++q) FR_ISSUE_REAL(A, kw, t, q); }             \
+      kw = kw + 1 == k_all ? 0 : kw + 1;                                                                   \
+    }                                                                                                      \
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * NLI) : "memory");                                   \
     __builtin_amdgcn_s_barrier();                                                                          \
     FR_READ_FRAGS_REAL(0, 0, 0);                                                                           \
@@ -526,6 +549,7 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   // Whole pipeline for an issuing (ISS_ = true) or a non-issuing wavefront.
 #define FR_PERSIST(ISS_)                                                                                   \
   {                                                                                                        \
+    int kw = first_k_tile(ntA, expert, pid_f, kb); /* the K tile the next refill fetches */                \
     FR_FILL(ISS_)                                                                                          \
     int sl = 0;                                                                                            \
     int unit = 0;                                                                                          \

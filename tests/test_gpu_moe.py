@@ -436,6 +436,36 @@ def test_rows_of_whole_and_partial_tiles(native, block, N):
         _assert_close(c.view(M * k, N), oracle.grouped_gemm(x, w, wt, ids, True, k), dtype, f"{dtype}")
 
 
+@pytest.mark.parametrize("split", [1, 3])
+@pytest.mark.parametrize("H,Fd", [(384, 1152), (640, 1664), (2432, 2176)])
+@pytest.mark.parametrize("block", [64, 128, 160])
+def test_k_starts_of_tiles_alone_on_their_weights(native, block, H, Fd, split):
+    """A tile that is alone on its weight tile walks its K tiles from a place of its own, round the end: K loops from the
+    shortest the persistent kernels take (6 K tiles) up, odd counts, K slices and cut last rounds, experts with one
+    block next to experts with several and with none."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_experts
+    E = 12
+    counts = np.array([block, block - 1, 1, 0, 17, 3 * block + 5, block // 2, 0, block + 1, 33, 2, block])
+    rng = np.random.default_rng(H + block)
+    ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E), counts))).int().view(-1, 1)
+    M = ids.shape[0]
+    _say(f"K starts block={block} H={H} F={Fd} split={split}")
+    for dtype in (torch.bfloat16, torch.float16):
+        x, _, w1, w2 = _inputs(M, H, Fd, E, 5 + H, dtype)
+        wts = torch.rand(M, 1, generator=torch.Generator().manual_seed(M)) + 0.5
+        ref = oracle.moe_experts(x, w1, w2, wts, ids)
+        xd, w1d, w2d, wd, idd = x.cuda(), w1.cuda(), w2.cuda(), wts.cuda(), ids.cuda()
+        try:
+            with fr.tunables(block=block, split_k=split, no_quad=True):
+                out, again = fused_experts(xd, w1d, w2d, wd, idd), fused_experts(xd, w1d, w2d, wd, idd)
+        finally:
+            fr.reset_tunables()
+        torch.cuda.synchronize()
+        assert torch.equal(out, again)
+        _assert_close(out, ref, dtype, f"{dtype}")
+
+
 def test_stable_and_vllm_route_layers(native):
     """Gate-matrix entry points of both reference layers."""
     from fast_route_amd.layers import stable_route, vllm_route
