@@ -54,6 +54,7 @@ int gateup_rows_routed(const void* x, const void* w1, const void* logits, int lo
 int prepare_static_scratch();
 
 constexpr int kTailDescBytes = 8192;  // what TailScratch::cuts points to
+constexpr int64_t kTallTailBytes = int64_t(256) * 288 * 256 * 4;  // slice buffers of the tallest tiles, one per workgroup
 
 // Scratch of a grouped GEMM for cutting the tiles of its last round along K (plan.tail_bytes, or nullptr), a place for the
 // list of the tiles cut (kTailDescBytes, or nullptr: taken from the scratch's end), and whether the tiles' heights may
@@ -63,6 +64,7 @@ struct TailScratch {
   float* buffers = nullptr;
   int* cuts = nullptr;
   bool any_height = false;
+  bool tall = false;  // buffers holds kTallTailBytes (at least plan.tail_bytes)
 };
 
 bool plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block);

@@ -61,7 +61,7 @@ struct Carve {
   void* actq;
   float* act_scale;
   int64_t total;
-  TailScratch tail_scratch() const { return TailScratch{tail, tail_cuts, any_height}; }
+  TailScratch tail_scratch() const { return TailScratch{tail, tail_cuts, any_height, tail != nullptr}; }
 };
 
 // the activated intermediate is stored in half precision also on the fp8 path
@@ -82,7 +82,7 @@ Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dt
   c.align_ws = take(c.align_ws_bytes);
   c.act = take(p.sorted_len * F * act_elem_size(dtype));
   c.partial = reinterpret_cast<float*>(take(static_cast<int64_t>(p.split_k) * n * H * 4));
-  c.tail = p.tail_bytes > 0 ? reinterpret_cast<float*>(take(p.tail_bytes)) : nullptr;
+  c.tail = p.tail_bytes > 0 ? reinterpret_cast<float*>(take(p.tail_bytes > kTallTailBytes ? p.tail_bytes : kTallTailBytes)) : nullptr;
   c.any_height = any_height(M, H, F, E, topk, dtype, p);
   c.tail_cuts = p.tail_bytes > 0 ? reinterpret_cast<int*>(take(kTailDescBytes)) : nullptr;
   c.xq = nullptr; c.x_scale = nullptr; c.actq = nullptr; c.act_scale = nullptr;

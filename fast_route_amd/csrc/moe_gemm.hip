@@ -181,6 +181,7 @@ int gateup_impl(const void* x, const float* x_scale, const void* w1, const float
   a.num_experts = E;
   a.tail_ws = tail.buffers;
   a.tail_desc = tail.cuts;
+  a.tail_tall = tail.tall;
   a.any_height = tail.any_height;
   a.w_tiled = w_tiled;
   // batches the routed form of the row kernel takes run the row kernel here too (same kernel, same sums, whoever
@@ -242,6 +243,7 @@ int down_impl(const void* act, const float* act_scale, const void* w2, const flo
   a.num_experts = E;
   a.tail_ws = tail.buffers;
   a.tail_desc = tail.cuts;
+  a.tail_tall = tail.tall;
   a.any_height = tail.any_height;
   a.long_k = 1;
   a.w_tiled = w_tiled;

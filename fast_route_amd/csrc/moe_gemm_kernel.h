@@ -61,7 +61,9 @@ struct GemmArgs {
   int long_k;           // down projection (few feature tiles, long K): hint for the form of the 128- and 16-row tiles
   float* tail_ws;       // persistent form only: slice buffers for splitting the last round of tiles along K, or nullptr
   int* tail_desc;       // one-wavefront-per-SIMD form only: kTailDescBytes next to tail_ws, or nullptr (they are taken from its end)
+  int tail_tall;        // tail_ws holds kTallTailBytes
   int tail_buffers;     // slice buffers of 256 x 256 fp32 per XCD
+  int tall_buffers;     // of 288 x 256
   unsigned x_span;      // bytes of X the tile loads may address (from X in gather mode, from a block's first row otherwise), or 0:
                         // with it, the loads of padding slots fall outside the buffer resource and fetch nothing
   int add_div;          // EPI_PLAIN: 0 = store row `sorted id` of out; k > 0 = add into row (sorted id / k) of a zero-filled out (packed atomics)

@@ -64,17 +64,21 @@ constexpr int kTileCost = 26;
 // whole one: 8 units 264 / 283, 4 experts, 16 units 203 / 231.
 constexpr int kCutCost = 4, kCutStretch = 8;
 constexpr int kQuadRing = 2 * (kUnitRows * kMaxUnits + 256) * 128;
-// Slice buffers of the cut last round, per XCD of 32 workgroups: 32 of 256 x 256 fp32 or, with 288-row tiles, 28 of 288 x 256.
+// Slice buffers of the cut last round, per XCD of 32 workgroups: 32 of 256 x 256 fp32 or, with 288-row tiles, as many of 288 x 256:
+// the layers' scratch has room for 32 of these too, a staged caller's (fr_moe_plan.tail_bytes) for 28.  Half a round of 288-row tiles
+// takes 32 for two slices each: H = 4096, F = 14336, 8 experts, one tile per expert and feature tile (gate/up: 3 1/2 rounds), layer
+// with 28 / 32 buffers 1031 tokens 780 / 769 us, 950 771 / 767; H = 6144, 1031 tokens 1320 / 1311.
 // What the fix-up launch needs to know about a cut tile is left next to them (QuadCut), in the scratch itself where the
 // caller has no other place for it: then there are 31 buffers of 256 rows.  (Working it out again in the fix-up launch instead
 // costs staged calls 8 to 12 us: down projection, 8 experts, 1300 tokens 302 / 314, 2048 381 / 393.)
 constexpr int kQuadTallBuffers = 28;
 __device__ __forceinline__ int quad_buffer_rows(int tallest) { return tallest > 8 ? kUnitRows * kMaxUnits : 256; }
-__device__ __forceinline__ int quad_buffers(const GemmArgs& a, int tallest) { return tallest > 8 ? kQuadTallBuffers : a.tail_buffers; }
+__device__ __forceinline__ int quad_buffers(const GemmArgs& a, int tallest) { return tallest > 8 ? a.tall_buffers : a.tail_buffers; }
 struct QuadCut {
   int row0, units, f, expert, slices, rest, buffers, buffer_rows;  // slices 0: tile is not cut
 };
 static_assert(sizeof(QuadCut) * kTailUnits <= kTailDescBytes, "a tile per workgroup");
+static_assert(static_cast<int64_t>(kTailUnits) * kUnitRows * kMaxUnits * 256 * 4 == kTallTailBytes, "32 buffers per XCD in the layers' scratch");
 static_assert(8 * kQuadTallBuffers * kUnitRows * kMaxUnits * 256 * 4 + kTailDescBytes <= kTailUnits * 256 * 256 * 4 &&
                   8 * 31 * 256 * 256 * 4 + kTailDescBytes <= kTailUnits * 256 * 256 * 4, "fits the scratch");
 
@@ -961,6 +965,7 @@ int launch_gemm_quad(const GemmArgs& a_in, int block, int splits, hipStream_t st
   const bool tail = a.tail_ws && a.K / BK >= kTailMinTiles && a.N % COLS == 0 && worst * block < max_rounds * resident * 256;
   if (!tail) a.tail_ws = nullptr;
   a.tail_buffers = 32;
+  a.tall_buffers = a.tail_tall ? 32 : kQuadTallBuffers;
   if (tail && !a.tail_desc) {
     a.tail_desc = reinterpret_cast<int*>(a.tail_ws + kTailUnits * 256 * 256) - kTailDescBytes / 4;
     a.tail_buffers = 31;
