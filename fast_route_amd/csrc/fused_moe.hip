@@ -21,14 +21,25 @@ double expected_blocks(double avg, int E, int rows) {
 
 // A layer whose plan routes for 128 or 160 rows and runs the one-wavefront-per-SIMD kernel all the same, with tiles as tall as
 // the experts' runs (moe_gemm_quad.h).  Layer in us, the plan's own tiles / that kernel:
-//   H = 4096, F = 14336, 8 experts   bf16 1031 tokens (258 pairs per expert) 800 / 797, 1100 815 / 819, 1180 864 / 865,
-//                                    1240 (310) 973 / 893, 1280 995 / 908, 1430 1078 / 945, 1500 1133 / 969, 2300 1480 / 1406,
-//                                    2420 1520 / 1478; fp8 1100 511 / 524, 1180 542 / 564, 1250 614 / 556
-//   16 experts, F = 8192, fp16       2300 (288) 1022 / 1046, 2490 (311) 1108 / 1065, 4400 1727 / 1581
+//   H = 4096, F = 14336, 8 experts   bf16 1240 tokens (310 pairs per expert) 973 / 893, 1280 995 / 908, 1430 1078 / 945, 1500
+//                                    1133 / 969, 2300 1480 / 1406, 2420 1520 / 1478; fp8 1250 614 / 556
+//   16 experts, F = 8192, fp16       2490 (311) 1108 / 1065, 4400 1727 / 1581
 //   H = 3072, F = 4096, 16 experts   4500 (562) 0.96, 5000 0.92 of the plan's tiles
 //   H = 2048, F = 1408, 64 experts, top-6, Zipf-skewed: 5600 (525) 1.04 to 1.06, 5900 (553) 0.96, 6200 0.96 to 0.99, 7100 0.97
 //   H = 2048, F = 8192, 8 experts    2200 (550) 0.98, 2500 0.92; fp8 0.92, 0.85
 //   H = 1024, F = 3584, 8 experts    2200 to 4096 0.93 to 1.03, 4142 (1036) 0.87
+// With fewer pairs (H >= 4096), where an expert's run is one tile of it and the plan's rows make it two: the weights pass through the
+// CUs once.  Up to 7 units (fp8: 6) such a tile streams its weights (moe_gemm_quad.h); 8 and 9 units gain less and lose to
+// the plan's tiles in a launch of few.
+//   H = 4096, F = 14336, 8 experts   645 (161) 735 / 635, 700 735 / 637, 850 783 / 702, 950 802 / 778, 1031 (258) 832 / 797, 1080
+//                                    845 / 826, but 1120 (280: some experts two tiles) 841 / 851, 1160 855 / 881, 1200 880 / 890
+//                                    fp8 640 441 / 397, 700 426 / 401, but 740 (185) 437 / 433, 800 442 / 452, 950 475 / 473
+//   H = 6144, F = 16384              700 1280 / 1108, 1000 1425 / 1342; one block of 160 rows per expert: 580 (145) 958 / 1097
+//   16 experts, F = 8192, fp16       1240 (155) 753 / 679, 1300 837 / 688, 1900 963 / 866, 2200 (275) 1008 / 1037; one block: 700
+//                                    593 / 611, 960 (120) 610 / 650, 1100 652 / 668
+//   H = 5120, F = 8192, 16 experts   1350 (169) 1075 / 922, 2000 1214 / 1099; H = 7168, F = 2048, 64 experts, top-8 1350 1487 / 1311
+//   H = 4096, F = 4096, 8 experts    640 250 / 203, 750 251 / 220, but 1000 (250; 256 gate/up tiles) 270 / 281; F = 1536, 32
+//                                    experts, top-4 1350 358 / 333, 1700 382 / 367, 2000 (250; 384) 400 / 409
 // A few tiles leave the chip idle whatever their height, and the smaller ones less of it: one expert, F = 4096 (64 gate/up
 // tiles) 350 tokens 1.20, 570 1.11, F = 2048 1.21, 1.13; 8 experts, F = 1024 (128 and 192 tiles) 1400 1.02, 2300 1.07; but one
 // expert, F = 14336 (224) 0.97, 8 experts, F = 2048 (256) 1400 0.87.
@@ -39,8 +50,10 @@ bool any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, con
   if ((p.block != 128 && p.block != 160) || p.split_k > 1 || t.no_quad || t.block || E > 1022) return false;
   const int es = dtype == FR_FP8_E4M3 ? 1 : 2;
   if (H * es < 2048 || F * es < 2048) return false;  // 16 K tiles in both GEMMs
-  const double avg = static_cast<double>(M) * topk / E;
-  return avg >= (H >= 4096 ? 310.0 : H >= 2048 ? 550.0 : 1030.0) && E * expected_blocks(avg, E, 288) * (F / 128) >= 200.0;
+  const double avg = static_cast<double>(M) * topk / E, tall = expected_blocks(avg, E, 288), tiles = E * tall * (F / 128);
+  if (avg >= (H >= 4096 ? 310.0 : H >= 2048 ? 550.0 : 1030.0)) return tiles >= 200.0;
+  if (H < 4096 || expected_blocks(avg, E, p.block) < 1.3) return false;
+  return (expected_blocks(avg, E, es == 2 ? 224 : 192) <= 1.13 && tiles >= 200.0) || (es == 2 && tall <= 1.13 && tiles >= 450.0);
 }
 
 struct Carve {

@@ -32,6 +32,17 @@ enum { EPI_PLAIN = 0, EPI_SILU = 1, EPI_DOWN = 2 };
 #define FR_W_AUX (C::BT <= 64 ? 2 : 0)
 #endif
 
+// Start of a K loop of k_all K tiles for number `n` of a set of tiles, from its own start kb on round the end: multiples of the golden
+// ratio, so that any run of consecutive numbers is spread evenly.  Why: see SPREAD_K in moe_gemm_persistent.h.
+__device__ __forceinline__ int spread_k_start(int kb, int n, int k_all) {
+  const int k = kb + static_cast<int>(__umulhi(static_cast<unsigned>(n) * 2654435769u, static_cast<unsigned>(k_all)));
+  return k >= k_all ? k - k_all : k;
+}
+// The 256-row kernels give an expert whose run fits a block of 256 rows (8 units of 32) a start per four feature tiles: with up to 256
+// token rows next to the weights, feature tiles that share the rows in L2 are kept in step.  Widths that are no
+// multiple of a tile's are not spread (the one-wavefront-per-SIMD kernel computes some of their columns twice).
+__device__ __forceinline__ int spread_k_start256(int expert, int f, int f_tiles, int kb, int k_all) { return spread_k_start(kb, (expert * f_tiles + f) >> 2, k_all); }
+
 struct GemmArgs {
   const void* X;        // token rows [*, K]
   int64_t ldx;          // row stride of X in elements
@@ -70,6 +81,7 @@ struct GemmArgs {
   unsigned div_mul;     // division by top_k of the one-wavefront-per-SIMD form (quad_divisor)
   int div_shift;
   int any_height;       // the tiles' heights need not be the routing block's (TailScratch::any_height)
+  int spread_k;         // one-wavefront-per-SIMD form: units of short runs start their K loop at spread places
   int w_tiled;          // W is in the prepared layout (see w_byte_offset), not [E, w_rows, K] row-major
   int setup_only;       // do the per-device set-up of the kernel a launch would take (LDS limit, occupancy) and launch nothing
 };
@@ -546,6 +558,11 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_kernel(const GemmArgs
   const T* W = static_cast<const T*>(a.W) + static_cast<int64_t>(expert) * a.w_expert_stride;
   const int k0 = split * a.k_per_split;
   const int k_tiles = min(a.k_per_split, a.K - k0) / BK;
+  int k_first = 0;  // K tile the walk starts at (the 256-row tile of fp8's gate/up GEMM only; as in the kernels it stands in for)
+  if constexpr (BT == 256 && E::SCALED) {
+    if (a.N % (EPI == EPI_SILU ? BF / 2 : BF) == 0 && (pid_t == 0 || a.expert_ids[pid_t - 1] != expert) && (pid_t == nt - 1 || a.expert_ids[pid_t + 1] != expert))
+      k_first = __builtin_amdgcn_readfirstlane(spread_k_start256(expert, pid_f, a.num_f_tiles, 0, k_tiles));
+  }
 
   // X row of a tile row (gathered through the routing arrays) and W row of a tile row
   auto x_src_row = [&](int rr) -> int64_t {
@@ -730,17 +747,18 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_kernel(const GemmArgs
     // first: in the prologue they depend only on the expert id, so they are in flight while the
     // sorted ids that the token-tile addresses need are still being fetched.  The IW virtual
     // wavefronts of one load index are adjacent.
+#define FR_KPOS(tile_) ((tile_) + k_first >= k_tiles ? (tile_) + k_first - k_tiles : (tile_) + k_first)
 #define FR_ISSUE_ONE(tile_, slot_, q_)                                                                     \
   {                                                                                                        \
     const int vw_ = wave_u + ((q_) % IW) * (NW / IW);                                                      \
     if ((q_) < WIW) {                                                                                  \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                            \
           wrs, (lptr_t)(lds_raw + (WBASE + (slot_) * C::WCH) * 16 + (((q_) / IW) * NW + vw_) * (kWave * 16)), \
-          16, wsrc[(q_) < WIW ? (q_) : 0], (tile_) * wstep, 0, FR_W_AUX);                                    \
+          16, wsrc[(q_) < WIW ? (q_) : 0], FR_KPOS(tile_) * wstep, 0, FR_W_AUX);                             \
     } else {                                                                                               \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                            \
           xrs, (lptr_t)(lds_raw + (slot_) * (C::XCH * 16) + ((((q_) - WIW) / IW) * NW + vw_) * (kWave * 16)), \
-          16, xsrc[(q_) < WIW ? 0 : (q_) - WIW], (tile_) * C::BKB, 0, 0);                          \
+          16, xsrc[(q_) < WIW ? 0 : (q_) - WIW], FR_KPOS(tile_) * C::BKB, 0, 0);                   \
     }                                                                                                      \
   }
 #define FR_ISSUE_PART(tile_, slot_, p_)                                                                    \
@@ -847,6 +865,7 @@ _Pragma("unroll") \
 #undef FR_KSTEP
 #undef FR_ISSUE_PART
 #undef FR_ISSUE_ONE
+#undef FR_KPOS
 #endif
   }
 #undef FR_READ_FRAGS

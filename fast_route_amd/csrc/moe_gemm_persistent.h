@@ -308,7 +308,7 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
     asm volatile("" : "+s"(kfirst_)); /* or the lanes' parts of the offsets stay in registers between units */ \
     xrs_ = uniform_rsrc(X + xrow0_ * a.ldx, a.x_span ? a.x_span : 0xFFFFFFFFu);                              \
     wrs_ = uniform_rsrc(static_cast<const T*>(a.W) + static_cast<int64_t>(ex_) * a.w_expert_stride);         \
-    nt_ = NTW && !expert_off[kMaxExperts + 1] && expert_off[(ex_) + 1] - expert_off[ex_] == 1;               \
+    nt_ = !expert_off[kMaxExperts + 1] && expert_off[(ex_) + 1] - expert_off[ex_] == 1;               \
     _Pragma("unroll") for (int ih = 0; ih < XIW; ++ih) {                                                 \
       FR_SLOT_ROW(ih, rr, c, BT)                                                                              \
       int64_t row_ = rr;                                                                                     \
@@ -333,13 +333,13 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   // F = 16384 400 tokens 884 / 814; fp8 150 tokens 274 / 268, 300 330 / 307.  Two blocks per expert spread as well (1031 tokens
   // 818 / 833, H = 6144 900 tokens 1297 / 1317): one of them finds its rows gone from L2.  Not for 2-byte tiles of 256-byte row pieces
   // (64 rows, 150 tokens 452 / 461), which touch two channels' worth of every row at a time.
-  constexpr bool SPREAD_K = NTW && BT >= 64 && (C::BKB == 128 || sizeof(T) == 1);
+  constexpr bool SPREAD_K = BT >= 64 && (C::BKB == 128 || sizeof(T) == 1);
   auto first_k_tile = [&](bool alone, int ex, int pf, int kb_) -> int {
     const int kb_u = __builtin_amdgcn_readfirstlane(kb_);
     if (!SPREAD_K || !__builtin_amdgcn_readfirstlane(alone)) return kb_u;
-    const unsigned tile = __builtin_amdgcn_readfirstlane(ex * a.num_f_tiles + pf);
-    const int k = kb_u + static_cast<int>(__umulhi(tile * 2654435769u, static_cast<unsigned>(k_all)));
-    return k >= k_all ? k - k_all : k;
+    const int e_u = __builtin_amdgcn_readfirstlane(ex), f_u = __builtin_amdgcn_readfirstlane(pf);
+    if constexpr (BT == 256) return a.N % (EPI == EPI_SILU ? BF / 2 : BF) == 0 ? spread_k_start256(e_u, f_u, a.num_f_tiles, kb_u, k_all) : kb_u;
+    return spread_k_start(kb_u, e_u * a.num_f_tiles + f_u, k_all);
   };
   FR_UNIT(0, pid_t, pid_f, expert, kb, kn, tu)
   FR_MAKE_SET(pid_t, pid_f, expert, a.sorted[pid_t * BT + rr], xsrcA, wsrcA, xrsA, wrsA, ntA)

@@ -34,6 +34,17 @@
 // rows), and each of them asks for its share of the rows of a K tile several K tiles ahead - one dword per
 // 128-byte row piece, into a sink in LDS - so that the tile loads proper find their lines in L2.
 //
+// Tiles alone on their weight tile.  Where an expert's run is one tile, nobody shares its weight tiles: the touch only passes them
+// through L1 twice.  Up to 7 units (fp8: 6) such a tile has a K loop without touches, its weight loads non-temporal, so that the
+// stream leaves the token rows in L2; and every run of up to 8 units starts its K loops at spread places (spread_k_start256, why:
+// SPREAD_K in moe_gemm_persistent.h), which keeps the bits of the eight-wavefront kernels that do the same.  Layer on these tiles, in
+// parts of the time with touches from column 0, without touches / and spread: H = 4096, F = 14336, 8 experts 700 tokens (6 units)
+// 0.95 / 0.90, 850 1.00 / 0.95; fp16, 16 experts, F = 8192, 700 (3) 0.90 / 0.855, 1100 0.92 / 0.89, 1500 0.96 / 0.91; H = 6144 700
+// 0.93 / 0.89; H = 2048, 64 experts, Zipf-skewed 3000 0.975 / 0.97, 6500 0.99 / 0.98.  With 8 and 9 units it is even or slower (the ring's
+// two slots need the L2 hits, and the rows of a start of its own the L2): 1031 tokens 820 without touches, 782 with.  Non-temporal
+// touches are evicted before their loads come (20 to 25 % slower); non-temporal loads behind ordinary touches change nothing there
+// and cost 14 % where weight tiles are shared.
+//
 // Same tail split and LDS swizzle as moe_gemm_persistent_kernel; the result is bit-identical to the eight-wavefront kernels on
 // the same MFMA shape (same K order per accumulator, same roundings in the epilogue).
 #pragma once
@@ -205,7 +216,7 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
 struct QuadUnit {
   int row0, units;    // first slot, height
   int f, expert;      // feature tile, expert
-  int kb, kn, tu;     // first K tile, K tiles, slice buffer (-1: a whole tile)
+  int kb, kn, tu;     // K tile it starts at, K tiles (round the end of K), slice buffer (-1: a whole tile)
   int share;          // tiles of its chunk (which share its weight tile) and its index among them: count << 16 | index
 };
 constexpr int kUnitTable = 64;  // units a wavefront works out at a time, one per lane
@@ -213,7 +224,7 @@ constexpr int kUnitTable = 64;  // units a wavefront works out at a time, one pe
 // Tile number lin of the walk: experts in order, an expert's run in chunks of at most group_t tiles, a chunk tile-fastest
 // over all feature tiles (see tile_coords).  even_heights: all tiles
 // of an expert but the last have the mean height rounded up to even, the last what is left.
-__device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& w, int block, bool even_heights, int lin, QuadUnit& u) {
+__device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& w, int block, bool even_heights, int lin, int k_all, QuadUnit& u) {
   const int F = a.num_f_tiles, t = lin / F;
   if (w.off[kMaxExperts + 1]) {
     u.row0 = t * block;
@@ -255,6 +266,7 @@ __device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& 
   }
   u.expert = lo;
   u.share = gsz << 16 | index;
+  if (un <= 8 && a.spread_k) u.kb = spread_k_start256(lo, u.f, F, u.kb, k_all);
 }
 
 // One MFMA, written out so that an accumulator stays in the registers it has: those of the first kQuadAgpr token tiles in
@@ -265,7 +277,7 @@ __device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& 
 // instruction 18 wait states after the last MFMA on it at the earliest (run_unit's s_nops wait 20; MFMAs on one accumulator are
 // as many MFMAs apart as a K-step has), and no vector instruction may write an operand right before the MFMA (two wait states).
 // Operands are LDS reads, which are waited for, and accumulators start from zero in an MFMA, so there is nothing to write one;
-// a change here is checked in the assembly: the 4592 MFMAs of a 2-byte kernel and the 812 of an fp8 one have no vector write
+// a change here is checked in the assembly: the 6720 MFMAs of a 2-byte kernel and the 1148 of an fp8 one have no vector write
 // of an operand among the four instructions before.
 constexpr int kQuadAgpr = 8;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -473,7 +485,7 @@ __device__ __forceinline__ QuadCut quad_cut(const GemmArgs& a, const QuadWalk& w
   QuadCut c = {};
   if (p.xs.slices > 1 && t < p.xs.rest) {
     QuadUnit u;
-    quad_tile_at(a, walk, block, p.even_heights, p.xs.tail_base + t, u);
+    quad_tile_at(a, walk, block, p.even_heights, p.xs.tail_base + t, 1, u);
     c = QuadCut{u.row0, u.units, u.f, u.expert, p.xs.slices, p.xs.rest, quad_buffers(a, p.tallest), quad_buffer_rows(p.tallest)};
   }
   return c;
@@ -490,6 +502,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
   constexpr int BF = CM::BF, CPR = CM::CPR, BKB = CM::BKB, BK = BKB / ES, FC = E::FC;
   constexpr int TILE = CM::TILE, KG = CM::KGROUPS;
   constexpr int COLS = EPI == EPI_SILU ? BF / 2 : BF;
+  constexpr int kAloneUnits = sizeof(T) == 1 ? 6 : 7;  // tallest tile with a loop of its own for being alone on its weight tile
   constexpr int NW = 4, XI = kMaxUnits, WI = 8;        // tile loads per wavefront and K tile, at most: a load per unit of rows
   constexpr int XBYTES = kUnitRows * kMaxUnits * BKB, SLOT = XBYTES + BF * BKB;  // a ring slot: X rows, then W rows
   static_assert(2 * SLOT == kQuadRing && CM::WIW == WI && CM::XIW == XI && CPR == 8 && CPR / (KG * FC) == 2, "two K-steps per K tile");
@@ -534,7 +547,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
       u.kn = (s + 1) * k_all / xs.slices - u.kb;
       u.tu = xs.slices > 1 ? s * xs.rest + t : -1;
     }
-    quad_tile_at(a, walk, block, plan.even_heights, lin, u);
+    quad_tile_at(a, walk, block, plan.even_heights, lin, k_all, u);
     unit_table[(j0 / kUnitTable) & 1][lane] = u;
   };
   auto unit_at = [&](int j) {
@@ -626,9 +639,8 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     xrs_ = uniform_rsrc(X + xrow0_ * a.ldx, (a.x_span ? a.x_span : 0xFFFFFFFFu) * static_cast<unsigned>(live_)); \
     wrs_ = uniform_rsrc(static_cast<const T*>(a.W) + static_cast<int64_t>((u_).expert) * a.w_expert_stride, 0xFFFFFFFFu * static_cast<unsigned>(live_)); \
     const int f0_ = first_col((u_).f);                                                                       \
-    const unsigned kbytes_ = static_cast<unsigned>((u_).kb) * wstep;                                         \
-    wl_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, f0_, 0, ES)) + kbytes_;                 \
-    wh_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_row(f0_, BF / 2), 0, ES)) + kbytes_;  \
+    wl_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, f0_, 0, ES));                           \
+    wh_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_row(f0_, BF / 2), 0, ES));            \
   }
 #define FQ_SET_ROW(u_, sid_, q_, xsrc_)                                                                      \
   {                                                                                                          \
@@ -637,18 +649,18 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     const bool pad_ = (q_) >= (u_).units || (sid_) >= a.num_valid;                                           \
     unsigned row_ = a.top_k > 0 ? div_top_k(sid_) : (q_) * kUnitRows + lrow_;                                \
     row_ = pad_ ? 0u : row_;                                                                                 \
-    const unsigned off_ = row_ * xpitch + static_cast<unsigned>((u_).kb) * BKB + lchunk * 16;                \
+    const unsigned off_ = row_ * xpitch + lchunk * 16;                                                       \
     xsrc_ = a.x_span && pad_ ? kSkipOffset : off_;                                                           \
   }
 #define FQ_SET_TOUCH(u_, tsid_, tw_, tx_)                                                                    \
   {                                                                                                          \
     int wrow_, xrow_; bool xon_;                                                                             \
     FQ_TOUCH_ROWS(u_, wrow_, xrow_, xon_)                                                                    \
-    tw_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_row(first_col((u_).f), wrow_), 0, ES)) + static_cast<unsigned>((u_).kb) * wstep; \
+    tw_ = static_cast<unsigned>(w_byte_offset(a.w_tiled, a.ldw, a.K, w_row(first_col((u_).f), wrow_), 0, ES)); \
     const bool tpad_ = !xon_ || (tsid_) >= a.num_valid;                                                      \
     unsigned trow_ = a.top_k > 0 ? div_top_k(tsid_) : static_cast<unsigned>(xrow_);                          \
     trow_ = tpad_ ? 0u : trow_;                                                                              \
-    tx_ = a.x_span && tpad_ ? kSkipOffset : trow_ * xpitch + static_cast<unsigned>((u_).kb) * BKB;           \
+    tx_ = a.x_span && tpad_ ? kSkipOffset : trow_ * xpitch;                                                  \
   }
   // tile load q (weight rows first) of K tile tile_ of set SET into ring slot slot_
 #define FQ_ISSUE(SET, tile_, slot_, q_)                                                                     \
@@ -656,7 +668,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     if ((q_) < WI) {                                                                                        \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                             \
           wrs##SET, (lptr_t)(lds_raw + (slot_) * SLOT + XBYTES + ((q_) * NW + wave_u) * (kWave * 16)),      \
-          16, wlane, (((q_) & 4) ? wh##SET : wl##SET) + (((q_) & 2) ? wgap2 : 0) + (((q_) & 1) ? wgap1 : 0) + (tile_) * wstep, 0, 0); \
+          16, wlane, (((q_) & 4) ? wh##SET : wl##SET) + (((q_) & 2) ? wgap2 : 0) + (((q_) & 1) ? wgap1 : 0) + (tile_) * wstep, 0, WAUX); \
     } else {                                                                                                \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                             \
           xrs##SET, (lptr_t)(lds_raw + (slot_) * SLOT + (((q_) - WI) * NW + wave_u) * (kWave * 16)),        \
@@ -704,7 +716,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
             FQ_FENCE                                                                                       \
           }                                                                                                \
         }                                                                                                  \
-        if (m == NM - 1) {                                                                                 \
+        if (m == NM - 1 && TOUCH) {                                                                        \
           FQ_TOUCH_ISSUE(TSET, ttile_)                                                                     \
           FQ_FENCE                                                                                         \
         }                                                                                                  \
@@ -737,7 +749,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
 #define FQ_PERIOD(FIRST, RDLAST, NLD_, LSET, ltile_, TSET, ttile_, HOOK)                 \
   {                                                                                      \
     FQ_KSTEP(0, FIRST, true, par, 0, LSET, 0, 0, TSET, 0, HOOK)                          \
-    FQ_SYNC((FIRST) ? 0 : 2)                                                             \
+    FQ_SYNC((FIRST) || !TOUCH ? 0 : 2)                                                   \
     FQ_KSTEP(1, false, RDLAST, par ^ 1, NLD_, LSET, ltile_, par, TSET, ttile_, FQ_NO_HOOK) \
     par ^= 1;                                                                            \
   }
@@ -776,21 +788,31 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     for (int q = 0; q < XI; ++q) FQ_SET_ROW(uA, sid0[q], q, xsrcA[q])
     FQ_SET_TOUCH(uA, tsid0, twA, txA)
   }
-  // fill: K tiles 0 and 1 into slots 0 and 1
+  // K tiles the next loads and the next touches ask for: a unit's follow each other round the end of K
+  auto next_k = [&](int k) { return k + 1 == k_all ? 0 : k + 1; };
+  int lw = uA.kb, tw;
+  // fill: the first two K tiles into slots 0 and 1
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < 2; ++t) {
+    constexpr int WAUX = 0;
 #pragma unroll
-    for (int q = 0; q < WI + XI; ++q) FQ_ISSUE(A, t, t, q)
+    for (int q = 0; q < WI + XI; ++q) FQ_ISSUE(A, lw, t, q)
+    lw = next_k(lw);
+  }
+  tw = next_k(lw);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WI + XI) : "memory");
   __builtin_amdgcn_s_barrier();
   int par = 0, unit = 0;
 
-  // One work unit of UN units of rows (or fewer: rows beyond the tile are padding): kn >= kQuadMinTiles K tiles.  The ring
+  // One work unit of UN units of rows (or fewer: rows beyond the tile are padding): kn >= kQuadMinTiles K tiles; ALONE: the only
+  // tile on its weight tile (no touch, weights non-temporal).  The ring
   // holds the unit's first two K tiles when it starts.  The next unit's routing data is asked for five K tiles before the end
   // and turned into the address set B in the next one (the K loop proper keeps one set in registers); the last three K tiles
   // touch its first three, and its first two refill the ring during the last two.
-  auto run_unit = [&](auto height) __attribute__((always_inline)) {
+  auto run_unit = [&](auto height, auto alone) __attribute__((always_inline)) {
     constexpr int UN = decltype(height)::value;
+    constexpr bool ALONE = decltype(alone)::value, TOUCH = !ALONE;
+    constexpr int WAUX = ALONE ? 2 : 0;  // cache policy of the weight loads (2: non-temporal)
     typedef QuadCfg<T, UN> C;
     // the operand walked slowest: the weights, or the token rows where a wavefront has all of them
     constexpr bool WOUT = C::WT == 2;
@@ -812,14 +834,27 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     const int live = min(n_units - 1 - unit, 1);  // 0: this is the workgroup's last unit
     if (live && (unit + 1) % kUnitTable == 0) fill_units(unit + 1);
     const int kn = uA.kn;
-    FQ_PERIOD(true, true, WI + UN, A, 2, A, 3, FQ_NO_HOOK)
+#define FQ_NEXT { lw = next_k(lw); tw = next_k(tw); }
+    FQ_PERIOD(true, true, WI + UN, A, lw, A, tw, FQ_NO_HOOK)
+    FQ_NEXT
     __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0): no scalar load pending inside the loop */
-    for (int t = 1; t < kn - 5; ++t) FQ_PERIOD(false, true, WI + UN, A, t + 2, A, t + 3, FQ_NO_HOOK)
-    FQ_PERIOD(false, true, WI + UN, A, kn - 3, A, kn - 2, FQ_HOOK_IDS)
-    FQ_PERIOD(false, true, WI + UN, A, kn - 2, A, kn - 1, FQ_HOOK_SET)
-    FQ_PERIOD(false, true, WI + UN, A, kn - 1, B, 0, FQ_NO_HOOK)
-    FQ_PERIOD(false, true, WI + XI, B, 0, B, 1, FQ_NO_HOOK)
-    FQ_PERIOD(false, false, WI + XI, B, 1, B, 2, FQ_NO_HOOK)
+    for (int t = 1; t < kn - 5; ++t) {
+      FQ_PERIOD(false, true, WI + UN, A, lw, A, tw, FQ_NO_HOOK)
+      FQ_NEXT
+    }
+    FQ_PERIOD(false, true, WI + UN, A, lw, A, tw, FQ_HOOK_IDS)
+    FQ_NEXT
+    FQ_PERIOD(false, true, WI + UN, A, lw, A, tw, FQ_HOOK_SET)
+    lw = next_k(lw);
+    tw = uB.kb;
+    FQ_PERIOD(false, true, WI + UN, A, lw, B, tw, FQ_NO_HOOK)
+    lw = tw;
+    tw = next_k(tw);
+    FQ_PERIOD(false, true, WI + XI, B, lw, B, tw, FQ_NO_HOOK)
+    FQ_NEXT
+    FQ_PERIOD(false, false, WI + XI, B, lw, B, tw, FQ_NO_HOOK)
+    FQ_NEXT
+#undef FQ_NEXT
     // the last MFMA's result is up to 19 wait states away, which the compiler does not know
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory");
     FQ_FENCE
@@ -834,17 +869,22 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
           acc, wt, wf, frow_e, kgrp_e);
   };
   for (;; ++unit) {
-    // a loop of its own for every height from 4 on (fp8: 9 and the even ones), 2 and 4 for those below
+    // a loop of its own for every height from 4 on (fp8: 9 and the even ones), 2 and 4 for those below; alone: 7, 6, 4 and 2
     const int height = uA.units;
-    if (height == 9) run_unit(std::integral_constant<int, 9>());
-    else if (height == 8 || (sizeof(T) == 1 && height == 7)) run_unit(std::integral_constant<int, 8>());
+    if (uA.share == 1 << 16 && height <= kAloneUnits && a.spread_k) {
+      if (height == 7) run_unit(std::integral_constant<int, kAloneUnits>(), std::true_type());
+      else if (height >= 5) run_unit(std::integral_constant<int, 6>(), std::true_type());
+      else if (height >= 3) run_unit(std::integral_constant<int, 4>(), std::true_type());
+      else run_unit(std::integral_constant<int, 2>(), std::true_type());
+    } else if (height == 9) run_unit(std::integral_constant<int, 9>(), std::false_type());
+    else if (height == 8 || (sizeof(T) == 1 && height == 7)) run_unit(std::integral_constant<int, 8>(), std::false_type());
     else if (sizeof(T) != 1 && height == 7) {
-      if constexpr (sizeof(T) != 1) run_unit(std::integral_constant<int, 7>());
-    } else if (height == 6 || (sizeof(T) == 1 && height == 5)) run_unit(std::integral_constant<int, 6>());
+      if constexpr (sizeof(T) != 1) run_unit(std::integral_constant<int, 7>(), std::false_type());
+    } else if (height == 6 || (sizeof(T) == 1 && height == 5)) run_unit(std::integral_constant<int, 6>(), std::false_type());
     else if (sizeof(T) != 1 && height == 5) {
-      if constexpr (sizeof(T) != 1) run_unit(std::integral_constant<int, 5>());
-    } else if (height >= 3) run_unit(std::integral_constant<int, 4>());
-    else run_unit(std::integral_constant<int, 2>());
+      if constexpr (sizeof(T) != 1) run_unit(std::integral_constant<int, 5>(), std::false_type());
+    } else if (height >= 3) run_unit(std::integral_constant<int, 4>(), std::false_type());
+    else run_unit(std::integral_constant<int, 2>(), std::false_type());
     if (unit + 1 >= n_units) break;
     uA = uB; xrsA = xrsB; wrsA = wrsB; wlA = wlB; whA = whB; twA = twB; txA = txB;
 #pragma unroll
@@ -949,6 +989,7 @@ int launch_gemm_quad(const GemmArgs& a_in, int block, int splits, hipStream_t st
                 (long long)x_rows, (long long)a.ldx, (long long)w_rows, (long long)a.ldw);
   a.group_t = tunables().group_m ? tunables().group_m : kChunkBlocks;
   if (tunables().no_tail_split) a.tail_ws = nullptr;
+  a.spread_k = a.N % COLS == 0;
   quad_divisor(a.top_k, &a.div_mul, &a.div_shift);
   a.x_span = x_rows * a.ldx * ES < (int64_t(1) << 31) ? static_cast<unsigned>(x_rows * a.ldx * ES) : 0u;
   int resident = 0;

@@ -257,6 +257,26 @@ def test_fp8_layer_leaves_the_heights_to_the_kernel(native, kernels_of):
     assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
 
 
+def test_fp8_one_tile_per_expert_where_the_plan_has_two(native, kernels_of):
+    """Runs of about five units, one tile each alone on its weight tile, where the plan's 160 rows cut them in two."""
+    from fast_route_amd import _native as N, fused_moe_fp8, prepare_weights_fp8
+    from fast_route_amd.layers.fused_moe import plan
+    M, H, Fd, E, k = 645, 4096, 3328, 8, 2
+    _say("fp8, one tile per expert")
+    assert plan(M, H, Fd, E, k, None, code=N.FR_FP8_E4M3).block == 160
+    x, logits, w1, w2 = oracle.make_inputs(M, H, Fd, E, seed=98)
+    x, w1, w2 = x.bfloat16(), w1.bfloat16(), w2.bfloat16()
+    args = [x.cuda(), *prepare_weights_fp8(w1.cuda(), w2.cuda()), logits.cuda()]
+    out, names = kernels_of(lambda: fused_moe_fp8(*args, k, True))
+    assert sum("moe_gemm_quad_kernel" in n for n in names) == 2, names
+    assert torch.equal(out, fused_moe_fp8(*args, k, True))
+    ref, _ = oracle.fused_moe_fp8(x, w1, w2, logits, k, True)
+    o = out.float().cpu()
+    assert torch.isfinite(o).all()
+    assert (o - ref).norm() / ref.norm() <= 1e-2
+    assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
 def test_fp8_cut_tiles_of_nine_units(native):
     """Both GEMMs' last round cut along K with tiles of 9 units (9 experts of two tiles each, 32 and 16 feature tiles, 32 K
     tiles): the result differs from that of whole tiles by the order of fp32 sums (and the codes of activated rows that

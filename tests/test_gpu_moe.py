@@ -833,6 +833,32 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
     assert ((out.float() - eight.float()).abs() <= 2 * ulp * eight.float().abs().max()).all()
 
 
+@pytest.mark.parametrize("M,Fd", [(645, 3200), (860, 7552)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_one_tile_per_expert_where_the_plan_has_two(native, kernels_of, dtype, M, Fd):
+    """Runs of five to seven units that the plan's 128 or 160 rows cut in two: both GEMMs multiply them as one tile each, alone on its
+    weight tile (K loop from a place of its own; 25 and 59 feature tiles, the last round cut).  One expert has a run of 8 units and
+    one of 9 (no loop of its own), one a single pair and one none."""
+    from fast_route_amd import fused_experts
+    from fast_route_amd.layers.fused_moe import plan
+    H, E, k = 4096, 8, 2
+    _say(f"one tile per expert M={M} F={Fd} {dtype}")
+    n = M * k
+    counts = np.array([1, 0, 250, 260, 0, 0, 0, 0])
+    counts[4:] = (n - counts.sum()) // 4
+    counts[4] += n - counts.sum()
+    rng = np.random.default_rng(M)
+    ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E), counts))).int().view(M, k)
+    x, _, w1, w2 = _inputs(M, H, Fd, E, 11 + M, dtype)
+    wts = torch.rand(M, k, generator=torch.Generator().manual_seed(M)) + 0.5
+    args = [x.cuda(), w1.cuda(), w2.cuda(), wts.cuda(), ids.cuda()]
+    assert plan(M, H, Fd, E, k, dtype).block in (128, 160)
+    out, names = kernels_of(lambda: fused_experts(*args))
+    assert sum("moe_gemm_quad_kernel" in x for x in names) == 2, names
+    assert torch.equal(out, fused_experts(*args))
+    _assert_close(out, oracle.moe_experts(x, w1, w2, wts, ids), dtype, "one tile per expert")
+
+
 @pytest.mark.parametrize("M,H,Fd,E,k,quad", [(1350, 4096, 2048, 8, 2, 2), (1430, 4096, 2048, 8, 2, 2), (2300, 2048, 2048, 8, 2, 2),
                                               (1200, 4096, 2048, 8, 2, 0), (2100, 2048, 2048, 8, 2, 0), (2850, 1024, 3584, 8, 2, 0),
                                               (350, 4096, 2048, 1, 1, 0), (1055, 2048, 5632, 4, 2, 0)])
