@@ -105,8 +105,14 @@ __device__ __forceinline__ int quad_tiles(int units, int limit) {
 struct QuadWalk {
   int off[kWalkTable], units[kWalkTable], tiles[kWalkTable];
   int tallest;  // units of the tallest tile
+  int count[6], high[6];  // tiles and tallest tile under each limit of a tile's height: see quad_walk
 };
-// all 256 threads; `block` rows per routing block (a multiple of 32, at most 256), nt > 0 blocks, nper workgroups per XCD
+// all 256 threads; `block` rows per routing block (a multiple of 32, at most 256), nt > 0 blocks, nper workgroups per XCD.
+// Nothing of a launch runs beside it, so it is written for few dependent loads and little code (which comes from memory, too):
+// from the start of the launch to the first K tile's arrival 64 experts take 11.5 - 12.1 us (gate/up, down projection), 8 experts 9.4 -
+// 10.2, of which 3 to 4 are the first tiles' own loads; 15.5 - 16.7 and 11.7 - 12.6 when a wavefront went through its experts' last blocks
+// and all limits, the cut tile was worked out apart and the first weights waited for the sorted ids.  Layer H = 2048, 64 experts,
+// top-6, 8192 tokens 883 -> 875 us, 6200 703 -> 696; H = 4096, 1031 tokens 773 -> 770; fp8 650 387 -> 384.
 __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int block, int nt, int tid, int nper, int k_tiles) {
   expert_block_offsets(a, nt, w.off, tid, 256);
   if (w.off[kMaxExperts + 1]) {
@@ -114,88 +120,92 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
     __syncthreads();
     return;
   }
-  const int E = a.num_experts, lane = tid & 63, wave = tid >> 6;
-  // the last block of every run: its last 32-slot group with a pair (sixteen experts' ids in flight per wavefront)
-  constexpr int XE = 16;
-  for (int e0 = wave; e0 < E; e0 += 4 * XE) {
-    int id[XE][4];
+  const int E = a.num_experts, lane = tid & 63, wave = tid >> 6, groups = block / kUnitRows;
+  for (int e = tid; e < E; e += 256) w.units[e] = max(w.off[e + 1] - w.off[e] - 1, 0) * groups;
+  __syncthreads();
+  // the last block of every run: its last 32-slot group with a pair, a group per thread (two at a time), their ids in flight together
+  for (int i0 = tid; i0 < E * 8; i0 += 2 * 256) {
+    typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int V = kUnitRows / 4;
+    i32x4_a4 id[2][V];
+    int e[2], run[2];  // expert, units of its run up to this group (0: no such group)
 #pragma unroll
-    for (int x = 0; x < XE; ++x) {
-      if (e0 + 4 * x >= E) break;
-      const int last = max(w.off[e0 + 4 * x + 1] - 1, 0);
+    for (int p = 0; p < 2; ++p) {
+      const int i = min(i0 + p * 256, E * 8 - 1), g = i & 7;
+      e[p] = i >> 3;
+      const int len = w.off[e[p] + 1] - w.off[e[p]];
+      run[p] = len > 0 && g < groups ? (len - 1) * groups + g + 1 : 0;
+      const i32x4_a4* ids = reinterpret_cast<const i32x4_a4*>(a.sorted + (run[p] ? (w.off[e[p]] + len - 1) * block + g * kUnitRows : 0));
 #pragma unroll
-      for (int p = 0; p < 4; ++p) id[x][p] = a.sorted[last * block + min(p * kWave + lane, block - 1)];
+      for (int x = 0; x < V; ++x) id[p][x] = ids[x];
     }
 #pragma unroll
-    for (int x = 0; x < XE; ++x) {
-      const int e = e0 + 4 * x;
-      if (e >= E) break;
-      int groups = 0;
+    for (int p = 0; p < 2; ++p) {
+      int least = id[p][0][0];
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const unsigned long long b = __ballot(p * kWave + lane < block && id[x][p] < a.num_valid);
-        if (b) groups = 2 * p + (b >> 32 ? 2 : 1);
-      }
-      if (lane == 0) {
-        const int len = w.off[e + 1] - w.off[e];
-        w.units[e] = len > 0 ? (len - 1) * (block / kUnitRows) + groups : 0;
-      }
+      for (int x = 0; x < V; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) least = min(least, id[p][x][r]);
+      if (least < a.num_valid) atomicMax(&w.units[e[p]], run[p]);
     }
   }
   __syncthreads();
-  if (wave == 0) {
-    // The limit of a tile's height.  Tall tiles cost least per row, but a launch of few rounds is over when its busiest
-    // workgroup is: a round takes as long as kTileCost + height, and the tiles behind the whole rounds as long as a round
-    // unless the schedule cuts them along K.  (Down projection, 8 experts x 16 feature tiles, limit 9 / 8 / 7 / 6 / 5 / 4 in us:
-    // 20 units each 574 / 574 / 576 / 498 / 483 / 693 (6 taken), 26 units 715 / 622 / 622 / 790 / 767 / 923 (8 taken), 33 units
-    // 752 / 907 / 910 / 867 / 1002 / 1068 (9 taken).  Over 186 launches, 8 to 50 units on 1 to 16 experts, the limit taken costs
-    // 1.0 % more than the best on average.)
-    constexpr int NL = 6;  // limits 9 to 4
-    int count[NL] = {}, high[NL] = {};
+  // The limit of a tile's height.  Tall tiles cost least per row, but a launch of few rounds is over when its busiest
+  // workgroup is: a round takes as long as kTileCost + height, and the tiles behind the whole rounds as long as a round
+  // unless the schedule cuts them along K.  (Down projection, 8 experts x 16 feature tiles, limit 9 / 8 / 7 / 6 / 5 / 4 in us:
+  // 20 units each 574 / 574 / 576 / 498 / 483 / 693 (6 taken), 26 units 715 / 622 / 622 / 790 / 767 / 923 (8 taken), 33 units
+  // 752 / 907 / 910 / 867 / 1002 / 1068 (9 taken).  Over 186 launches, 8 to 50 units on 1 to 16 experts, the limit taken costs
+  // 1.0 % more than the best on average.)
+  constexpr int NL = 6;  // limits 9 to 4: tiles and tallest tile of limits 9 - wave and 5 - wave
+  {
+    int n[2] = {}, tall[2] = {};
     for (int e0 = 0; e0 < E; e0 += kWave) {
       const int u = e0 + lane < E ? w.units[e0 + lane] : 0;
 #pragma unroll
-      for (int l = 0; l < NL; ++l) {
-        const int c = quad_tiles(u, kMaxUnits - l);
-        count[l] += c;
-        high[l] = max(high[l], c ? (u + c - 1) / c : 0);
+      for (int p = 0; p < 2; ++p) {
+        const int c = quad_tiles(u, kMaxUnits - min(wave + 4 * p, NL - 1));
+        n[p] += c;
+        tall[p] = max(tall[p], c ? (u + c - 1) / c : 0);
       }
     }
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1)
 #pragma unroll
-      for (int l = 0; l < NL; ++l) {  // the limits' chains of exchanges overlap
-        count[l] += __shfl_xor(count[l], d);
-        high[l] = max(high[l], __shfl_xor(high[l], d));
+      for (int p = 0; p < 2; ++p) {
+        n[p] += __shfl_xor(n[p], d);
+        tall[p] = max(tall[p], __shfl_xor(tall[p], d));
       }
-    unsigned cost = ~0u;  // lane l: of limit 9 - l
-    {
-      int n = 0, tall = 0;
 #pragma unroll
-      for (int l = 0; l < NL; ++l) {
-        n = lane == l ? count[l] : n;
-        tall = lane == l ? high[l] : tall;
+    for (int p = 0; p < 2; ++p)
+      if (lane == 0 && wave + 4 * p < NL) {
+        w.count[wave + 4 * p] = n[p];
+        w.high[wave + 4 * p] = tall[p];
       }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    unsigned cost;  // lane l: of limit 9 - l
+    {
+      const int n = w.count[min(lane, NL - 1)], tall = w.high[min(lane, NL - 1)];
       // XCD 0 has the largest share
       const XcdSchedule xs = xcd_schedule(n * a.num_f_tiles, nper, 0, k_tiles, a.tail_ws != nullptr, schedule_by_rounds(n, E),
                                           quad_buffers(a, tall));
       const unsigned tile = kTileCost + 10 * tall, rounds = xs.rounds, slices = xs.slices;
       const unsigned cut = 32 * tile * (rounds ? kCutStretch : 5) / (5 * slices) + kCutCost * tile;
-      if (lane < NL) cost = 32 * rounds * tile + (xs.rest == 0 ? 0 : slices < 2 ? 32 * tile : cut);
+      cost = 32 * rounds * tile + (xs.rest == 0 ? 0 : slices < 2 ? 32 * tile : cut);
     }
-    int best = kMaxUnits;
+    int best = 0;
     unsigned least = __builtin_amdgcn_readlane(cost, 0);
-#pragma unroll
     for (int l = 1; l < NL; ++l) {  // a lower limit has to be 3 % cheaper
       const unsigned c = __builtin_amdgcn_readlane(cost, l);
       if (c < least - least / 32) {
         least = c;
-        best = kMaxUnits - l;
+        best = l;
       }
     }
-    int base = 0, tall = 0;
+    int base = 0;
     for (int e0 = 0; e0 <= E; e0 += kWave) {
-      const int e = e0 + lane, u = e < E ? w.units[e] : 0, c = e < E ? quad_tiles(u, best) : 0;
+      const int e = e0 + lane, c = e < E ? quad_tiles(w.units[e], kMaxUnits - best) : 0;
       int s = c;
 #pragma unroll
       for (int d = 1; d < kWave; d <<= 1) {
@@ -204,10 +214,8 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
       }
       if (e <= E) w.tiles[e] = base + s - c;
       base += __shfl(s, kWave - 1);
-      for (int h = tall + 1; h <= kMaxUnits; ++h)
-        if (__any(c && (u + c - 1) / c >= h)) tall = h;
     }
-    if (lane == 0) w.tallest = tall;
+    if (lane == 0) w.tallest = w.high[best];
   }
   __syncthreads();
 }
@@ -480,17 +488,6 @@ __device__ __forceinline__ QuadPlan quad_plan(const GemmArgs& a, QuadWalk& walk,
                       quad_buffers(a, p.tallest));
   return p;
 }
-// tile t of the XCD's last round
-__device__ __forceinline__ QuadCut quad_cut(const GemmArgs& a, const QuadWalk& walk, int block, const QuadPlan& p, int t) {
-  QuadCut c = {};
-  if (p.xs.slices > 1 && t < p.xs.rest) {
-    QuadUnit u;
-    quad_tile_at(a, walk, block, p.even_heights, p.xs.tail_base + t, 1, u);
-    c = QuadCut{u.row0, u.units, u.f, u.expert, p.xs.slices, p.xs.rest, quad_buffers(a, p.tallest), quad_buffer_rows(p.tallest)};
-  }
-  return c;
-}
-
 template <typename T, int EPI>
 __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -517,7 +514,10 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
   const int k_all = a.K / BK;
   const QuadPlan plan = quad_plan<T>(a, walk, block, xcd, nper, tid);
   const XcdSchedule& xs = plan.xs;
-  if (a.tail_ws != nullptr && tid == 0) reinterpret_cast<QuadCut*>(a.tail_desc)[xcd * nper + loc] = quad_cut(a, walk, block, plan, loc);
+  // what the fix-up launch asks for: tile `loc` of the XCD's last round, if that is cut (then it is this workgroup's last unit)
+  QuadCut* const cut_at = a.tail_ws != nullptr ? reinterpret_cast<QuadCut*>(a.tail_desc) + (xcd * nper + loc) : nullptr;
+  const bool cut = xs.slices > 1 && loc < xs.rest;
+  if (cut_at && !cut && tid == 0) *cut_at = QuadCut{};
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
   if (n_units == 0) return;
 
@@ -549,6 +549,8 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     }
     quad_tile_at(a, walk, block, plan.even_heights, lin, k_all, u);
     unit_table[(j0 / kUnitTable) & 1][lane] = u;
+    if (cut_at && cut && tid == n_units - 1 - j0)
+      *cut_at = QuadCut{u.row0, u.units, u.f, u.expert, xs.slices, xs.rest, quad_buffers(a, plan.tallest), quad_buffer_rows(plan.tallest)};
   };
   auto unit_at = [&](int j) {
     const QuadUnit& s = unit_table[(j / kUnitTable) & 1][j % kUnitTable];
@@ -780,27 +782,33 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
 
   fill_units(0);
   uA = unit_at(0);
-  {
-    int sid0[XI], tsid0;
-    FQ_IDS(uA, sid0, tsid0)
-    FQ_SET_RSRC(uA, 1, wlA, whA, xrsA, wrsA)
-#pragma unroll
-    for (int q = 0; q < XI; ++q) FQ_SET_ROW(uA, sid0[q], q, xsrcA[q])
-    FQ_SET_TOUCH(uA, tsid0, twA, txA)
-  }
   // K tiles the next loads and the next touches ask for: a unit's follow each other round the end of K
   auto next_k = [&](int k) { return k + 1 == k_all ? 0 : k + 1; };
   int lw = uA.kb, tw;
-  // fill: the first two K tiles into slots 0 and 1
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
+  {
+    // fill: the first two K tiles into slots 0 and 1, the weights while the sorted ids are on their way
     constexpr int WAUX = 0;
+    const int k1 = next_k(lw);
+    int sid0[XI], tsid0;
+    FQ_IDS(uA, sid0, tsid0)
+    FQ_SET_RSRC(uA, 1, wlA, whA, xrsA, wrsA)
+    FQ_FENCE
 #pragma unroll
-    for (int q = 0; q < WI + XI; ++q) FQ_ISSUE(A, lw, t, q)
-    lw = next_k(lw);
+    for (int q = 0; q < WI; ++q) FQ_ISSUE(A, lw, 0, q)
+#pragma unroll
+    for (int q = 0; q < WI; ++q) FQ_ISSUE(A, k1, 1, q)
+    FQ_FENCE
+#pragma unroll
+    for (int q = 0; q < XI; ++q) FQ_SET_ROW(uA, sid0[q], q, xsrcA[q])
+#pragma unroll
+    for (int q = WI; q < WI + XI; ++q) FQ_ISSUE(A, lw, 0, q)
+#pragma unroll
+    for (int q = WI; q < WI + XI; ++q) FQ_ISSUE(A, k1, 1, q)
+    FQ_SET_TOUCH(uA, tsid0, twA, txA)
+    lw = next_k(k1);
+    tw = next_k(lw);
   }
-  tw = next_k(lw);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WI + XI) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XI) : "memory");
   __builtin_amdgcn_s_barrier();
   int par = 0, unit = 0;
 
@@ -832,7 +840,6 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
 #pragma unroll
     for (int j = 0; j < JF; ++j) FQ_READ_W(0, j, 0, par)
     const int live = min(n_units - 1 - unit, 1);  // 0: this is the workgroup's last unit
-    if (live && (unit + 1) % kUnitTable == 0) fill_units(unit + 1);
     const int kn = uA.kn;
 #define FQ_NEXT { lw = next_k(lw); tw = next_k(tw); }
     FQ_PERIOD(true, true, WI + UN, A, lw, A, tw, FQ_NO_HOOK)
@@ -871,6 +878,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
   for (;; ++unit) {
     // a loop of its own for every height from 4 on (fp8: 9 and the even ones), 2 and 4 for those below; alone: 7, 6, 4 and 2
     const int height = uA.units;
+    if (unit + 1 < n_units && (unit + 1) % kUnitTable == 0) fill_units(unit + 1);
     if (uA.share == 1 << 16 && height <= kAloneUnits && a.spread_k) {
       if (height == 7) run_unit(std::integral_constant<int, kAloneUnits>(), std::true_type());
       else if (height >= 5) run_unit(std::integral_constant<int, 6>(), std::true_type());

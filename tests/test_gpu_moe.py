@@ -413,6 +413,44 @@ def test_grouped_gemm_with_blocks_in_any_order(native, block):
     _assert_close(c1.view(M * k, -1), oracle.grouped_gemm(x, w1, w, ids, False, k), dtype, "reversed blocks")
 
 
+@pytest.mark.parametrize("block", [32, 64, 128, 160, 256])
+@pytest.mark.parametrize("E", [3, 70, 300])
+def test_grouped_gemm_with_pairs_anywhere_in_their_block(native, block, E):
+    """Routing arrays of another producer: pairs and padding of a block in any order, a run's last block with one pair in
+    its last slot, more experts than a workgroup has threads for, experts without a block."""
+    from fast_route_amd.ops.fused_moe import invoke_fused_moe_kernel
+    _say(f"grouped GEMM, shuffled blocks, block={block} E={E}")
+    dtype, K, N = torch.bfloat16, 1024, 256
+    rng = np.random.default_rng(E + block)
+    counts = rng.integers(0, 2 * block + 1, E) * (rng.random(E) < 40 / (E + 20))
+    counts[E // 2] = block + 1
+    n = int(counts.sum())
+    pairs = rng.permutation(n)
+    s, e, at = [], [], 0
+    for x in range(E):
+        left = pairs[at : at + counts[x]]
+        at += counts[x]
+        while len(left):
+            b = np.full(block, n)
+            take = left[: 1 if x == E // 2 and len(left) == counts[x] else block]
+            left = left[len(take):]
+            b[[block - 1] if len(take) == 1 else rng.choice(block, len(take), replace=False)] = take
+            s.append(b)
+            e.append(x)
+    a = torch.randn(n, K, generator=torch.Generator().manual_seed(E)).to(dtype)
+    w = (torch.randn(E, N, K, generator=torch.Generator().manual_seed(block)) * 0.02).to(dtype)
+    sid, eid = torch.from_numpy(np.concatenate(s)).int().cuda(), torch.tensor(e, dtype=torch.int32, device="cuda")
+    npost = torch.tensor([len(e) * block], dtype=torch.int32, device="cuda")
+    ids = torch.empty(n, 1, dtype=torch.int32)
+    ids[torch.from_numpy(pairs).long(), 0] = torch.from_numpy(np.repeat(np.arange(E), counts)).int()
+    c = torch.zeros(n, 1, N, dtype=dtype, device="cuda")
+    cfg = {"BLOCK_SIZE_M": block, "BLOCK_SIZE_N": 64, "BLOCK_SIZE_K": 32, "GROUP_SIZE_M": 8}
+    wt = torch.ones(n, 1)
+    invoke_fused_moe_kernel(a.cuda(), w.cuda(), c, wt.cuda(), ids.cuda(), sid, eid, npost, False, 1, cfg)
+    torch.cuda.synchronize()
+    _assert_close(c.view(n, N), oracle.grouped_gemm(a, w, wt, ids, False, 1), dtype, "pairs anywhere")
+
+
 @pytest.mark.parametrize("N", [256, 260, 388, 516])
 @pytest.mark.parametrize("block", [16, 32, 64, 128, 160, 256])
 def test_rows_of_whole_and_partial_tiles(native, block, N):
