@@ -154,11 +154,10 @@ extern "C" int fr_moe_get_tunables(fr_moe_tunables* t) {
   return FR_OK;
 }
 
-extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, fr_moe_plan* plan) {
-  FR_REQUIRE(plan, FR_E_NULL, "fr_moe_get_plan: null plan");
-  dtype &= ~FR_W_TILED;  // the plan does not depend on the weight layout
-  int rc = check_layer_shapes("fr_moe_get_plan", M, H, F, E, topk, dtype);
-  if (rc != FR_OK) return rc;
+namespace fr {
+namespace {
+// the plan's routing block
+int plan_block(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype) {
   const int64_t n = M * topk;
   const double avg = static_cast<double>(n) / E;  // expected pairs per expert under uniform load
   // Routing block = token rows per GEMM tile.  Decode sizes want one block per expert
@@ -222,6 +221,14 @@ extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk,
   if (g_tunables.block) block = g_tunables.block;
   // the fp8 160-row tile exists in the persistent form only (five K tiles per K slice at least, 1022 experts at most)
   if (block == 160 && !two_byte && (H < 640 || F < 1024 || E > 1022)) block = 128;
+  return block;
+}
+
+// The plan for that block: K slices of the down projection, scratch.
+fr_moe_plan plan_for(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block) {
+  const int64_t n = M * topk;
+  const double avg = static_cast<double>(n) / E;
+  auto expected = [&](int rows) { return expected_blocks(avg, E, rows); };
   // Down projection: N = H gives few feature tiles, so K is split.
   const int bf = block == 16 ? 64 : (block == 32 ? 128 : 256);
   // expected token blocks: one per pair or per expert in the decode regime, else the expected blocks per expert
@@ -271,11 +278,54 @@ extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk,
     while (split > 1 && F / split < 8 * bk_elems) --split;
   }
   if (g_tunables.no_tail_split) tail_bytes = 0;
-  plan->block = block;
-  plan->split_k = split;
-  plan->sorted_len = n + static_cast<int64_t>(E) * (block - 1);
-  plan->tail_bytes = tail_bytes;
-  plan->workspace_bytes = carve(nullptr, M, H, F, E, topk, dtype, *plan).total;
+  fr_moe_plan plan;
+  plan.block = block;
+  plan.split_k = split;
+  plan.sorted_len = n + static_cast<int64_t>(E) * (block - 1);
+  plan.tail_bytes = tail_bytes;
+  plan.workspace_bytes = carve(nullptr, M, H, F, E, topk, dtype, plan).total;
+  return plan;
+}
+
+// The layers route for another block than the plan's where that has been found faster (2-byte operands; a block set by hand
+// stands).  Never for fewer K slices that are summed from fp32 rows: a single slice's rows are rounded.
+// Layer in parts of the time with the plan's block:
+//   Many narrow experts with skewed loads (H = 2048, F = 1408, 64 experts, top-6, Zipf): the heavy experts take several small tiles.  (Up
+//   to 128 experts and F = 2816: the routing blocks' padding is E x block rows of F activated values.)
+//     plan 16: 32 rows 20 tokens (1.9 pairs per expert) 0.96, 32 0.98, 40 0.905, 48 0.997, 72 0.94, 80 0.92, but 6 to 16 tokens 1.01 to 1.05;
+//     plan 32: 64 rows 90 (8.4) 0.99, 110 0.95, 180 0.86, 230 (21.6) 0.86; 128 rows 260 (24.4) 0.85 (64: 0.84), 290 0.80 (0.78), 335 0.74 (0.79)
+//   H = 1024, F = 3584, 8 experts: the plan's 64-row range begins at H = 4096, and the 128-row tile has 16 short K tiles there.
+//     16 rows 33 to 48 tokens (8 to 12 pairs) 0.91, 56 (14) 0.96; 64 rows 56 0.96, 100 0.95, 120 0.84, 128 (32) 0.80, 240 0.91, 460 (115) 0.95,
+//     500 (125) 1.00, 520 1.03
+//   160 rows instead of 128 where an expert is likely to exceed 128 rows: a block more costs a round of tiles, the larger tile 1 %.
+//     16 experts, F = 8192, fp16: 880 tokens (110 pairs; one expert above 128) 0.90, 920 0.88, 800 (none) 0.99; H = 6144 460 (115) 0.95;
+//     H = 4096, F = 14336, 8 experts none above 128: 300 and 420 1.01.
+int layer_block(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
+  if ((dtype != FR_F16 && dtype != FR_BF16) || g_tunables.block) return p.block;
+  const double avg = static_cast<double>(M) * topk / E;
+  if (E >= 32 && E <= 128 && H >= 2048 && H < 4096 && F <= 2816 && p.block <= 32 && avg >= 1.75) return avg < 8.5 ? 32 : avg < 24 ? 64 : 128;
+  if (E <= 16 && H >= 640 && H <= 1024 && F >= 1024 && (p.block == 32 || p.block == 128) && avg < 118) return avg <= 12 ? 16 : 64;
+  if (E <= 16 && H >= 4096 && F >= 1024 && p.block == 128 && avg < 128 && E * (expected_blocks(avg, E, 128) - 1.0) >= 0.15) return 160;
+  return p.block;
+}
+// `p`: the plan
+fr_moe_plan layer_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
+  const int block = layer_block(M, H, F, E, topk, dtype, p);
+  if (block == p.block) return p;
+  const fr_moe_plan q = plan_for(M, H, F, E, topk, dtype, block);
+  return p.split_k > 1 && q.split_k == 1 ? p : q;
+}
+}  // namespace
+}  // namespace fr
+
+extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, fr_moe_plan* plan) {
+  FR_REQUIRE(plan, FR_E_NULL, "fr_moe_get_plan: null plan");
+  dtype &= ~FR_W_TILED;  // the plan does not depend on the weight layout
+  int rc = check_layer_shapes("fr_moe_get_plan", M, H, F, E, topk, dtype);
+  if (rc != FR_OK) return rc;
+  *plan = plan_for(M, H, F, E, topk, dtype, plan_block(M, H, F, E, topk, dtype));
+  const int64_t layer_bytes = layer_plan(M, H, F, E, topk, dtype, *plan).workspace_bytes;
+  if (layer_bytes > plan->workspace_bytes) plan->workspace_bytes = layer_bytes;
   return FR_OK;
 }
 
@@ -309,6 +359,7 @@ extern "C" int fr_fused_experts(const void* x, const void* w1, const void* w2, c
   FR_REQUIRE(x && w1 && w2 && topk_weights && topk_ids && out, FR_E_NULL, "fr_fused_experts: null pointer");
   FR_REQUIRE(workspace && workspace_bytes >= p.workspace_bytes, FR_E_WORKSPACE, "fr_fused_experts: workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)p.workspace_bytes);
   FR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, FR_E_ALIGN, "fr_fused_experts: workspace must be 256-byte aligned");
+  p = layer_plan(M, H, F, E, topk, dtype & ~FR_W_TILED, p);
   Carve c = carve(workspace, M, H, F, E, topk, dtype & ~FR_W_TILED, p);
   rc = fr_moe_align(topk_ids, FR_I32, M * topk, E, p.block, c.sorted, c.expert_ids, c.npost, c.align_ws, c.align_ws_bytes, stream);
   if (rc != FR_OK) return rc;
@@ -320,15 +371,15 @@ extern "C" int fr_fused_experts(const void* x, const void* w1, const void* w2, c
                    "fr_fused_experts", (dtype & FR_W2_TILED) ? 1 : 0, topk_ids);
 }
 
-extern "C" int fr_fused_moe(const void* x, const void* w1, const void* w2, const void* logits, int logits_dtype,
-                            int64_t M, int64_t H, int64_t F, int E, int topk, int renormalize, int dtype,
-                            void* out, void* workspace, int64_t workspace_bytes, void* stream) {
-  fr_moe_plan p;
-  int rc = fr_moe_get_plan(M, H, F, E, topk, dtype, &p);
-  if (rc != FR_OK) return rc;
-  if (M == 0) return FR_OK;
+namespace fr {
+namespace {
+// the layer with the blocks and slices of `p`; need: what the caller was told the workspace has to hold
+int fused_moe_run(const fr_moe_plan& p, int64_t need, const void* x, const void* w1, const void* w2, const void* logits, int logits_dtype,
+                  int64_t M, int64_t H, int64_t F, int E, int topk, int renormalize, int dtype, void* out, void* workspace,
+                  int64_t workspace_bytes, void* stream) {
+  int rc;
   FR_REQUIRE(x && w1 && w2 && logits && out, FR_E_NULL, "fr_fused_moe: null pointer");
-  FR_REQUIRE(workspace && workspace_bytes >= p.workspace_bytes, FR_E_WORKSPACE, "fr_fused_moe: workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)p.workspace_bytes);
+  FR_REQUIRE(workspace && workspace_bytes >= need, FR_E_WORKSPACE, "fr_fused_moe: workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
   FR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, FR_E_ALIGN, "fr_fused_moe: workspace must be 256-byte aligned");
   Carve c = carve(workspace, M, H, F, E, topk, dtype & ~FR_W_TILED, p);
   // a handful of tokens: the gate/up launch gates and sorts by itself (row-major weights only)
@@ -346,6 +397,19 @@ extern "C" int fr_fused_moe(const void* x, const void* w1, const void* w2, const
   return down_impl(c.act, nullptr, w2, nullptr, c.topk_w, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block,
                    p.split_k, dtype & ~FR_W_TILED, dtype & ~FR_W_TILED, c.partial, out, c.tail_scratch(), static_cast<hipStream_t>(stream),
                    "fr_fused_moe", (dtype & FR_W2_TILED) ? 1 : 0, c.topk_ids);
+}
+}  // namespace
+}  // namespace fr
+
+extern "C" int fr_fused_moe(const void* x, const void* w1, const void* w2, const void* logits, int logits_dtype,
+                            int64_t M, int64_t H, int64_t F, int E, int topk, int renormalize, int dtype,
+                            void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  fr_moe_plan p;
+  int rc = fr_moe_get_plan(M, H, F, E, topk, dtype, &p);
+  if (rc != FR_OK) return rc;
+  if (M == 0) return FR_OK;
+  return fused_moe_run(layer_plan(M, H, F, E, topk, dtype & ~FR_W_TILED, p), p.workspace_bytes, x, w1, w2, logits, logits_dtype, M, H, F, E,
+                       topk, renormalize, dtype, out, workspace, workspace_bytes, stream);
 }
 
 extern "C" int fr_fused_moe_fp8(const void* x, int x_dtype, const void* w1q, const float* w1_scale, const void* w2q,
@@ -418,6 +482,9 @@ extern "C" int fr_fused_moe_noalloc(const void* x, const void* w1, const void* w
   int rc = fr_moe_get_plan(M, H, F, E, topk, dtype, &p);
   if (rc != FR_OK) return rc;
   FR_REQUIRE((dtype & ~FR_W_TILED) == FR_F16 || (dtype & ~FR_W_TILED) == FR_BF16, FR_E_DTYPE, "fr_fused_moe_noalloc: dtype %d not in {f16, bf16}", dtype);
+  // the plan's own bytes decide, and where the block the layers route for instead would not fit, its block is taken, too
+  const int op_dtype = dtype & ~FR_W_TILED;
+  p = plan_for(M, H, F, E, topk, op_dtype, p.block);
   FR_REQUIRE(p.workspace_bytes <= kStaticScratchBytes, FR_E_WORKSPACE,
              "fr_fused_moe_noalloc: these sizes need %lld bytes of scratch, the library's static scratch holds %lld; use fr_fused_moe with a workspace",
              (long long)p.workspace_bytes, (long long)kStaticScratchBytes);
@@ -425,5 +492,7 @@ extern "C" int fr_fused_moe_noalloc(const void* x, const void* w1, const void* w
   void* ws = nullptr;
   rc = static_scratch(&ws);
   if (rc != FR_OK) return rc;
-  return fr_fused_moe(x, w1, w2, logits, logits_dtype, M, H, F, E, topk, renormalize, dtype, out, ws, kStaticScratchBytes, stream);
+  fr_moe_plan q = layer_plan(M, H, F, E, topk, op_dtype, p);
+  if (q.workspace_bytes > kStaticScratchBytes) q = p;
+  return fused_moe_run(q, q.workspace_bytes, x, w1, w2, logits, logits_dtype, M, H, F, E, topk, renormalize, dtype, out, ws, kStaticScratchBytes, stream);
 }

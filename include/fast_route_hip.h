@@ -136,7 +136,10 @@ int fr_moe_prepare_weights(const void* w, int dtype, int64_t E, int64_t rows, in
  * The block is the token rows per GEMM tile up to 64.  From 128 on the GEMMs
  * may cut an expert's run of slots into tiles of 32 to 288 rows instead,
  * whatever the block: always where the block is 256 and K is 16 tiles of 128
- * bytes or more, under some plans of 128 and 160 with one K slice.           */
+ * bytes or more, under some plans of 128 and 160 with one K slice.
+ * fr_fused_moe, fr_fused_experts and fr_fused_moe_noalloc may route for another
+ * block than the plan's where that is faster (layer_block in fused_moe.hip);
+ * workspace_bytes covers both.                                                */
 typedef struct fr_moe_plan {
   int32_t block;      /* routing block                                       */
   int32_t split_k;    /* K splits of the down projection                     */
@@ -249,7 +252,7 @@ int fr_fused_moe(const void* x, const void* w1, const void* w2, const void* logi
  * 64 MiB device array inside this library, which every GPU the library runs on holds
  * until the process ends.  No counterpart in the reference; it is for callers that
  * cannot allocate: code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc.  Sizes whose fr_moe_get_plan().workspace_bytes exceed 64 MiB are
+ * forbid hipMalloc.  Sizes whose scratch with the plan's block exceeds 64 MiB are
  * rejected with FR_E_WORKSPACE (Mixtral-8x7B shape: up to 207 tokens).  The array's
  * device address is looked up by fr_moe_prepare, or else on the first call on each device
  * (with that device current): before capturing a call, call fr_moe_prepare or make one

@@ -871,6 +871,29 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
     assert ((out.float() - eight.float()).abs() <= 2 * ulp * eight.float().abs().max()).all()
 
 
+@pytest.mark.parametrize("M,H,Fd,E,k,planned,rows", [
+    (17, 2048, 256, 32, 4, 16, 32), (67, 2048, 256, 32, 4, 32, 32), (68, 2048, 256, 32, 4, 32, 64), (191, 2048, 256, 32, 4, 32, 64),
+    (192, 2048, 256, 32, 4, 32, 128), (255, 2048, 256, 32, 4, 32, 128), (36, 1024, 2048, 8, 2, 32, 16), (48, 1024, 2048, 8, 2, 32, 16),
+    (49, 1024, 2048, 8, 2, 32, 64), (471, 1024, 2048, 8, 2, 128, 64), (472, 1024, 2048, 8, 2, 128, 128), (900, 4096, 1024, 16, 2, 128, 160)])
+def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, Fd, E, k, planned, rows):
+    """At the edges of the ranges where the layers take other tiles than the plan's block stands for: the plan stays, its workspace
+    covers both, and results match the oracle."""
+    import re
+    from fast_route_amd import fused_experts, fused_moe
+    from fast_route_amd.layers.fused_moe import plan
+    dtype = torch.bfloat16
+    _say(f"layer's own block M={M} H={H} F={Fd} E={E}")
+    assert plan(M, H, Fd, E, k, dtype).block == planned
+    x, logits, w1, w2 = _inputs(M, H, Fd, E, 3 + M, dtype, zipf=E >= 32)
+    args = [x.cuda(), w1.cuda(), w2.cuda()]
+    out, names = kernels_of(lambda: fused_moe(*args, logits.cuda(), k, True))
+    tiles = {int(n) for x in names if "moe_gemm" in x for n in re.findall(r"Cfg(?:ILi|<)(\d+)", x)}
+    assert tiles == {rows}, names
+    w, ids = oracle.gating_topk(logits, k, True)
+    _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, "layer")
+    _assert_close(fused_experts(*args, w.cuda(), ids.cuda()), oracle.moe_experts(x, w1, w2, w, ids), dtype, "experts")
+
+
 @pytest.mark.parametrize("M,Fd", [(645, 3200), (860, 7552)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_one_tile_per_expert_where_the_plan_has_two(native, kernels_of, dtype, M, Fd):
