@@ -335,12 +335,12 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   // (64 rows, 150 tokens 452 / 461), which touch two channels' worth of every row at a time.
   // The 16-row down projection's tiles all start at places of their own: H = 4096, F = 14336, 8 experts 24 tokens 0.98, H = 6144 20 tokens
   // 0.95, fp16, 16 experts, F = 8192 10 / 50 tokens 0.97 / 0.985 of the time, but fp8 16 tokens 1.01; its gate/up GEMM (rows of up to
-  // 2 KB) is even.
+  // 2 KB) is even.  Not in a launch that leaves workgroups without a tile (8 experts, 5 and 10 tokens 1.005).
   constexpr bool SPREAD_ALL = BT == 16 && EPI != EPI_SILU && sizeof(T) == 2;
   constexpr bool SPREAD_K = SPREAD_ALL || (BT >= 64 && (C::BKB == 128 || sizeof(T) == 1));
   auto first_k_tile = [&](bool alone, int ex, int pf, int kb_) -> int {
     const int kb_u = __builtin_amdgcn_readfirstlane(kb_);
-    if (!SPREAD_K || (!SPREAD_ALL && !__builtin_amdgcn_readfirstlane(alone))) return kb_u;
+    if (!SPREAD_K || (SPREAD_ALL ? total < static_cast<int>(gridDim.x) : !__builtin_amdgcn_readfirstlane(alone))) return kb_u;
     const int e_u = __builtin_amdgcn_readfirstlane(ex), f_u = __builtin_amdgcn_readfirstlane(pf);
     if constexpr (BT == 256) return a.N % (EPI == EPI_SILU ? BF / 2 : BF) == 0 ? spread_k_start256(e_u, f_u, a.num_f_tiles, kb_u, k_all) : kb_u;
     return spread_k_start(kb_u, e_u * a.num_f_tiles + f_u, k_all);
