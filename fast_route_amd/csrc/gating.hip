@@ -60,11 +60,13 @@ __global__ __launch_bounds__(kGateThreads) void gating_topk_blocked_kernel(
 // The token rows [M, H] are the only real traffic (the gate matrix, [H, E] with experts
 // contiguous, stays in L2), so the kernel is shaped to stream them: a workgroup of 4
 // wavefronts owns 64 tokens (16 per wavefront), or, while there are too few tokens to fill
-// the CUs that way, 16 tokens whose K range the 4 wavefronts split and reduce through LDS.
+// the CUs that way, 16 tokens whose K range 4 or 16 wavefronts split and reduce through LDS.
 // The gate is taken in chunks of kRgKC rows, each transposed once through registers into
 // expert-major LDS rows (two K rows packed per 32-bit store) that the MFMA "A" operand reads
 // as 16-byte vectors; token rows come straight from HBM as the "B" operand, fetched for the
 // whole chunk before the barrier that publishes it.
+// tokens up to which a workgroup of the split form has 16 wavefronts: one workgroup per CU (up to 16 experts; more would not fit the LDS)
+constexpr int kRgWideTokens = 4096;
 constexpr int kRgMaxE = 128;  // the reference's own bound (ops/stable_route.py:134)
 
 template <typename T> struct Mfma16;
@@ -79,23 +81,28 @@ template <> struct Mfma16<f16_t> {
 
 // KC = K rows of the gate per LDS chunk; TT = 16-token tiles per wavefront in the unsplit form (many
 // experts: more tokens per transposed gate chunk).
+// NW = wavefronts of a workgroup (the split form).  Bound by the chain of chunks: gate rows -> LDS -> MFMA with two barriers, about 1 us
+// each, 16 of them at H = 4096 with four wavefronts; sixteen take chunks of four times as many rows.  Back to back, 4 / 16
+// wavefronts in us: 16 experts, H = 4096, fp16 1 token 10.6 / 6.3, 128 11.5 / 8.8, 700 13.8 / 8.8, 2048 15.2 / 10.2, 4096 15.7 / 11.9; 8 experts,
+// bf16 9.0 / 5.4, 10.0 / 7.5, 13.2 / 8.5, 13.5 / 9.2, 14.2 / 10.6; H = 8192 15.9 / 7.9 and 28.1 / 24.4; H = 1024 (one chunk) 4.5 / 4.7 and 5.6 / 4.9.
 // G lanes gate a token, VPL logits each: up to G * VPL experts (VPL = 2: 65..128 experts).
-template <typename T, int G, bool SPLITK, int KC, int TT, int VPL = 1>
-__global__ __launch_bounds__(kGateThreads) void route_gate_kernel(
+template <typename T, int G, bool SPLITK, int KC, int TT, int VPL = 1, int NW = 4>
+__global__ __launch_bounds__(NW * 64) void route_gate_kernel(
     const T* __restrict__ hidden, const T* __restrict__ gate, int64_t M, int H, int E, int topk,
     int renorm, float* __restrict__ w_out, int32_t* __restrict__ ids_out) {
   typedef typename Mfma16<T>::vec8 vec8;
-  static_assert(kGateThreads == 256, "4 wavefronts");
+  constexpr int NT = NW * 64;
+  static_assert(SPLITK || NW == 4, "the unsplit form has 4 wavefronts");
   static_assert(!SPLITK || TT == 1, "the split form has one token tile");
   constexpr int ET = (G * VPL + 15) / 16;        // expert tiles of 16
   constexpr int TPC = SPLITK ? 16 : 64 * TT;     // tokens per workgroup
-  constexpr int KW = SPLITK ? KC / 4 : KC;       // K elements of a chunk one wavefront multiplies
+  constexpr int KW = SPLITK ? KC / NW : KC;      // K elements of a chunk one wavefront multiplies
   constexpr int KSTEPS = KW / 32;
   constexpr int PITCH = KC + 8;                  // elements; keeps 16-byte alignment, spreads banks
   constexpr int LP = ET * 16 + 1;                // pitch of a logit row (floats)
   // the transposed gate chunk during the K loop; afterwards the same memory holds the logits (and the K slices' partial sums)
   constexpr int GT_BYTES = ET * 16 * PITCH * static_cast<int>(sizeof(T));
-  constexpr int LG_BYTES = (TPC * LP + (SPLITK ? 4 * 16 * LP : 0)) * 4;
+  constexpr int LG_BYTES = (TPC * LP + (SPLITK ? NW * 16 * LP : 0)) * 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[GT_BYTES > LG_BYTES ? GT_BYTES : LG_BYTES];
   static_assert(sizeof(smem) <= 65536, "LDS");
   T* gt = reinterpret_cast<T*>(smem);
@@ -113,7 +120,7 @@ __global__ __launch_bounds__(kGateThreads) void route_gate_kernel(
     xrow[t] = hidden + (tok < M ? tok : 0) * H + kw0 + (lane >> 4) * 8;
   }
 
-  for (int i = tid; i < ET * 16 * PITCH; i += kGateThreads) gt[i] = static_cast<T>(0.f);  // experts >= E stay 0
+  for (int i = tid; i < ET * 16 * PITCH; i += NT) gt[i] = static_cast<T>(0.f);  // experts >= E stay 0
   f32x4 acc[TT][ET];
 #pragma unroll
   for (int t = 0; t < TT; ++t)
@@ -137,7 +144,7 @@ __global__ __launch_bounds__(kGateThreads) void route_gate_kernel(
     if (vec_gate) {
       // item = (pair of K rows, 8 experts): two 16-byte loads, eight 32-bit stores of (k, k+1) pairs
       const int evs = E / 8;
-      for (int item = tid; item < (KC / 2) * evs; item += kGateThreads) {
+      for (int item = tid; item < (KC / 2) * evs; item += NT) {
         const int kp = item % (KC / 2), ev = item / (KC / 2);
         const int k = kc + 2 * kp;
         vec8 r0, r1;
@@ -153,7 +160,7 @@ __global__ __launch_bounds__(kGateThreads) void route_gate_kernel(
         }
       }
     } else {
-      for (int i = tid; i < KC * E; i += kGateThreads) {
+      for (int i = tid; i < KC * E; i += NT) {
         const int k = i / E, e = i % E;
         gt[e * PITCH + k] = kc + k < H ? gate[static_cast<int64_t>(kc + k) * E + e] : static_cast<T>(0.f);
       }
@@ -179,13 +186,17 @@ __global__ __launch_bounds__(kGateThreads) void route_gate_kernel(
       for (int r = 0; r < 4; ++r) dst[trow[t] * LP + j * 16 + (lane >> 4) * 4 + r] = acc[t][j][r];
   __syncthreads();
   if constexpr (SPLITK) {
-    for (int i = tid; i < 16 * ET * 16; i += kGateThreads) {
+    for (int i = tid; i < 16 * ET * 16; i += NT) {
       const int t = i / (ET * 16), e = i % (ET * 16);
-      logit[t * LP + e] = (part[t * LP + e] + part[(16 + t) * LP + e]) + (part[(32 + t) * LP + e] + part[(48 + t) * LP + e]);
+      float sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; w += 4)
+        sum += (part[(w * 16 + t) * LP + e] + part[((w + 1) * 16 + t) * LP + e]) + (part[((w + 2) * 16 + t) * LP + e] + part[((w + 3) * 16 + t) * LP + e]);
+      logit[t * LP + e] = sum;
     }
     __syncthreads();
   }
-  constexpr int PER_PASS = kGateThreads / G;
+  constexpr int PER_PASS = NT / G;
   for (int t = tid / G; t < TPC; t += PER_PASS) {
     const int64_t token = tok0 + t;
     const bool live = token < M;
@@ -279,6 +290,13 @@ void launch_route_gate(const void* hidden, const void* gate, int64_t M, int H, i
     hipLaunchKernelGGL((route_gate_kernel<T, G, false, KCU, TT, VPL>), dim3(static_cast<unsigned>(ceil_div(M, 64 * TT))), dim3(kGateThreads),
                        0, st, static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);
   } else {
+    if constexpr (ET == 1) {
+      if (M <= kRgWideTokens) {
+        hipLaunchKernelGGL((route_gate_kernel<T, G, true, 1024, 1, VPL, 16>), dim3(static_cast<unsigned>(ceil_div(M, 16))), dim3(1024), 0, st,
+                           static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);
+        return;
+      }
+    }
     constexpr int KC = VPL == 1 ? 256 : 128;  // longer chunks for few experts leave fewer workgroups per CU: slower at M = 8192, no gain at M = 1
     hipLaunchKernelGGL((route_gate_kernel<T, G, true, KC, 1, VPL>), dim3(static_cast<unsigned>(ceil_div(M, 16))), dim3(kGateThreads), 0, st,
                        static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);

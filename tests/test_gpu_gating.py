@@ -190,6 +190,27 @@ def test_route_gate_fused_gemm(native, E, topk, H, dtype):
         torch.testing.assert_close(w.cpu()[ok], ow[ok], atol=1e-4, rtol=0)
 
 
+@pytest.mark.parametrize("E,topk,H", [(16, 2, 2056), (3, 1, 1032), (9, 3, 4088)])
+@pytest.mark.parametrize("M", [17, 4096, 4097])
+def test_route_gate_sixteen_wavefronts(native, E, topk, H, M):
+    """Up to 16 experts and 4096 tokens a workgroup's sixteen wavefronts split chunks of 1024 K rows: a last chunk of a few rows,
+    a wavefront's share of it empty, a ragged last workgroup, and the batch size where the form changes."""
+    from fast_route_amd.ops.stable_route import fused_route
+    _say(f"route_gate E={E} H={H} M={M}")
+    g = torch.Generator().manual_seed(E * 7 + H)
+    h = (torch.randn(M, H, generator=g) / 4).to(torch.float16)
+    gate = (torch.randn(H, E, generator=g) / 4).to(torch.float16)
+    tw = torch.empty(M, topk, dtype=torch.float32, device="cuda")
+    ti = torch.empty(M, topk, dtype=torch.int32, device="cuda")
+    w, ids = fused_route(h.cuda(), gate.cuda(), topk, tw, ti, True)
+    torch.cuda.synchronize()
+    ow, oid = oracle.gating_topk((h.double() @ gate.double()).float(), topk, True)
+    flips = (ids.cpu() != oid)
+    assert flips.float().mean() < 0.002  # near-ties of fp32 sums
+    ok = ~flips.any(dim=1)
+    torch.testing.assert_close(w.cpu()[ok], ow[ok], atol=1e-4, rtol=0)
+
+
 @pytest.mark.parametrize("E,topk,H", [(8, 2, 264), (64, 6, 256), (24, 3, 512), (128, 8, 256), (100, 6, 512)])
 def test_route_gate_large_batch(native, E, topk, H):
     """From 16384 tokens on the kernel takes its unsplit form (64 or 128 tokens per workgroup,
