@@ -14,7 +14,7 @@ namespace fr {
 //                   in the 256-row tile one wavefront per SIMD issues the loads of both;
 //   64 rows:        3-slot ring, 8 wavefronts (4 with 256-byte row segments for the gate/up GEMM, persistent);
 //                   (the register-staged double buffer of STAGES == 0 is no longer used by any tile);
-//   32 / 16 rows:   decode regime, 16x16 MFMA, 3-slot ring, two workgroups per CU (the 16-row tile
+//   32 / 16 rows:   decode regime, 16x16 MFMA, 2- or 3-slot ring, two or more workgroups per CU (the 16-row tile
 //                   persistent or plain, see dispatch_block): weight streaming at HBM rate.  The gate/up GEMM
 //                   streams long weight rows faster in 512-byte segments: T32L (when H allows), T16L (rows over 2 KB, fp8 4 KB).
 template <typename T> struct Tiles {  // bf16 / fp16
@@ -36,11 +36,17 @@ template <typename T> struct Tiles {  // bf16 / fp16
   typedef Cfg<160, 256, 128, 2, 4, 16, 1, 3, 0, 2> T160P;
   typedef Cfg<64, 256, 128, 2, 4, 32, 1, 3, 3> T64;    // 3-slot ring like the 128-row tile (5 % over the register-staged form)
   typedef Cfg<64, 128, 256, 2, 2, 32, 1, 3> T64U;      // gate/up: 256-byte row segments, 4 wavefronts (another 5 %)
-  typedef Cfg<32, 128, 128, 1, 4, 16, 2, 3> T32;
+  // Two slots (40 KB: four workgroups per CU) instead of three (two): down projection, layer in parts of the time H = 2048, 64 experts, 32 tokens
+  // 0.99, H = 4096, F = 14336 60 0.988, fp16, 16 experts, F = 8192 100 0.985, H = 6144 60 0.98.
+  typedef Cfg<32, 128, 128, 1, 4, 16, 2, 2> T32;
   typedef Cfg<16, 64, 256, 1, 2, 16, 2, 3> T16;
   typedef Cfg<32, 128, 512, 1, 4, 16, 1, 2> T32L;
   typedef Cfg<16, 64, 512, 1, 2, 16, 2, 2> T16L;
+  typedef Cfg<32, 64, 256, 1, 2, 16, 2, 3> T32N;   // see dispatch_block
+  typedef Cfg<64, 256, 128, 2, 4, 16, 1, 3> T64W;
+  typedef Cfg<64, 128, 256, 2, 2, 16, 1, 3> T64N;
 };
+constexpr int kShortRow = 4096;  // bytes of a gate/up weight row up to which the 32- and 64-row tiles of 2-byte operands have forms of their own
 template <> struct Tiles<fp8_t> {  // the 16x16x128 MFMA eats 256 bytes of K per two K-steps
   // every wavefront issues its own tile loads: half the address registers per wavefront (the persistent down
   // projection spills 16 instead of 57 registers: 586 vs 595 us at M=4096 although no wavefront can then skip an
@@ -133,6 +139,24 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       // The persistent form hides each tile's ring fill behind its predecessor's last K tiles: the 64-row gate/up
       // GEMM streams the weights at 6.3 instead of 5.9 TB/s (128 tokens: 318 -> 298 us, fp8 192 -> 170 us).  The
       // down projection's 64-row tile gains nothing from it (147 us either way) and stays plain.
+      if constexpr (sizeof(T) == 2) {
+        // Rows of up to 4 KB: the 128-row tile's walk with half the rows.  Layer in parts of the time on T64U: H = 2048, 64 experts,
+        // top-6 100 tokens 0.95, 120 0.95, 150 0.99, 230 0.97; H = 1024, F = 3584 60 0.97, 100 0.975, 200 0.96, 400 0.92; longer rows 1.01 to
+        // 1.035 (H = 6144 0.98).
+        if (EPI == EPI_SILU && a.K * static_cast<int>(sizeof(T)) <= kShortRow && a.K % (TL::T64W::BKB / static_cast<int>(sizeof(T))) == 0) {
+          fill(64, TL::T64W::BF, TL::T64W::BKB);
+          return launch_gemm_persistent<T, typename TL::T64W, EPI>(a, splits, st);
+        }
+        // So few tiles that 256 features each leave CUs idle (in every K slice at most so many blocks, x feature tiles): 128 features,
+        // 256-byte row pieces.  H = 1024, F = 3584, 8 experts, layer in parts of the time on T64: 60 tokens (156 tiles at most) 0.94, 100 0.93,
+        // 200 (226) 0.92, but 400 (326) 1.05.
+        if (EPI != EPI_SILU && a.long_k && a.K % (TL::T64N::BKB / static_cast<int>(sizeof(T))) == 0) {
+          fill(64, TL::T64N::BF, TL::T64N::BKB);
+          if (static_cast<int64_t>(a.num_t_blocks) * ceil_div(a.N, TL::T64::BF) * splits < 256 &&
+              static_cast<int64_t>(a.k_per_split) * (splits - 1) < a.K)
+            return launch_gemm_persistent<T, typename TL::T64N, EPI>(a, splits, st);
+        }
+      }
       if (EPI == EPI_SILU && a.K % (TL::T64U::BKB / static_cast<int>(sizeof(T))) == 0) {
         fill(64, TL::T64U::BF, TL::T64U::BKB);
         return launch_gemm_persistent<T, typename TL::T64U, EPI>(a, splits, st);
@@ -140,6 +164,15 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       fill(64, TL::T64::BF, TL::T64::BKB);
       return launch_gemm<T, typename TL::T64, EPI>(a, splits, st);
     case 32:
+      if constexpr (sizeof(T) == 2) {
+        // Rows of up to 4 KB: half the features in 256-byte pieces on three slots, two workgroups per CU, whose start-up per tile
+        // overlaps (T32L has one).  H = 2048, 64 experts, top-6, layer in parts of the time on T32L: 20 tokens 0.96, 32 0.97, 48 0.96, 80 0.977
+        // (persistent 1.04, 1.005, 0.97, 0.95; on two slots 1.025, 0.98, 0.99, 1.00); longer rows 1.035 to 1.05.
+        if (EPI == EPI_SILU && a.K * static_cast<int>(sizeof(T)) <= kShortRow && a.K % (TL::T32N::BKB / static_cast<int>(sizeof(T))) == 0) {
+          fill(32, TL::T32N::BF, TL::T32N::BKB);
+          return launch_gemm<T, typename TL::T32N, EPI>(a, splits, st);
+        }
+      }
       if (EPI == EPI_SILU && a.K % (TL::T32L::BKB / static_cast<int>(sizeof(T))) == 0) {
         fill(32, TL::T32L::BF, TL::T32L::BKB);
         return launch_gemm<T, typename TL::T32L, EPI>(a, splits, st);
@@ -204,6 +237,14 @@ int prepare_tiles() {
   if (rc == FR_OK) rc = launch_gemm<T, typename TL::T64, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T16, EPI>(a, 1, nullptr);  // and its plain form
+  if constexpr (sizeof(T) == 2) {
+    if constexpr (EPI == EPI_SILU) {
+      if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32N, EPI>(a, 1, nullptr);
+      if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64W, EPI>(a, 1, nullptr);
+    } else {
+      if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64N, EPI>(a, 1, nullptr);
+    }
+  }
   if constexpr (EPI == EPI_SILU) {
     if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64U, EPI>(a, 1, nullptr);
     if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32L, EPI>(a, 1, nullptr);

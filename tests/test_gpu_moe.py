@@ -475,12 +475,13 @@ def test_rows_of_whole_and_partial_tiles(native, block, N):
 
 
 @pytest.mark.parametrize("split", [1, 3])
-@pytest.mark.parametrize("H,Fd", [(384, 1152), (640, 1664), (2432, 2176)])
+@pytest.mark.parametrize("H,Fd", [(384, 1152), (640, 1664), (2048, 1152), (2432, 2176)])
 @pytest.mark.parametrize("block", [16, 32, 64, 128, 160])
 def test_k_starts_of_tiles_alone_on_their_weights(native, block, H, Fd, split):
     """A tile that is alone on its weight tile (16 and 32 rows: any tile) walks its K tiles from a place of its own, round the end:
     K loops from the shortest the persistent kernels take (6 K tiles) up, odd counts, K slices and cut last rounds, experts with one
-    block next to experts with several and with none."""
+    block next to experts with several and with none; gate/up rows on both sides of 4 KB (2048 elements: the last of the short ones), where
+    32 and 64 rows have forms of their own, and 64-row down projections with fewer tiles than CUs (one slice) and with more (three)."""
     import fast_route_amd as fr
     from fast_route_amd import fused_experts
     E = 12
