@@ -69,19 +69,22 @@ struct Carve {
   float* tail;       // scratch for splitting the last round of 256-row tiles, or nullptr
   int* tail_cuts;    // and the list of the tiles cut
   bool any_height;   // the GEMMs' tiles need not be the plan's blocks
+  bool tall;         // the buffers in `tail` hold tiles of 288 rows
   void* xq;          // fp8 layer only
   float* x_scale;
   void* actq;
   float* act_scale;
   int64_t total;
-  TailScratch tail_scratch() const { return TailScratch{tail, tail_cuts, any_height, tail != nullptr}; }
+  TailScratch tail_scratch() const { return TailScratch{tail, tail_cuts, any_height, tail && tall}; }
 };
 
 // the activated intermediate is stored in half precision also on the fp8 path
 int act_elem_size(int) { return 2; }
 
-Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
+// tall: slice buffers for tiles of 288 rows; without them kTallTailBytes - tail_bytes (8.4 MB) less
+Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p, bool tall = true) {
   Carve c;
+  c.tall = tall;
   const int64_t n = M * topk;
   char* b = static_cast<char*>(base);
   int64_t off = 0;
@@ -95,7 +98,7 @@ Carve carve(void* base, int64_t M, int64_t H, int64_t F, int E, int topk, int dt
   c.align_ws = take(c.align_ws_bytes);
   c.act = take(p.sorted_len * F * act_elem_size(dtype));
   c.partial = reinterpret_cast<float*>(take(static_cast<int64_t>(p.split_k) * n * H * 4));
-  c.tail = p.tail_bytes > 0 ? reinterpret_cast<float*>(take(p.tail_bytes > kTallTailBytes ? p.tail_bytes : kTallTailBytes)) : nullptr;
+  c.tail = p.tail_bytes > 0 ? reinterpret_cast<float*>(take(tall && p.tail_bytes < kTallTailBytes ? kTallTailBytes : p.tail_bytes)) : nullptr;
   c.any_height = any_height(M, H, F, E, topk, dtype, p);
   c.tail_cuts = p.tail_bytes > 0 ? reinterpret_cast<int*>(take(kTailDescBytes)) : nullptr;
   c.xq = nullptr; c.x_scale = nullptr; c.actq = nullptr; c.act_scale = nullptr;
@@ -315,6 +318,26 @@ fr_moe_plan layer_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dty
   const fr_moe_plan q = plan_for(M, H, F, E, topk, dtype, block);
   return p.split_k > 1 && q.split_k == 1 ? p : q;
 }
+
+// The blocks, slices and buffers of a layer call in the workspace it was given (p: fr_moe_get_plan's result, whose bytes hold all of
+// them).  A smaller workspace, as a caller may have kept it for these sizes, is enough while it holds the plan's own block with slice
+// buffers of 256 rows: the call then does without what does not fit.
+int layer_carve(const char* who, int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, fr_moe_plan& p, void* workspace, int64_t bytes,
+                Carve& c) {
+  FR_REQUIRE(workspace, FR_E_WORKSPACE, "%s: no workspace (%lld bytes needed)", who, (long long)p.workspace_bytes);
+  bool tall = true;
+  fr_moe_plan q = layer_plan(M, H, F, E, topk, dtype, p);
+  if (bytes < p.workspace_bytes) {
+    const int64_t least = carve(nullptr, M, H, F, E, topk, dtype, p, false).total;
+    FR_REQUIRE(bytes >= least, FR_E_WORKSPACE, "%s: workspace %lld < %lld bytes", who, (long long)bytes, (long long)least);
+    if (carve(nullptr, M, H, F, E, topk, dtype, q, false).total > bytes) q = p;
+    tall = carve(nullptr, M, H, F, E, topk, dtype, q).total <= bytes;
+  }
+  FR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, FR_E_ALIGN, "%s: workspace must be 256-byte aligned", who);
+  p = q;
+  c = carve(workspace, M, H, F, E, topk, dtype, p, tall);
+  return FR_OK;
+}
 }  // namespace
 }  // namespace fr
 
@@ -357,10 +380,9 @@ extern "C" int fr_fused_experts(const void* x, const void* w1, const void* w2, c
   if (rc != FR_OK) return rc;
   if (M == 0) return FR_OK;
   FR_REQUIRE(x && w1 && w2 && topk_weights && topk_ids && out, FR_E_NULL, "fr_fused_experts: null pointer");
-  FR_REQUIRE(workspace && workspace_bytes >= p.workspace_bytes, FR_E_WORKSPACE, "fr_fused_experts: workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)p.workspace_bytes);
-  FR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, FR_E_ALIGN, "fr_fused_experts: workspace must be 256-byte aligned");
-  p = layer_plan(M, H, F, E, topk, dtype & ~FR_W_TILED, p);
-  Carve c = carve(workspace, M, H, F, E, topk, dtype & ~FR_W_TILED, p);
+  Carve c;
+  rc = layer_carve("fr_fused_experts", M, H, F, E, topk, dtype & ~FR_W_TILED, p, workspace, workspace_bytes, c);
+  if (rc != FR_OK) return rc;
   rc = fr_moe_align(topk_ids, FR_I32, M * topk, E, p.block, c.sorted, c.expert_ids, c.npost, c.align_ws, c.align_ws_bytes, stream);
   if (rc != FR_OK) return rc;
   rc = gateup_impl(x, nullptr, w1, nullptr, c.sorted, c.expert_ids, c.npost, M, H, F, E, topk, p.block, dtype & ~FR_W_TILED, c.act, c.tail_scratch(),
@@ -373,15 +395,15 @@ extern "C" int fr_fused_experts(const void* x, const void* w1, const void* w2, c
 
 namespace fr {
 namespace {
-// the layer with the blocks and slices of `p`; need: what the caller was told the workspace has to hold
-int fused_moe_run(const fr_moe_plan& p, int64_t need, const void* x, const void* w1, const void* w2, const void* logits, int logits_dtype,
+// p: fr_moe_get_plan's result
+int fused_moe_run(fr_moe_plan p, const void* x, const void* w1, const void* w2, const void* logits, int logits_dtype,
                   int64_t M, int64_t H, int64_t F, int E, int topk, int renormalize, int dtype, void* out, void* workspace,
                   int64_t workspace_bytes, void* stream) {
   int rc;
   FR_REQUIRE(x && w1 && w2 && logits && out, FR_E_NULL, "fr_fused_moe: null pointer");
-  FR_REQUIRE(workspace && workspace_bytes >= need, FR_E_WORKSPACE, "fr_fused_moe: workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
-  FR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, FR_E_ALIGN, "fr_fused_moe: workspace must be 256-byte aligned");
-  Carve c = carve(workspace, M, H, F, E, topk, dtype & ~FR_W_TILED, p);
+  Carve c;
+  rc = layer_carve("fr_fused_moe", M, H, F, E, topk, dtype & ~FR_W_TILED, p, workspace, workspace_bytes, c);
+  if (rc != FR_OK) return rc;
   // a handful of tokens: the gate/up launch gates and sorts by itself (row-major weights only)
   rc = (dtype & FR_W1_TILED) ? 1
                             : gateup_rows_routed(x, w1, logits, logits_dtype, M, H, F, E, topk, renormalize, p.block, dtype, c.act, c.topk_w,
@@ -408,8 +430,7 @@ extern "C" int fr_fused_moe(const void* x, const void* w1, const void* w2, const
   int rc = fr_moe_get_plan(M, H, F, E, topk, dtype, &p);
   if (rc != FR_OK) return rc;
   if (M == 0) return FR_OK;
-  return fused_moe_run(layer_plan(M, H, F, E, topk, dtype & ~FR_W_TILED, p), p.workspace_bytes, x, w1, w2, logits, logits_dtype, M, H, F, E,
-                       topk, renormalize, dtype, out, workspace, workspace_bytes, stream);
+  return fused_moe_run(p, x, w1, w2, logits, logits_dtype, M, H, F, E, topk, renormalize, dtype, out, workspace, workspace_bytes, stream);
 }
 
 extern "C" int fr_fused_moe_fp8(const void* x, int x_dtype, const void* w1q, const float* w1_scale, const void* w2q,
@@ -424,10 +445,10 @@ extern "C" int fr_fused_moe_fp8(const void* x, int x_dtype, const void* w1q, con
   x_dtype &= ~FR_W_TILED;
   FR_REQUIRE(x_dtype == FR_BF16, FR_E_DTYPE, "fr_fused_moe_fp8: activations must be bf16 (dtype %d)", x_dtype);
   FR_REQUIRE(x && w1q && w1_scale && w2q && w2_scale && logits && out, FR_E_NULL, "fr_fused_moe_fp8: null pointer");
-  FR_REQUIRE(workspace && workspace_bytes >= p.workspace_bytes, FR_E_WORKSPACE, "fr_fused_moe_fp8: workspace %lld < %lld bytes", (long long)workspace_bytes, (long long)p.workspace_bytes);
-  FR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, FR_E_ALIGN, "fr_fused_moe_fp8: workspace must be 256-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  Carve c = carve(workspace, M, H, F, E, topk, FR_FP8_E4M3, p);
+  Carve c;
+  rc = layer_carve("fr_fused_moe_fp8", M, H, F, E, topk, FR_FP8_E4M3, p, workspace, workspace_bytes, c);
+  if (rc != FR_OK) return rc;
   rc = route_and_align(logits, logits_dtype, M, E, topk, renormalize, p.block, c, x, H, stream);
   if (rc != FR_OK) return rc;
   // the eight-wavefront kernels' gate/up GEMM does not cut its last round in fp8
@@ -482,17 +503,14 @@ extern "C" int fr_fused_moe_noalloc(const void* x, const void* w1, const void* w
   int rc = fr_moe_get_plan(M, H, F, E, topk, dtype, &p);
   if (rc != FR_OK) return rc;
   FR_REQUIRE((dtype & ~FR_W_TILED) == FR_F16 || (dtype & ~FR_W_TILED) == FR_BF16, FR_E_DTYPE, "fr_fused_moe_noalloc: dtype %d not in {f16, bf16}", dtype);
-  // the plan's own bytes decide, and where the block the layers route for instead would not fit, its block is taken, too
-  const int op_dtype = dtype & ~FR_W_TILED;
-  p = plan_for(M, H, F, E, topk, op_dtype, p.block);
-  FR_REQUIRE(p.workspace_bytes <= kStaticScratchBytes, FR_E_WORKSPACE,
+  // the plan's own bytes decide; layer_carve takes its block, too, where the one the layers route for instead does not fit
+  const int64_t own_bytes = plan_for(M, H, F, E, topk, dtype & ~FR_W_TILED, p.block).workspace_bytes;
+  FR_REQUIRE(own_bytes <= kStaticScratchBytes, FR_E_WORKSPACE,
              "fr_fused_moe_noalloc: these sizes need %lld bytes of scratch, the library's static scratch holds %lld; use fr_fused_moe with a workspace",
-             (long long)p.workspace_bytes, (long long)kStaticScratchBytes);
+             (long long)own_bytes, (long long)kStaticScratchBytes);
   if (M == 0) return FR_OK;
   void* ws = nullptr;
   rc = static_scratch(&ws);
   if (rc != FR_OK) return rc;
-  fr_moe_plan q = layer_plan(M, H, F, E, topk, op_dtype, p);
-  if (q.workspace_bytes > kStaticScratchBytes) q = p;
-  return fused_moe_run(q, q.workspace_bytes, x, w1, w2, logits, logits_dtype, M, H, F, E, topk, renormalize, dtype, out, ws, kStaticScratchBytes, stream);
+  return fused_moe_run(p, x, w1, w2, logits, logits_dtype, M, H, F, E, topk, renormalize, dtype, out, ws, kStaticScratchBytes, stream);
 }

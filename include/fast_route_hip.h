@@ -139,7 +139,9 @@ int fr_moe_prepare_weights(const void* w, int dtype, int64_t E, int64_t rows, in
  * bytes or more, under some plans of 128 and 160 with one K slice.
  * fr_fused_moe, fr_fused_experts and fr_fused_moe_noalloc may route for another
  * block than the plan's where that is faster (layer_block in fused_moe.hip);
- * workspace_bytes covers both.                                                */
+ * workspace_bytes covers both.  They run in a workspace that holds no more than
+ * the plan's own block with 64 MiB of tail scratch, too, as earlier versions of
+ * this library asked for, on the plan's block and with fewer tail buffers.      */
 typedef struct fr_moe_plan {
   int32_t block;      /* routing block                                       */
   int32_t split_k;    /* K splits of the down projection                     */

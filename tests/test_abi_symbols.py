@@ -184,6 +184,38 @@ def test_recorded_traffic_matches_profiles_file():
     assert mod.recorded_traffic("no_such_workload", block) is None
 
 
+def test_layers_accept_the_scratch_of_the_plans_own_block():
+    """The plan's bytes also hold what the layers route for instead of its block, and tail buffers for 288-row tiles.  A workspace with
+    neither is enough, one byte less is refused.  (The workspace is misaligned, so that no call gets beyond its checks.)"""
+    import fast_route_amd as fr
+    from fast_route_amd import _native
+    lib = _native.lib()
+    taller = 256 * 256 * 4 * (288 - 256)
+    for M, H, F, E, k in ((16, 4096, 14336, 8, 2), (32, 2048, 1408, 64, 6), (240, 2048, 1408, 64, 6), (130, 1024, 3584, 8, 2),
+                          (900, 4096, 8192, 16, 2), (700, 4096, 14336, 8, 2), (4096, 4096, 14336, 8, 2)):
+        for dt in (_native.FR_BF16, _native.FR_F16) + ((_native.FR_FP8_E4M3,) if F % 256 == 0 else ()):
+            p, own = _native.FrMoePlan(), _native.FrMoePlan()
+            assert lib.fr_moe_get_plan(M, H, F, E, k, dt, p) == 0
+            try:
+                with fr.tunables(block=p.block, split_k=p.split_k):
+                    assert lib.fr_moe_get_plan(M, H, F, E, k, dt, own) == 0
+            finally:
+                fr.reset_tunables()
+            least = own.workspace_bytes - (taller if own.tail_bytes else 0)
+            assert (own.split_k, own.tail_bytes) == (p.split_k, p.tail_bytes) and least <= p.workspace_bytes
+
+            def call(n):
+                if dt == _native.FR_FP8_E4M3:
+                    rc = lib.fr_fused_moe_fp8(256, _native.FR_BF16, 256, 256, 256, 256, 256, _native.FR_BF16, M, H, F, E, k, 1, 256, 257, n, None)
+                else:
+                    rc = lib.fr_fused_moe(256, 256, 256, 256, _native.FR_BF16, M, H, F, E, k, 1, dt, 256, 257, n, None)
+                assert rc != 0
+                return lib.fr_last_error_string().decode()
+            for n in (least, p.workspace_bytes):
+                assert "aligned" in call(n), (M, dt, n)
+            assert "workspace" in call(least - 1) and "aligned" not in call(least - 1)
+
+
 def test_tunables_override_the_plan_and_reset():
     """fr_moe_set_tunables is host logic: the plan follows the overrides, rejects values outside its ranges,
     and NULL restores the library's own choices."""

@@ -895,6 +895,35 @@ def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, 
     _assert_close(fused_experts(*args, w.cuda(), ids.cuda()), oracle.moe_experts(x, w1, w2, w, ids), dtype, "experts")
 
 
+@pytest.mark.parametrize("M,H,Fd,E,k", [(68, 2048, 256, 32, 4), (900, 4096, 1024, 16, 2), (1031, 4096, 4096, 8, 2)])
+def test_layer_in_the_scratch_of_the_plans_own_block(native, M, H, Fd, E, k):
+    """A workspace that holds the plan's block and tail buffers of 256 rows only: the layer stays inside it and matches the oracle."""
+    import fast_route_amd as fr
+    from fast_route_amd import _native
+    from fast_route_amd.layers.fused_moe import plan
+    dtype = torch.bfloat16
+    _say(f"smaller workspace M={M} H={H} F={Fd} E={E}")
+    p = plan(M, H, Fd, E, k, dtype)
+    try:
+        with fr.tunables(block=p.block, split_k=p.split_k):
+            own = plan(M, H, Fd, E, k, dtype)
+    finally:
+        fr.reset_tunables()
+    least = own.workspace_bytes - (256 * 256 * 4 * (288 - 256) if own.tail_bytes else 0)
+    x, logits, w1, w2 = _inputs(M, H, Fd, E, 3 + M, dtype)
+    xd, ld, w1d, w2d = x.cuda(), logits.cuda(), w1.cuda(), w2.cuda()
+    guard = 4096
+    for n in (least, p.workspace_bytes):
+        buf = torch.full((n + 2 * guard,), 0x5A, dtype=torch.uint8, device="cuda")
+        ws, out = buf[guard:], torch.empty_like(xd)
+        assert ws.data_ptr() % 256 == 0
+        _native.check(_native.lib().fr_fused_moe(xd.data_ptr(), w1d.data_ptr(), w2d.data_ptr(), ld.data_ptr(), _native.dtype_code(ld.dtype), M, H, Fd,
+                                                 E, k, 1, _native.dtype_code(dtype), out.data_ptr(), ws.data_ptr(), n, _native.stream_ptr(xd.device)))
+        torch.cuda.synchronize()
+        assert (buf[:guard] == 0x5A).all() and (buf[guard + n:] == 0x5A).all()
+        _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, f"{n} bytes")
+
+
 @pytest.mark.parametrize("M,Fd", [(645, 3200), (860, 7552)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_one_tile_per_expert_where_the_plan_has_two(native, kernels_of, dtype, M, Fd):
