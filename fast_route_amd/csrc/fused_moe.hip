@@ -295,19 +295,22 @@ fr_moe_plan plan_for(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype
 // Layer in parts of the time with the plan's block:
 //   Many narrow experts with skewed loads (H = 2048, F = 1408, 64 experts, top-6, Zipf): the heavy experts take several small tiles.  (Up
 //   to 128 experts and F = 2816: the routing blocks' padding is E x block rows of F activated values.)
-//     plan 16: 32 rows 20 tokens (1.9 pairs per expert) 0.96, 32 0.98, 40 0.905, 48 0.997, 72 0.94, 80 0.92, but 6 to 16 tokens 1.01 to 1.05;
-//     plan 32: 64 rows 90 (8.4) 0.99, 110 0.95, 180 0.86, 230 (21.6) 0.86; 128 rows 260 (24.4) 0.85 (64: 0.84), 290 0.80 (0.78), 335 0.74 (0.79)
+//     plan 16: 32 rows 12 tokens (1.1 pairs per expert) 0.98, 18 0.96, 32 0.92, 40 0.87, 48 0.95, 72 0.89, 80 0.87, but 8 and 10 (0.9) 1.03;
+//     64 rows 12 to 20 tokens 0.93 to 0.96, but 22 to 40 1.05 to 1.12: where the active experts' tiles are two rounds, which depends
+//     on the routing;
+//     plan 32: 64 rows instead of 32 90 (8.4) 1.00, 110 0.92, 180 0.86, 230 0.80, 290 (27.2) 0.74; 128 rows 260 1.09, 290 1.11 of
+//     64 rows, 300 (28.1) 1.00, 310 to 335 0.92 to 0.98
 //   H = 1024, F = 3584, 8 experts: the plan's 64-row range begins at H = 4096, and the 128-row tile has 16 short K tiles there.
-//     16 rows 33 to 48 tokens (8 to 12 pairs) 0.91, 56 (14) 0.96; 64 rows 56 0.96, 100 0.95, 120 0.84, 128 (32) 0.80, 240 0.91, 460 (115) 0.95,
-//     500 (125) 1.00, 520 1.03
+//     16 rows 33 to 48 tokens (8 to 12 pairs) 0.91 (64 rows 0.97 of that, 0.98 to 1.07 below 33), 56 (14) 0.96; 64 rows 60 0.88, 90 0.86, 130
+//     (32.5) 0.70, 200 0.73, 300 0.80, 460 (115) 0.80, 490 0.97, 500 (125) 0.89, 525 1.01, 550 1.03, 600 1.08
 //   160 rows instead of 128 where an expert is likely to exceed 128 rows: a block more costs a round of tiles, the larger tile 1 %.
 //     16 experts, F = 8192, fp16: 880 tokens (110 pairs; one expert above 128) 0.90, 920 0.88, 800 (none) 0.99; H = 6144 460 (115) 0.95;
 //     H = 4096, F = 14336, 8 experts none above 128: 300 and 420 1.01.
 int layer_block(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
   if ((dtype != FR_F16 && dtype != FR_BF16) || g_tunables.block) return p.block;
   const double avg = static_cast<double>(M) * topk / E;
-  if (E >= 32 && E <= 128 && H >= 2048 && H < 4096 && F <= 2816 && p.block <= 32 && avg >= 1.75) return avg < 8.5 ? 32 : avg < 24 ? 64 : 128;
-  if (E <= 16 && H >= 640 && H <= 1024 && F >= 1024 && (p.block == 32 || p.block == 128) && avg < 118) return avg <= 12 ? 16 : 64;
+  if (E >= 32 && E <= 128 && H >= 2048 && H < 4096 && F <= 2816 && p.block <= 32 && avg >= 1.05) return avg < 8.5 ? 32 : avg < 28 ? 64 : 128;
+  if (E <= 16 && H >= 640 && H <= 1024 && F >= 1024 && (p.block == 32 || p.block == 128) && avg < 126) return avg <= 12 ? 16 : 64;
   if (E <= 16 && H >= 4096 && F >= 1024 && p.block == 128 && avg < 128 && E * (expected_blocks(avg, E, 128) - 1.0) >= 0.15) return 160;
   return p.block;
 }

@@ -873,9 +873,9 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
 
 
 @pytest.mark.parametrize("M,H,Fd,E,k,planned,rows", [
-    (17, 2048, 256, 32, 4, 16, 32), (67, 2048, 256, 32, 4, 32, 32), (68, 2048, 256, 32, 4, 32, 64), (191, 2048, 256, 32, 4, 32, 64),
-    (192, 2048, 256, 32, 4, 32, 128), (255, 2048, 256, 32, 4, 32, 128), (36, 1024, 2048, 8, 2, 32, 16), (48, 1024, 2048, 8, 2, 32, 16),
-    (49, 1024, 2048, 8, 2, 32, 64), (471, 1024, 2048, 8, 2, 128, 64), (472, 1024, 2048, 8, 2, 128, 128), (900, 4096, 1024, 16, 2, 128, 160)])
+    (8, 2048, 256, 32, 4, 16, 16), (9, 2048, 256, 32, 4, 16, 32), (67, 2048, 256, 32, 4, 32, 32), (68, 2048, 256, 32, 4, 32, 64), (223, 2048, 256, 32, 4, 32, 64),
+    (224, 2048, 256, 32, 4, 32, 128), (255, 2048, 256, 32, 4, 32, 128), (36, 1024, 2048, 8, 2, 32, 16), (48, 1024, 2048, 8, 2, 32, 16),
+    (49, 1024, 2048, 8, 2, 32, 64), (503, 1024, 2048, 8, 2, 128, 64), (504, 1024, 2048, 8, 2, 128, 128), (900, 4096, 1024, 16, 2, 128, 160)])
 def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, Fd, E, k, planned, rows):
     """At the edges of the ranges where the layers take other tiles than the plan's block stands for: the plan stays, its workspace
     covers both, and results match the oracle."""
