@@ -515,10 +515,18 @@ void dispatch_route_align(const void* logits, int64_t M, int E, int topk, int re
 
 // Gating and routing arrays in one launch for small batches; false when the shape is
 // outside what one workgroup should do (the caller then runs the two stages separately).
-// (one workgroup gates and sorts 1024 pairs in 10.5 us; from there on the gating kernel spread over the CUs
-// plus the one-workgroup sort are faster: 8.9 us + a launch gap at 1024 pairs, 12.6 against 26.8 us at 4096)
-bool route_align_fits(int64_t M, int E, int topk) {
-  return M >= 1 && M * topk <= kRouteAlignMaxN && use_small_path(M * topk, E) && M * E <= 16384 && topk <= E;
+// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = next power of two of E; two launches cost 2 us
+// more and spread the gating over the CUs.  A layer with H = F = 128 in us, one / two launches:
+//   64 experts, top-6   16 tokens (1 round) 17.8 / 19.8, 32 (2) 19.8 / 19.5, 48 (3) 21.9 / 19.8, 80 (5) 25.9 / 19.7, 168 38.4 / 20.8
+//   32, top-4           64 (2) 18.5 / 19.3, 96 (3) 21.0 / 19.8, 256 34.9 / 24.9
+//   16, top-2           192 (3) 18.7 / 19.9, 256 (4) 25.1 / 23.6, 512 29.2 / 24.4;  8, top-2 256 (2) 23.2 / 23.7, 384 (3) 24.9 / 24.6, 512 26.2 / 24.9
+//   128 (two logits per lane), top-8   16 (1) 22.6 / 22.3, 32 (2) 27.8 / 22.8, 127 57.5 / 24.5;  256 16 26.0 / 25.3, 64 48.9 / 29.5
+// quant: the launch also quantises the token rows, which would be a third one; it then keeps all that one workgroup holds.
+bool route_align_fits(int64_t M, int E, int topk, bool quant) {
+  if (M < 1 || M * topk > kRouteAlignMaxN || !use_small_path(M * topk, E) || M * E > 16384 || topk > E) return false;
+  int G = 1;
+  while (G < E && G < 64) G *= 2;
+  return quant || M * G <= 1024 * (E > 64 ? 1 : topk <= 2 ? 3 : 2);
 }
 int route_align_small(const void* logits, int logits_dtype, int64_t M, int E, int topk, int renorm, int block,
                       float* w, int32_t* ids, int32_t* sorted, int32_t* expert_ids, int32_t* npost,

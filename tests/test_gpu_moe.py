@@ -895,6 +895,20 @@ def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, 
     _assert_close(fused_experts(*args, w.cuda(), ids.cuda()), oracle.moe_experts(x, w1, w2, w, ids), dtype, "experts")
 
 
+@pytest.mark.parametrize("M,E,k,launches", [(32, 64, 6, 1), (33, 64, 6, 2), (31, 33, 4, 1), (33, 33, 4, 2), (64, 32, 4, 1), (65, 32, 4, 2),
+                                            (192, 16, 2, 1), (193, 16, 2, 2), (128, 16, 3, 1), (129, 16, 3, 2), (384, 8, 2, 1), (385, 8, 2, 2),
+                                            (16, 128, 8, 1), (17, 128, 8, 2), (16, 200, 6, 1), (17, 200, 6, 2)])
+def test_gating_and_sort_in_one_launch_or_two(native, kernels_of, M, E, k, launches):
+    """Both sides of the rule that leaves small batches' gating and sort to one workgroup; the layer matches the oracle."""
+    from fast_route_amd import fused_moe
+    dtype = torch.bfloat16
+    _say(f"routing launches M={M} E={E} k={k}")
+    x, logits, w1, w2 = _inputs(M, 128, 128, E, 5 + M, dtype)
+    out, names = kernels_of(lambda: fused_moe(x.cuda(), w1.cuda(), w2.cuda(), logits.cuda(), k, True))
+    assert sum("route_align_small" in n for n in names) == (launches == 1) and sum("gating_topk" in n for n in names) == (launches == 2), names
+    _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, "layer")
+
+
 @pytest.mark.parametrize("M,H,Fd,E,k", [(68, 2048, 256, 32, 4), (900, 4096, 1024, 16, 2), (1031, 4096, 4096, 8, 2)])
 def test_layer_in_the_scratch_of_the_plans_own_block(native, M, H, Fd, E, k):
     """A workspace that holds the plan's block and tail buffers of 256 rows only: the layer stays inside it and matches the oracle."""
