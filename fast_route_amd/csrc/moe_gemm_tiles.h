@@ -147,9 +147,9 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
           fill(64, TL::T64W::BF, TL::T64W::BKB);
           return launch_gemm_persistent<T, typename TL::T64W, EPI>(a, splits, st);
         }
-        // So few tiles that 256 features each leave CUs idle (in every K slice at most so many blocks, x feature tiles): 128 features,
-        // 256-byte row pieces.  H = 1024, F = 3584, 8 experts, layer in parts of the time on T64: 60 tokens (156 tiles at most) 0.94, 100 0.93,
-        // 200 (226) 0.92, but 400 (326) 1.05.
+        // Fewer tiles of 256 features than CUs, K slices included (by the worst-case block count, which is all the host knows): 128
+        // features in 256-byte row pieces.  H = 1024, F = 3584, 8 experts, layer in parts of the time on T64: 60 tokens (156 tiles at
+        // most) 0.94, 100 0.93, 200 (226) 0.92, but 400 (326) 1.05.
         if (EPI != EPI_SILU && a.long_k && a.K % (TL::T64N::BKB / static_cast<int>(sizeof(T))) == 0) {
           fill(64, TL::T64N::BF, TL::T64N::BKB);
           if (static_cast<int64_t>(a.num_t_blocks) * ceil_div(a.N, TL::T64::BF) * splits < 256 &&
