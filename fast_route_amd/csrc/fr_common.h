@@ -54,6 +54,9 @@ int gateup_rows_routed(const void* x, const void* w1, const void* logits, int lo
 int prepare_static_scratch();
 
 constexpr int kTailDescBytes = 8192;  // what TailScratch::cuts points to
+// Whether the tiles of a GEMM may have other heights than its routing block (plans of 128 and 160 rows): no; yes; or where the
+// experts' runs, which only the device knows, favour it (launch_gemm_by_runs).
+enum { kHeightsOfBlock = 0, kHeightsAny = 1, kHeightsByRuns = 2 };
 constexpr int64_t kTallTailBytes = int64_t(256) * 288 * 256 * 4;  // slice buffers of the tallest tiles, one per workgroup
 
 // Scratch of a grouped GEMM for cutting the tiles of its last round along K (plan.tail_bytes, or nullptr), a place for the
@@ -63,11 +66,11 @@ constexpr int64_t kTallTailBytes = int64_t(256) * 288 * 256 * 4;  // slice buffe
 struct TailScratch {
   float* buffers = nullptr;
   int* cuts = nullptr;
-  bool any_height = false;
+  int any_height = kHeightsOfBlock;
   bool tall = false;  // buffers holds kTallTailBytes (at least plan.tail_bytes)
 };
 
-bool plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block);
+int plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block);
 
 // Gate/up projection + SiLU * up (what fr_moe_gateup_silu / fr_moe_gateup_silu_fp8 launch).
 int gateup_impl(const void* x, const float* x_scale, const void* w1, const float* w1_scale,

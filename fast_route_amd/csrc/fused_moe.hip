@@ -30,7 +30,15 @@ double expected_blocks(double avg, int E, int rows) {
 //   H = 1024, F = 3584, 8 experts    2200 to 4096 0.93 to 1.03, 4142 (1036) 0.87
 // With fewer pairs (H >= 4096), where an expert's run is one tile of it and the plan's rows make it two: the weights pass through the
 // CUs once.  Up to 7 units (fp8: 6) such a tile streams its weights (moe_gemm_quad.h); 8 and 9 units gain less and lose to
-// the plan's tiles in a launch of few.
+// the plan's tiles in a launch of few.  That holds for runs of about the same length, which is all that is priced here: with skewed loads the
+// plan's tiles are faster, so the device chooses by the runs (launch_gemm_by_runs; its second launch of either GEMM costs 4 us).
+// Layer in parts of the time with the plan's tiles, near-uniform load tall tiles / chosen by runs, and Zipf-skewed load tall / by runs:
+//   H = 4096, F = 14336, 8 experts   645 tokens 0.845 / 0.855, 1.10 / 1.00; 850 0.94 / 0.94, 1.13 / 1.005; 1031 0.96 / 0.965, 1.07 / 1.01
+//                                    fp8 640 0.90 / 0.92, 1.01 / 1.02; 700 0.965 / 0.97, 1.05 / 1.02
+//   H = 6144, F = 16384              900 0.925 / 0.93, 1.20 / 1.01;  H = 5120, F = 8192, 16 experts 1350 0.86 / 0.865, 1.18 / 1.00
+//   16 experts, F = 8192, fp16       1300 0.84 / 0.85, 1.11 / 1.00;  H = 7168, F = 2048, 64 experts, top-8 1350 0.88 / 0.885, 1.09 / 1.005
+//   H = 4096, F = 4096, 8 experts    640 0.835 / 0.86, 1.15 / 1.025; F = 1536, 32 experts, top-4 1350 0.955 / 0.97, 1.15 / 1.02
+// Tall tiles for every load, near-uniform, the plan's tiles / tall:
 //   H = 4096, F = 14336, 8 experts   645 (161) 735 / 635, 700 735 / 637, 850 783 / 702, 950 802 / 778, 1031 (258) 832 / 797, 1080
 //                                    845 / 826, but 1120 (280: some experts two tiles) 841 / 851, 1160 855 / 881, 1200 880 / 890
 //                                    fp8 640 441 / 397, 700 426 / 401, but 740 (185) 437 / 433, 800 442 / 452, 950 475 / 473
@@ -45,15 +53,15 @@ double expected_blocks(double avg, int E, int rows) {
 // expert, F = 14336 (224) 0.97, 8 experts, F = 2048 (256) 1400 0.87.
 // Only where the plan has a single K slice: that kernel writes a pair's row once, in the operands' 2-byte type, where several
 // slices are summed from fp32 rows.
-bool any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
+int any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
   const fr_moe_tunables& t = g_tunables;
-  if ((p.block != 128 && p.block != 160) || p.split_k > 1 || t.no_quad || t.block || E > 1022) return false;
+  if ((p.block != 128 && p.block != 160) || p.split_k > 1 || t.no_quad || t.block || E > 1022) return kHeightsOfBlock;
   const int es = dtype == FR_FP8_E4M3 ? 1 : 2;
-  if (H * es < 2048 || F * es < 2048) return false;  // 16 K tiles in both GEMMs
+  if (H * es < 2048 || F * es < 2048) return kHeightsOfBlock;  // 16 K tiles in both GEMMs
   const double avg = static_cast<double>(M) * topk / E, tall = expected_blocks(avg, E, 288), tiles = E * tall * (F / 128);
-  if (avg >= (H >= 4096 ? 310.0 : H >= 2048 ? 550.0 : 1030.0)) return tiles >= 200.0;
-  if (H < 4096 || expected_blocks(avg, E, p.block) < 1.3) return false;
-  return (expected_blocks(avg, E, es == 2 ? 224 : 192) <= 1.13 && tiles >= 200.0) || (es == 2 && tall <= 1.13 && tiles >= 450.0);
+  if (avg >= (H >= 4096 ? 310.0 : H >= 2048 ? 550.0 : 1030.0)) return tiles >= 200.0 ? kHeightsAny : kHeightsOfBlock;
+  if (H < 4096 || expected_blocks(avg, E, p.block) < 1.3) return kHeightsOfBlock;
+  return (expected_blocks(avg, E, es == 2 ? 224 : 192) <= 1.13 && tiles >= 200.0) || (es == 2 && tall <= 1.13 && tiles >= 450.0) ? kHeightsByRuns : kHeightsOfBlock;
 }
 
 struct Carve {
@@ -68,7 +76,7 @@ struct Carve {
   float* partial;
   float* tail;       // scratch for splitting the last round of 256-row tiles, or nullptr
   int* tail_cuts;    // and the list of the tiles cut
-  bool any_height;   // the GEMMs' tiles need not be the plan's blocks
+  int any_height;    // the GEMMs' tiles need not be the plan's blocks
   bool tall;         // the buffers in `tail` hold tiles of 288 rows
   void* xq;          // fp8 layer only
   float* x_scale;
@@ -125,11 +133,11 @@ int check_layer_shapes(const char* who, int64_t M, int64_t H, int64_t F, int E, 
 }  // namespace
 const fr_moe_tunables& tunables() { return g_tunables; }
 
-bool plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block) {
+int plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block) {
   const int mult = dtype == FR_FP8_E4M3 ? 256 : 128;
-  if ((block != 128 && block != 160) || H % mult || F % mult || E > 1022 || topk > E) return false;  // shapes without a plan among them
+  if ((block != 128 && block != 160) || H % mult || F % mult || E > 1022 || topk > E) return kHeightsOfBlock;  // shapes without a plan among them
   fr_moe_plan p;
-  return fr_moe_get_plan(M, H, F, E, topk, dtype, &p) == FR_OK && p.block == block && any_height(M, H, F, E, topk, dtype, p);
+  return fr_moe_get_plan(M, H, F, E, topk, dtype, &p) == FR_OK && p.block == block ? any_height(M, H, F, E, topk, dtype, p) : kHeightsOfBlock;
 }
 }  // namespace fr
 

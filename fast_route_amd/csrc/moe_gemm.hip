@@ -377,7 +377,7 @@ extern "C" int fr_moe_down_combine(const void* act, const void* w2, const float*
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_down_combine: dtype %d not in {f16, bf16}", dtype);
   return down_impl(act, nullptr, w2, nullptr, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F,
                    E, topk, block, split_k, dtype, dtype, partial, out,
-                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 && plan_leaves_heights(M, H, F, E, topk, dtype, block)},
+                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 ? plan_leaves_heights(M, H, F, E, topk, dtype, block) : kHeightsOfBlock},
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine", w_tiled, nullptr);
 }
 
@@ -391,7 +391,7 @@ extern "C" int fr_moe_down_combine_fp8(const void* actq, const float* act_scale,
   FR_REQUIRE(act_scale && w2_scale, FR_E_NULL, "fr_moe_down_combine_fp8: null scale pointer");
   return down_impl(actq, act_scale, w2q, w2_scale, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M,
                    H, F, E, topk, block, split_k, FR_FP8_E4M3, out_dtype, partial, out,
-                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 && plan_leaves_heights(M, H, F, E, topk, FR_FP8_E4M3, block)},
+                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 ? plan_leaves_heights(M, H, F, E, topk, FR_FP8_E4M3, block) : kHeightsOfBlock},
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine_fp8", w_tiled, nullptr);
 }
 

@@ -118,6 +118,23 @@ __device__ __forceinline__ void expert_block_offsets(const GemmArgs& a, int nt, 
     if (a.expert_ids[b] < a.expert_ids[b - 1]) off[kMaxExperts + 1] = 1;
   __syncthreads();
 }
+// Of the two launches of launch_gemm_by_runs, the one with tall tiles: nearly every expert's run fits a tile of it and a good
+// part of them takes two blocks, as the host expects of near-uniform loads.  All lanes; off: expert_block_offsets of nt blocks.
+// (A run of three blocks or more is two tall tiles at least; one such run in eight is what the host's own rule admits.)
+__device__ __forceinline__ bool runs_fill_tall_tiles(const GemmArgs& a, const int* off, int nt, int lane) {
+  int runs = 0, doubled = 0;
+  for (int e0 = 0; e0 < a.num_experts; e0 += kWave) {
+    const int e = e0 + lane, len = e < a.num_experts ? off[e + 1] - off[e] : 0;
+    runs += __popcll(__ballot(len > 0));
+    doubled += __popcll(__ballot(len > 1));
+  }
+  return !off[kMaxExperts + 1] && 8 * (nt - runs - doubled) <= runs && 10 * doubled >= 3 * runs;
+}
+// What a fix-up launch that does not walk the tiles itself needs to know about a cut tile, one per workgroup (QuadPlan,
+// launch_gemm_by_runs).  Heights in units of 32 rows.
+struct TailCut {
+  int row0, units, f, expert, slices, rest, buffers, buffer_rows;  // slices 0: tile is not cut
+};
 __device__ __forceinline__ void tile_coords(const GemmArgs& a, const int* off, int lin, int& pid_t, int& pid_f,
                                             int& expert) {
   const int F = a.num_f_tiles;
@@ -233,11 +250,26 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   const int k_all = min(a.k_per_split, a.K - k0) / BK;  // K tiles of a whole unit, >= S + 2 (checked by the launcher)
   const XcdSchedule xs = xcd_schedule(total, nper, xcd, k_all, a.tail_ws != nullptr, schedule_by_rounds(nt, a.num_experts), nper);
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
-  if (n_units == 0) return;
+  constexpr bool BY_RUNS = (BT == 128 || BT == 160) && EPI != EPI_DOWN;
+  const bool by_runs = BY_RUNS && a.by_runs != 0;
+  if (n_units == 0 && !by_runs) return;
   __shared__ int expert_off[kWalkTable];
   expert_block_offsets(a, nt, expert_off, threadIdx.x, C::NT);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (by_runs) {
+    if (runs_fill_tall_tiles(a, expert_off, nt, lane)) return;
+    if (a.tail_desc && tid == 0) {  // the common fix-up launch: tile `loc` of the XCD's last round, if that is cut
+      TailCut c = {};
+      if (xs.slices > 1 && loc < xs.rest) {
+        int t, f, e;
+        tile_coords(a, expert_off, xs.tail_base + loc, t, f, e);
+        c = TailCut{t * BT, BT / 32, f, e, xs.slices, xs.rest, nper, BT};
+      }
+      reinterpret_cast<TailCut*>(a.tail_desc)[xcd * nper + loc] = c;
+    }
+    if (n_units == 0) return;
+  }
   const int wt = wave / C::WF, wf = wave % C::WF;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const bool issuer = wave_u < NW / IW;
@@ -799,13 +831,15 @@ int launch_gemm_persistent(const GemmArgs& a_in, int splits, hipStream_t st) {
   if (grid < 8) grid = 8;
   if (tail) {
     if (grid > kTailUnits) grid = kTailUnits;  // one slice buffer per workgroup
+  } else if (a.by_runs) {
+    if (grid > kTailUnits) grid = kTailUnits;
   } else if (grid > (worst + 7) / 8 * 8) {
     grid = (worst + 7) / 8 * 8;
   }
   hipLaunchKernelGGL((moe_gemm_persistent_kernel<T, C, EPI>), dim3(static_cast<unsigned>(grid), splits), dim3(C::NT),
                      C::LDS_BYTES, st, a FR_PROF_ARG);
   int lrc = check_launch("moe_gemm_persistent_kernel");
-  if (lrc != FR_OK || !tail) return lrc;
+  if (lrc != FR_OK || !tail || a.by_runs) return lrc;
   if constexpr (kFixable) {
     const int nper = static_cast<int>(grid / 8);
     if (nper >= 2) {

@@ -79,16 +79,13 @@ constexpr int kQuadRing = 2 * (kUnitRows * kMaxUnits + 256) * 128;
 // the layers' scratch has room for 32 of these too, a staged caller's (fr_moe_plan.tail_bytes) for 28.  Half a round of 288-row tiles
 // takes 32 for two slices each: H = 4096, F = 14336, 8 experts, one tile per expert and feature tile (gate/up: 3 1/2 rounds), layer
 // with 28 / 32 buffers 1031 tokens 780 / 769 us, 950 771 / 767; H = 6144, 1031 tokens 1320 / 1311.
-// What the fix-up launch needs to know about a cut tile is left next to them (QuadCut), in the scratch itself where the
+// What the fix-up launch needs to know about a cut tile is left next to them (TailCut), in the scratch itself where the
 // caller has no other place for it: then there are 31 buffers of 256 rows.  (Working it out again in the fix-up launch instead
 // costs staged calls 8 to 12 us: down projection, 8 experts, 1300 tokens 302 / 314, 2048 381 / 393.)
 constexpr int kQuadTallBuffers = 28;
 __device__ __forceinline__ int quad_buffer_rows(int tallest) { return tallest > 8 ? kUnitRows * kMaxUnits : 256; }
 __device__ __forceinline__ int quad_buffers(const GemmArgs& a, int tallest) { return tallest > 8 ? a.tall_buffers : a.tail_buffers; }
-struct QuadCut {
-  int row0, units, f, expert, slices, rest, buffers, buffer_rows;  // slices 0: tile is not cut
-};
-static_assert(sizeof(QuadCut) * kTailUnits <= kTailDescBytes, "a tile per workgroup");
+static_assert(sizeof(TailCut) * kTailUnits <= kTailDescBytes, "a tile per workgroup");
 static_assert(static_cast<int64_t>(kTailUnits) * kUnitRows * kMaxUnits * 256 * 4 == kTallTailBytes, "32 buffers per XCD in the layers' scratch");
 static_assert(8 * kQuadTallBuffers * kUnitRows * kMaxUnits * 256 * 4 + kTailDescBytes <= kTailUnits * 256 * 256 * 4 &&
                   8 * 31 * 256 * 256 * 4 + kTailDescBytes <= kTailUnits * 256 * 256 * 4, "fits the scratch");
@@ -113,12 +110,14 @@ struct QuadWalk {
 // 10.2, of which 3 to 4 are the first tiles' own loads; 15.5 - 16.7 and 11.7 - 12.6 when a wavefront went through its experts' last blocks
 // and all limits, the cut tile was worked out apart and the first weights waited for the sorted ids.  Layer H = 2048, 64 experts,
 // top-6, 8192 tokens 883 -> 875 us, 6200 703 -> 696; H = 4096, 1031 tokens 773 -> 770; fp8 650 387 -> 384.
-__device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int block, int nt, int tid, int nper, int k_tiles) {
+// false: the other launch of launch_gemm_by_runs works on these runs
+__device__ __forceinline__ bool quad_walk(const GemmArgs& a, QuadWalk& w, int block, int nt, int tid, int nper, int k_tiles) {
   expert_block_offsets(a, nt, w.off, tid, 256);
+  if (a.by_runs && !runs_fill_tall_tiles(a, w.off, nt, tid & 63)) return false;
   if (w.off[kMaxExperts + 1]) {
     if (tid == 0) w.tallest = block / kUnitRows;
     __syncthreads();
-    return;
+    return true;
   }
   const int E = a.num_experts, lane = tid & 63, wave = tid >> 6, groups = block / kUnitRows;
   for (int e = tid; e < E; e += 256) w.units[e] = max(w.off[e + 1] - w.off[e] - 1, 0) * groups;
@@ -218,6 +217,7 @@ __device__ __forceinline__ void quad_walk(const GemmArgs& a, QuadWalk& w, int bl
     if (lane == 0) w.tallest = w.high[best];
   }
   __syncthreads();
+  return true;
 }
 
 // A work unit: an output tile, or a K slice of one.
@@ -467,6 +467,7 @@ struct QuadPlan {
   XcdSchedule xs;
   int tallest;
   bool even_heights;
+  bool works;  // see quad_walk
 };
 template <typename T>
 __device__ __forceinline__ QuadPlan quad_plan(const GemmArgs& a, QuadWalk& walk, int block, int xcd, int nper, int tid) {
@@ -479,8 +480,10 @@ __device__ __forceinline__ QuadPlan quad_plan(const GemmArgs& a, QuadWalk& walk,
   p.even_heights = sizeof(T) == 1 || k_tiles <= 32;
   int tiles = 0;
   p.tallest = 0;
+  p.works = true;
   if (nt > 0) {
-    quad_walk(a, walk, block, nt, tid, nper, k_tiles);
+    p.works = quad_walk(a, walk, block, nt, tid, nper, k_tiles);
+    if (!p.works) return p;
     tiles = __builtin_amdgcn_readfirstlane(walk.off[kMaxExperts + 1] ? nt : walk.tiles[a.num_experts]);
     p.tallest = __builtin_amdgcn_readfirstlane(walk.tallest);
   }
@@ -513,11 +516,12 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
   const int xcd = blockIdx.x & 7, nper = gridDim.x >> 3, loc = blockIdx.x >> 3;
   const int k_all = a.K / BK;
   const QuadPlan plan = quad_plan<T>(a, walk, block, xcd, nper, tid);
+  if (!plan.works) return;
   const XcdSchedule& xs = plan.xs;
   // what the fix-up launch asks for: tile `loc` of the XCD's last round, if that is cut (then it is this workgroup's last unit)
-  QuadCut* const cut_at = a.tail_ws != nullptr ? reinterpret_cast<QuadCut*>(a.tail_desc) + (xcd * nper + loc) : nullptr;
+  TailCut* const cut_at = a.tail_desc != nullptr ? reinterpret_cast<TailCut*>(a.tail_desc) + (xcd * nper + loc) : nullptr;
   const bool cut = xs.slices > 1 && loc < xs.rest;
-  if (cut_at && !cut && tid == 0) *cut_at = QuadCut{};
+  if (cut_at && !cut && tid == 0) *cut_at = TailCut{};
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
   if (n_units == 0) return;
 
@@ -550,7 +554,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     quad_tile_at(a, walk, block, plan.even_heights, lin, k_all, u);
     unit_table[(j0 / kUnitTable) & 1][lane] = u;
     if (cut_at && cut && tid == n_units - 1 - j0)
-      *cut_at = QuadCut{u.row0, u.units, u.f, u.expert, xs.slices, xs.rest, quad_buffers(a, plan.tallest), quad_buffer_rows(plan.tallest)};
+      *cut_at = TailCut{u.row0, u.units, u.f, u.expert, xs.slices, xs.rest, quad_buffers(a, plan.tallest), quad_buffer_rows(plan.tallest)};
   };
   auto unit_at = [&](int j) {
     const QuadUnit& s = unit_table[(j / kUnitTable) & 1][j % kUnitTable];
@@ -929,7 +933,7 @@ __global__ __launch_bounds__(256) void quad_fixup_kernel(const GemmArgs a, int n
   constexpr int BF = QuadCfg<T, kMaxUnits>::BF;
   const int half = nper / 2;
   const int xcd = blockIdx.x / (half * kMaxUnits), t = (blockIdx.x / kMaxUnits) % half, rb = blockIdx.x % kMaxUnits;
-  const QuadCut c = reinterpret_cast<const QuadCut*>(a.tail_desc)[xcd * nper + t];
+  const TailCut c = reinterpret_cast<const TailCut*>(a.tail_desc)[xcd * nper + t];
   if (rb >= c.units || c.slices < 2) return;
   const int64_t buffer = static_cast<int64_t>(c.buffer_rows) * BF;
   const float* first = a.tail_ws + (xcd * c.buffers + t) * buffer;
@@ -972,6 +976,17 @@ inline void quad_divisor(int d, unsigned* mul, int* shift) {
   *shift = l > 0 ? l - 1 : 0;
 }
 
+// The list of cut tiles where the caller has no place for it but the scratch
+inline int* tail_desc_in(float* tail_ws) { return reinterpret_cast<int*>(tail_ws + kTailUnits * 256 * 256) - kTailDescBytes / 4; }
+
+// nper: workgroups per XCD of the GEMM launch
+template <typename T, int EPI>
+int launch_quad_fixup(const GemmArgs& a, int nper, hipStream_t st) {
+  if (nper < 2) return FR_OK;
+  hipLaunchKernelGGL((quad_fixup_kernel<T, EPI>), dim3(8 * (nper / 2) * kMaxUnits), dim3(256), 0, st, a, nper);
+  return check_launch("quad_fixup_kernel");
+}
+
 // Launches the one-wavefront-per-SIMD kernel on routing arrays of `block` rows (a multiple of 32, at most 256; num_t_blocks
 // and num_f_tiles filled for `block` rows and 256 features) for a single K split with at least kQuadMinTiles K tiles per work
 // unit.  Returns 1 when the shape is not one it takes (nothing launched: the caller takes another kernel).
@@ -1012,24 +1027,45 @@ int launch_gemm_quad(const GemmArgs& a_in, int block, int splits, hipStream_t st
   // at 10 rounds, 1442 / 1437 at 12.
   const int64_t max_rounds = a.K / BK >= 112 ? 16 : 8;
   const bool tail = a.tail_ws && a.K / BK >= kTailMinTiles && a.N % COLS == 0 && worst * block < max_rounds * resident * 256;
-  if (!tail) a.tail_ws = nullptr;
   a.tail_buffers = 32;
   a.tall_buffers = a.tail_tall ? 32 : kQuadTallBuffers;
-  if (tail && !a.tail_desc) {
-    a.tail_desc = reinterpret_cast<int*>(a.tail_ws + kTailUnits * 256 * 256) - kTailDescBytes / 4;
-    a.tail_buffers = 31;
-  }
+  if (a.tail_ws && !a.tail_desc) a.tail_desc = tail_desc_in(a.tail_ws);
+  if (a.tail_ws && a.tail_desc == tail_desc_in(a.tail_ws)) a.tail_buffers = 31;
+  if (!tail) a.tail_ws = nullptr;
+  if (!tail && !a.by_runs) a.tail_desc = nullptr;
   int64_t grid = resident;
-  if (grid > kTailUnits && tail) grid = kTailUnits;
+  if (grid > kTailUnits && (tail || a.by_runs)) grid = kTailUnits;
   hipLaunchKernelGGL((moe_gemm_quad_kernel<T, EPI>), dim3(static_cast<unsigned>(grid)), dim3(256), kQuadRing + kQuadSink, st, a, block);
   int lrc = check_launch("moe_gemm_quad_kernel");
-  if (lrc != FR_OK || !tail) return lrc;
-  const int nper = static_cast<int>(grid / 8);
-  if (nper >= 2) {
-    hipLaunchKernelGGL((quad_fixup_kernel<T, EPI>), dim3(8 * (nper / 2) * kMaxUnits), dim3(256), 0, st, a, nper);
-    lrc = check_launch("quad_fixup_kernel");
-  }
-  return lrc;
+  if (lrc != FR_OK || !tail || a.by_runs) return lrc;
+  return launch_quad_fixup<T, EPI>(a, static_cast<int>(grid / 8), st);
+}
+
+// A GEMM whose tile form only the experts' runs can decide: tall tiles and the tiles C of the routing block are both launched, and
+// the device has one of them return at once (runs_fill_tall_tiles).  The one that works lists the tiles it cuts, which one
+// fix-up launch sums.  a: filled for `block` rows and 256 features.  Returns 1 as launch_gemm_quad does.
+// Near-uniform loads, which is all the host can price, are multiplied up to a fifth faster by tall tiles, skewed ones up to a
+// quarter slower: an expert with several tiles leaves the others' short ones to wait for its rounds.
+template <typename T, typename C, int EPI>
+int launch_gemm_by_runs(const GemmArgs& a_in, int block, hipStream_t st) {
+  GemmArgs a = a_in;
+  int tall_grid = 0, block_grid = 0;
+  int rc = quad_grid<T, EPI>(&tall_grid);
+  if (rc == FR_OK) rc = persistent_grid<T, C, EPI>(&block_grid);
+  if (rc != FR_OK) return rc;
+  if (tall_grid != block_grid) return 1;  // the list of cut tiles is one per workgroup
+  if (tunables().no_tail_split) a.tail_ws = nullptr;
+  if (!a.tail_ws) a.tail_desc = nullptr;
+  else if (!a.tail_desc) a.tail_desc = tail_desc_in(a.tail_ws);
+  a.by_runs = 1;
+  rc = launch_gemm_quad<T, EPI>(a, block, 1, st);
+  if (rc != FR_OK) return rc;
+  GemmArgs b = a;
+  b.by_runs = 2;
+  if (sizeof(T) == 1 && EPI == EPI_SILU) b.tail_ws = nullptr;  // fp8's gate/up GEMM does not cut these tiles
+  rc = launch_gemm_persistent<T, C, EPI>(b, 1, st);
+  if (rc != FR_OK || !a.tail_desc) return rc;
+  return launch_quad_fixup<T, EPI>(a, (tall_grid < kTailUnits ? tall_grid : kTailUnits) / 8, st);
 }
 
 }  // namespace fr

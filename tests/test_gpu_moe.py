@@ -964,6 +964,58 @@ def test_one_tile_per_expert_where_the_plan_has_two(native, kernels_of, dtype, M
     _assert_close(out, oracle.moe_experts(x, w1, w2, wts, ids), dtype, "one tile per expert")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, "fp8"])
+@pytest.mark.parametrize("counts,tall", [((162, 162, 161, 161, 161, 161, 161, 161), True), ((330, 165, 165, 165, 165, 100, 100, 100), True),
+                                         ((330, 330, 165, 165, 100, 100, 50, 50), False), ((170, 170, 158, 158, 158, 158, 159, 159), False),
+                                         ((645, 400, 0, 200, 44, 1, 0, 0), False)])
+def test_skewed_runs_keep_the_plans_tiles(native, dtype, counts, tall):
+    """Where near-uniform loads would make every expert's run one tall tile, the experts' runs decide: tall tiles with one run of
+    three blocks among eight experts, the plan's tiles (bit for bit those of no_quad) with two, with few runs of two blocks and with a
+    skewed load; without cut tiles as well."""
+    import fast_route_amd as fr
+    from fast_route_amd import _native as N, fused_experts, fused_moe_fp8, prepare_weights_fp8
+    from fast_route_amd.layers.fused_moe import plan
+    M, H, Fd, E, k = 645, 4096, 3328, 8, 2
+    _say(f"tiles by runs {counts} {dtype}")
+    pairs = np.repeat(np.arange(E), counts).reshape(k, M).T  # an expert's pairs are consecutive: no token has one twice
+    pairs = torch.from_numpy(np.random.default_rng(5).permutation(pairs)).int().contiguous()
+    two_byte = torch.bfloat16 if dtype == "fp8" else dtype
+    assert plan(M, H, Fd, E, k, two_byte, N.FR_FP8_E4M3 if dtype == "fp8" else None).block == 160
+    g = torch.Generator(device="cuda").manual_seed(len(set(counts)))
+    x = torch.randn(M, H, generator=g, device="cuda").to(two_byte)
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g, device="cuda") * 0.02).to(two_byte)
+    w2 = (torch.randn(E, H, Fd, generator=g, device="cuda") * 0.02).to(two_byte)
+    if dtype == "fp8":
+        logits = torch.full((M, E), -8.0)
+        logits.scatter_(1, pairs.long(), 2.0)
+        args = [x, *prepare_weights_fp8(w1, w2), logits.cuda()]
+        run = lambda: fused_moe_fp8(*args, k, True)
+        ref = oracle.fused_moe_fp8(x.cpu(), w1.cpu(), w2.cpu(), logits, k, True)[0]
+    else:
+        wts = torch.full((M, k), 0.5)
+        args = [x, w1, w2, wts.cuda(), pairs.cuda()]
+        run = lambda: fused_experts(*args)
+        ref = oracle.moe_experts(x.cpu(), w1.cpu(), w2.cpu(), wts, pairs)
+    out, again = run(), run()
+    try:
+        with fr.tunables(no_quad=True):
+            tiles = run()
+        with fr.tunables(no_tail_split=True):
+            whole = run()
+            with fr.tunables(no_tail_split=True, no_quad=True):
+                whole_tiles = run()
+    finally:
+        fr.reset_tunables()
+    assert torch.equal(out, again)
+    assert torch.equal(out, tiles) != tall and torch.equal(whole, whole_tiles) != tall
+    for o in (out, tiles, whole):
+        if dtype == "fp8":
+            o = o.float().cpu()
+            assert (o - ref).norm() / ref.norm() <= 1e-2 and (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+        else:
+            _assert_close(o, ref, dtype, f"{counts}")
+
+
 @pytest.mark.parametrize("M,H,Fd,E,k,quad", [(1350, 4096, 2048, 8, 2, 2), (1430, 4096, 2048, 8, 2, 2), (2300, 2048, 2048, 8, 2, 2),
                                               (1200, 4096, 2048, 8, 2, 0), (2100, 2048, 2048, 8, 2, 0), (2850, 1024, 3584, 8, 2, 0),
                                               (350, 4096, 2048, 1, 1, 0), (1055, 2048, 5632, 4, 2, 0)])
