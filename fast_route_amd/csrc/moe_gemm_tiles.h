@@ -167,8 +167,10 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       if constexpr (sizeof(T) == 2) {
         // Rows of up to 4 KB: half the features in 256-byte pieces on three slots, two workgroups per CU, whose start-up per tile
         // overlaps (T32L has one).  H = 2048, 64 experts, top-6, layer in parts of the time on T32L: 20 tokens 0.96, 32 0.97, 48 0.96, 80 0.977
-        // (persistent 1.04, 1.005, 0.97, 0.95; on two slots 1.025, 0.98, 0.99, 1.00); longer rows 1.035 to 1.05.
-        if (EPI == EPI_SILU && a.K * static_cast<int>(sizeof(T)) <= kShortRow && a.K % (TL::T32N::BKB / static_cast<int>(sizeof(T))) == 0) {
+        // (persistent 1.04, 1.005, 0.97, 0.95; on two slots 1.025, 0.98, 0.99, 1.00); longer rows 1.035 to 1.05.  Where T32L does not
+        // fit either, T32 stays: gate/up in parts of its time H = 640, F = 2560, 8 experts 1.08, Zipf-skewed 1.13 to 1.25, H = 1152
+        // 1.07 to 1.25, H = 1408, 16 experts 1.11 to 1.18.
+        if (EPI == EPI_SILU && a.K * static_cast<int>(sizeof(T)) <= kShortRow && a.K % (TL::T32L::BKB / static_cast<int>(sizeof(T))) == 0) {
           fill(32, TL::T32N::BF, TL::T32N::BKB);
           return launch_gemm<T, typename TL::T32N, EPI>(a, splits, st);
         }

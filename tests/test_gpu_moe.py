@@ -7,6 +7,7 @@ evaluated on the same rounded operands we require
     max|out - ref| <= 2**-6 * max|ref|      (a few output ulps at the largest magnitude)
     ||out - ref||_F <= 6e-3 * ||ref||_F     (bf16; 1.5e-3 for fp16)
 """
+import re
 import sys
 import tempfile
 
@@ -503,6 +504,25 @@ def test_k_starts_of_tiles_alone_on_their_weights(native, block, H, Fd, split):
         torch.cuda.synchronize()
         assert torch.equal(out, again)
         _assert_close(out, ref, dtype, f"{dtype}")
+
+
+@pytest.mark.parametrize("H,form", [(640, "32, 128, 128"), (1152, "32, 128, 128"), (1024, "32, 64, 256"), (2048, "32, 64, 256"), (2304, "32, 128, 512"), (2176, "32, 128, 128")])
+def test_gate_up_forms_of_32_rows(native, kernels_of, H, form):
+    """Weight rows of up to 4 KB take the narrow 32-row tile only where whole 512-byte pieces make them up."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_moe
+    M, Fd, E, k = 100, 1024, 8, 2
+    _say(f"32-row gate/up H={H}")
+    x, logits, w1, w2 = _inputs(M, H, Fd, E, 7 + H, torch.bfloat16)
+    try:
+        with fr.tunables(block=32):
+            out, names = kernels_of(lambda: fused_moe(x.cuda(), w1.cuda(), w2.cuda(), logits.cuda(), k, True))
+    finally:
+        fr.reset_tunables()
+    gate_up = [n for n in names if "moe_gemm" in n and re.search(r"Li1EEEv|, 1>\(", n)]  # EPI_SILU
+    mangled = "CfgILi" + form.replace(", ", "ELi") + "E"
+    assert len(gate_up) == 1 and (mangled in gate_up[0] or "Cfg<" + form + "," in gate_up[0]), names
+    _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), torch.bfloat16, "layer")
 
 
 def test_stable_and_vllm_route_layers(native):
