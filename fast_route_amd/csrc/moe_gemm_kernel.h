@@ -560,13 +560,15 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_kernel(const GemmArgs
   const int k0 = split * a.k_per_split;
   const int k_tiles = min(a.k_per_split, a.K - k0) / BK;
   // K tile the walk starts at, round the end of K (why: SPREAD_K in moe_gemm_persistent.h).  32 rows: every tile at a place of
-  // its own; 16 rows in 512-byte pieces, rows of up to 4 KB: neighbours in step, with as many places as there are K tiles; the 256-row tile of fp8's gate/up GEMM as
+  // its own, in the down projection where weight rows are a power of two long; 16 rows in 512-byte pieces, rows of up to 4 KB: neighbours in step, with as many places as there are K tiles; the 256-row tile of fp8's gate/up GEMM as
   // the kernels it stands in for; the others gain nothing (16 rows in 256-byte pieces) or lose 1 to 2 % (64 rows).  Layer in parts of
   // the time from column 0: 32 rows, gate/up H = 2048, 64 experts, top-6, 100 tokens 0.98, fp8 80 tokens 0.975, fp16, 16 experts,
-  // F = 8192, 120 tokens 0.94, its down projection 0.91, H = 4096, F = 14336 60 / 90 tokens 1.00, down projection 0.98, but rows of 2 KB (H = 1024) 1.014; 16 rows, gate/up
+  // F = 8192, 120 tokens 0.94, but rows of 2 KB (H = 1024) 1.014; their down projection (three slots) 0.90, F = 8192 in four slices 0.89, H = F = 4096
+  // 0.885, H = 8192, F = 2048 0.975, other lengths F = 14336 1.004 to 1.016 (fp8 1.01), 3584 1.002, 2560 1.01, 1408 and 1536 1.00; 16 rows, gate/up
   // H = 2048 8 / 32 / 64 tokens 0.96 / 0.987 / 0.987, H = 4096 1.00 to 1.006 (every tile at its own place 0.97 to 0.99 and 1.01).
+  constexpr bool SPREAD = BT == 32 || (BT == 16 && C::BKB == 512) || (BT == 256 && E::SCALED);
   int k_first = 0;
-  if constexpr (BT == 32) k_first = k_tiles * C::BKB > 2048 ? __builtin_amdgcn_readfirstlane(spread_k_start(0, expert * a.num_f_tiles + pid_f, k_tiles)) : 0;
+  if constexpr (BT == 32) k_first = k_tiles * C::BKB > 2048 && (EPI == EPI_SILU || (a.K & (a.K - 1)) == 0) ? __builtin_amdgcn_readfirstlane(spread_k_start(0, expert * a.num_f_tiles + pid_f, k_tiles)) : 0;
   else if constexpr (BT == 16 && C::BKB == 512) k_first = k_tiles * C::BKB <= 4096 ? __builtin_amdgcn_readfirstlane((pid_f & 31) * k_tiles >> 5) : 0;
   else if constexpr (BT == 256 && E::SCALED) {
     if (a.N % (EPI == EPI_SILU ? BF / 2 : BF) == 0 && (pid_t == 0 || a.expert_ids[pid_t - 1] != expert) && (pid_t == nt - 1 || a.expert_ids[pid_t + 1] != expert))
@@ -756,7 +758,7 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_kernel(const GemmArgs
     // first: in the prologue they depend only on the expert id, so they are in flight while the
     // sorted ids that the token-tile addresses need are still being fetched.  The IW virtual
     // wavefronts of one load index are adjacent.
-#define FR_KPOS(tile_) ((tile_) + k_first >= k_tiles ? (tile_) + k_first - k_tiles : (tile_) + k_first)
+#define FR_KPOS(tile_) (!SPREAD ? (tile_) : (tile_) + k_first >= k_tiles ? (tile_) + k_first - k_tiles : (tile_) + k_first)
 #define FR_ISSUE_ONE(tile_, slot_, q_)                                                                     \
   {                                                                                                        \
     const int vw_ = wave_u + ((q_) % IW) * (NW / IW);                                                      \

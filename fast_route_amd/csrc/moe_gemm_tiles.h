@@ -36,9 +36,9 @@ template <typename T> struct Tiles {  // bf16 / fp16
   typedef Cfg<160, 256, 128, 2, 4, 16, 1, 3, 0, 2> T160P;
   typedef Cfg<64, 256, 128, 2, 4, 32, 1, 3, 3> T64;    // 3-slot ring like the 128-row tile (5 % over the register-staged form)
   typedef Cfg<64, 128, 256, 2, 2, 32, 1, 3> T64U;      // gate/up: 256-byte row segments, 4 wavefronts (another 5 %)
-  // Two slots (40 KB: four workgroups per CU) instead of three (two): down projection, layer in parts of the time H = 2048, 64 experts, 32 tokens
-  // 0.99, H = 4096, F = 14336 60 0.988, fp16, 16 experts, F = 8192 100 0.985, H = 6144 60 0.98.
-  typedef Cfg<32, 128, 128, 1, 4, 16, 2, 2> T32;
+  typedef Cfg<32, 128, 128, 1, 4, 16, 2, 3> T32;
+  // Two slots (40 KB: four workgroups per CU) instead of three (two), for long K slices of rows a power of two long, see dispatch_block
+  typedef Cfg<32, 128, 128, 1, 4, 16, 2, 2> T32D;
   typedef Cfg<16, 64, 256, 1, 2, 16, 2, 3> T16;
   typedef Cfg<32, 128, 512, 1, 4, 16, 1, 2> T32L;
   typedef Cfg<16, 64, 512, 1, 2, 16, 2, 2> T16L;
@@ -180,6 +180,15 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
         return launch_gemm<T, typename TL::T32L, EPI>(a, splits, st);
       }
       fill(32, TL::T32::BF, TL::T32::BKB);
+      if constexpr (sizeof(T) == 2 && EPI != EPI_SILU) {
+        // The layer's down projection with K slices of 16 KB or more, whose tiles start K at spread places (SPREAD in moe_gemm_kernel.h): half
+        // the bytes in flight per workgroup, twice the workgroups.  Layer in parts of the time on three slots, near-uniform / Zipf-skewed:
+        // fp16, 16 experts, F = 8192 72 to 160 tokens 0.985 / 0.98, H = 6144, F = 16384, 8 experts 36 to 100 0.975 / 0.965.  Shorter
+        // slices leave a CU too few bytes in flight or the workgroups uneven shares: H = 768 1.08, H = 512 1.07, 64 experts,
+        // F = 1408 1.01 / 0.98 to 1.02, 16 experts, F = 1408, 200 tokens 0.99 / 1.02, F = 8192 in four slices 1.03 / 1.0.
+        if (a.long_k && a.k_per_split * static_cast<int>(sizeof(T)) >= 16384 && (a.K & (a.K - 1)) == 0)
+          return launch_gemm<T, typename TL::T32D, EPI>(a, splits, st);
+      }
       return launch_gemm<T, typename TL::T32, EPI>(a, splits, st);
     case 16:
       // Plain or persistent.  A plain launch has two workgroups per CU that come and go: every tile pays its start-up
@@ -245,6 +254,7 @@ int prepare_tiles() {
       if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64W, EPI>(a, 1, nullptr);
     } else {
       if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64N, EPI>(a, 1, nullptr);
+      if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32D, EPI>(a, 1, nullptr);
     }
   }
   if constexpr (EPI == EPI_SILU) {

@@ -476,7 +476,7 @@ def test_rows_of_whole_and_partial_tiles(native, block, N):
 
 
 @pytest.mark.parametrize("split", [1, 3])
-@pytest.mark.parametrize("H,Fd", [(384, 1152), (640, 1664), (2048, 1152), (2432, 2176)])
+@pytest.mark.parametrize("H,Fd", [(384, 1152), (640, 1664), (2048, 1152), (2432, 2176), (384, 2048)])
 @pytest.mark.parametrize("block", [16, 32, 64, 128, 160])
 def test_k_starts_of_tiles_alone_on_their_weights(native, block, H, Fd, split):
     """A tile that is alone on its weight tile (16 and 32 rows: any tile) walks its K tiles from a place of its own, round the end:
@@ -523,6 +523,25 @@ def test_gate_up_forms_of_32_rows(native, kernels_of, H, form):
     mangled = "CfgILi" + form.replace(", ", "ELi") + "E"
     assert len(gate_up) == 1 and (mangled in gate_up[0] or "Cfg<" + form + "," in gate_up[0]), names
     _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), torch.bfloat16, "layer")
+
+
+@pytest.mark.parametrize("Fd,split,slots", [(8192, 1, 2), (8192, 2, 3), (8064, 1, 3), (8320, 1, 3), (16384, 2, 2), (1408, 1, 3), (4096, 1, 3)])
+def test_ring_slots_of_the_32_row_down_projection(native, kernels_of, Fd, split, slots):
+    """Two ring slots only for K slices of 16 KB or more of weight rows a power of two long, three otherwise."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_moe
+    M, H, E, k = 100, 384, 8, 2
+    _say(f"32-row down projection F={Fd} split={split}")
+    for dtype in (torch.bfloat16, torch.float16):
+        x, logits, w1, w2 = _inputs(M, H, Fd, E, 9 + Fd, dtype)
+        try:
+            with fr.tunables(block=32, split_k=split):
+                out, names = kernels_of(lambda: fused_moe(x.cuda(), w1.cuda(), w2.cuda(), logits.cuda(), k, True))
+        finally:
+            fr.reset_tunables()
+        down = [n for n in names if "moe_gemm" in n and not re.search(r"Li1EEEv|, 1>\(", n)]
+        assert len(down) == 1 and re.search(r"ILi32ELi128ELi128ELi1ELi4ELi16ELi2ELi%dE|<32, 128, 128, 1, 4, 16, 2, %d," % (slots, slots), down[0]), names
+        _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, f"{dtype}")
 
 
 def test_stable_and_vllm_route_layers(native):
