@@ -299,26 +299,55 @@ fr_moe_plan plan_for(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype
 }
 
 // The layers route for another block than the plan's where that has been found faster (2-byte operands; a block set by hand
-// stands).  Never for fewer K slices that are summed from fp32 rows: a single slice's rows are rounded.
-// Layer in parts of the time with the plan's block:
-//   Many narrow experts with skewed loads (H = 2048, F = 1408, 64 experts, top-6, Zipf): the heavy experts take several small tiles.  (Up
-//   to 128 experts and F = 2816: the routing blocks' padding is E x block rows of F activated values.)
-//     plan 16: 32 rows 12 tokens (1.1 pairs per expert) 0.98, 18 0.96, 32 0.92, 40 0.87, 48 0.95, 72 0.89, 80 0.87, but 8 and 10 (0.9) 1.03;
-//     64 rows 12 to 20 tokens 0.93 to 0.96, but 22 to 40 1.05 to 1.12: where the active experts' tiles are two rounds, which depends
-//     on the routing;
-//     plan 32: 64 rows instead of 32 90 (8.4) 1.00, 110 0.92, 180 0.86, 230 0.80, 290 (27.2) 0.74; 128 rows 260 1.09, 290 1.11 of
-//     64 rows, 300 (28.1) 1.00, 310 to 335 0.92 to 0.98
-//   H = 1024, F = 3584, 8 experts: the plan's 64-row range begins at H = 4096, and the 128-row tile has 16 short K tiles there.
-//     16 rows 33 to 48 tokens (8 to 12 pairs) 0.91 (64 rows 0.97 of that, 0.98 to 1.07 below 33), 56 (14) 0.96; 64 rows 60 0.88, 90 0.86, 130
-//     (32.5) 0.70, 200 0.73, 300 0.80, 460 (115) 0.80, 490 0.97, 500 (125) 0.89, 525 1.01, 550 1.03, 600 1.08
+// stands).  Never for fewer K slices that are summed from fp32 rows: a single slice's rows are rounded.  Only sizes are known here, so every
+// range holds for near-uniform as well as Zipf-skewed loads.  Layer in parts of the time with the plan's block, near-uniform / Zipf (two
+// routings):
+//   Many narrow experts (shapes: H, F, experts, top-k).  The heavy experts of a skewed load take several small tiles.  Up to 128 experts
+//   and F = 2816: the routing blocks' padding is E x block rows of F activated values.
+//     plan 16, 32 rows from 2 pairs per expert, where gate/up rows are short enough for the narrow 32-row tile (moe_gemm_tiles.h):
+//       2048, 1408, 64, 6   2 pairs 1.00 / 0.98, 3 0.99 / 0.96, 6 1.01 / 0.88, 8 1.01 / 0.905, but 1.1 1.01 / 1.02
+//       2048, 768, 128, 8   2 1.01 / 0.97, 4 1.00 / 0.96, 8 1.00 / 0.85;   2048, 1024, 60, 4   2 0.99 / 0.98, 3 1.03 / 1.01, 5 1.02 / 0.93, 8 0.995 / 0.90
+//       2048, 1408, 32, 2   3 1.00 / 0.95, 6 1.00 / 0.98;   2048, 2048, 64, 6   3 0.97 / 0.88, 8 0.96 / 0.88
+//       2048, 2816, 64, 6   3 1.06 / 0.965;   2560, 1536, 64, 8   3 1.03 / 0.98;   3072, 1536, 32, 4   2 1.01 / 1.055, 6 1.01 / 1.05
+//     64 rows instead of 32 from 12 pairs:
+//       2048, 1408, 64, 6   12 1.015 / 0.94, 16 1.01 / 0.87, 20 1.00 / 0.83, 27 0.89 / 0.805;   2048, 768, 128, 8   12 1.01 / 0.89, 20 1.00 / 0.82
+//       2048, 1024, 60, 4   8.5 0.95 / 1.07, 12 0.95 / 0.99, 20 0.95 / 0.84;   2048, 1408, 32, 2   12 1.02 / 0.875, 16 1.02 / 0.985, 24 0.92 / 0.86
+//       3072, 1536, 32, 4   8.5 1.02 / 1.07, 12 1.015 / 1.015, 16 0.995 / 0.89;   2560, 1536, 64, 8   12 1.02 / 0.93;   3072, 1024, 96, 4   12 1.00 / 0.84
+//       2048, 2816, 64, 6   12 1.02 / 0.875;   3072, 2816, 100, 8   12 1.00 / 0.88
+//       2048, 1024, 128, 8   12 0.98 / 0.91;   3584, 640, 64, 6   12 0.97 / 0.83
+//     but from 24 pairs where w2 has short rows, or rows of a power of two of 4 KB or more, whose 32-row tiles start K at spread places and 64-row
+//     ones do not:   2048, 512, 128, 8   12 1.08 / 1.01, 18 1.08 / 0.88, 26 0.97 / 0.81;   2048, 256, 64, 6   12 1.145 / 1.20, 26 1.00 / 0.99, 128 rows 28.5 1.08 / 1.07
+//       2048, 2048, 64, 6   12 1.12 / 0.96, 20 1.11 / 0.89, 24 1.04 / 0.81, 27 0.98 / 0.85
+//     128 rows from 28 pairs (64 rows): 2048, 1408, 64, 6 28.5 0.89 / 0.78 (0.83 / 0.83); 3072, 1024, 96, 4 0.90 / 0.62 (0.87 / 0.71)
+//   H = 640 to 1024, up to 16 experts: the plan's 64-row range begins at H = 4096, and the 128-row tile has up to 16 short K tiles there.
+//   t = gate/up tiles with one block per expert.
+//     plan 32, 64 rows where t is most of a round and leaves room for an expert's second block, H = 1024:
+//       F = 3584, 8 experts (t = 224) 8.5 0.915 / 0.91, 12 0.925 / 0.91, 20 0.90 / 0.94, 30 0.815 / 0.91;   F = 1536, 16 experts (192) 12 0.905 / 0.91, 30 0.89 / 0.895
+//       F = 7168, 4 (224) 12 0.91 / 0.91, 30 0.84 / 0.82;   F = 14336, 2 (224) 12 0.98, 30 0.90;   F = 4096, 8 (256) 12 0.93 / 0.84, 20 0.92 / 1.07
+//       F = 2048, 8 (128) 12 1.05 / 0.95;   H = 768, F = 2048, 16 (256) 1.05 / 1.04;   H = 896, F = 5120, 6 (240) 1.12 / 1.125;   t = 22 to 80 1.2 to 1.3
+//     plan 32, 16 rows up to 10 pairs from a whole round on: F = 4096, 8 experts (256) 10 0.965 / 0.94, H = 768, F = 2048, 16 (256) 0.905 / 0.945, F = 3072, 16
+//       (384) 0.91 / 0.96, F = 14336, 8 (896) 0.91 / 0.95;   but F = 2048, 8 (128) 0.955 / 1.02, H = 768, F = 3584, 8 (224) 0.925 / 1.12
+//     plan 128, 64 rows up to 48 pairs: F = 3584, 8 40 0.74 / 0.97, F = 14336, 8 0.86 / 0.92, H = 768, F = 3072, 16 0.79 / 0.76, F = 1024, 16 (128; two K slices)
+//       0.89 / 0.92;   but F = 1536, 16 (192; three K slices) 0.89 / 1.04, 48 0.89 / 1.12
+//     up to 90 pairs with t up to 224 and one K slice: F = 3584, 8 64 1.00 / 0.80, 80 0.96 / 0.765, F = 7168, 4 1.01 / 0.95, 0.89 / 0.76, F = 2048, 8 0.84 / 0.85, 0.74 / 0.77;
+//       but t = 256 F = 4096, 8 80 1.05 / 0.895, H = 768, F = 2048, 16 1.025 / 0.875;   F = 2048, 8 100 0.74 / 1.09
+//     up to 125 pairs with t up to 80: F = 4096, 2 0.62, F = 2816, 1 0.63, F = 1024, 8 0.90 / 0.91, H = 640, F = 2560, 4 0.74 / 0.74
 //   160 rows instead of 128 where an expert is likely to exceed 128 rows: a block more costs a round of tiles, the larger tile 1 %.
-//     16 experts, F = 8192, fp16: 880 tokens (110 pairs; one expert above 128) 0.90, 920 0.88, 800 (none) 0.99; H = 6144 460 (115) 0.95;
-//     H = 4096, F = 14336, 8 experts none above 128: 300 and 420 1.01.
+//     16 experts, F = 8192, fp16: 920 tokens (115 pairs) 0.895 / 1.005, 800 (100; no expert above 128) 0.99; H = 6144, F = 16384 460 0.87 / 1.045; H = 4096,
+//     F = 14336, 8 experts 460 0.955 / 1.005, none above 128: 300 and 420 1.01; 16 experts, F = 1536, top-4 460 0.86 / 0.955; 4 experts, F = 2048 230 0.985 / 1.045
 int layer_block(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, const fr_moe_plan& p) {
   if ((dtype != FR_F16 && dtype != FR_BF16) || g_tunables.block) return p.block;
   const double avg = static_cast<double>(M) * topk / E;
-  if (E >= 32 && E <= 128 && H >= 2048 && H < 4096 && F <= 2816 && p.block <= 32 && avg >= 1.05) return avg < 8.5 ? 32 : avg < 28 ? 64 : 128;
-  if (E <= 16 && H >= 640 && H <= 1024 && F >= 1024 && (p.block == 32 || p.block == 128) && avg < 126) return avg <= 12 ? 16 : 64;
+  if (E >= 32 && E <= 128 && H >= 2048 && H < 4096 && F <= 2816 && p.block <= 32) {
+    if (F >= 512 && avg >= 28) return 128;
+    if (F >= 512 && avg >= (F < 640 || (F > 1024 && (F & (F - 1)) == 0) ? 24 : 12)) return 64;
+    return avg >= 2 && H <= 2048 && F <= 2048 ? 32 : p.block;
+  }
+  if (E <= 16 && H >= 640 && H <= 1024 && F >= 1024) {
+    const int64_t t = E * ceil_div(F, 128);
+    if (p.block == 32) return H > 896 && t >= 192 && t <= 240 ? 64 : t >= 256 && avg <= 10 ? 16 : 32;
+    if (p.block == 128 && ((avg <= 48 && (p.split_k == 1 || t <= 128)) || (avg <= 90 && p.split_k == 1 && t <= 224) || (avg < 126 && t <= 80))) return 64;
+  }
   if (E <= 16 && H >= 4096 && F >= 1024 && p.block == 128 && avg < 128 && E * (expected_blocks(avg, E, 128) - 1.0) >= 0.15) return 160;
   return p.block;
 }

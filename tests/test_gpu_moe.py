@@ -912,15 +912,21 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
 
 
 @pytest.mark.parametrize("M,H,Fd,E,k,planned,rows", [
-    (8, 2048, 256, 32, 4, 16, 16), (9, 2048, 256, 32, 4, 16, 32), (67, 2048, 256, 32, 4, 32, 32), (68, 2048, 256, 32, 4, 32, 64), (223, 2048, 256, 32, 4, 32, 64),
-    (224, 2048, 256, 32, 4, 32, 128), (255, 2048, 256, 32, 4, 32, 128), (36, 1024, 2048, 8, 2, 32, 16), (48, 1024, 2048, 8, 2, 32, 16),
-    (49, 1024, 2048, 8, 2, 32, 64), (503, 1024, 2048, 8, 2, 128, 64), (504, 1024, 2048, 8, 2, 128, 128), (900, 4096, 1024, 16, 2, 128, 160)])
+    # many narrow experts: pairs per expert, w2 rows of other lengths and of a power of two, gate/up rows above 4 KB, wide experts
+    (15, 2048, 640, 32, 4, 16, 16), (16, 2048, 640, 32, 4, 16, 32), (64, 2048, 640, 32, 4, 16, 32), (95, 2048, 640, 32, 4, 32, 32), (96, 2048, 640, 32, 4, 32, 64),
+    (223, 2048, 640, 32, 4, 32, 64), (224, 2048, 640, 32, 4, 32, 128), (255, 2048, 640, 32, 4, 32, 128), (191, 2048, 512, 32, 4, 32, 32), (192, 2048, 512, 32, 4, 32, 64),
+    (96, 2048, 1024, 32, 4, 32, 64), (191, 2048, 2048, 32, 4, 32, 32), (192, 2048, 2048, 32, 4, 32, 64), (16, 2048, 256, 32, 4, 16, 32), (230, 2048, 256, 32, 4, 32, 32),
+    (32, 2176, 640, 32, 4, 16, 16), (16, 2048, 2176, 32, 4, 16, 16),
+    # H of 640 to 1024: gate/up tiles with one block per expert, pairs per expert, K slices
+    (36, 1024, 3584, 8, 2, 32, 64), (361, 1024, 3584, 8, 2, 128, 128), (360, 1024, 3584, 8, 2, 128, 64), (40, 1024, 4096, 8, 2, 32, 16), (41, 1024, 4096, 8, 2, 32, 32),
+    (192, 1024, 4096, 8, 2, 128, 64), (193, 1024, 4096, 8, 2, 128, 128), (36, 1024, 2048, 8, 2, 32, 32), (125, 1024, 2048, 2, 2, 128, 64), (126, 1024, 2048, 2, 2, 128, 128),
+    (72, 1024, 1536, 16, 2, 32, 64), (300, 1024, 1536, 16, 2, 128, 128), (36, 896, 3584, 8, 2, 32, 32),
+    (900, 4096, 1024, 16, 2, 128, 160)])
 def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, Fd, E, k, planned, rows):
     """At the edges of the ranges where the layers take other tiles than the plan's block stands for: the plan stays, its workspace
     covers both, and results match the oracle."""
-    import re
     from fast_route_amd import fused_experts, fused_moe
-    from fast_route_amd.layers.fused_moe import plan
+    from fast_route_amd.layers.fused_moe import plan, prepare_weights
     dtype = torch.bfloat16
     _say(f"layer's own block M={M} H={H} F={Fd} E={E}")
     assert plan(M, H, Fd, E, k, dtype).block == planned
@@ -932,6 +938,8 @@ def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, 
     w, ids = oracle.gating_topk(logits, k, True)
     _assert_close(out, oracle.fused_moe(x, w1, w2, logits, k, True), dtype, "layer")
     _assert_close(fused_experts(*args, w.cuda(), ids.cuda()), oracle.moe_experts(x, w1, w2, w, ids), dtype, "experts")
+    t1, t2, flags = prepare_weights(*args[1:], which="both")
+    assert torch.equal(fused_moe(args[0], t1, t2, logits.cuda(), k, True, weights_prepared=flags), out)
 
 
 @pytest.mark.parametrize("M,E,k,launches", [(32, 64, 6, 1), (33, 64, 6, 2), (31, 33, 4, 1), (33, 33, 4, 2), (64, 32, 4, 1), (65, 32, 4, 2),
