@@ -141,7 +141,10 @@ int fr_moe_prepare_weights(const void* w, int dtype, int64_t E, int64_t rows, in
  * block than the plan's where that is faster (layer_block in fused_moe.hip);
  * workspace_bytes covers both.  They run in a workspace that holds no more than
  * the plan's own block with 64 MiB of tail scratch, too, as earlier versions of
- * this library asked for, on the plan's block and with fewer tail buffers.      */
+ * this library asked for, on the plan's block and with fewer tail buffers: there
+ * the kernels, and with them the order of fp32 sums, depend on the bytes given.
+ * Where fr_fused_moe_noalloc takes the sizes, it runs the kernels that
+ * fr_fused_moe runs in workspace_bytes.                                         */
 typedef struct fr_moe_plan {
   int32_t block;      /* routing block                                       */
   int32_t split_k;    /* K splits of the down projection                     */

@@ -216,6 +216,26 @@ def test_layers_accept_the_scratch_of_the_plans_own_block():
             assert "workspace" in call(least - 1) and "aligned" not in call(least - 1)
 
 
+def test_layers_scratch_stays_static_where_the_plans_own_does():
+    """Sizes whose scratch with the plan's block fits the 64 MiB of the entry point that allocates nothing need no more for what the
+    layers route for instead (which would be other kernels there than with a workspace)."""
+    import fast_route_amd as fr
+    from fast_route_amd import _native
+    lib, limit, grown = _native.lib(), 64 << 20, 0
+    for H, F, E, k in ((2048, 1408, 64, 6), (2048, 768, 128, 8), (2048, 2816, 128, 8), (3072, 1024, 96, 4), (1024, 3584, 8, 2), (4096, 1024, 16, 2)):
+        for M in range(1, 900, 7):
+            p, own = _native.FrMoePlan(), _native.FrMoePlan()
+            assert lib.fr_moe_get_plan(M, H, F, E, k, _native.FR_BF16, p) == 0
+            try:
+                with fr.tunables(block=p.block, split_k=p.split_k):
+                    assert lib.fr_moe_get_plan(M, H, F, E, k, _native.FR_BF16, own) == 0
+            finally:
+                fr.reset_tunables()
+            grown += p.workspace_bytes > own.workspace_bytes
+            assert own.workspace_bytes > limit or p.workspace_bytes <= limit, (M, H, F, E, own.workspace_bytes, p.workspace_bytes)
+    assert grown > 0
+
+
 def test_tunables_override_the_plan_and_reset():
     """fr_moe_set_tunables is host logic: the plan follows the overrides, rejects values outside its ranges,
     and NULL restores the library's own choices."""

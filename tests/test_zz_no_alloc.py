@@ -50,6 +50,19 @@ def test_noalloc_matches_workspace_entry_twice(native):
         assert err <= 2.0 ** -6 * want.abs().max().item(), err
 
 
+@pytest.mark.parametrize("M,H,F,E,topk", [(298, 2048, 1408, 64, 6), (299, 2048, 1408, 64, 6), (341, 2048, 1408, 64, 6), (470, 2048, 640, 128, 8), (200, 2048, 2816, 128, 8)])
+def test_noalloc_takes_the_layers_tiles_for_many_experts(native, M, H, F, E, topk):
+    """Sizes at which the layers route for another block than the plan's: with its scratch inside the static one, and (the
+    last) where it would not fit."""
+    from fast_route_amd import _native as N
+    _say(f"noalloc M={M} H={H} F={F} E={E} topk={topk}")
+    g = torch.Generator(device="cuda").manual_seed(M)
+    normal = lambda std, *shape: torch.empty(shape, dtype=torch.bfloat16, device="cuda").normal_(0.0, std, generator=g)
+    x, w1, w2 = normal(1.0, M, H), normal(0.02, E, 2 * F, H), normal(0.02, E, H, F)
+    out, ref = _both(N, x, w1, w2, torch.randn(M, E, generator=g, device="cuda"), topk)
+    assert torch.isfinite(out).all() and torch.equal(out, ref)
+
+
 def test_noalloc_rejects_sizes_beyond_its_scratch(native):
     from fast_route_amd import _native as N
     _say("noalloc size limit")
