@@ -70,6 +70,11 @@ struct TailScratch {
   bool tall = false;  // buffers holds kTallTailBytes (at least plan.tail_bytes)
 };
 
+// a staged caller's: fr_moe_plan.tail_bytes or, with FR_LAYER_TAIL, what fr_moe_get_layer_plan asks for
+inline TailScratch staged_tail(void* tail_ws, bool layers, int any_height) {
+  float* b = static_cast<float*>(tail_ws);
+  return layers && b ? TailScratch{b, reinterpret_cast<int*>(b + kTallTailBytes / 4), any_height, true} : TailScratch{b, nullptr, any_height, false};
+}
 int plan_leaves_heights(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, int block);
 
 // Gate/up projection + SiLU * up (what fr_moe_gateup_silu / fr_moe_gateup_silu_fp8 launch).

@@ -398,6 +398,16 @@ extern "C" int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk,
   return FR_OK;
 }
 
+extern "C" int fr_moe_get_layer_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, fr_moe_plan* plan) {
+  int rc = fr_moe_get_plan(M, H, F, E, topk, dtype, plan);
+  if (rc != FR_OK) return rc;
+  const int64_t bytes = plan->workspace_bytes;
+  *plan = layer_plan(M, H, F, E, topk, dtype & ~FR_W_TILED, *plan);
+  plan->workspace_bytes = bytes;
+  if (plan->tail_bytes > 0) plan->tail_bytes = kTallTailBytes + kTailDescBytes;
+  return FR_OK;
+}
+
 namespace fr {
 namespace {
 // top-k gating of the logits and the routing arrays of the result: one launch for small

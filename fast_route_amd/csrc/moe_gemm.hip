@@ -350,10 +350,11 @@ extern "C" int fr_moe_gateup_silu(const void* x, const void* w1, const int32_t* 
                                   int64_t M, int64_t H, int64_t F, int E, int topk, int block, int dtype,
                                   void* act, void* tail_ws, void* stream) {
   const int w_tiled = (dtype & FR_W1_TILED) ? 1 : 0;
-  dtype &= ~FR_W_TILED;
+  const bool layer_tail = (dtype & FR_LAYER_TAIL) != 0;
+  dtype &= ~(FR_W_TILED | FR_LAYER_TAIL);
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_gateup_silu: dtype %d not in {f16, bf16}", dtype);
   return gateup_impl(x, nullptr, w1, nullptr, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F, E, topk,
-                     block, dtype, act, TailScratch{static_cast<float*>(tail_ws), nullptr, plan_leaves_heights(M, H, F, E, topk, dtype, block)},
+                     block, dtype, act, staged_tail(tail_ws, layer_tail, plan_leaves_heights(M, H, F, E, topk, dtype, block)),
                      static_cast<hipStream_t>(stream), "fr_moe_gateup_silu", w_tiled);
 }
 
@@ -373,11 +374,12 @@ extern "C" int fr_moe_down_combine(const void* act, const void* w2, const float*
                                    int E, int topk, int block, int split_k, int dtype, float* partial,
                                    void* out, void* tail_ws, void* stream) {
   const int w_tiled = (dtype & FR_W2_TILED) ? 1 : 0;
-  dtype &= ~FR_W_TILED;
+  const bool layer_tail = (dtype & FR_LAYER_TAIL) != 0;
+  dtype &= ~(FR_W_TILED | FR_LAYER_TAIL);
   FR_REQUIRE(dtype == FR_F16 || dtype == FR_BF16, FR_E_DTYPE, "fr_moe_down_combine: dtype %d not in {f16, bf16}", dtype);
   return down_impl(act, nullptr, w2, nullptr, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, M, H, F,
                    E, topk, block, split_k, dtype, dtype, partial, out,
-                   TailScratch{static_cast<float*>(tail_ws), nullptr, split_k == 1 ? plan_leaves_heights(M, H, F, E, topk, dtype, block) : kHeightsOfBlock},
+                   staged_tail(tail_ws, layer_tail, split_k == 1 ? plan_leaves_heights(M, H, F, E, topk, dtype, block) : kHeightsOfBlock),
                    static_cast<hipStream_t>(stream), "fr_moe_down_combine", w_tiled, nullptr);
 }
 

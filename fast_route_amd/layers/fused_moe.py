@@ -25,6 +25,14 @@ def plan(M: int, H: int, F: int, E: int, topk: int, dtype, code: int | None = No
     return p
 
 
+def layer_plan(M: int, H: int, F: int, E: int, topk: int, dtype) -> N.FrMoePlan:
+    """What the one-call layers run for these sizes (fr_moe_get_layer_plan): the block they route for, K slices, and the tail
+    scratch that the staged entry points take with FR_LAYER_TAIL."""
+    p = N.FrMoePlan()
+    N.check(N.lib().fr_moe_get_layer_plan(M, H, F, E, topk, N.dtype_code(dtype), p))
+    return p
+
+
 def workspace(M: int, H: int, F: int, E: int, topk: int, dtype, device) -> torch.Tensor:
     """Scratch the layer needs for these shapes (256-byte aligned by torch)."""
     return torch.empty((max(plan(M, H, F, E, topk, dtype).workspace_bytes, 256),), dtype=torch.uint8, device=device)

@@ -5,7 +5,8 @@ The reference wraps its five launches in torch.profiler ranges (data_alloc, rout
 moe_align, moe_1, silu_and_mul, moe_2) and exports a chrome trace to
 ./data/fused_breakdown_{M}_{K}_{E}_{N}_{topk}.json.  Here the same stages run through
 the op-level C entry points, each bracketed by HIP events on the launch stream, and the
-trace holds one complete ("X") event per stage with its GPU duration.  SiLU*mul is fused
+trace holds one complete ("X") event per stage with its GPU duration; they are the layer's
+own kernels (fr_moe_get_layer_plan).  SiLU*mul is fused
 into the first grouped GEMM and the top-k sum into the second, so those ranges are named
 "moe_1+silu_and_mul" and "moe_2+sum".
 """
@@ -18,7 +19,7 @@ import torch
 
 from .. import _native as N
 from ..ops.stable_route import fused_route
-from .fused_moe import _check_layer, plan
+from .fused_moe import _check_layer, layer_plan
 
 STAGES = ("data_alloc", "route", "moe_align", "moe_1+silu_and_mul", "moe_2+sum")
 
@@ -33,11 +34,11 @@ def fused_moe(hidden_states: torch.Tensor, gate: torch.Tensor, w1: torch.Tensor,
     E, N2, _ = w1.shape
     F = N2 // 2
     dev = hidden_states.device
-    lib, st, code = N.lib(), N.stream_ptr(dev), N.dtype_code(hidden_states.dtype)
+    lib, st, code = N.lib(), N.stream_ptr(dev), N.dtype_code(hidden_states.dtype) | N.FR_LAYER_TAIL
     ev = [torch.cuda.Event(enable_timing=True) for _ in range(len(STAGES) + 1)]
 
     ev[0].record()
-    p = plan(M, K, F, E, topk, hidden_states.dtype)
+    p = layer_plan(M, K, F, E, topk, hidden_states.dtype)
     n = M * topk
     topk_weights = torch.empty((M, topk), dtype=torch.float32, device=dev)
     topk_ids = torch.empty((M, topk), dtype=torch.int32, device=dev)

@@ -156,6 +156,12 @@ typedef struct fr_moe_plan {
 } fr_moe_plan;
 int fr_moe_get_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, fr_moe_plan* plan);
 
+/* What fr_fused_moe and fr_fused_experts run in workspace_bytes, for callers who run their stages one by one (2-byte
+ * dtypes): route with its block, pass its split_k, and give the two GEMM entry points below tail_bytes of scratch with
+ * FR_LAYER_TAIL OR-ed into their dtype.  They then run the layer's kernels, with its results bit for bit. */
+#define FR_LAYER_TAIL 0x400
+int fr_moe_get_layer_plan(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, fr_moe_plan* plan);
+
 /* Per-device set-up of every grouped-GEMM kernel of `dtype` (FR_F16, FR_BF16, FR_FP8_E4M3) on the
  * CURRENT device: raises the kernels' dynamic-LDS limits and caches the persistent kernels'
  * occupancy, and looks up the address of fr_fused_moe_noalloc's scratch.  The first call of each tile configuration does the same work lazily; a caller whose

@@ -1094,6 +1094,26 @@ def test_layers_and_staged_entry_points_take_the_same_kernels(native, kernels_of
     _assert_close(out, tiles.cpu(), torch.bfloat16, "one-wavefront-per-SIMD kernel against the plan's tiles")
 
 
+@pytest.mark.parametrize("M,H,Fd,E,k", [(900, 4096, 1024, 16, 2), (96, 2048, 640, 32, 4), (32, 2048, 1408, 64, 6), (240, 2048, 640, 32, 4), (130, 1024, 3584, 8, 2), (40, 1024, 4096, 8, 2),
+                                        (1031, 4096, 4096, 8, 2), (1056, 4096, 2048, 8, 2), (645, 4096, 4096, 8, 2), (2050, 4096, 2048, 8, 2), (3, 4096, 1024, 8, 2)])
+def test_stage_by_stage_twin_has_the_layers_result(native, kernels_of, M, H, Fd, E, k):
+    """The twin on the staged entry points runs the layer's kernels and has its result bit for bit: where the layer routes for another block
+    than the plan's, and where tiles are cut into as many slices as the layer's tail scratch has buffers for."""
+    from fast_route_amd.layers import profile_fused_route, stable_route
+    _say(f"twin M={M} H={H} F={Fd} E={E}")
+    g = torch.Generator(device="cuda").manual_seed(96)
+    x = torch.randn(M, H, generator=g, device="cuda").bfloat16()
+    gate = (torch.randn(H, E, generator=g, device="cuda") / 64).bfloat16()
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g, device="cuda") * 0.02).bfloat16()
+    w2 = (torch.randn(E, H, Fd, generator=g, device="cuda") * 0.02).bfloat16()
+    gemms = lambda names: [n for n in names if "moe_gemm" in n or "rows_kernel" in n]
+    out, names = kernels_of(lambda: stable_route.fused_moe(x, gate, w1, w2, k, True))
+    with tempfile.TemporaryDirectory() as d:
+        twin, twins = kernels_of(lambda: profile_fused_route.fused_moe(x, gate, w1, w2, k, True, save_dir=d))
+    assert gemms(names) == gemms(twins)
+    assert torch.equal(out, twin)
+
+
 def test_more_than_64_tiles_per_workgroup(native, kernels_of):
     """The one-wavefront-per-SIMD kernel works a workgroup's tiles out 64 at a time: 131 tiles of up to 288 rows x 128 feature
     tiles on 256 workgroups are 65 or 66 each.  Operands are small integers, whose sums are exact in any order: equal to the
