@@ -225,7 +225,7 @@ struct QuadUnit {
   int row0, units;    // first slot, height
   int f, expert;      // feature tile, expert
   int kb, kn, tu;     // K tile it starts at, K tiles (round the end of K), slice buffer (-1: a whole tile)
-  int share;          // tiles of its chunk (which share its weight tile) and its index among them: count << 16 | index
+  int share;          // tiles of its chunk (which share its weight tile) and its index among them: count << 16 | index; 0: blocks in no order
 };
 constexpr int kUnitTable = 64;  // units a wavefront works out at a time, one per lane
 
@@ -239,7 +239,7 @@ __device__ __forceinline__ void quad_tile_at(const GemmArgs& a, const QuadWalk& 
     u.units = block / kUnitRows;
     u.f = lin - t * F;
     u.expert = a.expert_ids[t];
-    u.share = 1 << 16;
+    u.share = 0;  // unknown: touched like a tile alone, but its weights are not taken for a stream
     return;
   }
   int lo = 0, hi = a.num_experts - 1;  // the last expert whose tiles start at or before t: it has some
@@ -553,7 +553,7 @@ __global__ __launch_bounds__(256, 1) void moe_gemm_quad_kernel(const GemmArgs a,
     }
     quad_tile_at(a, walk, block, plan.even_heights, lin, k_all, u);
     unit_table[(j0 / kUnitTable) & 1][lane] = u;
-    if (cut_at && cut && tid == n_units - 1 - j0)
+    if (cut_at && cut && tid < kUnitTable && tid == n_units - 1 - j0)  // (thread = lane: u is unit j0 + tid)
       *cut_at = TailCut{u.row0, u.units, u.f, u.expert, xs.slices, xs.rest, quad_buffers(a, plan.tallest), quad_buffer_rows(plan.tallest)};
   };
   auto unit_at = [&](int j) {
