@@ -283,7 +283,7 @@ void launch_route_gate(const void* hidden, const void* gate, int64_t M, int H, i
                        float* w, int32_t* ids, hipStream_t st) {
   constexpr int ET = (G * VPL + 15) / 16;
   // 64 (128 with many experts) tokens per workgroup once that gives every CU a workgroup or two; below,
-  // 16 tokens with K split over the wavefronts (more workgroups, a quarter of the row per wavefront)
+  // 16 tokens with K split over the wavefronts (more workgroups; a quarter or a sixteenth of a chunk per wavefront)
   if (M >= 16384) {
     constexpr int TT = (ET >= 2 && VPL == 1) ? 2 : 1;
     constexpr int KCU = VPL == 1 ? 256 : 128;  // 128 expert rows of 256 K elements would not fit the LDS

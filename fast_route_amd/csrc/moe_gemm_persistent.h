@@ -357,8 +357,9 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   }
   // K tile a unit starts at: it walks its K tiles from there on, round the end.  The rows of a weight matrix are a power of two
   // (or a multiple of 4 KB) long in most models, and workgroups that stream different rows of it at the same pace ask for the same
-  // columns, i.e. for a few of the memory channels, all at once: pure streaming with these loads and 128 token rows
-  // next to them reaches 5.4 TB/s (8 KB rows; 4 KB 5.6) and 6.5 (6.4) with the starts spread.  A tile that is alone on its
+  // columns, i.e. for a few of the memory channels, all at once: a stream of these loads with 128 token rows
+  // next to them from eight wavefronts reaches 5.3 TB/s with tiles dealt in eighths and 4.6 by rounds (8 KB rows; 4 KB 5.0 and 4.5), and
+  // 5.9 either way with the starts spread (6.4 to 6.5 when four wavefronts issue it).  A tile that is alone on its
   // weight tile starts at a place of its own (multiples of the golden ratio: any run of consecutive tiles is spread evenly); tiles
   // that share theirs go on in step.  Layer in us, from column 0 / spread: H = 2048, F = 1408, 64 experts, top-6, 509 tokens
   // 252 / 239, 1000 291 / 277, 2000 384 / 375; H = 4096, F = 14336, 8 experts 256 tokens 526 / 508, 400 547 / 520, 600 623 / 599; H = 6144,

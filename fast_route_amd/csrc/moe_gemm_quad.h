@@ -37,7 +37,7 @@
 // Tiles alone on their weight tile.  Where an expert's run is one tile, nobody shares its weight tiles: the touch only passes them
 // through L1 twice.  Up to 7 units (fp8: 6) such a tile has a K loop without touches, its weight loads non-temporal, so that the
 // stream leaves the token rows in L2; and every run of up to 8 units starts its K loops at spread places (spread_k_start256, why:
-// SPREAD_K in moe_gemm_persistent.h), which keeps the bits of the eight-wavefront kernels that do the same.  Layer on these tiles, in
+// SPREAD_K in moe_gemm_persistent.h), as the eight-wavefront 256-row kernels do.  Layer on these tiles, in
 // parts of the time with touches from column 0, without touches / and spread: H = 4096, F = 14336, 8 experts 700 tokens (6 units)
 // 0.95 / 0.90, 850 1.00 / 0.95; fp16, 16 experts, F = 8192, 700 (3) 0.90 / 0.855, 1100 0.92 / 0.89, 1500 0.96 / 0.91; H = 6144 700
 // 0.93 / 0.89; H = 2048, 64 experts, Zipf-skewed 3000 0.975 / 0.97, 6500 0.99 / 0.98.  With 8 and 9 units it is even or slower (the ring's
@@ -45,8 +45,9 @@
 // touches are evicted before their loads come (20 to 25 % slower); non-temporal loads behind ordinary touches change nothing there
 // and cost 14 % where weight tiles are shared.
 //
-// Same tail split and LDS swizzle as moe_gemm_persistent_kernel; the result is bit-identical to the eight-wavefront kernels on
-// the same MFMA shape (same K order per accumulator, same roundings in the epilogue).
+// Same tail split and LDS swizzle as moe_gemm_persistent_kernel; whole tiles are bit-identical to the eight-wavefront 256-row kernels' on
+// the same MFMA shape (same K order per accumulator, same roundings in the epilogue).  The 128- and 160-row tiles that this
+// kernel stands in for start their K loops elsewhere, and a tile cut along K depends on the tiles' heights.
 #pragma once
 #include "moe_gemm_persistent.h"
 

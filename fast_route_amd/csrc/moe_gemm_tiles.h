@@ -138,7 +138,7 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
     case 64:
       // The persistent form hides each tile's ring fill behind its predecessor's last K tiles: the 64-row gate/up
       // GEMM streams the weights at 6.3 instead of 5.9 TB/s (128 tokens: 318 -> 298 us, fp8 192 -> 170 us).  The
-      // down projection's 64-row tile gains nothing from it (147 us either way) and stays plain.
+      // down projection's 64 x 256 tile gains nothing from it (147 us either way) and stays plain.
       if constexpr (sizeof(T) == 2) {
         // Rows of up to 4 KB: the 128-row tile's walk with half the rows.  Layer in parts of the time on T64U: H = 2048, 64 experts,
         // top-6 100 tokens 0.95, 120 0.95, 150 0.99, 230 0.97; H = 1024, F = 3584 60 0.97, 100 0.975, 200 0.96, 400 0.92; longer rows 1.01 to

@@ -18,7 +18,8 @@ def set_tunables(block: int = 0, split_k: int = 0, group_m: int = 0, no_tail_spl
     (16, 32, 64, 128, 160, 256); split_k: K slices of the down projection; group_m: token blocks
     walked together over the feature tiles; no_tail_split: never split the last round of tiles;
     epilogue_combine: top-2 combine by atomic adds in the down GEMM's epilogue (measured slower than the combine kernel);
-    no_quad: no GEMM takes the one-wavefront-per-SIMD kernel; the eight-wavefront ones run (same results)."""
+    no_quad: no GEMM takes the one-wavefront-per-SIMD kernel; the eight-wavefront ones run (fp32 sums in another
+    order under plans of 128 and 160 rows and in tiles cut along K)."""
     t = N.FrMoeTunables(int(block), int(split_k), int(group_m), int(bool(no_tail_split)), int(bool(epilogue_combine)),
                         int(bool(no_quad)))
     N.check(N.lib().fr_moe_set_tunables(ctypes.byref(t)))

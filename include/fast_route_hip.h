@@ -187,8 +187,9 @@ int fr_moe_prepare(int dtype);
  *              16384 tokens, 149 against 146 us at 16 tokens)
  *   no_quad    1: no GEMM takes the one-wavefront-per-SIMD kernel (four wavefronts, tiles as tall as the experts' runs;
  *              the default with 256-row blocks where K has 16 K tiles or more and the width is at least a
- *              feature tile, and under some plans of 128 and 160 rows) but the eight-wavefront ones; same
- *              results bit for bit on the same MFMA shape, for comparisons and tests
+ *              feature tile, and under some plans of 128 and 160 rows) but the eight-wavefront ones.  With
+ *              256-row blocks whole tiles are the same bit for bit on the same MFMA shape; elsewhere fp32
+ *              sums are added in another order.  For comparisons and tests
  * fr_moe_get_plan, fr_fused_moe, fr_fused_experts, fr_fused_moe_fp8 and the staged GEMM entry
  * points all see them.  fr_moe_set_tunables(NULL) restores the defaults.
  * The staged entry points read the knobs when they are called, not when the plan was made: a
