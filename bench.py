@@ -71,8 +71,13 @@ class Layer:
         else:
             self.logits = torch.randn(M, self.E, generator=g, device=dev)
         self.w1, self.w2 = w1, w2
+        # what the one-call layer runs: its block, K slices and tail scratch, so that the stages are its kernels (fp8: all but the
+        # last round of its gate/up GEMM, for which the staged call takes no scratch)
         self.plan = N.FrMoePlan()
-        N.check(N.lib().fr_moe_get_plan(M, self.H, self.F, self.E, self.topk, N.FR_FP8_E4M3 if fp8 else self.code, self.plan))
+        if fp8:
+            N.check(N.lib().fr_moe_get_plan(M, self.H, self.F, self.E, self.topk, N.FR_FP8_E4M3, self.plan))
+        else:
+            N.check(N.lib().fr_moe_get_layer_plan(M, self.H, self.F, self.E, self.topk, self.code, self.plan))
         p, n = self.plan, M * self.topk
         self.ws = torch.empty(max(p.workspace_bytes, 256), dtype=torch.uint8, device=dev)
         self.out = torch.empty(M, self.H, dtype=self.tdtype, device=dev)
@@ -116,13 +121,9 @@ class Layer:
         N.check(lib.fr_moe_align(self.ti.data_ptr(), N.FR_I32, self.M * self.topk, self.E, p.block, self.sorted.data_ptr(),
                                  self.eids.data_ptr(), self.npost.data_ptr(), self.aws.data_ptr(), self.aws_bytes, self.stream))
         rec(2)
+        self.gate_up()
         if self.fp8:
             w1q, w1s, w2q, w2s = self.fp8
-            N.check(lib.fr_quant_e4m3_rows(self.x.data_ptr(), N.FR_BF16, self.M, self.H, self.H, self.xq.data_ptr(),
-                                           self.xs.data_ptr(), self.stream))
-            N.check(lib.fr_moe_gateup_silu_fp8(self.xq.data_ptr(), self.xs.data_ptr(), w1q.data_ptr(), w1s.data_ptr(),
-                                               self.sorted.data_ptr(), self.eids.data_ptr(), self.npost.data_ptr(), self.M,
-                                               self.H, self.F, self.E, self.topk, p.block, self.act.data_ptr(), self.stream))
             rec(3)
             N.check(lib.fr_quant_e4m3_rows(self.act.data_ptr(), N.FR_BF16, p.sorted_len, self.F, self.F, self.actq.data_ptr(),
                                            self.acts.data_ptr(), self.stream))
@@ -133,17 +134,28 @@ class Layer:
                                                 self.tail.data_ptr() if self.tail is not None else None, self.stream))
             rec(4)
             return
-        N.check(lib.fr_moe_gateup_silu(self.x.data_ptr(), self.w1.data_ptr(), self.sorted.data_ptr(), self.eids.data_ptr(),
-                                       self.npost.data_ptr(), self.M, self.H, self.F, self.E, self.topk, p.block, self.wcode,
-                                       self.act.data_ptr(), self.tail.data_ptr() if self.tail is not None else None,
-                                       self.stream))
         rec(3)
         N.check(lib.fr_moe_down_combine(self.act.data_ptr(), self.w2.data_ptr(), self.tw.data_ptr(), self.sorted.data_ptr(),
                                         self.eids.data_ptr(), self.npost.data_ptr(), self.M, self.H, self.F, self.E,
-                                        self.topk, p.block, p.split_k, self.wcode, self.partial.data_ptr(),
+                                        self.topk, p.block, p.split_k, self.wcode | N.FR_LAYER_TAIL, self.partial.data_ptr(),
                                         self.out.data_ptr(), self.tail.data_ptr() if self.tail is not None else None,
                                         self.stream))
         rec(4)
+
+    def gate_up(self):
+        N, lib, p = self.N, self.N.lib(), self.plan
+        if self.fp8:
+            w1q, w1s, _, _ = self.fp8
+            N.check(lib.fr_quant_e4m3_rows(self.x.data_ptr(), N.FR_BF16, self.M, self.H, self.H, self.xq.data_ptr(),
+                                           self.xs.data_ptr(), self.stream))
+            N.check(lib.fr_moe_gateup_silu_fp8(self.xq.data_ptr(), self.xs.data_ptr(), w1q.data_ptr(), w1s.data_ptr(),
+                                               self.sorted.data_ptr(), self.eids.data_ptr(), self.npost.data_ptr(), self.M,
+                                               self.H, self.F, self.E, self.topk, p.block, self.act.data_ptr(), self.stream))
+            return
+        N.check(lib.fr_moe_gateup_silu(self.x.data_ptr(), self.w1.data_ptr(), self.sorted.data_ptr(), self.eids.data_ptr(),
+                                       self.npost.data_ptr(), self.M, self.H, self.F, self.E, self.topk, p.block, self.wcode | N.FR_LAYER_TAIL,
+                                       self.act.data_ptr(), self.tail.data_ptr() if self.tail is not None else None,
+                                       self.stream))
 
     def active_experts(self):
         return int(self.torch.unique(self.ti).numel())
@@ -253,37 +265,36 @@ def graph_replay_us(torch, layer, reps=20, per_graph=8):
     return round(sorted(times)[len(times) // 2], 2)
 
 
+GATE_UP_KERNELS = ("moe_gemm_quad_kernel", "moe_gemm_persistent_kernel", "moe_gemm_kernel", "gateup_rows_kernel")
+
+
+def gate_up_kernel(torch, layer):
+    """Name of the kernel that did the gate/up GEMM's work (two are launched where the experts' runs choose between
+    tile forms: the longer one), from a profile of that stage.  Taken after all timing."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        layer.gate_up()
+        torch.cuda.synchronize()
+    kernels = [(e.time_range.elapsed_us(), k) for e in prof.events() for k in GATE_UP_KERNELS if k in e.name]
+    name = max(kernels)[1] if kernels else None
+    return name + "<EPI_SILU>" if name in GATE_UP_KERNELS[:3] else name
+
+
 def kernel_roofline(shape, rec, fp8=False):
     """Roofline of the dominant kernel (gate/up grouped GEMM + SiLU*mul) from its
-    event-measured average duration."""
+    event-measured average duration; its name is filled in from a profile (gate_up_kernel)."""
     M, H, F, topk = rec["tokens"], shape["H"], shape["F"], shape["topk"]
     dur = rec["stage_us"]["moe_1+silu_and_mul"] * 1e-6
     flops = 4.0 * M * topk * H * F
     eb = 1 if fp8 else 2
     byts = rec["active_experts"] * 2 * F * H * eb + M * H * eb + M * topk * F * 2
     peak = PEAK_FP8_TFLOPS if fp8 else PEAK_BF16_TFLOPS
-    # which kernel the library picks for the gate/up GEMM: weight rows against token rows for up to 4
-    # tokens of 2-byte operands with H = 4096, 5120, 6144, 7168 or 8192, the one-wavefront-per-SIMD kernel for 256-row
-    # blocks with a K of 16 K tiles or more, that kernel or the persistent tile kernel (by the experts' expected runs) for
-    # 128- and 160-row blocks, the persistent one for 64-row blocks (and 256-row blocks of 2-byte operands with a short
-    # K), the plain tile kernel otherwise
-    if not fp8 and M <= 4 and H >= 4096 and H % 512 == 0 and any(H // 512 % c == 0 for c in (5, 6, 7, 8)) and M * H * 2 <= 65536:
-        name = "gateup_rows_kernel"
-    elif rec["block"] == 256 and H >= (2048 if fp8 else 1024):  # 16 K tiles of 128 bytes per row or more
-        name = "moe_gemm_quad_kernel<EPI_SILU>"
-    elif rec["block"] in (128, 160) and M * topk >= 310 * shape["E"]:
-        name = "moe_gemm_quad_kernel<EPI_SILU> or moe_gemm_persistent_kernel<EPI_SILU>"
-    elif rec["block"] in (64, 128, 160) or (rec["block"] == 256 and not fp8):
-        name = "moe_gemm_persistent_kernel<EPI_SILU>"
-    else:
-        name = "moe_gemm_kernel<EPI_SILU>"
     if flops / (peak * 1e12) >= byts / (PEAK_HBM_GBS * 1e9):
         ach = flops / dur / 1e12
-        return {"kernel": name, "bound": "mfma", "achieved": round(ach, 2), "peak": peak,
+        return {"kernel": None, "bound": "mfma", "achieved": round(ach, 2), "peak": peak,
                 "unit": "TFLOP/s", "frac": round(ach / peak, 4), "traffic": None,
                 "avg_launch_us": round(dur * 1e6, 2), "algorithmic_flops_per_launch": flops}
     ach = byts / dur / 1e9
-    return {"kernel": name, "bound": "hbm", "achieved": round(ach, 1), "peak": PEAK_HBM_GBS,
+    return {"kernel": None, "bound": "hbm", "achieved": round(ach, 1), "peak": PEAK_HBM_GBS,
             "unit": "GB/s", "frac": round(ach / PEAK_HBM_GBS, 4), "traffic": None,
             "avg_launch_us": round(dur * 1e6, 2), "algorithmic_bytes_per_launch": byts}
 
@@ -314,8 +325,8 @@ def recorded_traffic(metric, block):
     """HBM bytes per launch of the dominant kernel for this workload, as measured offline with
     rocprofv3 --pmc (FETCH_SIZE and WRITE_SIZE runs, scaled by the copy probe) and recorded
     in profiles/hbm_traffic.json; None when the workload has no record, when the record was taken
-    with other GEMM kernel sources than the ones present, or when the plan now picks another
-    routing block (i.e. another tile) for this workload than the one that was measured."""
+    with other GEMM kernel sources than the ones present, or when the layer now routes for another
+    block (i.e. another tile) for this workload than the one that was measured."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "hbm_traffic.json")
     try:
         with open(path) as f:
@@ -525,7 +536,7 @@ def reference_protocol(torch, N, args):
     included, as the reference times them), median of the repetitions (its do_bench quantile 0.5), and its "TFLOPS"
     figure 2*m*n*k / t (a sixth of the layer's real work at top-2) next to the real one."""
     from fast_route_amd.layers.stable_route import fused_moe as gate_matrix_layer
-    from fast_route_amd.layers.fused_moe import plan
+    from fast_route_amd.layers.fused_moe import layer_plan
     shape = dict(H=args.k, F=args.n, E=args.e, topk=args.topk, zipf=False)
     w1, w2 = make_weights(torch, shape, args.seed, torch.float16, 0.1)
     g = torch.Generator(device="cuda").manual_seed(args.seed)
@@ -545,7 +556,7 @@ def reference_protocol(torch, N, args):
         t = sorted(e0.elapsed_time(e1) for e0, e1 in ev)[len(ev) // 2] * 1e-3
         rows.append({"m": m, "us_per_layer": round(t * 1e6, 2), "ref_2mnk_tflops": round(2.0 * m * args.n * args.k / t / 1e12, 3),
                      "tflops": round(layer_flops(m, args.k, args.n, args.topk) / t / 1e12, 3),
-                     "block": plan(m, args.k, args.n, args.e, args.topk, torch.float16).block})
+                     "block": layer_plan(m, args.k, args.n, args.e, args.topk, torch.float16).block})
     return {"protocol": "fp16, randn/10, n=%d k=%d e=%d topk=%d, gate-matrix layer fused_moe(a, gate, w1, w2, topk, True, False), "
                         "median of %d event-timed calls" % (args.n, args.k, args.e, args.topk, args.steps),
             "ref_2mnk_tflops_is": "2*m*n*k / t, the figure the reference plots (README moe_bench.png)", "rows": rows}
@@ -722,12 +733,14 @@ def main():
         result["routing_stress"] = routing_bench(torch, N, args.steps, args.warmup, args.seed)
     if not args.no_cpu and fp8 is None:
         result["cpu_baseline"] = cpu_baseline(torch, shape, layer, args.cpu_tokens)
+    headline = layer
     default_run = args.shape == "mixtral" and args.dtype == "bf16" and not args.no_sweep
     if default_run and not args.no_configs:
         del layer
         result["configs"] = other_configs(torch, N, args, (w1, w2))
         rp_args = argparse.Namespace(**{**vars(args), "no_sweep": True, "tokens": 4096})
         result["reference_protocol_row"] = reference_protocol(torch, N, rp_args)
+    result["roofline"]["kernel"] = gate_up_kernel(torch, headline)
     print(json.dumps(result))
 
 

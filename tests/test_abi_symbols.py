@@ -176,12 +176,14 @@ def test_recorded_traffic_matches_profiles_file():
     rec = json.load(open(os.path.join(root, "profiles", "hbm_traffic.json")))
     key = "moe_layer_tflops_mixtral_bf16_M4096"
     assert rec[key]["traffic_bytes"] == rec[key]["fetch_bytes"] + rec[key]["write_bytes"]
-    # the record counts only for the kernel sources it was measured with
     block = rec[key]["block"]
-    want = rec[key]["traffic_bytes"] if rec.get("kernel_sources_sha") == mod.kernel_sources_sha() else None
-    assert mod.recorded_traffic(key, block) == want
     assert mod.recorded_traffic(key, block + 1) is None
     assert mod.recorded_traffic("no_such_workload", block) is None
+    # the record counts only for the kernel sources it was measured with
+    if rec["kernel_sources_sha"] != mod.kernel_sources_sha():
+        assert mod.recorded_traffic(key, block) is None
+        pytest.skip("profiles/hbm_traffic.json was taken with other kernel sources than these: bench.py reports no traffic")
+    assert mod.recorded_traffic(key, block) == rec[key]["traffic_bytes"]
 
 
 def test_layers_accept_the_scratch_of_the_plans_own_block():
