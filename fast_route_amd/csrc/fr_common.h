@@ -56,7 +56,7 @@ int prepare_static_scratch();
 constexpr int kTailDescBytes = 8192;  // what TailScratch::cuts points to
 // Whether the tiles of a GEMM may have other heights than its routing block (plans of 128 and 160 rows): no; yes; or where the
 // experts' runs, which only the device knows, favour it (launch_gemm_by_runs).
-enum { kHeightsOfBlock = 0, kHeightsAny = 1, kHeightsByRuns = 2 };
+enum { kHeightsOfBlock = 0, kHeightsAny = 1, kHeightsByRuns = 2, kHeightsByRuns128 = 3, kHeightsByLongRuns128 = 4 };
 constexpr int64_t kTallTailBytes = int64_t(256) * 288 * 256 * 4;  // slice buffers of the tallest tiles, one per workgroup
 
 // Scratch of a grouped GEMM for cutting the tiles of its last round along K (plan.tail_bytes, or nullptr), a place for the

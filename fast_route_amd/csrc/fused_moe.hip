@@ -35,7 +35,7 @@ double expected_blocks(double avg, int E, int rows) {
 // plan's tiles are faster, so the device chooses by the runs (launch_gemm_by_runs; its second launch of either GEMM costs 4 us).
 // Layer in parts of the time with the plan's tiles, near-uniform load tall tiles / chosen by runs, and Zipf-skewed load tall / by runs:
 //   H = 4096, F = 14336, 8 experts   645 tokens 0.845 / 0.855, 1.10 / 1.00; 850 0.94 / 0.94, 1.13 / 1.005; 1031 0.96 / 0.965, 1.07 / 1.01
-//                                    fp8 640 0.90 / 0.92, 1.01 / 1.02; 700 0.965 / 0.97, 1.05 / 1.02
+//                                    fp8 640 0.83 / 0.84, 1.10 / 1.03, but 700 (175 pairs) 0.99 / 1.005, 1.06 / 1.02: up to 167
 //   H = 6144, F = 16384              900 0.925 / 0.93, 1.20 / 1.01;  H = 5120, F = 8192, 16 experts 1350 0.86 / 0.865, 1.18 / 1.00
 //   16 experts, F = 8192, fp16       1300 0.84 / 0.85, 1.11 / 1.00;  H = 7168, F = 2048, 64 experts, top-8 1350 0.88 / 0.885, 1.09 / 1.005
 //   H = 4096, F = 4096, 8 experts    640 0.835 / 0.86, 1.15 / 1.025; F = 1536, 32 experts, top-4 1350 0.955 / 0.97, 1.15 / 1.02
@@ -62,7 +62,10 @@ int any_height(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, cons
   const double avg = static_cast<double>(M) * topk / E, tall = expected_blocks(avg, E, 288), tiles = E * tall * (F / 128);
   if (avg >= (H >= 4096 ? 310.0 : H >= 2048 ? 550.0 : 1030.0)) return tiles >= 200.0 ? kHeightsAny : kHeightsOfBlock;
   if (H < 4096 || expected_blocks(avg, E, p.block) < 1.3) return kHeightsOfBlock;
-  return (expected_blocks(avg, E, es == 2 ? 224 : 192) <= 1.13 && tiles >= 200.0) || (es == 2 && tall <= 1.13 && tiles >= 450.0) ? kHeightsByRuns : kHeightsOfBlock;
+  if (!((expected_blocks(avg, E, es == 2 ? 224 : 180) <= 1.13 && tiles >= 200.0) || (es == 2 && tall <= 1.13 && tiles >= 450.0))) return kHeightsOfBlock;
+  if (p.block != 128 || avg < 222.0) return kHeightsByRuns;
+  const int64_t up = E * ceil_div(F, 128);  // gate/up tiles with one per expert and feature tile; the plan has two
+  return up % 256 != 0 && 2 * up % 256 == 0 ? kHeightsByLongRuns128 : kHeightsByRuns128;
 }
 
 struct Carve {
@@ -330,7 +333,7 @@ fr_moe_plan plan_for(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype
 //       (384) 0.91 / 0.96, F = 14336, 8 (896) 0.91 / 0.95;   but F = 2048, 8 (128) 0.955 / 1.02, H = 768, F = 3584, 8 (224) 0.925 / 1.12
 //     plan 128, 64 rows up to 48 pairs: F = 3584, 8 40 0.74 / 0.97, F = 14336, 8 0.86 / 0.92, H = 768, F = 3072, 16 0.79 / 0.76, F = 1024, 16 (128; two K slices)
 //       0.89 / 0.92;   but F = 1536, 16 (192; three K slices) 0.89 / 1.04, 48 0.89 / 1.12
-//     up to 90 pairs with t up to 224 and one K slice: F = 3584, 8 64 1.00 / 0.80, 80 0.96 / 0.765, F = 7168, 4 1.01 / 0.95, 0.89 / 0.76, F = 2048, 8 0.84 / 0.85, 0.74 / 0.77;
+//     up to 90 pairs (t above 128: 104) with t up to 224 and one K slice: F = 3584, 8 64 1.00 / 0.80, 80 0.96 / 0.765, 100 0.95 / 0.75, F = 7168, 4 1.01 / 0.95, 0.89 / 0.76, F = 2048, 8 0.84 / 0.85, 0.74 / 0.77;
 //       but t = 256 F = 4096, 8 80 1.05 / 0.895, H = 768, F = 2048, 16 1.025 / 0.875;   F = 2048, 8 100 0.74 / 1.09
 //     up to 125 pairs with t up to 80: F = 4096, 2 0.62, F = 2816, 1 0.63, F = 1024, 8 0.90 / 0.91, H = 640, F = 2560, 4 0.74 / 0.74
 //   160 rows instead of 128 where an expert is likely to exceed 128 rows: a block more costs a round of tiles, the larger tile 1 %.
@@ -347,7 +350,7 @@ int layer_block(int64_t M, int64_t H, int64_t F, int E, int topk, int dtype, con
   if (E <= 16 && H >= 640 && H <= 1024 && F >= 1024) {
     const int64_t t = E * ceil_div(F, 128);
     if (p.block == 32) return H > 896 && t >= 192 && t <= 240 ? 64 : t >= 256 && avg <= 10 ? 16 : 32;
-    if (p.block == 128 && ((avg <= 48 && (p.split_k == 1 || t <= 128)) || (avg <= 90 && p.split_k == 1 && t <= 224) || (avg < 126 && t <= 80))) return 64;
+    if (p.block == 128 && ((avg <= 48 && (p.split_k == 1 || t <= 128)) || (avg <= (t > 128 ? 104 : 90) && p.split_k == 1 && t <= 224) || (avg < 126 && t <= 80))) return 64;
   }
   if (E <= 16 && H >= 4096 && F >= 1024 && p.block == 128 && avg < 128 && E * (expected_blocks(avg, E, 128) - 1.0) >= 0.15) return 160;
   return p.block;

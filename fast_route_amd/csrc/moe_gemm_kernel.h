@@ -81,7 +81,7 @@ struct GemmArgs {
   unsigned div_mul;     // division by top_k of the one-wavefront-per-SIMD form (quad_divisor)
   int div_shift;
   int any_height;       // the tiles' heights need not be the routing block's (TailScratch::any_height)
-  int by_runs;          // launch_gemm_by_runs: 1 = this launch works where runs_fill_tall_tiles, 2 = where they do not, 0 = always
+  int by_runs;          // launch_gemm_by_runs: which runs fill tall tiles (runs_fill_tall_tiles), 0 = not launched by it
   int spread_k;         // one-wavefront-per-SIMD form: units of short runs start their K loop at spread places
   int w_tiled;          // W is in the prepared layout (see w_byte_offset), not [E, w_rows, K] row-major
   int setup_only;       // do the per-device set-up of the kernel a launch would take (LDS limit, occupancy) and launch nothing

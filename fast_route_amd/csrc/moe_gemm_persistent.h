@@ -118,9 +118,15 @@ __device__ __forceinline__ void expert_block_offsets(const GemmArgs& a, int nt, 
     if (a.expert_ids[b] < a.expert_ids[b - 1]) off[kMaxExperts + 1] = 1;
   __syncthreads();
 }
-// Of the two launches of launch_gemm_by_runs, the one with tall tiles: nearly every expert's run fits a tile of it and a good
+// Of the two launches of launch_gemm_by_runs, the one with tall tiles works: nearly every expert's run fits a tile of it and a good
 // part of them takes two blocks, as the host expects of near-uniform loads.  All lanes; off: expert_block_offsets of nt blocks.
-// (A run of three blocks or more is two tall tiles at least; one such run in eight is what the host's own rule admits.)
+// A run of three 160-row blocks is two tall tiles, and so is most often one of three 128-row blocks (257 to 384 rows); one such run in eight
+// is what the host's own rule admits.  Where the mean run nearly fills two blocks of 128 rows (by_runs 2 and 3), three mean just over
+// 256 rows, one tile of 288 still, while the plan's tiles grow by half: up to three runs in eight.  Layer on the plan's tiles / tall ones,
+// 8 experts, H = 4096, F = 14336, 232 pairs per expert, 0 / 1 / 2 / 3 runs of 265: 1 / 1.03, 0.93, 0.91, 0.89; H = 6144, F = 16384 0.955, 0.89, 0.86, 0.86;
+// 16 experts, fp16, F = 8192 0.96, 0.885, 0.90, 0.88.  The one loss is of half rounds of tiles where the plan's make whole ones
+// (by_runs 3, by the host: there has to be such a run).  Runs of two blocks, 16 experts of 154 pairs, fp16, F = 8192: 0 1.08, 1 0.92, 3 0.87, 5 0.81;
+// H = 5120, 1 1.005, 3 0.95, 6 0.91; 8 experts, H = 6144 1 1.04, 2 1.00, 3 0.89; 32 experts, F = 1536 4 1.06, 8 1.035, 12 0.90.
 __device__ __forceinline__ bool runs_fill_tall_tiles(const GemmArgs& a, const int* off, int nt, int lane) {
   int runs = 0, doubled = 0;
   for (int e0 = 0; e0 < a.num_experts; e0 += kWave) {
@@ -128,7 +134,8 @@ __device__ __forceinline__ bool runs_fill_tall_tiles(const GemmArgs& a, const in
     runs += __popcll(__ballot(len > 0));
     doubled += __popcll(__ballot(len > 1));
   }
-  return !off[kMaxExperts + 1] && 8 * (nt - runs - doubled) <= runs && 10 * doubled >= 3 * runs;
+  const int extra = nt - runs - doubled;  // blocks beyond two of a run
+  return !off[kMaxExperts + 1] && 4 * doubled >= runs && 8 * extra <= (a.by_runs > 1 ? 3 : 1) * runs && (a.by_runs < 3 || extra > 0);
 }
 // What a fix-up launch that does not walk the tiles itself needs to know about a cut tile, one per workgroup (QuadPlan,
 // launch_gemm_by_runs).  Heights in units of 32 rows.
@@ -203,7 +210,8 @@ inline long long*& fr_prof_host() { static long long* p = nullptr; return p; }
 #define FR_PROF_PARAM
 #define FR_PROF_ARG
 #endif
-template <typename T, typename C, int EPI>
+// BY_RUNS: one of launch_gemm_by_runs's two launches (a form of its own: the fp8 kernels spill more for it, 3 % of the layer)
+template <typename T, typename C, int EPI, bool BY_RUNS = false>
 __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(const GemmArgs a FR_PROF_PARAM) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer resources and LDS-DMA builtins exist in the device pass only
   typedef Elem<T> E;
@@ -250,14 +258,12 @@ __global__ __launch_bounds__(C::NT, C::MINB) void moe_gemm_persistent_kernel(con
   const int k_all = min(a.k_per_split, a.K - k0) / BK;  // K tiles of a whole unit, >= S + 2 (checked by the launcher)
   const XcdSchedule xs = xcd_schedule(total, nper, xcd, k_all, a.tail_ws != nullptr, schedule_by_rounds(nt, a.num_experts), nper);
   const int n_units = xs.rounds + (loc < xs.rest * xs.slices ? 1 : 0);
-  constexpr bool BY_RUNS = (BT == 128 || BT == 160) && EPI != EPI_DOWN;
-  const bool by_runs = BY_RUNS && a.by_runs != 0;
-  if (n_units == 0 && !by_runs) return;
+  if (!BY_RUNS && n_units == 0) return;
   __shared__ int expert_off[kWalkTable];
   expert_block_offsets(a, nt, expert_off, threadIdx.x, C::NT);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (by_runs) {
+  if constexpr (BY_RUNS) {
     if (runs_fill_tall_tiles(a, expert_off, nt, lane)) return;
     if (a.tail_desc && tid == 0) {  // the common fix-up launch: tile `loc` of the XCD's last round, if that is cut
       TailCut c = {};
@@ -755,7 +761,7 @@ __global__ __launch_bounds__(256) void tail_fixup_kernel(const GemmArgs a, int n
 }
 
 // Workgroups resident at once on the current device (a multiple of 8, one share per XCD).
-template <typename T, typename C, int EPI>
+template <typename T, typename C, int EPI, bool BY_RUNS = false>
 int persistent_grid(int* grid_out) {
   constexpr int kMaxDevices = 64;
   static int cached[kMaxDevices] = {};  // per device; a race between threads writes the same value twice
@@ -764,12 +770,12 @@ int persistent_grid(int* grid_out) {
   if (e != hipSuccess || dev < 0 || dev >= kMaxDevices) return fail(FR_E_LAUNCH, "persistent GEMM: device %d (%s)", dev, hipGetErrorString(e));
   if (!cached[dev]) {
     if (C::LDS_BYTES > 65536)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_persistent_kernel<T, C, EPI>),
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_persistent_kernel<T, C, EPI, BY_RUNS>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
     int cus = 0, per_cu = 0;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess)
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_gemm_persistent_kernel<T, C, EPI>, C::NT, C::LDS_BYTES);
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_gemm_persistent_kernel<T, C, EPI, BY_RUNS>, C::NT, C::LDS_BYTES);
     if (e != hipSuccess) {
       (void)hipGetLastError();  // reported here: not to be found again by the next launch check
       return fail(FR_E_LAUNCH, "persistent GEMM set-up (%d B LDS): %s", C::LDS_BYTES, hipGetErrorString(e));
@@ -783,7 +789,7 @@ int persistent_grid(int* grid_out) {
 
 // Launches the persistent form when every split has at least STAGES + 2 K tiles, else the plain one.
 // a.tail_ws (kTailUnits buffers of BT x BF floats, or nullptr) enables the split of the last round.
-template <typename T, typename C, int EPI>
+template <typename T, typename C, int EPI, bool BY_RUNS = false>
 int launch_gemm_persistent(const GemmArgs& a_in, int splits, hipStream_t st) {
   GemmArgs a = a_in;
   constexpr int BK = C::BKB / static_cast<int>(sizeof(T));
@@ -802,7 +808,7 @@ int launch_gemm_persistent(const GemmArgs& a_in, int splits, hipStream_t st) {
   };
   if (a.setup_only) {  // both forms a launch may take
     int resident = 0;
-    const int rc = persistent_grid<T, C, EPI>(&resident);
+    const int rc = persistent_grid<T, C, EPI, BY_RUNS>(&resident);
     return rc != FR_OK ? rc : plain(a);
   }
   if (a.k_per_split / BK < C::STAGES + 2 || last_k / BK < C::STAGES + 2 || a.num_experts < 1 || a.num_experts > kMaxExperts) {
@@ -819,7 +825,7 @@ int launch_gemm_persistent(const GemmArgs& a_in, int splits, hipStream_t st) {
   if (tunables().no_tail_split) a.tail_ws = nullptr;
   a.x_span = x_rows * a.ldx * es < (int64_t(1) << 31) ? static_cast<unsigned>(x_rows * a.ldx * es) : 0u;
   int resident = 0;
-  const int rc = persistent_grid<T, C, EPI>(&resident);
+  const int rc = persistent_grid<T, C, EPI, BY_RUNS>(&resident);
   if (rc != FR_OK) return rc;
   // the fix-up writes whole tiles of 4-column groups: the feature count must be a multiple of the tile's
   constexpr int COLS = (EPI == EPI_SILU) ? C::BF / 2 : C::BF;
@@ -832,15 +838,15 @@ int launch_gemm_persistent(const GemmArgs& a_in, int splits, hipStream_t st) {
   if (grid < 8) grid = 8;
   if (tail) {
     if (grid > kTailUnits) grid = kTailUnits;  // one slice buffer per workgroup
-  } else if (a.by_runs) {
+  } else if (BY_RUNS) {
     if (grid > kTailUnits) grid = kTailUnits;
   } else if (grid > (worst + 7) / 8 * 8) {
     grid = (worst + 7) / 8 * 8;
   }
-  hipLaunchKernelGGL((moe_gemm_persistent_kernel<T, C, EPI>), dim3(static_cast<unsigned>(grid), splits), dim3(C::NT),
+  hipLaunchKernelGGL((moe_gemm_persistent_kernel<T, C, EPI, BY_RUNS>), dim3(static_cast<unsigned>(grid), splits), dim3(C::NT),
                      C::LDS_BYTES, st, a FR_PROF_ARG);
   int lrc = check_launch("moe_gemm_persistent_kernel");
-  if (lrc != FR_OK || !tail || a.by_runs) return lrc;
+  if (lrc != FR_OK || !tail || BY_RUNS) return lrc;
   if constexpr (kFixable) {
     const int nper = static_cast<int>(grid / 8);
     if (nper >= 2) {

@@ -1052,19 +1052,18 @@ int launch_gemm_by_runs(const GemmArgs& a_in, int block, hipStream_t st) {
   GemmArgs a = a_in;
   int tall_grid = 0, block_grid = 0;
   int rc = quad_grid<T, EPI>(&tall_grid);
-  if (rc == FR_OK) rc = persistent_grid<T, C, EPI>(&block_grid);
+  if (rc == FR_OK) rc = persistent_grid<T, C, EPI, true>(&block_grid);
   if (rc != FR_OK) return rc;
   if (tall_grid != block_grid) return 1;  // the list of cut tiles is one per workgroup
   if (tunables().no_tail_split) a.tail_ws = nullptr;
   if (!a.tail_ws) a.tail_desc = nullptr;
   else if (!a.tail_desc) a.tail_desc = tail_desc_in(a.tail_ws);
-  a.by_runs = 1;
+  a.by_runs = a.any_height - kHeightsByRuns + 1;
   rc = launch_gemm_quad<T, EPI>(a, block, 1, st);
   if (rc != FR_OK) return rc;
   GemmArgs b = a;
-  b.by_runs = 2;
   if (sizeof(T) == 1 && EPI == EPI_SILU) b.tail_ws = nullptr;  // fp8's gate/up GEMM does not cut these tiles
-  rc = launch_gemm_persistent<T, C, EPI>(b, 1, st);
+  rc = launch_gemm_persistent<T, C, EPI, true>(b, 1, st);
   if (rc != FR_OK || !a.tail_desc) return rc;
   return launch_quad_fixup<T, EPI>(a, (tall_grid < kTailUnits ? tall_grid : kTailUnits) / 8, st);
 }

@@ -111,7 +111,7 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       if constexpr (EPI != EPI_DOWN) {
         if (a.any_height) {  // tiles as tall as the experts' runs
           fill(128, TL::T256::BF, TL::T256::BKB);
-          const int rc = a.any_height == kHeightsByRuns && splits == 1 ? launch_gemm_by_runs<T, typename TL::T128P, EPI>(a, 128, st) : launch_gemm_quad<T, EPI>(a, 128, splits, st);
+          const int rc = a.any_height >= kHeightsByRuns && splits == 1 ? launch_gemm_by_runs<T, typename TL::T128P, EPI>(a, 128, st) : launch_gemm_quad<T, EPI>(a, 128, splits, st);
           if (rc != 1) return rc;
         }
       }
@@ -129,7 +129,7 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
       if constexpr (EPI != EPI_DOWN) {
         if (a.any_height) {  // tiles as tall as the experts' runs
           fill(160, TL::T256::BF, TL::T256::BKB);
-          const int rc = a.any_height == kHeightsByRuns && splits == 1 ? launch_gemm_by_runs<T, typename TL::T160P, EPI>(a, 160, st) : launch_gemm_quad<T, EPI>(a, 160, splits, st);
+          const int rc = a.any_height >= kHeightsByRuns && splits == 1 ? launch_gemm_by_runs<T, typename TL::T160P, EPI>(a, 160, st) : launch_gemm_quad<T, EPI>(a, 160, splits, st);
           if (rc != 1) return rc;
         }
       }
@@ -241,6 +241,8 @@ int prepare_tiles() {
   }
   if constexpr (EPI != EPI_DOWN) {
     if (rc == FR_OK) rc = launch_gemm_quad<T, EPI>(a, 256, 1, nullptr);
+    if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T128P, EPI, true>(a, 1, nullptr);
+    if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T160P, EPI, true>(a, 1, nullptr);
   }
   if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T128P, EPI>(a, 1, nullptr);
   if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T160P, EPI>(a, 1, nullptr);

@@ -918,9 +918,9 @@ def test_tiles_as_tall_as_the_experts_runs(native, kernels_of, dtype, case):
     (96, 2048, 1024, 32, 4, 32, 64), (191, 2048, 2048, 32, 4, 32, 32), (192, 2048, 2048, 32, 4, 32, 64), (16, 2048, 256, 32, 4, 16, 32), (230, 2048, 256, 32, 4, 32, 32),
     (32, 2176, 640, 32, 4, 16, 16), (16, 2048, 2176, 32, 4, 16, 16),
     # H of 640 to 1024: gate/up tiles with one block per expert, pairs per expert, K slices
-    (36, 1024, 3584, 8, 2, 32, 64), (361, 1024, 3584, 8, 2, 128, 128), (360, 1024, 3584, 8, 2, 128, 64), (40, 1024, 4096, 8, 2, 32, 16), (41, 1024, 4096, 8, 2, 32, 32),
+    (36, 1024, 3584, 8, 2, 32, 64), (417, 1024, 3584, 8, 2, 128, 128), (416, 1024, 3584, 8, 2, 128, 64), (40, 1024, 4096, 8, 2, 32, 16), (41, 1024, 4096, 8, 2, 32, 32),
     (192, 1024, 4096, 8, 2, 128, 64), (193, 1024, 4096, 8, 2, 128, 128), (36, 1024, 2048, 8, 2, 32, 32), (125, 1024, 2048, 2, 2, 128, 64), (126, 1024, 2048, 2, 2, 128, 128),
-    (72, 1024, 1536, 16, 2, 32, 64), (300, 1024, 1536, 16, 2, 128, 128), (36, 896, 3584, 8, 2, 32, 32),
+    (72, 1024, 1536, 16, 2, 32, 64), (300, 1024, 1536, 16, 2, 128, 128), (180, 1024, 2048, 4, 2, 128, 64), (253, 1024, 2048, 8, 2, 128, 64), (361, 1024, 2048, 8, 2, 128, 128), (36, 896, 3584, 8, 2, 32, 32),
     (900, 4096, 1024, 16, 2, 128, 160)])
 def test_layers_route_for_another_block_than_the_plan(native, kernels_of, M, H, Fd, E, k, planned, rows):
     """At the edges of the ranges where the layers take other tiles than the plan's block stands for: the plan stays, its workspace
@@ -1013,11 +1013,11 @@ def test_one_tile_per_expert_where_the_plan_has_two(native, kernels_of, dtype, M
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, "fp8"])
 @pytest.mark.parametrize("counts,tall", [((162, 162, 161, 161, 161, 161, 161, 161), True), ((330, 165, 165, 165, 165, 100, 100, 100), True),
-                                         ((330, 330, 165, 165, 100, 100, 50, 50), False), ((170, 170, 158, 158, 158, 158, 159, 159), False),
+                                         ((330, 330, 165, 165, 100, 100, 50, 50), False), ((170, 170, 158, 158, 158, 158, 159, 159), True), ((170, 160, 160, 160, 160, 160, 160, 160), False),
                                          ((645, 400, 0, 200, 44, 1, 0, 0), False)])
 def test_skewed_runs_keep_the_plans_tiles(native, dtype, counts, tall):
     """Where near-uniform loads would make every expert's run one tall tile, the experts' runs decide: tall tiles with one run of
-    three blocks among eight experts, the plan's tiles (bit for bit those of no_quad) with two, with few runs of two blocks and with a
+    three blocks among eight experts, the plan's tiles (bit for bit those of no_quad) with two, with one run of two blocks and with a
     skewed load; without cut tiles as well."""
     import fast_route_amd as fr
     from fast_route_amd import _native as N, fused_experts, fused_moe_fp8, prepare_weights_fp8
@@ -1061,6 +1061,30 @@ def test_skewed_runs_keep_the_plans_tiles(native, dtype, counts, tall):
             assert (o - ref).norm() / ref.norm() <= 1e-2 and (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
         else:
             _assert_close(o, ref, dtype, f"{counts}")
+
+
+@pytest.mark.parametrize("Fd,counts,tall", [
+    (7296, (232,) * 8, True), (7296, (265,) * 3 + (212,) * 4 + (213,), True), (7296, (265,) * 4 + (199,) * 4, False), (7296, (400, 232, 232, 232, 200, 200, 180, 180), True),
+    (10240, (232,) * 8, False), (10240, (265,) + (227,) * 5 + (228,) * 2, True), (10240, (265,) * 4 + (199,) * 4, False)])
+def test_runs_that_nearly_fill_two_blocks(native, Fd, counts, tall):
+    """128-row blocks and a mean run of nearly two of them: tall tiles with up to three runs of three blocks among eight experts; with
+    10240 features, where two blocks each are whole rounds of tiles and one tall tile each is not, with at least one."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_experts
+    from fast_route_amd.layers.fused_moe import plan
+    M, H, E, k = 928, 4096, 8, 2
+    _say(f"runs of nearly two blocks {Fd} {counts}")
+    assert plan(M, H, Fd, E, k, torch.bfloat16).block == 128
+    pairs = np.repeat(np.arange(E), counts).reshape(k, M).T
+    pairs = torch.from_numpy(np.random.default_rng(5).permutation(pairs)).int().contiguous()
+    g = torch.Generator(device="cuda").manual_seed(Fd)
+    normal = lambda std, *shape: torch.empty(shape, dtype=torch.bfloat16, device="cuda").normal_(0.0, std, generator=g)
+    args = [normal(1.0, M, H), normal(0.02, E, 2 * Fd, H), normal(0.02, E, H, Fd), torch.full((M, k), 0.5, device="cuda"), pairs.cuda()]
+    out, again = fused_experts(*args), fused_experts(*args)
+    with fr.tunables(no_quad=True):
+        tiles = fused_experts(*args)
+    assert torch.equal(out, again) and torch.equal(out, tiles) != tall
+    _assert_close(out, tiles.cpu(), torch.bfloat16, "tall tiles against the plan's")
 
 
 @pytest.mark.parametrize("M,H,Fd,E,k,quad", [(1350, 4096, 2048, 8, 2, 2), (1430, 4096, 2048, 8, 2, 2), (2300, 2048, 2048, 8, 2, 2),
