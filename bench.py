@@ -740,7 +740,8 @@ def main():
         result["configs"] = other_configs(torch, N, args, (w1, w2))
         rp_args = argparse.Namespace(**{**vars(args), "no_sweep": True, "tokens": 4096})
         result["reference_protocol_row"] = reference_protocol(torch, N, rp_args)
-    result["roofline"]["kernel"] = gate_up_kernel(torch, headline)
+    if not args.copy_probe:  # a run under a profiler of its own
+        result["roofline"]["kernel"] = gate_up_kernel(torch, headline)
     print(json.dumps(result))
 
 
