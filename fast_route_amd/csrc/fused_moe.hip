@@ -32,7 +32,7 @@ double expected_blocks(double avg, int E, int rows) {
 // With fewer pairs (H >= 4096), where an expert's run is one tile of it and the plan's rows make it two: the weights pass through the
 // CUs once.  Up to 7 units (fp8: 6) such a tile streams its weights (moe_gemm_quad.h); 8 and 9 units gain less and lose to
 // the plan's tiles in a launch of few.  That holds for runs of about the same length, which is all that is priced here: with skewed loads the
-// plan's tiles are faster, so the device chooses by the runs (launch_gemm_by_runs; its second launch of either GEMM costs 4 us).
+// plan's tiles are faster, so the device chooses by the runs (launch_gemm_by_runs; its second launch of either GEMM costs 4 to 5 us).
 // Layer in parts of the time with the plan's tiles, near-uniform load tall tiles / chosen by runs, and Zipf-skewed load tall / by runs:
 //   H = 4096, F = 14336, 8 experts   645 tokens 0.845 / 0.855, 1.10 / 1.00; 850 0.94 / 0.94, 1.13 / 1.005; 1031 0.96 / 0.965, 1.07 / 1.01
 //                                    fp8 640 0.83 / 0.84, 1.10 / 1.03, but 700 (175 pairs) 0.99 / 1.005, 1.06 / 1.02: up to 167
