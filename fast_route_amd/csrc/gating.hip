@@ -28,18 +28,6 @@ __global__ __launch_bounds__(kGateThreads) void gating_topk_kernel(
   }
 }
 
-// 4 consecutive logits as fp32 from a 4-element-aligned address
-template <typename T>
-__device__ __forceinline__ f32x4 load4_as_float(const T* p) {
-  if constexpr (sizeof(T) == 4) {
-    return *reinterpret_cast<const f32x4*>(p);
-  } else {
-    typedef T vec4 __attribute__((ext_vector_type(4)));
-    const vec4 t = *reinterpret_cast<const vec4*>(p);
-    return f32x4{to_float(t[0]), to_float(t[1]), to_float(t[2]), to_float(t[3])};
-  }
-}
-
 template <typename T, int G, int NV>
 __global__ __launch_bounds__(kGateThreads) void gating_topk_blocked_kernel(
     const T* __restrict__ logits, int64_t M, int E, int64_t ld, int topk, int renorm,

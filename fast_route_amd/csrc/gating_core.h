@@ -199,6 +199,18 @@ __device__ __forceinline__ void gate_token(Load load, bool live, int E, int topk
   }
 }
 
+// 4 consecutive logits as fp32 from a 4-element-aligned address
+template <typename T>
+__device__ __forceinline__ f32x4 load4_as_float(const T* p) {
+  if constexpr (sizeof(T) == 4) {
+    return *reinterpret_cast<const f32x4*>(p);
+  } else {
+    typedef T vec4 __attribute__((ext_vector_type(4)));
+    const vec4 t = *reinterpret_cast<const vec4*>(p);
+    return f32x4{to_float(t[0]), to_float(t[1]), to_float(t[2]), to_float(t[3])};
+  }
+}
+
 // Many experts: a group of only G lanes owns a token and every lane keeps NV vectors of 4
 // consecutive logits, vector j of lane g holding experts 4*(G*j + g) .. 4*(G*j + g) + 3, so
 // the G lanes read 4*G consecutive logits of the token per load and a wavefront gates 64/G
@@ -226,7 +238,8 @@ __device__ __forceinline__ void gate_token(Load load, bool live, int E, int topk
 // all but topk - 1 experts masked 11.5 / 12.7 / 9.9, all 64 logits within 70 units in the last place 12.5 / 12.5 / 12.3.
 constexpr int kBlockedSlots = 4;  // result slots per lane: topk <= kBlockedSlots * G
 
-template <int G, int NV, typename Load4, typename Load1>
+// RANKED: renormalised weights from the largest logit and their sum in the order of rank, as gate_token takes them.
+template <int G, int NV, bool RANKED = false, typename Load4, typename Load1>
 __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, bool live, int E, int topk, int renorm,
                                                    float* __restrict__ w_row, int32_t* __restrict__ id_row) {
   constexpr int VPL = 4 * NV;
@@ -372,7 +385,21 @@ __device__ __forceinline__ void gate_token_blocked(Load4 load4, Load1 load1, boo
   // top-1 first: with renormalised weights it is all the softmax statistics there are
   float m = top_v;
   float denom;
-  if (renorm) {
+  if (RANKED && renorm) {
+    float first = -INFINITY;  // (the first winner of a class refilled above is the packed order's, not always the largest)
+#pragma unroll
+    for (int sl = 0; sl < kBlockedSlots; ++sl)
+      if (sl * G + g < topk && place[sl] == 0) first = sel_v[sl];
+    m = group_max<G>(first);
+    denom = 0.f;
+    for (int r = 0; r < topk; ++r) {  // the one lane and slot that holds rank r adds it, the others zeros
+      float term = 0.f;
+#pragma unroll
+      for (int sl = 0; sl < kBlockedSlots; ++sl)
+        if (sl * G + g < topk && place[sl] == r) term = __expf(sel_v[sl] - m);
+      denom += group_sum<G>(term);
+    }
+  } else if (renorm) {
     denom = 0.f;
 #pragma unroll
     for (int sl = 0; sl < kBlockedSlots; ++sl)

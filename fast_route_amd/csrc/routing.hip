@@ -50,12 +50,15 @@ __device__ __forceinline__ unsigned long long same_expert_lanes(int e, bool vali
   return m;
 }
 
-__device__ __forceinline__ int wave_inclusive_scan(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int t = __shfl_up(v, d, kWave);
-    if (lane >= d) v += t;
-  }
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  // inside the rows of 16 lanes (row_shr), then each row's last value into the rows behind it (row_bcast): eight vector
+  // instructions where six __shfl_up steps are six LDS round trips one behind the other
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
   return v;
 }
 
@@ -132,36 +135,11 @@ __device__ __forceinline__ void scan_padded_totals(const int* total, int* start,
   for (int base = 0; base < E; base += kWave) {
     const int e = base + lane;
     const int c = (e < E) ? (total[e] + B - 1) / B * B : 0;
-    const int incl = wave_inclusive_scan(c, lane);
+    const int incl = wave_inclusive_scan(c);
     if (e < E) start[e] = running + incl - c;
-    running += __shfl(incl, kWave - 1, kWave);
+    running += __builtin_amdgcn_readlane(incl, kWave - 1);
   }
   if (lane == 0) start[E] = running;
-}
-
-// expert_ids for every block, padding slots of every run, and the tail.
-__device__ __forceinline__ void write_block_table(const int* total, const int* start, int E, int B,
-                                                  int64_t n, int64_t sorted_len, int tid, int nthreads,
-                                                  int32_t* __restrict__ sorted,
-                                                  int32_t* __restrict__ expert_ids,
-                                                  int32_t* __restrict__ npost_out) {
-  const int npost = start[E];
-  const int nblocks = npost / B;
-  for (int b = tid; b < nblocks; b += nthreads) {
-    const int pos = b * B;
-    int lo = 0, hi = E;  // largest e with start[e] <= pos and a non-empty run
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (start[mid] <= pos) lo = mid; else hi = mid;
-    }
-    expert_ids[b] = lo;
-  }
-  const int lane = tid % kWave, wave = tid / kWave, nwaves = nthreads / kWave;
-  for (int e = wave; e < E; e += nwaves) {
-    for (int s = start[e] + total[e] + lane; s < start[e + 1]; s += kWave) sorted[s] = static_cast<int32_t>(n);
-  }
-  for (int64_t s = npost + tid; s < sorted_len; s += nthreads) sorted[s] = static_cast<int32_t>(n);
-  if (tid == 0) npost_out[0] = npost;
 }
 
 // ---------------------------------------------------------------- small path
@@ -182,30 +160,72 @@ __device__ __forceinline__ void scan_segments(int* table, int* total, int E, int
   }
 }
 
+struct SmallTables {
+  int table[kSmallWaves * kSmallMaxE];  // [segment][expert]: counts, then next free slots
+  int total[kSmallMaxE];
+  int first_block[kSmallMaxE + 1];  // of an expert's run; [E]: blocks in all
+};
+// The sort of one workgroup: the segment of each wavefront is [lo, hi), `first` its first ids (segment_ids), the table is
+// zero and published.  A chain of dependent LDS steps that nothing runs beside, so it has few of them: up to 64 experts one
+// wavefront turns counts into slots without a barrier (a lane per expert), a wavefront then places its pairs from its own row of the table and the block
+// table and the padding are written behind that, by groups of lanes per expert instead of a search per block.
 template <typename IdT>
-__global__ __launch_bounds__(kSmallThreads) void align_small_kernel(
-    const IdT* __restrict__ ids, int64_t n, int E, int B, int seg_len, int64_t sorted_len,
-    int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids, int32_t* __restrict__ npost_out) {
-  __shared__ int table[kSmallWaves * kSmallMaxE];
-  __shared__ int total[kSmallMaxE];
-  __shared__ int start[kSmallMaxE + 1];
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int64_t lo = min64(n, static_cast<int64_t>(wave) * seg_len);
-  const int64_t hi = min64(n, lo + seg_len);
-  int first[kScatterPF];  // read once for the histogram and the placement
-  segment_ids(ids, lo, hi, lane, first);
-  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] = 0;
+__device__ __forceinline__ void small_sort(SmallTables& t, const IdT* ids, const int (&first)[kScatterPF], int64_t lo, int64_t hi,
+                                           int64_t n, int E, int B, int64_t sorted_len, int tid, int32_t* __restrict__ sorted,
+                                           int32_t* __restrict__ expert_ids, int32_t* __restrict__ npost_out) {
+  const int lane = tid % kWave, wave = tid / kWave;
+  int* mine = t.table + wave * E;
+  segment_histogram(ids, lo, hi, E, lane, mine, first);
   __syncthreads();
-  segment_histogram(ids, lo, hi, E, lane, &table[wave * E], first);
-  __syncthreads();
-  scan_segments(table, total, E, tid);
-  __syncthreads();
-  if (wave == 0) scan_padded_totals(total, start, E, B, lane);
-  __syncthreads();
-  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] += start[i % E];
-  write_block_table(total, start, E, B, n, sorted_len, tid, kSmallThreads, sorted, expert_ids, npost_out);
-  __syncthreads();
-  segment_scatter(ids, lo, hi, E, bits_for(E), lane, &table[wave * E], sorted, first);
+  if (E <= kWave) {
+    if (wave == 0) {
+      int c[kSmallWaves], all = 0;
+#pragma unroll
+      for (int w = 0; w < kSmallWaves; ++w) c[w] = lane < E ? t.table[w * E + lane] : 0;
+#pragma unroll
+      for (int w = 0; w < kSmallWaves; ++w) all += c[w];
+      const int blocks = static_cast<int>(static_cast<unsigned>(all + B - 1) / static_cast<unsigned>(B)), end = wave_inclusive_scan(blocks);
+      if (lane < E) {
+        int slot = (end - blocks) * B;
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) {
+          t.table[w * E + lane] = slot;
+          slot += c[w];
+        }
+        t.total[lane] = all;
+        t.first_block[lane] = end - blocks;
+        if (lane == E - 1) t.first_block[E] = end;
+      }
+    }
+    __syncthreads();
+  } else {
+    scan_segments(t.table, t.total, E, tid);
+    __syncthreads();
+    if (wave == 0) {
+      int running = 0;
+      for (int base = 0; base < E; base += kWave) {
+        const int e = base + lane;
+        const int blocks = e < E ? static_cast<int>(static_cast<unsigned>(t.total[e] + B - 1) / static_cast<unsigned>(B)) : 0;
+        const int end = running + wave_inclusive_scan(blocks);
+        if (e < E) t.first_block[e] = end - blocks;
+        running = __builtin_amdgcn_readlane(end, kWave - 1);
+      }
+      if (lane == 0) t.first_block[E] = running;
+    }
+    __syncthreads();
+    for (int e = lane; e < E; e += kWave) mine[e] += t.first_block[e] * B;
+    __builtin_amdgcn_wave_barrier();
+  }
+  segment_scatter(ids, lo, hi, E, bits_for(E), lane, mine, sorted, first);
+  const int group = E <= kSmallWaves ? 6 : 4;  // log2 of the lanes an expert gets
+  for (int e = tid >> group; e < E; e += kSmallThreads >> group) {
+    const int sub = tid & ((1 << group) - 1), b0 = t.first_block[e], b1 = t.first_block[e + 1];
+    for (int b = b0 + sub; b < b1; b += 1 << group) expert_ids[b] = e;
+    for (int s = b0 * B + t.total[e] + sub; s < b1 * B; s += 1 << group) sorted[s] = static_cast<int32_t>(n);
+  }
+  const int npost = t.first_block[E] * B;
+  for (int64_t s = npost + tid; s < sorted_len; s += kSmallThreads) sorted[s] = static_cast<int32_t>(n);
+  if (tid == 0) npost_out[0] = npost;
 }
 
 // bf16 token rows [M, K] to quantise to e4m3 alongside (x == nullptr: none)
@@ -216,32 +236,57 @@ struct RowQuant {
   int K;
 };
 
-// Small batches, whole routing in one launch: the workgroup first gates every token
-// (a group of G lanes per token, 1024/G tokens per pass; weights and ids go to their
-// global arrays), then sorts the ids it has just written exactly as above.
-template <typename T, int G, int VPL>
+// The token rows of workgroups 1 and up of a one-workgroup sort, a row per wavefront
+__device__ __forceinline__ void quant_rows_beside(const RowQuant& rq, int64_t M, int tid) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x - 1) * kSmallWaves + tid / kWave;
+  if (row < M) quant_row(rq.x + row * rq.K, rq.K, rq.q + row * rq.K, rq.scale + row, tid % kWave);
+}
+
+template <typename IdT>
+__global__ __launch_bounds__(kSmallThreads) void align_small_kernel(
+    const IdT* __restrict__ ids, int64_t n, int E, int B, int seg_len, int64_t sorted_len,
+    int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids, int32_t* __restrict__ npost_out) {
+  __shared__ SmallTables t;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int64_t lo = min64(n, static_cast<int64_t>(wave) * seg_len);
+  const int64_t hi = min64(n, lo + seg_len);
+  int first[kScatterPF];  // read once for the histogram and the placement
+  segment_ids(ids, lo, hi, lane, first);
+  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) t.table[i] = 0;
+  __syncthreads();
+  small_sort(t, ids, first, lo, hi, n, E, B, sorted_len, tid, sorted, expert_ids, npost_out);
+}
+
+// Small batches, whole routing in one launch: the workgroup first gates every token (a group of G lanes per token,
+// 1024/G tokens per pass; weights and ids go to their global arrays), then sorts the ids it has just written.  The gating of
+// one workgroup is bound by vector instructions.  NV > 0: each lane keeps 4 * NV logits (gate_token_blocked), which is
+// a quarter of them for 64 experts.
+template <typename T, int G, int VPL, int NV>
 __global__ __launch_bounds__(kSmallThreads) void route_align_small_kernel(
     const T* __restrict__ logits, int64_t M, int E, int topk, int renorm, int B, int seg_len, int64_t sorted_len,
     float* __restrict__ w_out, int32_t* __restrict__ ids_out, int32_t* __restrict__ sorted,
     int32_t* __restrict__ expert_ids, int32_t* __restrict__ npost_out, RowQuant rq) {
-  __shared__ int table[kSmallWaves * kSmallMaxE];
-  __shared__ int total[kSmallMaxE];
-  __shared__ int start[kSmallMaxE + 1];
+  __shared__ SmallTables t;
   __shared__ int32_t pair_id[kRouteAlignMaxN];  // the ids stay here for the sort: no way out to memory and back
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   if (blockIdx.x > 0) {  // the fp8 layer's token rows are quantised by further workgroups of the same launch
-    const int64_t row = static_cast<int64_t>(blockIdx.x - 1) * kSmallWaves + wave;
-    if (row < M) quant_row(rq.x + row * rq.K, rq.K, rq.q + row * rq.K, rq.scale + row, lane);
+    quant_rows_beside(rq, M, tid);
     return;
   }
-  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] = 0;
+  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) t.table[i] = 0;
   constexpr int kPerPass = kSmallThreads / G;
   for (int64_t base = 0; base < M; base += kPerPass) {  // uniform trip count: every lane joins the cross-lane ops
     const int64_t token = base + tid / G;
     const bool live = token < M;
     const T* row = logits + (live ? token : 0) * E;
-    gate_token<G, VPL>([&](int e) { return to_float(row[e]); }, live, E, topk, renorm, w_out + token * topk,
-                       pair_id + static_cast<int>(live ? token : 0) * topk);
+    float* w_row = w_out + token * topk;
+    int32_t* id_row = pair_id + static_cast<int>(live ? token : 0) * topk;
+    if constexpr (NV > 0) {
+      if (base + wave * (kWave / G) >= M) break;  // a wavefront without a token (it has none in later passes)
+      gate_token_blocked<G, NV, true>([&](int e0) { return load4_as_float(row + e0); }, [&](int e) { return to_float(row[e]); }, live, E, topk, renorm, w_row, id_row);
+    } else {
+      gate_token<G, VPL>([&](int e) { return to_float(row[e]); }, live, E, topk, renorm, w_row, id_row);
+    }
   }
   __syncthreads();
   const int64_t n = M * topk;
@@ -249,17 +294,8 @@ __global__ __launch_bounds__(kSmallThreads) void route_align_small_kernel(
   const int64_t hi = min64(n, lo + seg_len);
   int first[kScatterPF];
   segment_ids(pair_id, lo, hi, lane, first);
-  segment_histogram(pair_id, lo, hi, E, lane, &table[wave * E], first);
   for (int i = tid; i < n; i += kSmallThreads) ids_out[i] = pair_id[i];
-  __syncthreads();
-  scan_segments(table, total, E, tid);
-  __syncthreads();
-  if (wave == 0) scan_padded_totals(total, start, E, B, lane);
-  __syncthreads();
-  for (int i = tid; i < kSmallWaves * E; i += kSmallThreads) table[i] += start[i % E];
-  write_block_table(total, start, E, B, n, sorted_len, tid, kSmallThreads, sorted, expert_ids, npost_out);
-  __syncthreads();
-  segment_scatter(pair_id, lo, hi, E, bits_for(E), lane, &table[wave * E], sorted, first);
+  small_sort(t, pair_id, first, lo, hi, n, E, B, sorted_len, tid, sorted, expert_ids, npost_out);
 }
 
 // ---------------------------------------------------------------- large path
@@ -293,7 +329,7 @@ __global__ __launch_bounds__(kSegThreads) void align_segscan_kernel(int* __restr
   for (int base = 0; base < S; base += kSegThreads) {
     const int s = base + tid;
     const int c = (s < S) ? row[s] : 0;
-    const int incl = wave_inclusive_scan(c, lane);
+    const int incl = wave_inclusive_scan(c);
     if (lane == kWave - 1) wave_sum[wave] = incl;
     __syncthreads();
     int before = 0, all = 0;
@@ -482,14 +518,21 @@ int run(const void* ids_v, int64_t n, int E, int B, int32_t* sorted, int32_t* ex
   return check_launch("align kernels");
 }
 
-template <typename T, int G, int VPL>
+// Rows that 4-element vector loads can read, 17 to 64 experts: a few lanes per token in the one-workgroup form.  Renormalised weights
+// only: their sum is taken in the order of rank, as gate_token takes it, so that a weight has the same bits from either.
+// (Above 64 experts the two forms order NaN differently.)
+bool gated_blocked(const void* logits, size_t elem, int E, int topk, int renorm) {
+  return renorm && E > 16 && E <= 64 && E % 4 == 0 && reinterpret_cast<uintptr_t>(logits) % (4 * elem) == 0 && topk <= kBlockedSlots * (E <= 32 ? 8 : 16);
+}
+
+template <typename T, int G, int VPL, int NV>
 void launch_route_align(const void* logits, int64_t M, int E, int topk, int renorm, int B, int64_t sorted_len,
                         float* w, int32_t* ids, int32_t* sorted, int32_t* expert_ids, int32_t* npost, RowQuant rq,
                         hipStream_t st) {
   int seg_len = static_cast<int>(round_up(ceil_div(M * topk, kSmallWaves), kWave));
   if (seg_len == 0) seg_len = kWave;
   const unsigned grid = 1 + (rq.x ? static_cast<unsigned>(ceil_div(M, kSmallWaves)) : 0u);
-  hipLaunchKernelGGL((route_align_small_kernel<T, G, VPL>), dim3(grid), dim3(kSmallThreads), 0, st,
+  hipLaunchKernelGGL((route_align_small_kernel<T, G, VPL, NV>), dim3(grid), dim3(kSmallThreads), 0, st,
                      static_cast<const T*>(logits), M, E, topk, renorm, B, seg_len, sorted_len, w, ids, sorted,
                      expert_ids, npost, rq);
 }
@@ -498,16 +541,19 @@ template <typename T>
 void dispatch_route_align(const void* logits, int64_t M, int E, int topk, int renorm, int B, int64_t sorted_len,
                           float* w, int32_t* ids, int32_t* sorted, int32_t* expert_ids, int32_t* npost, RowQuant rq,
                           hipStream_t st) {
-#define FR_RA(G, VPL) launch_route_align<T, G, VPL>(logits, M, E, topk, renorm, B, sorted_len, w, ids, sorted, expert_ids, npost, rq, st)
-  if (E <= 1) FR_RA(1, 1);
-  else if (E <= 2) FR_RA(2, 1);
-  else if (E <= 4) FR_RA(4, 1);
-  else if (E <= 8) FR_RA(8, 1);
-  else if (E <= 16) FR_RA(16, 1);
-  else if (E <= 32) FR_RA(32, 1);
-  else if (E <= 64) FR_RA(64, 1);
-  else if (E <= 128) FR_RA(64, 2);
-  else FR_RA(64, 4);
+#define FR_RA(G, VPL, NV) launch_route_align<T, G, VPL, NV>(logits, M, E, topk, renorm, B, sorted_len, w, ids, sorted, expert_ids, npost, rq, st)
+  if (gated_blocked(logits, sizeof(T), E, topk, renorm)) {
+    if (E <= 32) FR_RA(8, 1, 1);
+    else FR_RA(16, 1, 1);
+  } else if (E <= 1) FR_RA(1, 1, 0);
+  else if (E <= 2) FR_RA(2, 1, 0);
+  else if (E <= 4) FR_RA(4, 1, 0);
+  else if (E <= 8) FR_RA(8, 1, 0);
+  else if (E <= 16) FR_RA(16, 1, 0);
+  else if (E <= 32) FR_RA(32, 1, 0);
+  else if (E <= 64) FR_RA(64, 1, 0);
+  else if (E <= 128) FR_RA(64, 2, 0);
+  else FR_RA(64, 4, 0);
 #undef FR_RA
 }
 
@@ -515,15 +561,20 @@ void dispatch_route_align(const void* logits, int64_t M, int E, int topk, int re
 
 // Gating and routing arrays in one launch for small batches; false when the shape is
 // outside what one workgroup should do (the caller then runs the two stages separately).
-// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = next power of two of E; two launches cost 2 us
-// more and spread the gating over the CUs.  A layer with H = F = 128 in us, one / two launches:
-//   64 experts, top-6   16 tokens (1 round) 17.8 / 19.8, 32 (2) 19.8 / 19.5, 48 (3) 21.9 / 19.8, 80 (5) 25.9 / 19.7, 168 38.4 / 20.8
-//   32, top-4           64 (2) 18.5 / 19.3, 96 (3) 21.0 / 19.8, 256 34.9 / 24.9
-//   16, top-2           192 (3) 18.7 / 19.9, 256 (4) 25.1 / 23.6, 512 29.2 / 24.4;  8, top-2 256 (2) 23.2 / 23.7, 384 (3) 24.9 / 24.6, 512 26.2 / 24.9
-//   128 (two logits per lane), top-8   16 (1) 22.6 / 22.3, 32 (2) 27.8 / 22.8, 127 57.5 / 24.5;  256 16 26.0 / 25.3, 64 48.9 / 29.5
+// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = lanes per token: the next power of two of E, or 8 or 16
+// (gated_blocked); two launches cost 1 to 3 us more and spread the gating over the CUs.  A layer with H = F = 128 in us.  One logit
+// per lane, one / two launches (with the sort as it was before, a microsecond longer):
+//   16 experts, top-2   192 (3) 18.7 / 19.9, 256 (4) 25.1 / 23.6, 512 29.2 / 24.4;  8, top-2 256 (2) 23.2 / 23.7, 384 (3) 24.9 / 24.6, 512 26.2 / 24.9
+//   64, top-6 (weights not renormalised)   16 tokens (1 round) 17.8 / 19.8, 32 (2) 19.8 / 19.5, 48 (3) 21.9 / 19.8, 80 (5) 25.9 / 19.7, 168 38.4 / 20.8
+// several logits per lane (gated_blocked), sixteen calls in a graph, one logit per lane where that took one launch, else two / now / two launches now:
+//   64 experts, top-6   8 tokens 16.7 / 15.6 / 16.4, 16 17.0 / 15.9 / 16.8, 32 19.1 / 16.2 / 17.5, 64 (1 round) 18.0 / 17.8 / 18.2; 96 (2) 19.4 / 19.5 / 18.6, 160 (3) 19.6 / 21.9 / 18.5
+//   32, top-4           64 18.1 / 15.6 / 16.9, 128 (1) 17.7 / 16.8 / 17.3; 256 (2) 24.0 / 24.6 / 22.9
+// above 64 experts (two and four logits per lane), one / two launches:
+//   128, top-8   16 tokens (1 round) 22.6 / 22.3, 32 (2) 27.8 / 22.8, 127 57.5 / 24.5;  256 16 26.0 / 25.3, 64 48.9 / 29.5
 // quant: the launch also quantises the token rows, which would be a third one; it then keeps all that one workgroup holds.
-bool route_align_fits(int64_t M, int E, int topk, bool quant) {
+bool route_align_fits(const void* logits, int logits_dtype, int64_t M, int E, int topk, int renorm, bool quant) {
   if (M < 1 || M * topk > kRouteAlignMaxN || !use_small_path(M * topk, E) || M * E > 16384 || topk > E) return false;
+  if (gated_blocked(logits, logits_dtype == FR_F32 ? 4 : 2, E, topk, renorm)) return quant || M * (E <= 32 ? 8 : 16) <= 1024;
   int G = 1;
   while (G < E && G < 64) G *= 2;
   return quant || M * G <= 1024 * (E > 64 ? 1 : topk <= 2 ? 3 : 2);

@@ -254,3 +254,37 @@ def test_fused_route_half_and_int64_buffers(native, E, topk, H):
         assert flips.float().mean() < 0.02   # fp32 against float64 logits: near-ties only
         ok = ~flips.any(dim=1)
         torch.testing.assert_close(w.cpu().float()[ok], ow[ok], atol=1e-3, rtol=0)  # fp16 storage of the weights
+
+
+@pytest.mark.parametrize("E,topk", [(20, 3), (32, 4), (32, 20), (36, 6), (64, 1), (64, 6), (64, 17), (68, 2), (256, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_launch_routing_is_the_separate_launches(native, E, topk, dtype):
+    """Small layers gate and sort in one launch, with several logits per lane for 17 to 64 experts; the layer is then bit
+    for bit that of the gating launch's ids and weights.  Token counts at the edges of the wavefronts' groups, of the one
+    launch and beyond it; rows of ties, of logits that differ below the packed keys, of infinities and NaN; logits that
+    vector loads cannot read and weights that are not renormalised, which take the other form."""
+    from fast_route_amd import fused_experts, fused_moe
+    H = Fd = 128
+    g = torch.Generator().manual_seed(E * 7 + topk)
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g) * 0.05).bfloat16().cuda()
+    w2 = (torch.randn(E, H, Fd, generator=g) * 0.05).bfloat16().cuda()
+    for M in (1, 3, 4, 15, 17, 63, 64, 65, 129):
+        x = torch.randn(M, H, generator=g).bfloat16().cuda()
+        noise = torch.randn(M, E, generator=g)
+        rows = {"random": noise, "ties": (noise * 2).round(), "near": 1.0 + noise * 2.0 ** -22,
+                "masked": torch.where(torch.rand(M, E, generator=g) < 0.5, noise, torch.tensor(-float("inf")))}
+        rows["nan"] = torch.where(torch.rand(M, E, generator=g) < 0.05, torch.tensor(float("nan")), noise)
+        for name, logits in rows.items():
+            for renorm in (True, False):
+                for odd in (False, True):
+                    if (odd or not renorm) and name not in ("random", "ties"):
+                        continue
+                    _say(f"one-launch routing E={E} k={topk} {dtype} M={M} {name} renorm={renorm} odd={odd}")
+                    buf = torch.empty(M * E + 1, dtype=dtype, device="cuda")
+                    dev = buf[int(odd):int(odd) + M * E].view(M, E)
+                    dev.copy_(logits)
+                    w, ids = _run_gating(dev, topk, renorm)
+                    out = fused_moe(x, w1, w2, dev, topk, renorm)
+                    ref = fused_experts(x, w1, w2, w.cuda(), ids.cuda())
+                    assert torch.equal(out.isnan(), ref.isnan()), "other rows are NaN"
+                    assert torch.equal(out.nan_to_num(), ref.nan_to_num()), "layer differs"
