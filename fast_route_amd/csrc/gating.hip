@@ -74,7 +74,11 @@ template <> struct Mfma16<f16_t> {
 // wavefronts in us: 16 experts, H = 4096, fp16 1 token 10.6 / 6.3, 128 11.5 / 8.8, 700 13.8 / 8.8, 2048 15.2 / 10.2, 4096 15.7 / 11.9; 8 experts,
 // bf16 9.0 / 5.4, 10.0 / 7.5, 13.2 / 8.5, 13.5 / 9.2, 14.2 / 10.6; H = 8192 15.9 / 7.9 and 28.1 / 24.4; H = 1024 (one chunk) 4.5 / 4.7 and 5.6 / 4.9.
 // G lanes gate a token, VPL logits each: up to G * VPL experts (VPL = 2: 65..128 experts).
-template <typename T, int G, bool SPLITK, int KC, int TT, int VPL = 1, int NW = 4>
+// PF > 1: the gate and token rows of PF chunks are asked for together and wait in registers (a chunk's gate rows are at most an
+// item per thread), so that H = 4096 is one memory latency and not four.  Back to back on other inputs each time, one chunk / four at a
+// time in us: 16 experts, H = 4096, fp16 700 tokens 9.3 / 9.1, 2048 9.9 / 9.2, 4096 12.5 / 11.2; 8 experts 700 8.8 / 8.5, H = 8192, 4096 tokens 22.4 /
+// 17.9; but H = 1024 (one chunk) 3.45 / 3.9.
+template <typename T, int G, bool SPLITK, int KC, int TT, int VPL = 1, int NW = 4, int PF = 1>
 __global__ __launch_bounds__(NW * 64) void route_gate_kernel(
     const T* __restrict__ hidden, const T* __restrict__ gate, int64_t M, int H, int E, int topk,
     int renorm, float* __restrict__ w_out, int32_t* __restrict__ ids_out) {
@@ -116,52 +120,93 @@ __global__ __launch_bounds__(NW * 64) void route_gate_kernel(
     for (int j = 0; j < ET; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const bool vec_gate = E % 8 == 0 && (reinterpret_cast<uintptr_t>(gate) & 15u) == 0;
 
-  for (int kc = 0; kc < H; kc += KC) {
-    vec8 xf[TT][KSTEPS];
+  if (PF > 1 && vec_gate) {
+    typedef T pair_t __attribute__((ext_vector_type(2)));
+    static_assert(PF == 1 || (KC / 2) * (ET * 16 / 8) <= NT, "an item per thread and chunk");
+    const int evs = E / 8, item = min(tid, (KC / 2) * evs - 1), kp = item / evs, ev = item - kp * evs;
+    for (int kc0 = 0; kc0 < H; kc0 += PF * KC) {
+      vec8 xf[PF][KSTEPS], row[PF][2];
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
+      for (int p = 0; p < PF; ++p) {
+        const int kc = kc0 + p * KC, k = kc + 2 * kp;
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int kk = kc + kw0 + ks * 32 + (lane >> 4) * 8;
-        if (kk + 8 <= H) xf[t][ks] = *reinterpret_cast<const vec8*>(xrow[t] + kc + ks * 32);
-        else
+        for (int h = 0; h < 2; ++h) {
+          row[p][h] = vec8{};
+          if (k + h < H) row[p][h] = *reinterpret_cast<const vec8*>(gate + static_cast<int64_t>(k + h) * E + ev * 8);
+        }
 #pragma unroll
-          for (int r = 0; r < 8; ++r) xf[t][ks][r] = static_cast<T>(0.f);
-      }
-    __syncthreads();  // the previous chunk has been read
-    if (vec_gate) {
-      // item = (pair of K rows, 8 experts): two 16-byte loads, eight 32-bit stores of (k, k+1) pairs
-      const int evs = E / 8;
-      for (int item = tid; item < (KC / 2) * evs; item += NT) {
-        const int kp = item % (KC / 2), ev = item / (KC / 2);
-        const int k = kc + 2 * kp;
-        vec8 r0, r1;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) { r0[r] = static_cast<T>(0.f); r1[r] = static_cast<T>(0.f); }
-        if (k < H) r0 = *reinterpret_cast<const vec8*>(gate + static_cast<int64_t>(k) * E + ev * 8);
-        if (k + 1 < H) r1 = *reinterpret_cast<const vec8*>(gate + static_cast<int64_t>(k + 1) * E + ev * 8);
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          typedef T pair_t __attribute__((ext_vector_type(2)));
-          const pair_t pr = {r0[r], r1[r]};
-          *reinterpret_cast<pair_t*>(&gt[(ev * 8 + r) * PITCH + 2 * kp]) = pr;
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          xf[p][ks] = vec8{};
+          if (kc + kw0 + ks * 32 + (lane >> 4) * 8 + 8 <= H) xf[p][ks] = *reinterpret_cast<const vec8*>(xrow[0] + kc + ks * 32);
         }
       }
-    } else {
-      for (int i = tid; i < KC * E; i += NT) {
-        const int k = i / E, e = i % E;
-        gt[e * PITCH + k] = kc + k < H ? gate[static_cast<int64_t>(kc + k) * E + e] : static_cast<T>(0.f);
+#pragma unroll
+      for (int p = 0; p < PF; ++p) {
+        if (kc0 + p * KC >= H) break;
+        __syncthreads();  // the previous chunk has been read
+        if (tid == item)
+#pragma unroll
+          for (int r = 0; r < 8; ++r) *reinterpret_cast<pair_t*>(&gt[(ev * 8 + r) * PITCH + 2 * kp]) = pair_t{row[p][0][r], row[p][1][r]};
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          const vec8 gf = *reinterpret_cast<const vec8*>(&gt[(lane & 15) * PITCH + kw0 + ks * 32 + (lane >> 4) * 8]);
+          acc[0][0] = Mfma16<T>::mma(gf, xf[p][ks], acc[0][0]);
+        }
       }
     }
-    __syncthreads();
+  } else {
+    static_assert(PF == 1 || (ET == 1 && TT == 1), "one tile of experts and of tokens");
+    for (int kc = 0; kc < H; kc += KC) {
+      vec8 xf[TT][KSTEPS];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks)
+      for (int t = 0; t < TT; ++t)
 #pragma unroll
-      for (int j = 0; j < ET; ++j) {
-        const vec8 gf = *reinterpret_cast<const vec8*>(&gt[(j * 16 + (lane & 15)) * PITCH + kw0 + ks * 32 + (lane >> 4) * 8]);
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          const int kk = kc + kw0 + ks * 32 + (lane >> 4) * 8;
+          if (kk + 8 <= H) xf[t][ks] = *reinterpret_cast<const vec8*>(xrow[t] + kc + ks * 32);
+          else
 #pragma unroll
-        for (int t = 0; t < TT; ++t) acc[t][j] = Mfma16<T>::mma(gf, xf[t][ks], acc[t][j]);
+            for (int r = 0; r < 8; ++r) xf[t][ks][r] = static_cast<T>(0.f);
+        }
+      __syncthreads();  // the previous chunk has been read
+      if (vec_gate) {
+        // item = (pair of K rows, 8 experts): two 16-byte loads, eight 32-bit stores of (k, k+1) pairs.  With one or two groups of 8
+        // (sixteen wavefronts) the groups of a row are neighbouring lanes: a load of a wavefront touches 16 lines and not 32 (16
+        // experts, H = 4096, fp16, 1 / 700 tokens 6.7 -> 6.05 and 9.9 -> 9.3 us); with eight the stores would meet in the banks (64
+        // experts, 700 tokens 22 -> 25).
+        const int evs = E / 8;
+        for (int item = tid; item < (KC / 2) * evs; item += NT) {
+          const int kp = NW == 16 ? item / evs : item % (KC / 2), ev = NW == 16 ? item - kp * evs : item / (KC / 2);
+          const int k = kc + 2 * kp;
+          vec8 r0, r1;
+#pragma unroll
+          for (int r = 0; r < 8; ++r) { r0[r] = static_cast<T>(0.f); r1[r] = static_cast<T>(0.f); }
+          if (k < H) r0 = *reinterpret_cast<const vec8*>(gate + static_cast<int64_t>(k) * E + ev * 8);
+          if (k + 1 < H) r1 = *reinterpret_cast<const vec8*>(gate + static_cast<int64_t>(k + 1) * E + ev * 8);
+#pragma unroll
+          for (int r = 0; r < 8; ++r) {
+            typedef T pair_t __attribute__((ext_vector_type(2)));
+            const pair_t pr = {r0[r], r1[r]};
+            *reinterpret_cast<pair_t*>(&gt[(ev * 8 + r) * PITCH + 2 * kp]) = pr;
+          }
+        }
+      } else {
+        for (int i = tid; i < KC * E; i += NT) {
+          const int k = i / E, e = i % E;
+          gt[e * PITCH + k] = kc + k < H ? gate[static_cast<int64_t>(kc + k) * E + e] : static_cast<T>(0.f);
+        }
       }
+      __syncthreads();
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+        for (int j = 0; j < ET; ++j) {
+          const vec8 gf = *reinterpret_cast<const vec8*>(&gt[(j * 16 + (lane & 15)) * PITCH + kw0 + ks * 32 + (lane >> 4) * 8]);
+#pragma unroll
+          for (int t = 0; t < TT; ++t) acc[t][j] = Mfma16<T>::mma(gf, xf[t][ks], acc[t][j]);
+        }
+    }
   }
   __syncthreads();  // every wavefront has read its last gate chunk: the memory becomes the logit rows
   // accumulator rows are experts (lane/16*4 + r inside tile j), columns tokens
@@ -280,8 +325,12 @@ void launch_route_gate(const void* hidden, const void* gate, int64_t M, int H, i
   } else {
     if constexpr (ET == 1) {
       if (M <= kRgWideTokens) {
-        hipLaunchKernelGGL((route_gate_kernel<T, G, true, 1024, 1, VPL, 16>), dim3(static_cast<unsigned>(ceil_div(M, 16))), dim3(1024), 0, st,
-                           static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);
+        if (H > 1024)  // several chunks
+          hipLaunchKernelGGL((route_gate_kernel<T, G, true, 1024, 1, VPL, 16, 4>), dim3(static_cast<unsigned>(ceil_div(M, 16))), dim3(1024), 0, st,
+                             static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);
+        else
+          hipLaunchKernelGGL((route_gate_kernel<T, G, true, 1024, 1, VPL, 16>), dim3(static_cast<unsigned>(ceil_div(M, 16))), dim3(1024), 0, st,
+                             static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);
         return;
       }
     }
