@@ -354,3 +354,23 @@ def test_fp8_random_shapes_against_oracle(native):
         assert torch.isfinite(o).all()
         assert (o - ref).norm() / ref.norm() <= 1e-2, f"case {case}"
         assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max(), f"case {case}"
+
+
+@pytest.mark.parametrize("H", [256, 8192, 8448, 16384, 16640])
+@pytest.mark.parametrize("M", [1, 17])
+def test_fp8_token_rows_of_the_routing_launch(native, H, M):
+    """A small layer's token rows are quantised beside its routing: one chunk per thread of a workgroup, two, the last one partly
+    filled, and beyond those a wavefront to a row.  Bounds as in test_fp8_layer_vs_oracle: 256 of 16640 elements left out or taken from
+    the wrong place would be 12 % of the norm."""
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8
+    _say(f"fp8 token rows H={H} M={M}")
+    Fd, E, k = 256, 2, 1
+    x, logits, w1, w2 = oracle.make_inputs(M, H, Fd, E, seed=79)
+    x, w1, w2 = x.bfloat16(), w1.bfloat16(), w2.bfloat16()
+    out = fused_moe_fp8(x.cuda(), *prepare_weights_fp8(w1.cuda(), w2.cuda()), logits.cuda(), k, True)
+    torch.cuda.synchronize()
+    ref, _ = oracle.fused_moe_fp8(x, w1, w2, logits, k, True)
+    o = out.float().cpu()
+    assert torch.isfinite(o).all()
+    assert (o - ref).norm() / ref.norm() <= 1e-2
+    assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
