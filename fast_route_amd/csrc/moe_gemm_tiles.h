@@ -39,6 +39,7 @@ template <typename T> struct Tiles {  // bf16 / fp16
   typedef Cfg<32, 128, 128, 1, 4, 16, 2, 3> T32;
   // Two slots (40 KB: four workgroups per CU) instead of three (two), for long K slices of rows a power of two long, see dispatch_block
   typedef Cfg<32, 128, 128, 1, 4, 16, 2, 2> T32D;
+  typedef Cfg<32, 128, 128, 1, 4, 16, 2, 4> T32S;  // four slots (80 KB) for short K slices, see dispatch_block
   typedef Cfg<16, 64, 256, 1, 2, 16, 2, 3> T16;
   typedef Cfg<32, 128, 512, 1, 4, 16, 1, 2> T32L;
   typedef Cfg<16, 64, 512, 1, 2, 16, 2, 2> T16L;
@@ -188,6 +189,12 @@ int dispatch_block(GemmArgs a, int block, int splits, int64_t sorted_len, hipStr
         // F = 1408 1.01 / 0.98 to 1.02, 16 experts, F = 1408, 200 tokens 0.99 / 1.02, F = 8192 in four slices 1.03 / 1.0.
         if (a.long_k && a.k_per_split * static_cast<int>(sizeof(T)) >= 16384 && (a.K & (a.K - 1)) == 0)
           return launch_gemm<T, typename TL::T32D, EPI>(a, splits, st);
+        // Short slices (weight rows of up to 4 KB): a tile's rate is what it has in flight over the latency of memory, and a CU holds two
+        // workgroups on four slots as on three.  Layer in parts of the time on three: H = 2048, F = 1408, 64 experts, top-6 24 to 48 tokens 0.995 to
+        // 1.00, 64 0.987, 80 0.973, 100 0.988, 120 0.982; long slices lose (H = 4096, F = 14336, 8 experts 36 to 100 tokens 1.00 to 1.02),
+        // and a launch that cannot fill two workgroups per CU, by the worst-case tile count, has nothing of it (H = 384 and 512, 8 and 16 experts).
+        if (a.long_k && a.k_per_split * static_cast<int>(sizeof(T)) <= kShortRow && static_cast<int64_t>(a.num_t_blocks) * a.num_f_tiles * splits >= 512)
+          return launch_gemm<T, typename TL::T32S, EPI>(a, splits, st);
       }
       return launch_gemm<T, typename TL::T32, EPI>(a, splits, st);
     case 16:
@@ -257,6 +264,7 @@ int prepare_tiles() {
     } else {
       if (rc == FR_OK) rc = launch_gemm_persistent<T, typename TL::T64N, EPI>(a, 1, nullptr);
       if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32D, EPI>(a, 1, nullptr);
+      if (rc == FR_OK) rc = launch_gemm<T, typename TL::T32S, EPI>(a, 1, nullptr);
     }
   }
   if constexpr (EPI == EPI_SILU) {
