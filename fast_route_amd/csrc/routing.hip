@@ -391,43 +391,40 @@ __global__ __launch_bounds__(kSegThreads) void align_scatter_kernel(
 // ---------------------------------------------------------------- large path, two launches
 // The per-expert scan over segments costs a launch of its own only because every scatter workgroup needs
 // (a) each expert's total and (b) the pairs of each expert in the segments before its own.  Here a count
-// workgroup covers 16 segments, leaves each segment's offset INSIDE the workgroup in counts[e][seg] and the
-// workgroup's sums in wgcnt[b][e]; a scatter workgroup then gets (a) and (b) from one pass over the NB x E
-// workgroup sums (6144 values for 64 experts and 393 216 pairs: six loads per thread, all of one expert, summed in
-// registers before two integer LDS atomics, so the order does not matter).  Used while NB x E stays small.
+// workgroup covers 16 segments and leaves their sums in wgcnt[b][e]; a scatter workgroup gets (a) and (b) from one pass
+// over the NB x E sums (12288 values for 64 experts and 393 216 pairs: twelve loads per thread, all of one expert, summed in
+// registers before two integer LDS atomics, so the order does not matter), and counts its own 16 segments again while these are
+// on their way: the ids are in its registers anyway.  Used while NB x E stays small.
+// A wavefront places its 64-pair rounds one behind the other, so segments are short (two_level_seg_len); 256 pairs and more each left most
+// CUs without a wavefront.  Both launches, ids that change from call to call, us, segments of 256 pairs (a 2048th from 524 288 on)
+// and a table of every segment's counts in memory / now:
+//   64 experts    6200 pairs 8.9 / 6.4, 20000 9.5 / 7.1, 100000 10.3 / 7.8, 200000 10.9 / 8.2, 393216 11.5 / 9.1, 1000000 16.7 / 12.8, 4000000 42.6 / 32.3
+//   8 experts     20000 9.0 / 6.5, 100000 9.1 / 6.7, 400000 9.4 / 9.3, 1000000 14.3 / 11.4, 4000000 38.1 / 26.7
+//   256 experts   200000 15.8 / 11.9;  512 50000 20.1 / 11.2
 constexpr int kSeg2Threads = 1024;
 constexpr int kSeg2Waves = kSeg2Threads / kWave;
 constexpr int64_t kTwoLevelMaxEntries = 16384;
 
 template <typename IdT>
 __global__ __launch_bounds__(kSeg2Threads) void align_count2_kernel(
-    const IdT* __restrict__ ids, int64_t n, int E, int seg_len, int S, int* __restrict__ counts,
-    int* __restrict__ wgcnt) {
-  extern __shared__ int hist[];  // [kSeg2Waves][E]
+    const IdT* __restrict__ ids, int64_t n, int E, int seg_len, int* __restrict__ wgcnt) {
+  extern __shared__ int hist[];  // [E]
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int seg0 = blockIdx.x * kSeg2Waves, seg = seg0 + wave;
-  int* mine = hist + wave * E;
-  const int64_t lo = min64(n, static_cast<int64_t>(seg) * seg_len);
-  const int64_t hi = seg < S ? min64(n, lo + seg_len) : lo;
+  const int64_t lo = min64(n, (static_cast<int64_t>(blockIdx.x) * kSeg2Waves + wave) * seg_len);
+  const int64_t hi = min64(n, lo + seg_len);
   int first[kScatterPF];
   segment_ids(ids, lo, hi, lane, first);
-  for (int e = lane; e < E; e += kWave) mine[e] = 0;
-  __builtin_amdgcn_wave_barrier();
-  segment_histogram(ids, lo, hi, E, lane, mine, first);
+  for (int e = tid; e < E; e += kSeg2Threads) hist[e] = 0;
   __syncthreads();
-  for (int i = tid; i < E * kSeg2Waves; i += kSeg2Threads) {  // (expert, segment of this workgroup)
-    const int e = i % E, w = i / E;
-    int before = 0;
-    for (int v = 0; v < w; ++v) before += hist[v * E + e];
-    if (seg0 + w < S) counts[static_cast<int64_t>(e) * S + seg0 + w] = before;
-    if (w == kSeg2Waves - 1) wgcnt[static_cast<int64_t>(blockIdx.x) * E + e] = before + hist[w * E + e];
-  }
+  segment_histogram(ids, lo, hi, E, lane, hist, first);
+  __syncthreads();
+  for (int e = tid; e < E; e += kSeg2Threads) wgcnt[static_cast<int64_t>(blockIdx.x) * E + e] = hist[e];
 }
 
 template <typename IdT>
 __global__ __launch_bounds__(kSeg2Threads) void align_scatter2_kernel(
-    const IdT* __restrict__ ids, int64_t n, int E, int B, int seg_len, int S, int NB, int64_t sorted_len,
-    const int* __restrict__ counts, const int* __restrict__ wgcnt, int32_t* __restrict__ sorted,
+    const IdT* __restrict__ ids, int64_t n, int E, int B, int seg_len, int NB, int64_t sorted_len,
+    const int* __restrict__ wgcnt, int32_t* __restrict__ sorted,
     int32_t* __restrict__ expert_ids, int32_t* __restrict__ npost_out) {
   extern __shared__ int hist[];  // [kSeg2Waves][E]
   __shared__ int start[kMaxE + 1];
@@ -435,15 +432,12 @@ __global__ __launch_bounds__(kSeg2Threads) void align_scatter2_kernel(
   __shared__ int before[kMaxE];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int wg = blockIdx.x;
-  // this wavefront's segment: its first ids and its offsets inside the workgroup are asked for now, so that
-  // their latency passes together with that of the workgroup sums below
-  const int seg = wg * kSeg2Waves + wave;
-  const int64_t lo = min64(n, static_cast<int64_t>(seg) * seg_len);
-  const int64_t hi = seg < S ? min64(n, lo + seg_len) : lo;
+  const int64_t lo = min64(n, (static_cast<int64_t>(wg) * kSeg2Waves + wave) * seg_len);
+  const int64_t hi = min64(n, lo + seg_len);
   int first[kScatterPF];
   segment_ids(ids, lo, hi, lane, first);
-  const int in_wg0 = (seg < S && lane < E) ? counts[static_cast<int64_t>(lane) * S + seg] : 0;
   for (int e = tid; e < E; e += kSeg2Threads) total[e] = before[e] = 0;
+  for (int i = tid; i < kSeg2Waves * E; i += kSeg2Threads) hist[i] = 0;
   __syncthreads();
   // expert e: all pairs, and the pairs in the workgroups before this one.  A thread keeps one expert and sums every
   // (1024 / E)-th workgroup in registers: independent loads, two LDS atomics at the end.  E <= 512 (the launcher).
@@ -465,9 +459,22 @@ __global__ __launch_bounds__(kSeg2Threads) void align_scatter2_kernel(
     if (all != 0) atomicAdd(&total[my_e], all);
     if (below != 0) atomicAdd(&before[my_e], below);
   }
+  int* mine = hist + wave * E;
+  segment_histogram(ids, lo, hi, E, lane, mine, first);
   __syncthreads();
   if (wave == 0) scan_padded_totals(total, start, E, B, lane);
   __syncthreads();
+  // a segment's counts -> its next free slots
+  for (int e = tid; e < E; e += kSeg2Threads) {
+    int c[kSeg2Waves], slot = start[e] + before[e];
+#pragma unroll
+    for (int w = 0; w < kSeg2Waves; ++w) c[w] = hist[w * E + e];
+#pragma unroll
+    for (int w = 0; w < kSeg2Waves; ++w) {
+      hist[w * E + e] = slot;
+      slot += c[w];
+    }
+  }
   if (wg < E) {
     const int e = wg;
     for (int b = start[e] / B + tid; b < start[e + 1] / B; b += kSeg2Threads) expert_ids[b] = e;
@@ -477,11 +484,7 @@ __global__ __launch_bounds__(kSeg2Threads) void align_scatter2_kernel(
     for (int64_t s = start[E] + tid; s < sorted_len; s += kSeg2Threads) sorted[s] = static_cast<int32_t>(n);
     if (tid == 0) npost_out[0] = start[E];
   }
-  if (seg >= S) return;
-  int* mine = hist + wave * E;
-  if (lane < E) mine[lane] = start[lane] + before[lane] + in_wg0;
-  for (int e = lane + kWave; e < E; e += kWave) mine[e] = start[e] + before[e] + counts[static_cast<int64_t>(e) * S + seg];
-  __builtin_amdgcn_wave_barrier();
+  __syncthreads();
   segment_scatter(ids, lo, hi, E, bits_for(E), lane, mine, sorted, first);
 }
 
@@ -490,6 +493,16 @@ bool use_small_path(int64_t n, int E) { return n <= kSmallMaxN && E <= kSmallMax
 int large_seg_len(int64_t n) {
   const int64_t want = round_up(ceil_div(n, 2048), kWave);
   return static_cast<int>(want < 256 ? 256 : want);
+}
+// Pairs per segment of the two launches: one 64-pair round up to 524 288 pairs and an 8192nd beyond, or as many more as keep the workgroup sums
+// within kTwoLevelMaxEntries (a 2048th of the pairs from the start: 393216 pairs on 64 experts 9.8 us and not 9.1, 1000000 on 8 16.4 and not 11.4);
+// 0: too many sums all the same, the three launches.
+int two_level_seg_len(int64_t n, int E) {
+  if (E > 512) return 0;
+  const int longest = large_seg_len(n);
+  for (int64_t len = n > 0 ? round_up(ceil_div(n, 8192), kWave) : kWave; len <= longest; len += kWave)
+    if (E * ceil_div(ceil_div(n, len), kSeg2Waves) <= kTwoLevelMaxEntries) return static_cast<int>(len);
+  return 0;
 }
 
 template <typename IdT>
@@ -511,13 +524,11 @@ int run(const void* ids_v, int64_t n, int E, int B, int32_t* sorted, int32_t* ex
   const unsigned blocks = static_cast<unsigned>(ceil_div(S, kSegWaves));
   const unsigned scatter_blocks = blocks > static_cast<unsigned>(E) ? blocks : static_cast<unsigned>(E);
   const size_t lds = sizeof(int) * kSegWaves * E;
-  const int NB = static_cast<int>(ceil_div(S, kSeg2Waves));
-  if (static_cast<int64_t>(E) * NB <= kTwoLevelMaxEntries && E <= 512) {  // count (+ workgroup sums), scatter: two launches
-    const size_t lds2 = sizeof(int) * kSeg2Waves * E;
-    int* wgcnt = counts + static_cast<int64_t>(E) * S;
-    hipLaunchKernelGGL((align_count2_kernel<IdT>), dim3(NB), dim3(kSeg2Threads), lds2, st, ids, n, E, seg_len, S, counts, wgcnt);
-    hipLaunchKernelGGL((align_scatter2_kernel<IdT>), dim3(NB > E ? NB : E), dim3(kSeg2Threads), lds2, st, ids, n, E, B,
-                       seg_len, S, NB, sorted_len, counts, wgcnt, sorted, expert_ids, npost);
+  if (const int len = two_level_seg_len(n, E)) {  // workgroup sums, scatter: two launches (the sums take a part of the workspace)
+    const int NB = static_cast<int>(n > 0 ? ceil_div(ceil_div(n, len), kSeg2Waves) : 1);
+    hipLaunchKernelGGL((align_count2_kernel<IdT>), dim3(NB), dim3(kSeg2Threads), sizeof(int) * E, st, ids, n, E, len, counts);
+    hipLaunchKernelGGL((align_scatter2_kernel<IdT>), dim3(NB > E ? NB : E), dim3(kSeg2Threads), sizeof(int) * kSeg2Waves * E, st, ids, n, E, B,
+                       len, NB, sorted_len, counts, sorted, expert_ids, npost);
     return check_launch("align kernels");
   }
   hipLaunchKernelGGL((align_count_kernel<IdT>), dim3(blocks), dim3(kSegThreads), lds, st, ids, n, E,

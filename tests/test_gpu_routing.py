@@ -82,3 +82,25 @@ def test_align_medium_sizes_cross_path_boundary(native):
         rng = np.random.default_rng(n_tokens)
         ids = rng.integers(0, 64, size=(n_tokens, 6)).astype(np.int32)
         _check(torch.from_numpy(ids), 32, 64)
+
+
+@pytest.mark.parametrize("n,E", [(6145, 64), (6145, 1), (8193, 8), (262144, 64), (262145, 64), (524289, 8), (700001, 100), (300, 257),
+                                 (32768, 512), (32769, 512), (131072, 512), (131073, 512)])
+def test_align_segment_lengths_of_the_large_sort(native, n, E):
+    """Batches beyond one workgroup: the first size, one pair into a new workgroup, the sizes up to which 64 experts keep one-round
+    segments and from which long batches take longer ones, more experts than the one-workgroup form has, and 512 experts
+    at the last sizes of one round per segment and of the two launches."""
+    from fast_route_amd.ops.fused_moe import moe_align_block_size
+    _say(f"align n={n} E={E}")
+    g = torch.Generator().manual_seed(n + E)
+    p = (torch.arange(E) + 1.0) ** -1.2
+    for B in (16, 160):
+        ids = torch.multinomial(p, n, replacement=True, generator=g).int().view(n, 1)
+        if E > 2:
+            ids[ids == E // 2] = 0  # an expert without a pair
+        s, e, npost = moe_align_block_size(ids.cuda(), B, E)
+        rs, re_, rn = oracle.moe_align_block_size(ids, B, E)
+        total = int(rn[0])
+        assert int(npost.cpu()[0]) == total
+        assert (s.cpu().numpy() == rs).all()
+        assert (e.cpu().numpy()[: total // B] == re_[: total // B]).all()
