@@ -38,7 +38,7 @@ int quant_rows(const void* x, int dtype, int64_t rows, RowFilter rf, int64_t K, 
 const fr_moe_tunables& tunables();
 
 // gating + routing arrays in one launch (small batches); see routing.hip
-bool route_align_fits(const void* logits, int logits_dtype, int64_t M, int E, int topk, int renorm, bool quant);
+bool route_align_fits(int64_t M, int E, int topk, bool quant);
 // qx (optional): bf16 token rows [M, qK] quantised per row to e4m3 (qq, qscale) by further workgroups of the launch
 int route_align_small(const void* logits, int logits_dtype, int64_t M, int E, int topk, int renorm, int block,
                       float* w, int32_t* ids, int32_t* sorted, int32_t* expert_ids, int32_t* npost,

@@ -419,7 +419,7 @@ namespace {
 int route_and_align(const void* logits, int logits_dtype, int64_t M, int E, int topk, int renormalize, int block,
                     const Carve& c, const void* qx, int64_t H, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (route_align_fits(logits, logits_dtype, M, E, topk, renormalize, qx != nullptr))
+  if (route_align_fits(M, E, topk, qx != nullptr))
     return route_align_small(logits, logits_dtype, M, E, topk, renormalize, block, c.topk_w, c.topk_ids, c.sorted,
                              c.expert_ids, c.npost, qx, H, c.xq, c.x_scale, st);
   int rc = fr_gating_topk(logits, logits_dtype, M, E, E, topk, renormalize, c.topk_w, c.topk_ids, stream);

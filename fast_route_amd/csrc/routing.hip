@@ -582,8 +582,8 @@ void dispatch_route_align(const void* logits, int64_t M, int E, int topk, int re
 
 // Gating and routing arrays in one launch for small batches; false when the shape is
 // outside what one workgroup should do (the caller then runs the two stages separately).
-// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = lanes per token: the next power of two of E, or 8 or 16
-// (gated_blocked); two launches cost 1 to 3 us more and spread the gating over the CUs.  A layer with H = F = 128 in us.  One logit
+// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = next power of two of E (with several logits per lane,
+// gated_blocked, it has fewer; the line is where it was without); two launches cost 1 to 3 us more and spread the gating over the CUs.  A layer with H = F = 128 in us.  One logit
 // per lane, one / two launches (with the sort as it was before, a microsecond longer):
 //   16 experts, top-2   192 (3) 18.7 / 19.9, 256 (4) 25.1 / 23.6, 512 29.2 / 24.4;  8, top-2 256 (2) 23.2 / 23.7, 384 (3) 24.9 / 24.6, 512 26.2 / 24.9
 //   64, top-6 (weights not renormalised)   16 tokens (1 round) 17.8 / 19.8, 32 (2) 19.8 / 19.5, 48 (3) 21.9 / 19.8, 80 (5) 25.9 / 19.7, 168 38.4 / 20.8
@@ -593,9 +593,8 @@ void dispatch_route_align(const void* logits, int64_t M, int E, int topk, int re
 // above 64 experts (two and four logits per lane), one / two launches:
 //   128, top-8   16 tokens (1 round) 22.6 / 22.3, 32 (2) 27.8 / 22.8, 127 57.5 / 24.5;  256 16 26.0 / 25.3, 64 48.9 / 29.5
 // quant: the launch also quantises the token rows, which would be a third one; it then keeps all that one workgroup holds.
-bool route_align_fits(const void* logits, int logits_dtype, int64_t M, int E, int topk, int renorm, bool quant) {
+bool route_align_fits(int64_t M, int E, int topk, bool quant) {
   if (M < 1 || M * topk > kRouteAlignMaxN || !use_small_path(M * topk, E) || M * E > 16384 || topk > E) return false;
-  if (gated_blocked(logits, logits_dtype == FR_F32 ? 4 : 2, E, topk, renorm)) return quant || M * (E <= 32 ? 8 : 16) <= 1024;
   int G = 1;
   while (G < E && G < 64) G *= 2;
   return quant || M * G <= 1024 * (E > 64 ? 1 : topk <= 2 ? 3 : 2);
