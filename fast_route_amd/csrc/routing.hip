@@ -20,9 +20,9 @@ namespace {
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / kWave;
 constexpr int kSmallMaxE = 256;
-// One workgroup sorts up to this many pairs; above, two launches spread over the CUs are faster.  Measured, gating +
-// sort back to back, one workgroup against two launches: 4096 pairs 12.9 / 14.7 us (8 experts), 15.2 / 16.1 (64 experts);
-// 8192 pairs 16.2 / 15.4 and 20.0 / 17.7 us.
+// One workgroup sorts up to this many pairs.  Sort alone, replayed from a graph: one workgroup 4000 / 6100 pairs 6.5 / 8.4 us,
+// two launches 6.4 at 6200 (64 experts), so they would win from about 4000; the line stays because callers of up to 6144
+// pairs are told that they need no workspace.
 constexpr int64_t kSmallMaxN = 6144;
 // Gating and sort in ONE launch up to this many pairs (above, the gating kernel spread over the CUs plus the
 // one-workgroup sort win: 2048 pairs 31.6 against 29.5 us for a small layer, 1536 pairs on 64 experts 51.8 against 26.5)
