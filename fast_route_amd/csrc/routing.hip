@@ -8,9 +8,9 @@
 // 64 pairs at a time and ranks the pairs of one expert among themselves with
 // wavefront ballots, so flat order survives inside each expert: the result is
 // the stable sort.  Small inputs run all three phases in one workgroup with the
-// tables in LDS; large ones use a global table and two launches (count + sums per count
-// workgroup, scatter + block table) or, with many experts, three (count, per-expert
-// segment scan, scatter + block table).
+// tables in LDS; large ones take two launches, between which only the sums of every count
+// workgroup go through memory (count, scatter + block table), or, with many experts, three
+// on a table of every segment's counts (count, per-expert segment scan, scatter + block table).
 #include "gating_core.h"
 #include "quant_core.h"
 
@@ -504,6 +504,8 @@ int two_level_seg_len(int64_t n, int E) {
     if (E * ceil_div(ceil_div(n, len), kSeg2Waves) <= kTwoLevelMaxEntries) return static_cast<int>(len);
   return 0;
 }
+// workgroups of the count launch, a set of sums each
+int two_level_groups(int64_t n, int len) { return static_cast<int>(n > 0 ? ceil_div(ceil_div(n, len), kSeg2Waves) : 1); }
 
 template <typename IdT>
 int run(const void* ids_v, int64_t n, int E, int B, int32_t* sorted, int32_t* expert_ids,
@@ -524,8 +526,8 @@ int run(const void* ids_v, int64_t n, int E, int B, int32_t* sorted, int32_t* ex
   const unsigned blocks = static_cast<unsigned>(ceil_div(S, kSegWaves));
   const unsigned scatter_blocks = blocks > static_cast<unsigned>(E) ? blocks : static_cast<unsigned>(E);
   const size_t lds = sizeof(int) * kSegWaves * E;
-  if (const int len = two_level_seg_len(n, E)) {  // workgroup sums, scatter: two launches (the sums take a part of the workspace)
-    const int NB = static_cast<int>(n > 0 ? ceil_div(ceil_div(n, len), kSeg2Waves) : 1);
+  if (const int len = two_level_seg_len(n, E)) {  // workgroup sums, scatter: two launches
+    const int NB = two_level_groups(n, len);
     hipLaunchKernelGGL((align_count2_kernel<IdT>), dim3(NB), dim3(kSeg2Threads), sizeof(int) * E, st, ids, n, E, len, counts);
     hipLaunchKernelGGL((align_scatter2_kernel<IdT>), dim3(NB > E ? NB : E), dim3(kSeg2Threads), sizeof(int) * kSeg2Waves * E, st, ids, n, E, B,
                        len, NB, sorted_len, counts, sorted, expert_ids, npost);
@@ -619,9 +621,10 @@ extern "C" int64_t fr_moe_align_workspace_bytes(int64_t n, int E) {
   using namespace fr;
   if (n < 0 || E < 1 || E > kMaxE) return -1;
   if (use_small_path(n, E)) return 0;
+  // two launches: the count workgroups' sums; three: [E][S] counts and E totals
+  if (const int len = two_level_seg_len(n, E)) return static_cast<int64_t>(sizeof(int)) * E * two_level_groups(n, len);
   const int64_t S = n > 0 ? ceil_div(n, large_seg_len(n)) : 1;
-  // [E][S] counts, then E totals (three launches) or [E][ceil(S / 4)] workgroup sums (two launches)
-  return static_cast<int64_t>(sizeof(int)) * (static_cast<int64_t>(E) * S + static_cast<int64_t>(E) * (ceil_div(S, kSegWaves) + 1));
+  return static_cast<int64_t>(sizeof(int)) * E * (S + 1);
 }
 
 extern "C" int fr_moe_align(const void* topk_ids, int ids_dtype, int64_t n, int E, int block,

@@ -271,3 +271,20 @@ def test_tunables_override_the_plan_and_reset():
     p = plan(4096)
     assert (p.block, p.split_k, p.tail_bytes) == (base.block, base.split_k, base.tail_bytes)
     assert lib.fr_moe_prepare(_native.FR_F32) == -3
+
+
+@pytest.mark.parametrize("n,E,block", [(6145, 64, 16), (8192, 512, 16), (20000, 256, 64), (393216, 64, 64), (524289, 8, 128), (1000000, 64, 32)])
+def test_workspace_of_a_two_launch_sort(n, E, block):
+    """Up to 512 experts a sort keeps one number per expert and count workgroup, 16384 at most: the size it states is that, and it
+    fits the entries of expert_ids behind the last block's, where moe_align_block_size puts it."""
+    from fast_route_amd import _native
+    need = _native.lib().fr_moe_align_workspace_bytes(n, E)
+    assert 4 * E <= need <= 4 * 16384 and need % (4 * E) == 0
+    assert 4 * (n + E - -(-(n + E * (block - 1)) // block)) >= need
+
+
+def test_workspace_of_a_three_launch_sort():
+    """More than 512 experts, or too many sums: every segment's counts and the experts' totals."""
+    from fast_route_amd import _native
+    assert _native.lib().fr_moe_align_workspace_bytes(100000, 600) == 4 * 600 * (-(-100000 // 256) + 1)
+    assert _native.lib().fr_moe_align_workspace_bytes(0, 600) == 4 * 600 * 2

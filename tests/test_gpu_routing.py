@@ -104,3 +104,25 @@ def test_align_segment_lengths_of_the_large_sort(native, n, E):
         assert int(npost.cpu()[0]) == total
         assert (s.cpu().numpy() == rs).all()
         assert (e.cpu().numpy()[: total // B] == re_[: total // B]).all()
+
+
+@pytest.mark.parametrize("n,E", [(6145, 64), (0, 257), (1025, 300), (32768, 512), (131073, 512), (524289, 8), (5000, 600), (0, 1024)])
+def test_align_stays_in_the_workspace_it_asks_for(native, n, E):
+    """Two and three launches in a workspace of exactly the stated size: the result is the oracle's, the words behind it are untouched,
+    and a byte less is refused."""
+    from fast_route_amd import _native as N
+    _say(f"align workspace n={n} E={E}")
+    B, lib = 32, N.lib()
+    ids = torch.randint(0, E, (n, 1), generator=torch.Generator().manual_seed(n + E)).int()
+    need = lib.fr_moe_align_workspace_bytes(n, E)
+    assert need > 0
+    dev, ws = ids.cuda(), torch.full((need // 4 + 64,), -7, dtype=torch.int32, device="cuda")
+    out = [torch.empty(k, dtype=torch.int32, device="cuda") for k in (n + E * (B - 1), n + E, 1)]
+    call = lambda size: lib.fr_moe_align(dev.data_ptr() or None, N.FR_I32, n, E, B, *(t.data_ptr() for t in out), ws.data_ptr(), size, N.stream_ptr(dev.device))
+    assert call(need - 1) != 0
+    N.check(call(need))
+    torch.cuda.synchronize()
+    rs, re_, rn = oracle.moe_align_block_size(ids, B, E)
+    total = int(rn[0])
+    assert int(out[2]) == total and (out[0].cpu().numpy() == rs).all() and (out[1].cpu().numpy()[: total // B] == re_[: total // B]).all()
+    assert (ws[need // 4:] == -7).all()
