@@ -75,9 +75,7 @@ template <> struct Mfma16<f16_t> {
 // bf16 9.0 / 5.4, 10.0 / 7.5, 13.2 / 8.5, 13.5 / 9.2, 14.2 / 10.6; H = 8192 15.9 / 7.9 and 28.1 / 24.4; H = 1024 (one chunk) 4.5 / 4.7 and 5.6 / 4.9.
 // G lanes gate a token, VPL logits each: up to G * VPL experts (VPL = 2: 65..128 experts).
 // PF > 1: the gate and token rows of PF chunks are asked for together and wait in registers (a chunk's gate rows are at most an
-// item per thread), so that H = 4096 is one memory latency and not four.  Back to back on other inputs each time, one chunk / four at a
-// time in us: 16 experts, H = 4096, fp16 700 tokens 9.3 / 9.1, 2048 9.9 / 9.2, 4096 12.5 / 11.2; 8 experts 700 8.8 / 8.5, H = 8192, 4096 tokens 22.4 /
-// 17.9; but H = 1024 (one chunk) 3.45 / 3.9.
+// item per thread), so that H = 4096 is one memory latency and not four (the rule and its figures: gate_chunks_together).
 template <typename T, int G, bool SPLITK, int KC, int TT, int VPL = 1, int NW = 4, int PF = 1>
 __global__ __launch_bounds__(NW * 64) void route_gate_kernel(
     const T* __restrict__ hidden, const T* __restrict__ gate, int64_t M, int H, int E, int topk,
@@ -311,6 +309,16 @@ extern "C" int fr_gating_topk(const void* logits, int logits_dtype, int64_t M, i
 
 namespace fr {
 namespace {
+// Four chunks of 1024 gate rows asked for together, or each behind the one before.  Together they are one memory latency; with 16 experts they
+// are also 128 KB of gate rows that a CU asks for in front of its first MFMA, which loses where some tens of workgroups ask for them from memory at
+// once (few do not get in each other's way, and at 4096 tokens two workgroups to a CU cover for one another).  Other gate and
+// token rows every time, none in a cache, one / four at a time in us:
+//   16 experts, H = 4096   1 token 8.2 / 7.0, 16 10.4 / 9.9, 128 10.4 / 10.4, 256 10.36 / 10.46, 700 10.4 / 10.7, 1000 10.25 / 10.8, 2048 11.4 / 11.35, 4096 13.7 / 12.0
+//   H = 2048               1 4.45 / 4.2, 128 6.6 / 6.6, 700 6.6 / 6.9, 1000 6.5 / 7.0, 4096 8.6 / 8.0;  H = 8192 16 18.3 / 17.5, 700 17.75 / 18.2, 4096 23.8 / 20.6
+//   8 experts, H = 4096    1 5.95 / 5.2, 16 9.15 / 8.6, 700 9.65 / 9.2, 4096 12.8 / 11.6;  H = 2048 4.2 / 3.9, 5.6 / 5.5, 6.15 / 6.15, 8.3 / 7.8
+// (On rows that L2 still holds 8 experts lose 0.1 to 0.5 us below 256 tokens: H = 4096, 33 tokens 7.7 / 8.05.)  H = 1024 is one chunk: 3.45 / 3.9.
+bool gate_chunks_together(int64_t M, int H, int E) { return H > 1024 && (E <= 8 || M <= 128 || M > 2048); }
+
 template <typename T, int G, int VPL = 1>
 void launch_route_gate(const void* hidden, const void* gate, int64_t M, int H, int E, int topk, int renorm,
                        float* w, int32_t* ids, hipStream_t st) {
@@ -325,7 +333,7 @@ void launch_route_gate(const void* hidden, const void* gate, int64_t M, int H, i
   } else {
     if constexpr (ET == 1) {
       if (M <= kRgWideTokens) {
-        if (H > 1024)  // several chunks
+        if (gate_chunks_together(M, H, E))
           hipLaunchKernelGGL((route_gate_kernel<T, G, true, 1024, 1, VPL, 16, 4>), dim3(static_cast<unsigned>(ceil_div(M, 16))), dim3(1024), 0, st,
                              static_cast<const T*>(hidden), static_cast<const T*>(gate), M, H, E, topk, renorm, w, ids);
         else

@@ -313,3 +313,27 @@ def test_route_gate_chunks_asked_for_together(native, E, topk, H):
         assert clear.float().mean() > 0.9
         assert torch.equal(ids.cpu()[clear], oid[clear])
         torch.testing.assert_close(w.cpu()[clear], ow[clear], atol=1e-4, rtol=0)
+
+
+@pytest.mark.parametrize("E,M,H,together", [(16, 128, 1032, 4), (16, 129, 1032, 1), (16, 2048, 4104, 1), (16, 2049, 2048, 4), (16, 128, 1024, 1), (8, 129, 4096, 4),
+                                            (8, 2048, 1032, 4), (12, 129, 4096, 1), (5, 129, 4096, 4)])
+def test_route_gate_chunks_by_experts_and_tokens(native, kernels_of, E, M, H, together):
+    """Where four chunks of gate rows are asked for together and where one: both sides of the rule, against float64 logits.  Bounds as in
+    test_route_gate_chunks_asked_for_together."""
+    import re
+    from fast_route_amd.ops.stable_route import fused_route
+    _say(f"route_gate chunks E={E} M={M} H={H}")
+    g, k = torch.Generator().manual_seed(E * 7 + M), 2
+    h = (torch.randn(M, H, generator=g) / 4).to(torch.float16)
+    gate = (torch.randn(H, E, generator=g) / 4).to(torch.float16)
+    tw, ti = torch.empty(M, k, dtype=torch.float32, device="cuda"), torch.empty(M, k, dtype=torch.int32, device="cuda")
+    (w, ids), names = kernels_of(lambda: fused_route(h.cuda(), gate.cuda(), k, tw, ti, True))
+    used = [n for n in names if "route_gate_kernel" in n]
+    assert len(used) == 1 and re.search(r"Li16ELi%dEE|, 16, %d>" % (together, together), used[0]), names
+    logits = h.double() @ gate.double()
+    ow, oid = oracle.gating_topk(logits.float(), k, True)
+    top = torch.sort(logits, dim=1, descending=True).values
+    clear = (top[:, :k] - top[:, 1:k + 1]).min(dim=1).values > 2e-4
+    assert clear.float().mean() > 0.9
+    assert torch.equal(ids.cpu()[clear], oid[clear])
+    torch.testing.assert_close(w.cpu()[clear], ow[clear], atol=1e-4, rtol=0)
