@@ -236,20 +236,29 @@ struct RowQuant {
   int K;
 };
 
-// Workgroups 1 and up of the one-launch routing: the fp8 layer's token rows, a workgroup to a row, whose loads then are all in flight at once; rows
-// beyond its registers a wavefront to a row.  (A wavefront to every row, in two passes, was the longest chain of the launch: 8.2 us against
-// 5.0 without the rows at 16 tokens, H = 4096.)
+// Workgroups 1 and up of the one-launch routing: the fp8 layer's token rows.  A workgroup to a row has all of the row's loads in flight at
+// once (a wavefront to a row, in two passes, was the longest chain of the launch: 8.2 us against 5.0 without the rows at 16 tokens, H = 4096);
+// rows beyond its registers take a wavefront each.  So do short rows, of which most of a workgroup's threads have nothing.  Layer with F = 256, 8 experts, top-1, a wavefront / a workgroup to a row, us:
+//   16 tokens     H = 256 16.5 / 16.7, 1024 17.5 / 17.6, 1280 20.5 / 20.2, 2048 21.7 / 21.2, 4096 28.9 / 25.6, 8192 45.8 / 37.8, 16384 81.3 / 58.5
+//   128           1024 21.6 / 21.65, 1280 22.8 / 22.4, 1792 24.1 / 23.8, 2048 25.6 / 25.0, 4096 36.2 / 32.7, 8192 58.8 / 48.8
+//   512           1024 31.9 / 32.4, 1792 36.9 / 37.6, 2048 39.95 / 39.1, 3072 50.0 / 49.5, 4096 57.6 / 55.6, 8192 89.9 / 82.4
+//   700           1280 36.9 / 36.7, 2048 42.4 / 42.8, 3072 53.5 / 53.5, 4096 60.7 / 59.6, 5120 74.7 / 71.6
+//   1024          1024 38.9 / 39.4, 2048 48.4 / 48.7, 3072 58.5 / 58.8, 4096 63.5 / 64.0, 8192 104.7 / 100.3, 16384 184.5 / 161.1
 constexpr int kRowOfBlock = 2 * 8 * kSmallThreads;  // longest row of a workgroup
-__host__ __device__ inline int64_t quant_blocks(int64_t M, int K) { return K <= kRowOfBlock ? M : (M + kSmallWaves - 1) / kSmallWaves; }
+__host__ __device__ inline bool block_per_row(int64_t M, int K) {
+  return K <= kRowOfBlock && (M <= 128 ? K > 1024 : K >= 2048);
+}
+__host__ __device__ inline int64_t quant_blocks(int64_t M, int K) { return block_per_row(M, K) ? M : (M + kSmallWaves - 1) / kSmallWaves; }
 __device__ __forceinline__ void quant_rows_beside(const RowQuant& rq, int64_t M, int tid, float* red) {
   const int64_t block = static_cast<int64_t>(blockIdx.x) - 1;
-  const int64_t row = rq.K <= kRowOfBlock ? block : block * kSmallWaves + tid / kWave;
+  const bool whole = block_per_row(M, rq.K);
+  const int64_t row = whole ? block : block * kSmallWaves + tid / kWave;
   if (row >= M) return;
   const bf16_t* x = rq.x + row * rq.K;
   unsigned char* q = rq.q + row * rq.K;
-  if (rq.K <= kRowOfBlock / 2) quant_row_block<bf16_t, 1, kSmallWaves>(x, rq.K, q, rq.scale + row, tid, red);
-  else if (rq.K <= kRowOfBlock) quant_row_block<bf16_t, 2, kSmallWaves>(x, rq.K, q, rq.scale + row, tid, red);
-  else quant_row(x, rq.K, q, rq.scale + row, tid % kWave);
+  if (!whole) quant_row(x, rq.K, q, rq.scale + row, tid % kWave);
+  else if (rq.K <= kRowOfBlock / 2) quant_row_block<bf16_t, 1, kSmallWaves>(x, rq.K, q, rq.scale + row, tid, red);
+  else quant_row_block<bf16_t, 2, kSmallWaves>(x, rq.K, q, rq.scale + row, tid, red);
 }
 
 template <typename IdT>

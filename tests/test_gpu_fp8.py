@@ -374,3 +374,21 @@ def test_fp8_token_rows_of_the_routing_launch(native, H, M):
     assert torch.isfinite(o).all()
     assert (o - ref).norm() / ref.norm() <= 1e-2
     assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("M,H", [(128, 1024), (128, 1280), (129, 1280), (129, 1792), (129, 2048), (513, 4096), (1024, 512), (1024, 2048)])
+def test_fp8_token_rows_by_length_and_count(native, M, H):
+    """Both sides of the rule that gives a token row beside the routing a wavefront or a workgroup: a wavefront to every row with the last
+    workgroup partly filled, a workgroup to every row.  Bounds as in test_fp8_layer_vs_oracle."""
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8
+    _say(f"fp8 token rows M={M} H={H}")
+    Fd, E, k = 256, 2, 1
+    x, logits, w1, w2 = oracle.make_inputs(M, H, Fd, E, seed=83)
+    x, w1, w2 = x.bfloat16(), w1.bfloat16(), w2.bfloat16()
+    out = fused_moe_fp8(x.cuda(), *prepare_weights_fp8(w1.cuda(), w2.cuda()), logits.cuda(), k, True)
+    torch.cuda.synchronize()
+    ref, _ = oracle.fused_moe_fp8(x, w1, w2, logits, k, True)
+    o = out.float().cpu()
+    assert torch.isfinite(o).all()
+    assert (o - ref).norm() / ref.norm() <= 1e-2
+    assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
