@@ -392,3 +392,24 @@ def test_fp8_token_rows_by_length_and_count(native, M, H):
     assert torch.isfinite(o).all()
     assert (o - ref).norm() / ref.norm() <= 1e-2
     assert (o - ref).abs().max() <= 2.0 ** -5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("E,topk,Ms", [(32, 4, (128, 129, 250)), (32, 1, (256, 257, 511)), (64, 6, (64, 65, 129, 170)), (64, 1, (193, 256))])
+def test_fp8_routing_passes_of_several_logits_per_lane(native, E, topk, Ms):
+    """fp8 layers gate up to 1024 pairs in one workgroup: one to four passes of 128 (64) tokens with several logits per lane, wavefronts
+    without a token in the last one.  The same logits at an address that vector loads cannot read take one per lane in the same launch:
+    the outputs are bit-equal."""
+    from fast_route_amd import fused_moe_fp8, prepare_weights_fp8
+    H = Fd = 256
+    for M in Ms:
+        _say(f"fp8 routing passes E={E} k={topk} M={M}")
+        x, logits, w1, w2 = oracle.make_inputs(M, H, Fd, E, seed=89 + M)
+        args = (x.bfloat16().cuda(), *prepare_weights_fp8(w1.bfloat16().cuda(), w2.bfloat16().cuda()))
+        buf = torch.empty(M * E + 1, device="cuda")
+        outs = []
+        for odd in (0, 1):
+            dev = buf[odd:odd + M * E].view(M, E)
+            dev.copy_(logits)
+            outs.append(fused_moe_fp8(*args, dev, topk, True))
+        assert torch.isfinite(outs[0].float()).all() and outs[0].abs().max() > 0
+        assert torch.equal(outs[0], outs[1])

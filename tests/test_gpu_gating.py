@@ -337,3 +337,29 @@ def test_route_gate_chunks_by_experts_and_tokens(native, kernels_of, E, M, H, to
     assert clear.float().mean() > 0.9
     assert torch.equal(ids.cpu()[clear], oid[clear])
     torch.testing.assert_close(w.cpu()[clear], ow[clear], atol=1e-4, rtol=0)
+
+
+@pytest.mark.parametrize("E,topk,Ms", [(64, 6, (31, 32, 33)), (64, 2, (32, 33, 48, 49)), (36, 6, (32, 33)), (32, 4, (32, 33, 64, 65)), (20, 1, (65, 96, 97))])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_one_launch_routing_at_its_last_sizes(native, E, topk, Ms, dtype):
+    """The last token counts of the one launch, the first of two, and more than one pass of the one workgroup; rows with +inf, with
+    both infinities, of -inf alone, masked with the type's lowest value, and with NaN.  Bit for bit the separate launches' layer."""
+    from fast_route_amd import fused_experts, fused_moe
+    H = Fd = 128
+    g = torch.Generator().manual_seed(E * 11 + topk)
+    w1 = (torch.randn(E, 2 * Fd, H, generator=g) * 0.05).bfloat16().cuda()
+    w2 = (torch.randn(E, H, Fd, generator=g) * 0.05).bfloat16().cuda()
+    for M in Ms:
+        x = torch.randn(M, H, generator=g).bfloat16().cuda()
+        noise, u = torch.randn(M, E, generator=g), torch.rand(M, E, generator=g)
+        inf, lowest = torch.tensor(float("inf")), torch.tensor(torch.finfo(dtype).min)
+        rows = {"random": noise, "+inf": torch.where(u < 0.03, inf, noise), "both": torch.where(u < 0.03, inf, torch.where(u > 0.6, -inf, noise)),
+                "lowest": torch.where(u < 0.95, lowest, noise), "nan": torch.where(u < 0.03, torch.tensor(float("nan")), noise)}
+        rows["-inf"] = torch.where(torch.arange(M)[:, None] % 3 == 0, -inf, noise)
+        for name, logits in rows.items():
+            _say(f"one-launch routing at its last sizes E={E} k={topk} {dtype} M={M} {name}")
+            dev = logits.to(dtype).cuda()
+            w, ids = _run_gating(dev, topk, True)
+            out, ref = fused_moe(x, w1, w2, dev, topk, True), fused_experts(x, w1, w2, w.cuda(), ids.cuda())
+            assert torch.equal(out.isnan(), ref.isnan()), "other rows are NaN"
+            assert torch.equal(out.nan_to_num(), ref.nan_to_num()), "layer differs"
