@@ -571,6 +571,32 @@ def test_four_ring_slots_of_short_down_projections(native, kernels_of, Fd, H, sl
         _assert_close(out, ref.cpu(), dtype, f"{dtype}")
 
 
+@pytest.mark.parametrize("Fd,slots", [(4096, 4), (4352, 3)])
+def test_four_ring_slots_of_split_down_projections(native, kernels_of, Fd, slots):
+    """Two K slices of longer weight rows: four ring slots up to 4 KB of a slice, three beyond.  Reference: float32 on the operands."""
+    import fast_route_amd as fr
+    from fast_route_amd import fused_moe
+    M, E, k, H = 64, 32, 4, 1024
+    _say(f"slots of a split 32-row down projection F={Fd}")
+    for dtype in (torch.bfloat16, torch.float16):
+        g = torch.Generator(device="cuda").manual_seed(17 + Fd)
+        x = torch.randn(M, H, generator=g, device="cuda").to(dtype)
+        w1 = (torch.randn(E, 2 * Fd, H, generator=g, device="cuda") * 0.02).to(dtype)
+        w2 = (torch.randn(E, H, Fd, generator=g, device="cuda") * 0.02).to(dtype)
+        logits = torch.randn(M, E, generator=g, device="cuda")
+        with fr.tunables(block=32, split_k=2):
+            out, names = kernels_of(lambda: fused_moe(x, w1, w2, logits, k, True))
+        down = [n for n in names if "moe_gemm" in n and not re.search(r"Li1EEEv|, 1>\(", n)]
+        assert len(down) == 1 and re.search(r"ILi32ELi128ELi128ELi1ELi4ELi16ELi2ELi%dE|<32, 128, 128, 1, 4, 16, 2, %d," % (slots, slots), down[0]), names
+        top, ids = torch.topk(logits, k, dim=1)
+        weights, ref = torch.softmax(top, dim=1), torch.zeros(M, H, device="cuda")
+        for e in range(E):
+            token, slot = (ids == e).nonzero(as_tuple=True)
+            gate, up = (x[token].float() @ w1[e].float().t()).chunk(2, dim=1)
+            ref.index_add_(0, token, ((torch.nn.functional.silu(gate) * up) @ w2[e].float().t()) * weights[token, slot][:, None])
+        _assert_close(out, ref.cpu(), dtype, f"{dtype}")
+
+
 def test_stable_and_vllm_route_layers(native):
     """Gate-matrix entry points of both reference layers."""
     from fast_route_amd.layers import stable_route, vllm_route
