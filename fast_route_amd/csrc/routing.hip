@@ -20,9 +20,13 @@ namespace {
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / kWave;
 constexpr int kSmallMaxE = 256;
-// One workgroup sorts up to this many pairs.  Sort alone, replayed from a graph: one workgroup 4000 / 6100 pairs 6.5 / 8.4 us,
-// two launches 6.4 at 6200 (64 experts), so they would win from about 4000; the line stays because callers of up to 6144
-// pairs are told that they need no workspace.
+// One workgroup sorts up to this many pairs.  As kernels two launches are the faster form from about 4000 pairs on (replayed from a graph,
+// Zipf-skewed, one workgroup / two launches, us: 8 experts 4096 pairs 6.0 / 6.4, 5120 6.9 / 6.4, 6144 7.8 / 6.5; 64 experts 3072 5.75 / 6.2, 4096 6.6 / 6.6, 5120
+// 7.7 / 6.6, 6144 8.6 / 6.6; 256 experts 2048 6.9 / 7.2, 3072 7.8 / 7.3, 6144 10.8 / 8.0).  But a program that calls moe_align_block_size by itself waits for the
+// host side of the call, to which a second launch adds 2.5 us and more: 64 experts, 4200 / 6144 pairs 8.9 and 8.9 us with one, 11.7 and 11.7 with
+// two among other calls, 21.7 and 22.5 against 23.1 and 23.2 alone; with topk_softmax in front 14.6 and 14.5 against 17.5 and 17.6.  The layers, whose
+// GEMMs hide their host side, take the same line, at a cost of up to 2 us, 3 to 5 with 256 experts (H = 2048, F = 1408, 64 experts, 4200 pairs 234.0 / 232.6,
+// 6144 240.7 / 236.7; H = 1024, F = 512, 256 experts, 4800 181.1 / 177.7; H = 1024, F = 3584, 8 experts, 5200 153.5 / 154.2, 6144 164.1 / 162.4).
 constexpr int64_t kSmallMaxN = 6144;
 // Gating and sort in ONE launch up to this many pairs (above, the gating kernel spread over the CUs plus the
 // one-workgroup sort win: 2048 pairs 31.6 against 29.5 us for a small layer, 1536 pairs on 64 experts 51.8 against 26.5)
@@ -593,16 +597,15 @@ void dispatch_route_align(const void* logits, int64_t M, int E, int topk, int re
 
 // Gating and routing arrays in one launch for small batches; false when the shape is
 // outside what one workgroup should do (the caller then runs the two stages separately).
-// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = next power of two of E (with several logits per lane,
-// gated_blocked, it has fewer; the line is where it was without); two launches cost 1 to 3 us more and spread the gating over the CUs.  A layer with H = F = 128 in us.  One logit
-// per lane, one / two launches (with the sort as it was before, a microsecond longer):
-//   16 experts, top-2   192 (3) 18.7 / 19.9, 256 (4) 25.1 / 23.6, 512 29.2 / 24.4;  8, top-2 256 (2) 23.2 / 23.7, 384 (3) 24.9 / 24.6, 512 26.2 / 24.9
-//   64, top-6 (weights not renormalised)   16 tokens (1 round) 17.8 / 19.8, 32 (2) 19.8 / 19.5, 48 (3) 21.9 / 19.8, 80 (5) 25.9 / 19.7, 168 38.4 / 20.8
-// several logits per lane (gated_blocked), sixteen calls in a graph, one logit per lane where that took one launch, else two / now / two launches now:
-//   64 experts, top-6   8 tokens 16.7 / 15.6 / 16.4, 16 17.0 / 15.9 / 16.8, 32 19.1 / 16.2 / 17.5, 64 (1 round) 18.0 / 17.8 / 18.2; 96 (2) 19.4 / 19.5 / 18.6, 160 (3) 19.6 / 21.9 / 18.5
-//   32, top-4           64 18.1 / 15.6 / 16.9, 128 (1) 17.7 / 16.8 / 17.3; 256 (2) 24.0 / 24.6 / 22.9
-// above 64 experts (two and four logits per lane), one / two launches:
-//   128, top-8   16 tokens (1 round) 22.6 / 22.3, 32 (2) 27.8 / 22.8, 127 57.5 / 24.5;  256 16 26.0 / 25.3, 64 48.9 / 29.5
+// One workgroup's gating is a chain of rounds of 16 wavefronts x 64 / G tokens, G = next power of two of E; two launches cost 1 to 3 us more and
+// spread the gating over the CUs.  A layer with H = F = 128, one / two launches, us (the sort of then, a microsecond longer in either):
+//   16 experts, top-2   192 tokens (3 rounds) 18.7 / 19.9, 256 (4) 25.1 / 23.6, 512 29.2 / 24.4;  8, top-2 256 (2) 23.2 / 23.7, 384 (3) 24.9 / 24.6, 512 26.2 / 24.9
+//   64, top-6           16 (1) 17.8 / 19.8, 32 (2) 19.8 / 19.5, 48 (3) 21.9 / 19.8, 80 (5) 25.9 / 19.7, 168 38.4 / 20.8
+//   128, top-8 (two logits per lane)   16 (1) 22.6 / 22.3, 32 (2) 27.8 / 22.8, 127 57.5 / 24.5;  256 16 26.0 / 25.3, 64 48.9 / 29.5
+// With several logits per lane (gated_blocked) there are fewer rounds, and at the line one launch is the clearly better one: 64 experts, top-6, 32 tokens
+// 16.2 / 17.5, 32, top-4, 64 tokens 15.6 / 16.9.  The line is all the same that of one logit per lane, which weights that are not renormalised and
+// unaligned logits still take: a further one would be 0.4 to 0.5 us better at 64 (128) tokens and worse from 96 (256) on (builds with the line
+// moved there: 64 experts 64 tokens 17.8 / 18.2, 96 19.5 / 18.6, 160 21.9 / 18.5; 32 experts 128 16.8 / 17.3, 256 24.6 / 22.9).
 // quant: the launch also quantises the token rows, which would be a third one; it then keeps all that one workgroup holds.
 bool route_align_fits(int64_t M, int E, int topk, bool quant) {
   if (M < 1 || M * topk > kRouteAlignMaxN || !use_small_path(M * topk, E) || M * E > 16384 || topk > E) return false;
