@@ -35,7 +35,7 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     ids_ptr, ws, ws_ptr = expert_ids.data_ptr(), None, 0
     if ws_bytes:  # small inputs sort in LDS
         # entries that may hold a block's expert: at most ceil(sorted length / block)
-        used = -(-(n + num_experts * (block_size - 1)) // block_size) if block_size > 0 else n + num_experts
+        used = int(-(-(n + num_experts * (block_size - 1)) // block_size)) if block_size > 0 else n + int(num_experts)
         if 4 * (n + num_experts - used) >= ws_bytes:
             ws_ptr = ids_ptr + 4 * used
         else:

@@ -126,3 +126,15 @@ def test_align_stays_in_the_workspace_it_asks_for(native, n, E):
     total = int(rn[0])
     assert int(out[2]) == total and (out[0].cpu().numpy() == rs).all() and (out[1].cpu().numpy()[: total // B] == re_[: total // B]).all()
     assert (ws[need // 4:] == -7).all()
+
+
+@pytest.mark.parametrize("n", [100, 20000])
+@pytest.mark.parametrize("integer", [np.int64, np.int32, torch.tensor], ids=["int64", "int32", "tensor"])
+def test_align_takes_any_integer(native, n, integer):
+    """block_size and num_experts as numpy or torch integers, with and without scratch for the sort."""
+    from fast_route_amd.ops.fused_moe import moe_align_block_size
+    _say(f"align integers n={n} {integer}")
+    ids = (torch.arange(n, dtype=torch.int32) * 7 % 64).view(n, 1).cuda()
+    for got, want in zip(moe_align_block_size(ids, integer(32), integer(64)), moe_align_block_size(ids, 32, 64)):
+        used = want.numel() if want.numel() != n + 64 else n // 32
+        assert torch.equal(got[:used], want[:used])
