@@ -25,7 +25,8 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     assert topk_ids.is_contiguous(), "topk_ids must be contiguous"
     n = topk_ids.numel()
     dev = topk_ids.device
-    int32 = topk_ids if topk_ids.dtype == torch.int32 else torch.empty((0,), dtype=torch.int32, device=dev)
+    plain = type(topk_ids) is torch.Tensor  # new_empty of a subclass is one too
+    int32 = topk_ids if plain and topk_ids.dtype == torch.int32 else torch.empty((0,), dtype=torch.int32, device=dev)
     sorted_ids = int32.new_empty(n + num_experts * (block_size - 1))
     expert_ids = int32.new_empty(n + num_experts)
     num_tokens_post_pad = int32.new_empty(1)

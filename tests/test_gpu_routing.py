@@ -138,3 +138,19 @@ def test_align_takes_any_integer(native, n, integer):
     for got, want in zip(moe_align_block_size(ids, integer(32), integer(64)), moe_align_block_size(ids, 32, 64)):
         used = want.numel() if want.numel() != n + 64 else n // 32
         assert torch.equal(got[:used], want[:used])
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_align_returns_plain_tensors(native, dtype):
+    """Ids of a torch.Tensor subclass: the routing arrays are plain tensors all the same."""
+    from fast_route_amd.ops.fused_moe import moe_align_block_size
+
+    class Ids(torch.Tensor):
+        pass
+
+    _say(f"align subclass {dtype}")
+    for n in (100, 20000):
+        ids = (torch.arange(n, dtype=dtype) * 7 % 64).view(n, 1).cuda()
+        got, want = moe_align_block_size(ids.as_subclass(Ids), 32, 64), moe_align_block_size(ids, 32, 64)
+        assert all(type(t) is torch.Tensor for t in got)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1][: n // 32], want[1][: n // 32]) and torch.equal(got[2], want[2])
