@@ -556,7 +556,10 @@ int run(const void* ids_v, int64_t n, int E, int B, int32_t* sorted, int32_t* ex
 
 // Rows that 4-element vector loads can read, 17 to 64 experts: a few lanes per token in the one-workgroup form.  Renormalised weights
 // only: their sum is taken in the order of rank, as gate_token takes it, so that a weight has the same bits from either.
-// (Above 64 experts the two forms order NaN differently.)
+// (Above 64 experts the two forms order NaN differently.)  Any topk: from 24 tokens on the several logits win at each, with fewer tokens the two are within
+// 0.3 us.  Layer with H = F = 128, one / several, us: 64 experts, 48 tokens, top-1 16.4 / 15.0, top-2 16.8 / 14.9, 32 tokens, top-8 19.2 / 16.9, top-16 23.9 / 20.2, top-32
+// 34.8 / 27.7, 16 tokens, top-64 39.4 / 39.6; 32 experts, 64 tokens, top-8 20.25 / 17.7, top-16 31.2 / 27.0, 32, top-32 33.1 / 31.9; fp8 layers (F = 256), 64 experts, 64 tokens,
+// top-16 39.1 / 29.3, 170, top-6 42.2 / 29.4, 250, top-1 32.05 / 24.2, 32 experts, 250, top-4 33.0 / 25.0.
 bool gated_blocked(const void* logits, size_t elem, int E, int topk, int renorm) {
   return renorm && E > 16 && E <= 64 && E % 4 == 0 && reinterpret_cast<uintptr_t>(logits) % (4 * elem) == 0 && topk <= kBlockedSlots * (E <= 32 ? 8 : 16);
 }
